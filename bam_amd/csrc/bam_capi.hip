@@ -111,23 +111,29 @@ __global__ void k_array_read_n_whole(array_d_t<uint64_t>* dr, uint64_t n_reqs, c
 }
 
 /*
- * A launch of scattered requests in two launches (arrays of one range).  The first, this kernel: thread t takes requests
- * t, t + threads, ... (N at a time for `rounds` rounds, `threads` a multiple of 64) and reads those whose page is resident, without a reference
- * (array_d_t::seq_read_n_resident); bit t of missed[] says whether request t is left for the second launch
- * (k_array_read_deferred).  No call, no atomic but the checksum's and the counters', no stack: a kernel that can miss
+ * A launch of scattered requests in several launches (arrays of one range).  The first, this kernel: a wave takes
+ * 64 * N * rounds consecutive requests, N per lane at a time, and reads those whose page is resident, without a reference
+ * (array_d_t::seq_read_n_resident); bit t of missed[] says whether request t is left for the launches that follow, and
+ * wanted[] (may be NULL) gets a byte set for the page it needs.  GATHER: the elements go to out[], otherwise they are summed.
+ * No call, no atomic but the checksum's and the counters', no stack: a kernel that can miss
  * carries the registers of the miss path (four waves per SIMD) and its frame in scratch memory through every read.  The
- * last workgroup folds the checksum of what was read; the second launch adds what it reads.
+ * last workgroup folds the checksum of what was read; the later launches add what they read.
+ * A request outside the range reads as 0 and is not counted, as array_d_t::operator[] has it.
+ * Bound by the requests the vector L1s keep in flight (three per read: descriptor, element, descriptor) and by the 128-byte
+ * line of HBM behind each element.  2^26 reads of a resident 1 GiB: 1.52 ms summed, 1.83 ms handed out (2.03 as one launch with
+ * one read per thread); N = 4 instead of 8: 1.91.
  */
-template <int N>
-__global__ __launch_bounds__(256) void k_array_read_n(array_d_t<uint64_t>* dr, uint64_t n_reqs, const uint64_t* __restrict__ assignment, uint64_t threads, uint32_t rounds,
-                                                      unsigned long long* partials, uint64_t* missed, unsigned long long* sum, uint32_t* finished, uint32_t call)
+template <int N, bool GATHER>
+__global__ __launch_bounds__(256) void k_array_read_n(array_d_t<uint64_t>* dr, uint64_t n_reqs, const uint64_t* __restrict__ assignment, uint32_t rounds,
+                                                      unsigned long long* partials, uint64_t* missed, uint64_t n_words, uint8_t* wanted, unsigned long long* sum, uint64_t* out_list, uint32_t* finished, uint32_t call)
 {
-    const uint64_t tid = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const uint32_t lane = bam::lane();
+    /* the wave's requests: 64 * N * rounds consecutive ones, lane l taking l, l + 64, ..., N at a time: what a wave, a workgroup
+     * and the launch do once (the range's descriptor, the counters, the checksum) is shared by more reads the more rounds there are */
+    const uint64_t wave = bam::first(((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) / BAM_WAVE_SIZE), w0 = wave * N * rounds, t0 = w0 * BAM_WAVE_SIZE + lane;
     bam::range_view<uint64_t> view;
     view.load(dr->d_ranges);
     uint64_t v = 0, any_left = 0;
-    /* thread t takes requests t + k * threads, k = 0 .. N * rounds - 1, N at a time: what a wave, a workgroup and the launch
-     * do once (the range's descriptor, the counters, the checksum) is shared by more reads the more rounds there are */
     /* the indices of a round are asked for a round ahead: a read is four trips to memory one after the other (index,
      * descriptor, element, descriptor again), and this takes the first out of the chain (44 against 41 thousand million reads
      * a second with eight reads per lane).  Every lane loads (one without a request the first index): N loads side by side,
@@ -135,8 +141,8 @@ __global__ __launch_bounds__(256) void k_array_read_n(array_d_t<uint64_t>* dr, u
     size_t ahead[N];
 #pragma unroll
     for (int j = 0; j < N; j++) {
-        const uint64_t t = tid + (uint64_t)j * threads;
-        ahead[j] = __builtin_nontemporal_load(assignment + (tid < threads && t < n_reqs ? t : 0));
+        const uint64_t t = t0 + (uint32_t)j * BAM_WAVE_SIZE;
+        ahead[j] = __builtin_nontemporal_load(assignment + (t < n_reqs ? t : 0));
     }
     for (uint32_t r = 0; r < rounds; r++) {
         size_t idx[N];
@@ -144,15 +150,14 @@ __global__ __launch_bounds__(256) void k_array_read_n(array_d_t<uint64_t>* dr, u
         uint64_t out[N];
 #pragma unroll
         for (int j = 0; j < N; j++) {
-            const uint64_t t = tid + (uint64_t)(r * N + j) * threads;
-            want[j] = tid < threads && t < n_reqs;
+            want[j] = t0 + (r * N + j) * BAM_WAVE_SIZE < n_reqs;
             idx[j] = ahead[j];
         }
         if (r + 1 < rounds) {
 #pragma unroll
             for (int j = 0; j < N; j++) {
-                const uint64_t t = tid + (uint64_t)((r + 1) * N + j) * threads;
-                ahead[j] = __builtin_nontemporal_load(assignment + (tid < threads && t < n_reqs ? t : 0));
+                const uint64_t t = t0 + ((r + 1) * N + j) * BAM_WAVE_SIZE;
+                ahead[j] = __builtin_nontemporal_load(assignment + (t < n_reqs ? t : 0));
             }
         }
         dr->template seq_read_n_resident<N, true>(idx, want, out, got, view);
@@ -160,70 +165,161 @@ __global__ __launch_bounds__(256) void k_array_read_n(array_d_t<uint64_t>* dr, u
         uint64_t mine = 0;
 #pragma unroll
         for (int j = 0; j < N; j++) {
-            v += got[j] ? out[j] : 0;
-            const uint64_t m = bam::ballot(want[j] & !got[j]);
-            if (bam::lane() == (uint32_t)j) mine = m;
+            const bool left = want[j] & !got[j] & (idx[j] - view.index_start < view.index_end - view.index_start);
+            if constexpr (GATHER) { if (want[j] & !left) __builtin_nontemporal_store(got[j] ? out[j] : 0, out_list + t0 + (r * N + j) * BAM_WAVE_SIZE); }
+            else v += got[j] ? out[j] : 0;
+            const uint64_t m = bam::ballot(left);
+            if (lane == (uint32_t)j) mine = m;
             any_left |= m;
+            if (m && wanted && left) wanted[view.page_of(idx[j])] = 1;
         }
-        if (bam::lane() < (uint32_t)N && tid - bam::lane() < threads)
-            missed[(tid - bam::lane() + (uint64_t)(r * N + bam::lane()) * threads) / BAM_WAVE_SIZE] = mine;
+        if (lane < (uint32_t)N && w0 + r * N + lane < n_words) missed[w0 + r * N + lane] = mine;
     }
     view.flush_stats();
     if (any_left) note_work_left(finished, call);
-    block_accumulate(partials, v);
-    fold_by_last_block(partials, sum, finished);
+    if constexpr (!GATHER) {
+        block_accumulate(partials, v);
+        fold_by_last_block(partials, sum, finished);
+    }
 }
 
 /*
- * The second launch: the requests the first one left, one per lane through array_d_t::operator[], which has the miss
- * path.  A wave takes `words` words of missed[] at a time (1 to 16, a power of two: lane l looks after `words` bits),
- * lines the requests noted there up in LDS and reads them 64 at a time: whatever the share of misses, the batches of
- * commands that go to the store are whole waves' worth.  The last workgroup to finish adds the checksum of these reads
- * to the first launch's.  When the first launch left nothing (it says so in a word of its own) this one ends at once.
+ * The pages of [first, last) that the first launch left somebody waiting for, asked for in batches of 64 commands, each page
+ * once.  With many requests per page and a cache smaller than the array, request by request is the wrong order: a page comes
+ * in for one request and has left again before the next one for it is looked at (2^22 random requests over 2^19 pages
+ * behind a cache of half of them: 2.05 million reads from the store where 262144 pages are missing), and the batches of a
+ * wave thin out as the pages come in.  Here a wave collects the numbers of wanted pages in LDS until it has 64, so every
+ * batch but its last is a whole one.  The bytes are cleared as they are taken up.  wanted[] is padded to whole words of
+ * eight and `first` is a multiple of 512.
+ */
+#define BAM_FETCH_PAGE_WAVES 512       /* 32768 pages on their way: 20.1 ms for 2^22 requests and 262144 pages with 512 to 2048 waves, 20.5 with 256, 20.7 with 128 */
+#define BAM_FETCH_FLAGS (8u * BAM_WAVE_SIZE)       /* page bytes a wave looks at per turn: a word per lane */
+__global__ __launch_bounds__(256) void k_fetch_wanted(array_d_t<uint64_t>* dr, uint64_t* wanted8, uint64_t first, uint64_t last, const uint32_t* finished, uint32_t call)
+{
+    __shared__ uint32_t list[256 / BAM_WAVE_SIZE][BAM_FETCH_FLAGS + BAM_WAVE_SIZE];
+    if (__hip_atomic_load(finished + BAM_LEFT_WORD, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != call) return;      /* nothing was left */
+    const uint32_t lane = bam::lane();
+    uint32_t* const mine = list[threadIdx.x / BAM_WAVE_SIZE];
+    const uint64_t gwave = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) / BAM_WAVE_SIZE, n_gwaves = (uint64_t)gridDim.x * blockDim.x / BAM_WAVE_SIZE;
+    bam::range_view<uint64_t> view;
+    view.load(dr->d_ranges);
+    view.place = BAM_PLACE_PULLED;
+    auto touch = [](uint32_t) { return true; };
+    uint32_t have = 0;
+    for (uint64_t c = first + gwave * BAM_FETCH_FLAGS;; c += n_gwaves * BAM_FETCH_FLAGS) {
+        const bool more = c < last;
+        if (more) {
+            const uint64_t p = c + lane * 8u;
+            uint64_t f = p < last ? wanted8[p / 8] : 0ull;
+            if (f) wanted8[p / 8] = 0;
+            const uint32_t n = bam::popc(f);
+            uint32_t incl = n;
+#pragma unroll
+            for (uint32_t o = 1; o < BAM_WAVE_SIZE; o <<= 1) {
+                const uint32_t u = bam::shfl(incl, lane >= o ? lane - o : lane);
+                if (lane >= o) incl += u;
+            }
+            uint32_t at = have + incl - n;
+            for (; f; f &= f - 1) mine[at++] = (uint32_t)(p - first) + (uint32_t)__builtin_ctzll(f) / 8u;
+            have += bam::bcast(incl, BAM_WAVE_SIZE - 1);
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        }
+        while (have >= BAM_WAVE_SIZE || (!more && have)) {
+            const uint32_t n = have < BAM_WAVE_SIZE ? have : BAM_WAVE_SIZE;
+            have -= n;
+            const uint64_t page = first + mine[have + (lane < n ? lane : 0)];
+            const bool take = lane < n && page_absent(view, page);
+            if (bam::ballot(take)) view.acquire_helped(page, take, false, touch, touch);
+        }
+        if (!more) break;
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    }
+    view.n_access = view.n_hit = 0;
+}
+
+/*
+ * A later launch: the requests the first one left whose page lies in [page_first, page_last), with the miss path for those
+ * whose page is not there.  A wave takes `words` words of missed[] at a time (1 to 16: a request per lane and word), lines
+ * the requests up in LDS, index and all, and reads them four per lane side by side as far as they are resident
+ * (k_fetch_wanted has just brought their pages in, where it ran), what is not one after the other, 64 to a wave: whatever
+ * the share of misses, the batches of commands that go to the store are whole waves' worth.  The bits of what was read are
+ * cleared.  All of them count as misses: the first launch looked and did not find their page.  The last workgroup to finish
+ * adds the checksum of these reads to the first launch's.  When the first launch left nothing (it says so in a word of its
+ * own) this one ends at once.
  */
 #define BAM_DEFER_MAX_WORDS 16u
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_array_read_deferred(array_d_t<uint64_t>* dr, uint64_t n_reqs, const uint64_t* __restrict__ assignment, const uint64_t* missed,
-                                                             uint64_t n_words, uint32_t words, unsigned long long* partials, unsigned long long* sum, uint32_t* finished, uint32_t call)
+template <bool GATHER>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_array_read_deferred(array_d_t<uint64_t>* dr, uint64_t n_reqs, const uint64_t* __restrict__ assignment, uint64_t* missed,
+                                                             uint64_t n_words, uint32_t words, uint64_t page_first, uint64_t page_last, unsigned long long* partials, unsigned long long* sum,
+                                                             uint64_t* out_list, uint32_t* finished, uint32_t call)
 {
-    __shared__ uint16_t ids[256 / BAM_WAVE_SIZE][BAM_DEFER_MAX_WORDS * BAM_WAVE_SIZE];
+    __shared__ uint64_t list[256 / BAM_WAVE_SIZE][BAM_DEFER_MAX_WORDS * BAM_WAVE_SIZE];      /* index of the request's element */
+    __shared__ uint16_t ids[256 / BAM_WAVE_SIZE][BAM_DEFER_MAX_WORDS * BAM_WAVE_SIZE];       /* which request of the chunk it is */
     if (__hip_atomic_load(finished + BAM_LEFT_WORD, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != call) return;      /* nothing was left */
     const uint32_t lane = bam::lane(), w_in_block = threadIdx.x / BAM_WAVE_SIZE;
     const uint64_t gwave = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) / BAM_WAVE_SIZE, n_gwaves = (uint64_t)gridDim.x * blockDim.x / BAM_WAVE_SIZE;
     const uint64_t n_chunks = (n_words + words - 1) / words;
+    bam::range_view<uint64_t> view;
+    view.load(dr->d_ranges);
     uint64_t v = 0;
     bool any = false;
     for (uint64_t c = gwave; c < n_chunks; c += n_gwaves) {
-        /* lane l: bits [l * words, (l + 1) * words) of the chunk's 64 * words */
-        const uint32_t bit0 = lane * words;
-        const uint64_t word = c * words + bit0 / 64;
-        const uint32_t seg = word < n_words ? (uint32_t)((missed[word] >> (bit0 % 64)) & ((1u << words) - 1u)) : 0u;
-        uint32_t incl = bam::popc((uint64_t)seg);
-        const uint32_t mine = incl;
-#pragma unroll
-        for (uint32_t o = 1; o < BAM_WAVE_SIZE; o <<= 1) {
-            const uint32_t u = bam::shfl(incl, lane >= o ? lane - o : lane);
-            if (lane >= o) incl += u;
+        const uint64_t w0 = c * words;
+        uint64_t bits = lane < words && w0 + lane < n_words ? missed[w0 + lane] : 0ull;      /* lane w looks after word w */
+        if (!bam::ballot(bits != 0)) continue;
+        uint32_t total = 0;
+        uint64_t rest = bits;
+        for (uint64_t m = bam::ballot(bits != 0); m; m &= m - 1) {
+            const uint32_t w = bam::first_lane(m);
+            const uint64_t word = bam::bcast(bits, w), t = (w0 + w) * BAM_WAVE_SIZE + lane;
+            bool mine = ((word >> lane) & 1) != 0;
+            const uint64_t i = mine ? assignment[t] : 0;
+            const uint64_t page = mine ? view.page_of(i) : 0;
+            mine = mine && page >= page_first && page < page_last;
+            const uint64_t take = bam::ballot(mine);
+            if (mine) { const uint32_t at = total + bam::popc(take & bam::lanes_below(lane)); list[w_in_block][at] = i; ids[w_in_block][at] = (uint16_t)(w * BAM_WAVE_SIZE + lane); }
+            total += bam::popc(take);
+            if (lane == w) rest &= ~take;
         }
-        const uint32_t total = bam::bcast(incl, BAM_WAVE_SIZE - 1);
         if (!total) continue;
         any = true;
-        uint32_t at = incl - mine;
-        for (uint32_t m = seg; m; m &= m - 1) ids[w_in_block][at++] = (uint16_t)(bit0 + (uint32_t)__builtin_ctz(m));
+        if (rest != bits) missed[w0 + lane] = rest;
         /* written and read by the lanes of one wave, which runs its LDS operations in order */
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        for (uint32_t b = 0; b < total; b += BAM_WAVE_SIZE) {
-            if (b + lane < total) {
-                const uint64_t t = c * words * BAM_WAVE_SIZE + ids[w_in_block][b + lane];
-                if (t < n_reqs) v += (*dr)[assignment[t]];
+        for (uint32_t b = 0; b < total; b += 4 * BAM_WAVE_SIZE) {
+            size_t idx[4];
+            bool want[4], got[4];
+            uint64_t x[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const uint32_t k = b + j * BAM_WAVE_SIZE + lane;
+                want[j] = k < total;
+                idx[j] = list[w_in_block][want[j] ? k : 0];
+            }
+            dr->template seq_read_n_resident<4, true>(idx, want, x, got, view);
+#pragma unroll 1
+            for (int j = 0; j < 4; j++)
+                if (want[j] && !got[j]) x[j] = dr->seq_read_call(idx[j]);
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                if constexpr (GATHER) { if (want[j]) out_list[w0 * BAM_WAVE_SIZE + ids[w_in_block][b + j * BAM_WAVE_SIZE + lane]] = x[j]; }
+                else v += want[j] ? x[j] : 0;
             }
         }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
     }
-    if (bam::ballot(any)) block_accumulate(partials, v);
-    fold_by_last_block(partials, sum, finished);
+    view.n_hit = 0;
+    view.flush_stats();
+    if constexpr (!GATHER) {
+        if (bam::ballot(any)) block_accumulate(partials, v);
+        fold_by_last_block(partials, sum, finished);
+    }
 }
 
 /* thread t hands out the element it read instead of adding it to a sum */
@@ -380,7 +476,7 @@ __device__ __forceinline__ void stream_fetch_role(array_d_t<uint64_t>* dr, const
     if (dr->n_ranges != 1) return;
     bam::range_view<uint64_t> view;
     view.load(dr->d_ranges);
-    view.read_ahead = true;
+    view.place = BAM_PLACE_AHEAD;
     const uint64_t epp = dr->d_ranges->n_elems_per_page;
     const uint64_t fwave = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) / BAM_WAVE_SIZE, n_fwaves = (uint64_t)fp.blocks * blockDim.x / BAM_WAVE_SIZE;
     const uint64_t total = n_waves * ppw, n_batches = (total + BAM_WAVE_SIZE - 1) / BAM_WAVE_SIZE;
@@ -1318,6 +1414,78 @@ static bool two_launches_ok(bam_array_t* a)
     return a->a->adt.n_ranges == 1 && a->a->h_ranges[0].cache.fast_reads != 0;
 }
 
+extern "C++" {
+namespace {
+/* whether a gather is better off as several launches than as one that can miss; they keep notes between launches, which a
+ * stream under capture must not (the graph may be replayed beside other calls) */
+bool scattered_launches_pay(bam_array_t* a, uint64_t n_reqs, hipStream_t st)
+{
+    if (!two_launches_ok(a)) return false;
+    const range_d_t<uint64_t>& range = a->a->h_ranges[0];
+    if (n_reqs < (range.page_count > range.cache.n_pages ? 1ull << 14 : 1ull << 20)) return false;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &cap) != hipSuccess) { (void)hipGetLastError(); return false; }
+    return cap == hipStreamCaptureStatusNone;
+}
+/*
+ * Scattered reads in several launches: what is resident (k_array_read_n), then the rest.  Where the array is larger than
+ * its cache and there are enough requests for them to meet on pages, the rest goes page by page: the pages somebody waits
+ * for are fetched, each once, in whole batches (k_fetch_wanted), and then the requests for them are read
+ * (k_array_read_deferred), a stretch of the range at a time so that what is fetched is still there when it is read.
+ */
+template <bool GATHER>
+void scattered_reads(bam_array_t* a, uint64_t n_reqs, const uint64_t* d_assignment, uint32_t N, unsigned long long* sum, uint64_t* d_out, hipStream_t st)
+{
+    const range_d_t<uint64_t>& range = a->a->h_ranges[0];
+    const uint64_t cache_pages = range.cache.n_pages, pages = range.page_count;
+    array_d_t<uint64_t>* d = a->a->d_array_ptr;
+    /* rounds of N reads per thread: as many as leave sixteen thousand workgroups, several times what the device holds at a time
+     * (a launch of about as many workgroups as the device holds ends with most of the device idle) */
+    uint32_t rounds = 1;
+    while (rounds < 32 && n_reqs / ((uint64_t)N * rounds * 2 * 256) >= 16384) rounds *= 2;
+    const uint64_t per_thread = (uint64_t)N * rounds;
+    const uint64_t n_words = (n_reqs + BAM_WAVE_SIZE - 1) / BAM_WAVE_SIZE, n_waves = (n_words + per_thread - 1) / per_thread;
+    /* page by page: with a request for every other page or more (below that nearly every request has its page to itself, and
+     * the requests by themselves make whole batches), and a cache that takes 64 pages from each of 32 waves and has room
+     * for as many again */
+    const bool by_page = pages > cache_pages && n_reqs >= pages / 2 && cache_pages >= 4096;
+    const uint64_t wanted_bytes = by_page ? (pages + 511) / 512 * 512 : 0;
+    std::lock_guard<std::mutex> guard(a->scatter_mu);
+    bam_array::scatter_set* set = a->scatter_for(st, n_words * sizeof(uint64_t), wanted_bytes);
+    uint64_t* missed = (uint64_t*)set->notes.get();
+    uint8_t* wanted = by_page ? (uint8_t*)set->wanted.get() : nullptr;
+    unsigned long long* part = set->partials();
+    uint32_t* fin = set->finished();
+    const uint32_t call = set->next_call();
+    const dim3 grid(blocks_for(n_waves * BAM_WAVE_SIZE, 256)), block(256);
+    switch (N) {
+    case 1: hipLaunchKernelGGL((k_array_read_n<1, GATHER>), grid, block, 0, st, d, n_reqs, d_assignment, rounds, part, missed, n_words, wanted, sum, d_out, fin, call); break;
+    case 2: hipLaunchKernelGGL((k_array_read_n<2, GATHER>), grid, block, 0, st, d, n_reqs, d_assignment, rounds, part, missed, n_words, wanted, sum, d_out, fin, call); break;
+    case 4: hipLaunchKernelGGL((k_array_read_n<4, GATHER>), grid, block, 0, st, d, n_reqs, d_assignment, rounds, part, missed, n_words, wanted, sum, d_out, fin, call); break;
+    default: hipLaunchKernelGGL((k_array_read_n<8, GATHER>), grid, block, 0, st, d, n_reqs, d_assignment, rounds, part, missed, n_words, wanted, sum, d_out, fin, call); break;
+    }
+    /* the later launches: as many words per wave as leave some eight thousand waves' worth of chunks */
+    uint32_t words = 1;
+    while (words < BAM_DEFER_MAX_WORDS && n_words / (words * 2) >= 8192) words *= 2;
+    const uint64_t n_chunks = (n_words + words - 1) / words;
+    const uint64_t waves = n_chunks < 16384 ? n_chunks : 16384;
+    const dim3 grid_d(blocks_for(waves * BAM_WAVE_SIZE, 256));
+    /* stretches of which at most three quarters of the cache can be wanted (all of it is when the requests are spread evenly) */
+    const uint64_t room = cache_pages - cache_pages / 4, most = pages < n_reqs ? pages : n_reqs;
+    const uint64_t stretches = by_page ? (most + room - 1) / room : 1;
+    const uint64_t step = ((pages + stretches - 1) / stretches + 511) / 512 * 512;
+    const uint64_t f_waves = std::min<uint64_t>(BAM_FETCH_PAGE_WAVES, cache_pages / (2 * BAM_WAVE_SIZE));
+    for (uint64_t p = 0; p < pages; p += step) {
+        const uint64_t q = p + step < pages ? p + step : pages;
+        if (by_page)
+            hipLaunchKernelGGL(k_fetch_wanted, dim3(blocks_for(f_waves * BAM_WAVE_SIZE, 256)), block, 0, st, d, (uint64_t*)wanted, p, q, fin, call);
+        hipLaunchKernelGGL(k_array_read_deferred<GATHER>, grid_d, block, 0, st, d, n_reqs, d_assignment, missed, n_words, words, p, q, part, sum, d_out, fin, call);
+    }
+    hip_err_chk(hipGetLastError());
+}
+} // namespace
+} // extern "C++"
+
 int bam_array_read_shaped(bam_array_t* a, uint64_t n_reqs, const uint64_t* d_assignment, int shape, uint32_t reads_per_lane, uint32_t block_size,
                           uint64_t* d_sum, void* stream)
 {
@@ -1339,34 +1507,8 @@ int bam_array_read_shaped(bam_array_t* a, uint64_t n_reqs, const uint64_t* d_ass
         const uint64_t threads = (n_reqs + BAM_READS_PER_LANE - 1) / BAM_READS_PER_LANE;
         hipLaunchKernelGGL(k_array_read_n_whole, dim3(blocks_for(threads, block_size)), dim3(block_size), 0, st, d, n_reqs, d_assignment, threads, part);
         hipLaunchKernelGGL(k_fold_partials, dim3(1), dim3(1024), 0, st, part, (unsigned long long*)d_sum);
-    } else {
-        const uint32_t N = reads_per_lane;
-        /* rounds of N reads per thread: as many as leave sixteen thousand workgroups, several times what the device holds at a time
-         * (a launch of about as many workgroups as the device holds ends with most of the device idle) */
-        uint32_t rounds = 1;
-        while (rounds < 32 && n_reqs / ((uint64_t)N * rounds * 2 * 256) >= 16384) rounds *= 2;
-        const uint64_t per_thread = (uint64_t)N * rounds;
-        const uint64_t threads = ((n_reqs + per_thread - 1) / per_thread + BAM_WAVE_SIZE - 1) / BAM_WAVE_SIZE * BAM_WAVE_SIZE;
-        const uint64_t n_words = threads / BAM_WAVE_SIZE * per_thread;
-        uint64_t* missed = (uint64_t*)a->notes_for(n_words * sizeof(uint64_t));
-        const dim3 grid(blocks_for(threads, 256)), block(256);
-        unsigned long long* sum = (unsigned long long*)d_sum;
-        uint32_t* fin = (uint32_t*)a->finished.get();
-        const uint32_t call = a->next_call();
-        switch (N) {
-        case 1: hipLaunchKernelGGL(k_array_read_n<1>, grid, block, 0, st, d, n_reqs, d_assignment, threads, rounds, part, missed, sum, fin, call); break;
-        case 2: hipLaunchKernelGGL(k_array_read_n<2>, grid, block, 0, st, d, n_reqs, d_assignment, threads, rounds, part, missed, sum, fin, call); break;
-        case 4: hipLaunchKernelGGL(k_array_read_n<4>, grid, block, 0, st, d, n_reqs, d_assignment, threads, rounds, part, missed, sum, fin, call); break;
-        default: hipLaunchKernelGGL(k_array_read_n<8>, grid, block, 0, st, d, n_reqs, d_assignment, threads, rounds, part, missed, sum, fin, call); break;
-        }
-        /* the second launch: as many words per wave as leave some eight thousand waves' worth of chunks */
-        uint32_t words = 1;
-        while (words < BAM_DEFER_MAX_WORDS && n_words / (words * 2) >= 8192) words *= 2;
-        const uint64_t n_chunks = (n_words + words - 1) / words;
-        const uint64_t waves = n_chunks < 16384 ? n_chunks : 16384;
-        hipLaunchKernelGGL(k_array_read_deferred, dim3(blocks_for(waves * BAM_WAVE_SIZE, 256)), dim3(256), 0, st, d, n_reqs, d_assignment, missed, n_words, words,
-                           part, sum, fin, call);
-    }
+    } else
+        scattered_reads<false>(a, n_reqs, d_assignment, reads_per_lane, (unsigned long long*)d_sum, nullptr, st);
     hip_err_chk(hipGetLastError());
     BAM_API_END
 }
@@ -1402,6 +1544,10 @@ int bam_array_gather(bam_array_t* a, uint64_t n_reqs, const uint64_t* d_assignme
     if (!block_size || block_size % BAM_WAVE_SIZE || block_size > 1024) return fail(EINVAL, "bam_array_gather: block size must be a multiple of 64, at most 1024");
     if (!n_reqs) return 0;
     BAM_API_BEGIN
+    if (d_assignment && scattered_launches_pay(a, n_reqs, (hipStream_t)stream)) {
+        scattered_reads<true>(a, n_reqs, d_assignment, 8, nullptr, d_out, (hipStream_t)stream);
+        return 0;
+    }
     hipLaunchKernelGGL(k_array_gather, dim3(blocks_for(n_reqs, block_size)), dim3(block_size), 0, (hipStream_t)stream,
                        a->a->d_array_ptr, n_reqs, d_assignment, stride, d_out);
     hip_err_chk(hipGetLastError());

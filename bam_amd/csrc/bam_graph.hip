@@ -36,7 +36,7 @@ struct list_read_ahead {
         view.load(da->d_ranges);
         /* what is touched ahead may be placed directly up to the higher of the cache's two bounds: measured on the per-vertex
          * BFS (RMAT-24) 4.55 GTEPS with at most 1024 directly placed commands in flight, 4.7 with 4096 to 8192, 4.46 with 16384 */
-        view.read_ahead = true;
+        view.place = BAM_PLACE_AHEAD;
         const uint64_t r = da->d_ranges[0].cache.n_pages >> 6;
         reach = r > BAM_WAVE_SIZE ? BAM_WAVE_SIZE : (uint32_t)r;
     }

@@ -103,8 +103,8 @@ int bam_array_stats(bam_array_t* a, uint64_t* out, int reset);
  * One thread per request: thread t reads element d_assignment[t] (or t * stride when d_assignment is NULL)
  * reqs_per_thread times through array_d_t::operator[] and the launch adds every value read into *d_sum
  * (mod 2^64).  The reference discards the values; the checksum is what makes the result checkable.  A launch of 2^16 or
- * more scattered requests read once each runs with a quarter of the threads, thread t taking requests t, t + n/4, t + 2n/4
- * and t + 3n/4 side by side (array_d_t::seq_read_n): the same reads, sum and counters, four of them in flight per lane. */
+ * more scattered requests read once each takes another shape (bam_array_read_shaped): the same reads, sum and counters of
+ * accesses, several of them in flight per lane. */
 int bam_array_read(bam_array_t* a, uint64_t n_reqs, const uint64_t* d_assignment, uint64_t stride, uint64_t reqs_per_thread,
                    uint32_t block_size, uint64_t* d_sum, void* stream);
 /* The same scattered requests (thread t reads element d_assignment[t] once; sum into *d_sum) with the launch shape named,
@@ -113,8 +113,12 @@ int bam_array_read(bam_array_t* a, uint64_t n_reqs, const uint64_t* d_assignment
  *   BAM_READ_FOUR_PER_THREAD  a quarter of the threads, four requests per thread side by side, one launch
  *   BAM_READ_TWO_LAUNCHES     a first launch reads what is resident, reads_per_lane (1, 2, 4, 8) requests per thread, with a
  *                             kernel that cannot miss (no call, no stack, a fraction of the registers) and notes the rest;
- *                             a second launch reads the rest, one request per lane and 64 per wave whatever the share of
- *                             misses was.  Arrays of one range only (EINVAL otherwise).
+ *                             a second launch reads the rest, 64 requests to a wave whatever the share of misses was.
+ *                             Where the array is larger than its cache and there is a request for every other page or more,
+ *                             the rest goes page by page: launches that fetch the pages somebody waits for, each once, in
+ *                             batches of 64 commands, alternate with launches that read the requests for them.  Arrays of
+ *                             one range only (EINVAL otherwise).  A request that did not find its page in the first launch
+ *                             counts as a miss.
  * bam_array_read picks BAM_READ_TWO_LAUNCHES with eight reads per lane for launches of 2^16 requests and more where the array
  * allows it (BAM_READ_FOUR_PER_THREAD where not) and BAM_READ_ONE_PER_THREAD below that. */
 #define BAM_READ_ONE_PER_THREAD  1
@@ -123,7 +127,9 @@ int bam_array_read(bam_array_t* a, uint64_t n_reqs, const uint64_t* d_assignment
 int bam_array_read_shaped(bam_array_t* a, uint64_t n_reqs, const uint64_t* d_assignment, int shape, uint32_t reads_per_lane, uint32_t block_size,
                           uint64_t* d_sum, void* stream);
 /* the same requests with the values handed out: d_out[t] = element d_assignment[t] (or t * stride); what a kernel of the
- * reference's benchmark would hold in its register after array_d_t::operator[] (benchmarks/array/main.cu:57) */
+ * reference's benchmark would hold in its register after array_d_t::operator[] (benchmarks/array/main.cu:57).  Launches of
+ * 2^20 requests and more, 2^14 where the array is larger than its cache, run as BAM_READ_TWO_LAUNCHES does (arrays of one
+ * range, streams that are not being captured) */
 int bam_array_gather(bam_array_t* a, uint64_t n_reqs, const uint64_t* d_assignment, uint64_t stride, uint32_t block_size, uint64_t* d_out, void* stream);
 /* The read pattern of bam_array_read (one thread per request, element d_assignment[t] or t * span) through the other
  * access routes of array_d_t (include/page_cache.h:1240-1716, 414-485): api 1 get_raw/release_raw, 2 get_page_gid +

@@ -80,6 +80,17 @@ enum data_dist_t { REPLICATE = 0, STRIPE = 1 };
 #define BAM_DIRECT_MIN_BATCH 24u
 #endif
 
+/*
+ * Where the payload of a read batch of the miss path goes, as the caller sees it.  NORMAL: somebody waits for it, placed by
+ * load up to direct_limit; AHEAD: the wave fetches for others that compute meanwhile, up to direct_limit_ahead; PULLED:
+ * the wave has nothing else to do and nobody computes beside it, so it pulls all of it from the staging pages itself
+ * (waves that only fetch, alone on the device: 262144 pages in 19.9 ms = 13.2 M pages/s all pulled; 20.7 ms with at most
+ * 1024 commands placed by the controller, 22.9 with 8192: what the controller pushes takes it ten times as long)
+ */
+#define BAM_PLACE_NORMAL 0u
+#define BAM_PLACE_AHEAD  1u
+#define BAM_PLACE_PULLED 2u
+
 #define BAM_TOKEN_SLOTS 4096u
 #define BAM_STAT_SHARDS 4096
 
@@ -126,7 +137,7 @@ struct page_cache_d_t {
     uint32_t* page_ticket;
     uint64_t* prp1;                  /* [n_pages] bus address of each slot (direct transfers) */
     uint32_t direct_share;           /* with staging available: of every 8 read batches of the cache's miss path, this many go direct all the same */
-    uint32_t direct_limit_ahead;     /* the same bound for batches of waves that only fetch ahead of others (range_view::read_ahead): nobody copies for them */
+    uint32_t direct_limit_ahead;     /* the same bound for batches of waves that only fetch ahead of others (range_view::place): nobody copies for them */
     uint32_t direct_limit;           /* not 0: instead of that share, a read batch of the miss path goes direct while fewer than this many directly placed commands are in flight on the whole cache (*direct_gauge) */
     uint32_t* direct_gauge;
     uint32_t direct_share_raw;       /* the same for reads through read_data / access_data (raw block I/O into slots the caller names) */
@@ -411,7 +422,7 @@ inline __device__ void access_data(page_cache_d_t* pc, QueuePair* qp, const uint
  * with several groups each one runs its whole transfer before the next starts, and `held` comes back false.
  */
 inline __device__ void read_begin(page_cache_d_t* pc, QueuePair* qp, const uint64_t starting_lba, const uint64_t n_blocks, const unsigned long long pc_entry,
-                                  uint32_t& cid, uint8_t*& stage, bool& held, bool& ok, const bool ahead = false)
+                                  uint32_t& cid, uint8_t*& stage, bool& held, bool& ok, const uint32_t place = BAM_PLACE_NORMAL)
 {
     const uint64_t all = bam::active_mask();
     bool one_group = bam::ballot(qp == (QueuePair*)bam::first((uint64_t)qp) && pc == (page_cache_d_t*)bam::first((uint64_t)pc)) == all;
@@ -424,7 +435,8 @@ inline __device__ void read_begin(page_cache_d_t* pc, QueuePair* qp, const uint6
     if (!one_group) {
         bam::for_each_group((uint64_t)qp, (uint64_t)pc, [&](uint64_t q, uint64_t c) {
             bam::for_each_chunk(((QueuePair*)q)->sq.qs >> 1, [&]() {
-                ok = bam::io_group((page_cache_d_t*)c, (QueuePair*)q, starting_lba, (uint32_t)n_blocks, pc_entry, NVM_IO_READ, ((page_cache_d_t*)c)->direct_share);
+                ok = bam::io_group((page_cache_d_t*)c, (QueuePair*)q, starting_lba, (uint32_t)n_blocks, pc_entry, NVM_IO_READ,
+                                   place == BAM_PLACE_PULLED ? 0u : ((page_cache_d_t*)c)->direct_share);
             });
         });
         return;
@@ -432,8 +444,8 @@ inline __device__ void read_begin(page_cache_d_t* pc, QueuePair* qp, const uint6
     QueuePair* cur = (QueuePair*)bam::first((uint64_t)qp);
     page_cache_d_t* cpc = (page_cache_d_t*)bam::first((uint64_t)pc);
     uint32_t pos;
-    uint32_t gauged = ahead ? 2u : 1u;
-    cid = bam::io_submit_group(cpc, cur, starting_lba, (uint32_t)n_blocks, pc_entry, NVM_IO_READ, stage, pos, cpc->direct_share, gauged);
+    uint32_t gauged = place == BAM_PLACE_PULLED ? 0u : place == BAM_PLACE_AHEAD ? 2u : 1u;
+    cid = bam::io_submit_group(cpc, cur, starting_lba, (uint32_t)n_blocks, pc_entry, NVM_IO_READ, stage, pos, place == BAM_PLACE_PULLED ? 0u : cpc->direct_share, gauged);
 #ifdef BAM_PROFILE
     const uint64_t pt2 = wall_clock64();
 #endif
@@ -625,7 +637,7 @@ struct range_d_t {
     /* spread by workgroup so that no counter word is shared by more than a few waves at a time */
     __forceinline__ __device__ bam_stat_shard_t* shard() const { return stats + (((blockIdx.x + blockIdx.y * gridDim.x) * 0x9E3779B1u) >> 20) % BAM_STAT_SHARDS; }
     __forceinline__ __device__ bool slow_step(const size_t pg, const bool write, const uint32_t queue, uint64_t& sv, uint32_t& slot, bool& was_hit, bool& progressed, const bool take_part = true,
-                                              const bool may_load = true, bool* wants_load = nullptr, const bool ahead = false);
+                                              const bool may_load = true, bool* wants_load = nullptr, const uint32_t place = BAM_PLACE_NORMAL);
 };
 
 /*
@@ -731,7 +743,7 @@ __device__ __forceinline__ void stat_add(unsigned long long* ctr, uint32_t v)
 template <typename T>
 __forceinline__ __device__
 bool range_d_t<T>::slow_step(const size_t pg, const bool write, const uint32_t queue, uint64_t& sv, uint32_t& slot, bool& was_hit, bool& progressed, const bool take_part,
-                             const bool may_load, bool* wants_load, const bool ahead)
+                             const bool may_load, bool* wants_load, const uint32_t place)
 {
     using namespace bam;
     data_page_t* dp = &pages[pg];
@@ -779,7 +791,7 @@ bool range_d_t<T>::slow_step(const size_t pg, const bool write, const uint32_t q
             stat_add((unsigned long long*)&ctl->access_counter, 1);
             stat_add(&shard()->read_io_cnt, 1);
             qp = ctl->d_qps + (queue % ctl->n_qps);
-            read_begin(&cache, qp, get_backing_page(pg) * cache.n_blocks_per_page, cache.n_blocks_per_page, found, cid, stage, held, io_ok, ahead);
+            read_begin(&cache, qp, get_backing_page(pg) * cache.n_blocks_per_page, cache.n_blocks_per_page, found, cid, stage, held, io_ok, place);
         }
     }
     /* staged payload is moved by every lane that came in, whether it loaded a page itself or not */
@@ -857,13 +869,13 @@ struct bam_pass_t { uint64_t sv; uint32_t slot; uint32_t flags; };
 #define BAM_PASS_WRITE      16u     /* in: */
 #define BAM_PASS_TAKE_PART  32u
 #define BAM_PASS_MAY_LOAD   64u
-#define BAM_PASS_AHEAD      128u    /* the caller fetches for others (placement: page_cache_d_t::direct_limit_ahead) */
+#define BAM_PASS_PLACE_SHIFT 7u     /* BAM_PLACE_* in the two bits from here on */
 template <typename T>
 __forceinline__ __device__ bam_pass_t bam_slow_pass_inline(range_d_t<T>* r, const uint64_t pg, const uint32_t queue, uint64_t sv, uint32_t slot, const uint32_t in)
 {
     bool hit = false, progressed = false, wants = false;
     const bool resolved = r->slow_step(pg, (in & BAM_PASS_WRITE) != 0, queue, sv, slot, hit, progressed, (in & BAM_PASS_TAKE_PART) != 0,
-                                       (in & BAM_PASS_MAY_LOAD) != 0, &wants, (in & BAM_PASS_AHEAD) != 0);
+                                       (in & BAM_PASS_MAY_LOAD) != 0, &wants, (in >> BAM_PASS_PLACE_SHIFT) & 3u);
     bam_pass_t out;
     out.sv = sv;
     out.slot = slot;
@@ -932,7 +944,7 @@ struct range_view {
     uint64_t index_start, index_end, pso;
     uint32_t page_size_log, page_size;
     uint32_t n_access = 0, n_hit = 0;   /* this lane's accesses since the last flush_stats() */
-    bool read_ahead = false;            /* set by waves that fetch for others: their batches may be placed directly up to the higher bound */
+    uint32_t place = BAM_PLACE_NORMAL;  /* waves that only fetch say so: BAM_PLACE_AHEAD, BAM_PLACE_PULLED */
 
     __forceinline__ __device__ void load(range_d_t<T>* r_)
     {
@@ -1061,7 +1073,7 @@ struct range_view {
                 const bool part = !done && master == me;
                 const bam_pass_t ps = bam_slow_pass<OUTLINE>(r, page, queue, sv, slot,
                                                     (dirty ? BAM_PASS_WRITE : 0u) | (part ? BAM_PASS_TAKE_PART : 0u) | (admitted ? BAM_PASS_MAY_LOAD : 0u) |
-                                                    (read_ahead ? BAM_PASS_AHEAD : 0u));
+                                                    (place << BAM_PASS_PLACE_SHIFT));
                 const bool progressed = (ps.flags & BAM_PASS_PROGRESSED) != 0, wants = (ps.flags & BAM_PASS_WANTS) != 0;
                 if (part) {
                     sv = ps.sv;
