@@ -30,15 +30,9 @@ __global__ __launch_bounds__(64) void k_vectoradd_ptr_pc(array_d_t<uint64_t>* da
 }
 
 // ---- reduction (benchmarks/reduction/main.cu:166-195 kernel_reduce_baseline_ptr_pc): output[b] = sum of the 2 x blockDim elements of block b ----
-__global__ void k_reduce_ptr_pc(array_d_t<uint64_t>* da, unsigned long long* output, uint64_t len, const fetch_plan fp)
+/* one output; by all threads of the workgroup */
+__device__ __forceinline__ void reduce_output(array_d_t<uint64_t>* da, unsigned long long* output, const uint64_t len, const uint64_t bid, uint64_t* wave_total)
 {
-    __shared__ uint64_t wave_total[1024 / BAM_WAVE_SIZE];
-    if (fp.done && blockIdx.x < fp.blocks) {
-        array_d_t<uint64_t>* const arrays[1] = {da};
-        fetch_role(arrays, len, fp);
-        return;
-    }
-    const uint64_t bid = blockIdx.x - (fp.done ? fp.blocks : 0u);
     const uint64_t tid = threadIdx.x, start = 2ull * blockDim.x * bid;
     uint64_t v = 0;
     {
@@ -57,8 +51,152 @@ __global__ void k_reduce_ptr_pc(array_d_t<uint64_t>* da, unsigned long long* out
     if (tid < BAM_WAVE_SIZE) {
         v = wave_sum(tid < blockDim.x / BAM_WAVE_SIZE ? wave_total[tid] : 0);
         if (tid == 0) output[bid] = v;
-        if (fp.done && tid == 0) __hip_atomic_fetch_add(fp.done, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
+}
+
+__global__ void k_reduce_ptr_pc(array_d_t<uint64_t>* da, unsigned long long* output, uint64_t len, const fetch_plan fp)
+{
+    __shared__ uint64_t wave_total[1024 / BAM_WAVE_SIZE];
+    if (fp.done && blockIdx.x < fp.blocks) {
+        array_d_t<uint64_t>* const arrays[1] = {da};
+        fetch_role(arrays, len, fp);
+        return;
+    }
+    const uint64_t bid = blockIdx.x - (fp.done ? fp.blocks : 0u);
+    reduce_output(da, output, len, bid, wave_total);
+    if (fp.done && threadIdx.x == 0) __hip_atomic_fetch_add(fp.done, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+/*
+ * The outputs k_reduce_resident left, by as many workgroups as the device holds at a time: what is resident was summed
+ * there, and a grid with a workgroup per output would take longer to find nothing to do (131072 workgroups) than that
+ * kernel takes.  notes[k] covers `per_note` consecutive outputs.
+ */
+__global__ void k_reduce_rest(array_d_t<uint64_t>* da, unsigned long long* output, uint64_t len, uint64_t n_outputs, uint32_t per_note, const uint8_t* notes,
+                              const uint32_t* finished, uint32_t call, const fetch_plan fp)
+{
+    __shared__ uint64_t wave_total[1024 / BAM_WAVE_SIZE];
+    if (__hip_atomic_load(finished + BAM_LEFT_WORD, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != call) return;      /* nothing was left */
+    const uint32_t fetching = fp.done ? fp.blocks : 0u;
+    if (blockIdx.x < fetching) {
+        array_d_t<uint64_t>* const arrays[1] = {da};
+        fetch_role(arrays, len, fp);
+        return;
+    }
+    for (uint64_t bid = blockIdx.x - fetching; bid < n_outputs; bid += gridDim.x - fetching) {
+        if (notes[bid / per_note]) {
+            reduce_output(da, output, len, bid, wave_total);
+            __syncthreads();
+        }
+        if (fp.done && threadIdx.x == 0) __hip_atomic_fetch_add(fp.done, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+}
+
+// ---- reading consecutive elements that are resident ----
+/*
+ * Eight rows of 128 elements from element `first` (a multiple of 128; the same in every lane) of a range that starts on a
+ * page boundary with element 0: lane l gets elements first + 128 r + 2 l and the one behind it in x[r], zero from element n
+ * on.  True (in every lane) if every page with elements below n was resident, by two looks at its descriptor, before and
+ * after the loads, as in bam_read_unpinned; nothing is counted.  The look is one load per page and wave instead of one
+ * atomic pair per page and wave, and a page's payload one 16-byte load per lane and KiB.
+ */
+#define BAM_ROW_ELEMS (2u * BAM_WAVE_SIZE)
+#define BAM_WAVE_ROWS 8u
+#define BAM_WAVE_ELEMS (BAM_WAVE_ROWS * BAM_ROW_ELEMS)
+__device__ __forceinline__ bool read_rows_resident(const bam::range_view<uint64_t>& view, const uint64_t first, const uint64_t n, bam::u64x2_t (&x)[BAM_WAVE_ROWS])
+{
+    using bam::u64x2_t;
+    const uint32_t lane = bam::lane(), log = view.page_size_log;
+#pragma unroll
+    for (uint32_t r = 0; r < BAM_WAVE_ROWS; r++) x[r] = u64x2_t{0, 0};
+    if (first >= n) return true;
+    const uint64_t end = first + BAM_WAVE_ELEMS < n ? first + BAM_WAVE_ELEMS : n;
+    const uint64_t byte0 = first * 8, p0 = byte0 >> log;
+    const uint32_t np = (uint32_t)(((end - 1) * 8 >> log) - p0) + 1;          /* at most 16: pages are of 512 bytes and more */
+    const uint64_t* dp = (const uint64_t*)(view.pages + p0 + (lane < np ? lane : 0));
+    const uint64_t s1 = __hip_atomic_load(dp, __ATOMIC_RELAXED, BAM_AGENT);
+    if (bam::ballot(((uint32_t)s1 >> (CNT_SHIFT + 1)) != V_NB)) return false;
+    const uint32_t slot = (uint32_t)(s1 >> 32) & BAM_SLOT_MASK;
+    const u64x2_t* p[BAM_WAVE_ROWS];
+#pragma unroll
+    for (uint32_t r = 0; r < BAM_WAVE_ROWS; r++) {
+        /* a row spans two pages of 512 bytes or lies in one larger one; rows behind the last page with elements below n read
+         * that page once more */
+        const uint64_t byte = byte0 + r * (BAM_ROW_ELEMS * 8u);
+        const uint32_t a = (uint32_t)((byte >> log) - p0), b = (uint32_t)(((byte + BAM_ROW_ELEMS * 4u) >> log) - p0);
+        const uint32_t slot_a = bam::bcast(slot, a < np ? a : np - 1), slot_b = bam::bcast(slot, b < np ? b : np - 1);
+        p[r] = (const u64x2_t*)(view.base_addr + ((uint64_t)(lane < BAM_WAVE_SIZE / 2 ? slot_a : slot_b) << log) + ((byte + lane * 16u) & (view.page_size - 1)));
+    }
+    bam::ld_payload_stream8x2(p, x);                /* with its wait: the elements are here before the second look goes out */
+    const uint64_t s2 = __hip_atomic_load(dp, __ATOMIC_RELAXED, BAM_AGENT);
+    if (end - first < BAM_WAVE_ELEMS) {
+#pragma unroll
+        for (uint32_t r = 0; r < BAM_WAVE_ROWS; r++) {
+            const uint64_t e = first + r * BAM_ROW_ELEMS + 2u * lane;
+            if (e >= n) x[r].x = 0;
+            if (e + 1 >= n) x[r].y = 0;
+        }
+    }
+    return bam::ballot(((s1 ^ s2) & 0xFFFFFFFFC0000000ull) != 0) == 0;
+}
+
+/*
+ * The outputs of bam_reduce whose elements are resident.  A wave takes as many outputs at a time as fit its 1024 elements,
+ * or one larger one, and goes on to the next; the outputs it could not read are left to k_reduce_rest (a byte per turn says
+ * so).  The accesses are counted as the bam_ptr of k_reduce_ptr_pc counts them: one per lane and page, the lane's second
+ * element, block_size further on, on its own only where it lies on another page.
+ * Bound by HBM: 8 bytes read per element.  2^26 elements in outputs of 512: 95 us, 5.6 TB/s (4221 through bam_ptr); the call takes 16 us
+ * whatever its size below 2^22.
+ */
+__global__ __launch_bounds__(256) void k_reduce_resident(array_d_t<uint64_t>* da, unsigned long long* output, uint64_t len, uint64_t n_outputs, uint32_t half_groups, uint32_t per_note,
+                                                         uint8_t* notes, uint32_t* finished, uint32_t call, unsigned long long* done)
+{
+    const uint32_t lane = bam::lane(), rows = half_groups;          /* rows of an output: 2 x 64 x half_groups elements, 128 to a row */
+    const uint64_t wave = bam::first(((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) / BAM_WAVE_SIZE), n_waves = (uint64_t)gridDim.x * blockDim.x / BAM_WAVE_SIZE;
+    if (blockIdx.x == 0 && threadIdx.x == 0) *done = 0;              /* for the fetching workgroups of the launch behind this one */
+    bam::range_view<uint64_t> view;
+    view.load(da->d_ranges);
+    const uint64_t n_turns = (n_outputs + per_note - 1) / per_note;
+    bool any_left = false;
+    for (uint64_t t = wave; t < n_turns; t += n_waves) {
+        const uint64_t o0 = t * per_note, first = o0 * rows * BAM_ROW_ELEMS;
+        bam::u64x2_t x[BAM_WAVE_ROWS];
+        /* what the lanes hold of the output at hand, and how many of its rows are still to come */
+        uint64_t acc = 0, o = o0;
+        uint32_t rest = rows;
+        bool left = false;
+        const uint32_t turn_rows = per_note * rows;
+        for (uint32_t r0 = 0; r0 < turn_rows && !left; r0 += BAM_WAVE_ROWS) {
+            if (!read_rows_resident(view, first + (uint64_t)r0 * BAM_ROW_ELEMS, len, x)) { left = true; break; }
+#pragma unroll
+            for (uint32_t r = 0; r < BAM_WAVE_ROWS; r++) {
+                if (r0 + r < turn_rows) {
+                    acc += x[r].x + x[r].y;
+                    if (--rest == 0) {
+                        const uint64_t sum = bam::wave_running_sum(acc);
+                        if (lane == BAM_WAVE_SIZE - 1 && o < n_outputs) output[o] = sum;
+                        acc = 0; rest = rows; o++;
+                    }
+                }
+            }
+        }
+        if (lane == 0) notes[t] = left ? 1 : 0;
+        any_left |= left;
+        if (!left && lane < 2u * turn_rows) {
+            /* lane l: the l-th group of 64 elements of the turn; the first half of an output's groups are read by its threads first */
+            const uint64_t e = first + lane * 64ull;
+            const uint32_t within = lane % (2u * rows);
+            if (within < half_groups && e < len) {
+                const uint64_t e2 = e + half_groups * 64ull;
+                uint32_t n = (uint32_t)(len - e < 64 ? len - e : 64);
+                if (e2 < len && view.page_of(e) != view.page_of(e2)) n += (uint32_t)(len - e2 < 64 ? len - e2 : 64);
+                view.n_access += n;
+                view.n_hit += n;
+            }
+        }
+    }
+    if (any_left) note_work_left(finished, call);
+    view.flush_stats();
 }
 
 // ---- scan (benchmarks/scan/main.cu:147-190 kernel_scan_baseline_ptr_pc, :89-100 finalsum) ----
@@ -117,6 +255,106 @@ __global__ void k_scan_ptr_pc(array_d_t<uint64_t>* da, unsigned long long* outpu
     if (fp.done && t == 0) __hip_atomic_fetch_add(fp.done, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+/*
+ * The scan of elements that are resident, in two launches: the sums of all pieces of 1024 elements and of all chunks of
+ * 8 x `pieces` pieces, and then, chunk by chunk, what comes before the chunk, before each of its pieces, and the running
+ * sums.  The first launch reads the array, the second reads it again and writes the result; no workgroup waits for another.
+ * Bound by HBM: 16 bytes per element at least, 24 here (2^26 elements: 312 us with the wait at the end, 5 TB/s of what is moved; 4690
+ * through bam_ptr with a pass over the result to add the block totals; 2^20: 27 against 73).  One pass in which a workgroup waits
+ * for the sums of the ones before it reads the array once, but took 350 us there and 92 for 2^22: the number of the next
+ * tile, drawn from one word, costs the device 20 ns each, and a workgroup's registers sit idle for the 12 us it waits.
+ * A page that is not resident: the wave tells the second launch and the host, which then runs the kernels that can miss.
+ */
+#define BAM_CHUNK_WAVES 8u
+__device__ __forceinline__ void scan_gives_up(uint32_t* finished, const uint32_t call, volatile uint32_t* host_left)
+{
+    if (bam::lane() == 0 && __hip_atomic_load(finished + BAM_LEFT_WORD, __ATOMIC_RELAXED, BAM_AGENT) != call &&
+        __hip_atomic_exchange(finished + BAM_LEFT_WORD, call, __ATOMIC_RELAXED, BAM_AGENT) != call) *host_left = call;
+}
+__global__ __launch_bounds__(BAM_CHUNK_WAVES * BAM_WAVE_SIZE) void k_scan_sums(array_d_t<uint64_t>* da, const uint64_t n, const uint32_t pieces, uint64_t* piece_sums,
+                                                                               uint64_t* chunk_sums, uint32_t* finished, const uint32_t call, volatile uint32_t* host_left)
+{
+    __shared__ uint64_t wave_sums[BAM_CHUNK_WAVES];
+    const uint32_t lane = bam::lane(), w = threadIdx.x / BAM_WAVE_SIZE;
+    const uint64_t chunk = blockIdx.x, p0 = bam::first(chunk * BAM_CHUNK_WAVES * pieces + w);
+    bam::range_view<uint64_t> view;
+    view.load(da->d_ranges);
+    uint64_t total = 0;
+    bool missing = false;
+    for (uint32_t k = 0; k < pieces; k++) {
+        const uint64_t piece = p0 + k * BAM_CHUNK_WAVES;
+        bam::u64x2_t x[BAM_WAVE_ROWS];
+        if (!read_rows_resident(view, piece * BAM_WAVE_ELEMS, n, x)) { missing = true; break; }
+        uint64_t v = 0;
+#pragma unroll
+        for (uint32_t r = 0; r < BAM_WAVE_ROWS; r++) v += x[r].x + x[r].y;
+        v = bam::wave_running_sum(v);
+        if (lane == BAM_WAVE_SIZE - 1) piece_sums[piece] = v;
+        total += v;
+    }
+    if (missing) scan_gives_up(finished, call, host_left);
+    if (lane == BAM_WAVE_SIZE - 1) wave_sums[w] = total;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        uint64_t v = 0;
+#pragma unroll
+        for (uint32_t k = 0; k < BAM_CHUNK_WAVES; k++) v += wave_sums[k];
+        chunk_sums[chunk] = v;
+    }
+}
+
+/* n_access: what the scan counts, as the kernels that can miss count it */
+__global__ __launch_bounds__(BAM_CHUNK_WAVES * BAM_WAVE_SIZE) void k_scan_write(array_d_t<uint64_t>* da, uint64_t* result, const uint64_t n, const uint32_t pieces,
+                                                                                const uint64_t* piece_sums, const uint64_t* chunk_sums, uint32_t* finished, const uint32_t call,
+                                                                                volatile uint32_t* host_left, const uint64_t n_access)
+{
+    __shared__ uint64_t wave_sums[BAM_CHUNK_WAVES];
+    const uint32_t lane = bam::lane(), w = threadIdx.x / BAM_WAVE_SIZE;
+    bam::range_view<uint64_t> view;
+    view.load(da->d_ranges);
+    if (__hip_atomic_load(finished + BAM_LEFT_WORD, __ATOMIC_RELAXED, BAM_AGENT) == call) {
+        if (blockIdx.x == 0 && threadIdx.x == 0) *host_left = call;
+        return;
+    }
+    const uint64_t chunk = blockIdx.x, p0 = chunk * BAM_CHUNK_WAVES * pieces;
+    uint64_t before = 0;
+    for (uint64_t c = threadIdx.x; c < chunk; c += BAM_CHUNK_WAVES * BAM_WAVE_SIZE) before += chunk_sums[c];
+    /* lane l: the sum of the chunk's l-th piece (there are at most 64); the sums of pieces behind the last element are 0 */
+    const uint64_t mine = lane < BAM_CHUNK_WAVES * pieces ? piece_sums[p0 + lane] : 0;
+    const uint64_t pieces_before = bam::wave_running_sum(mine) - mine;
+    before = bam::wave_running_sum(before);
+    if (lane == BAM_WAVE_SIZE - 1) wave_sums[w] = before;
+    __syncthreads();
+    before = 0;
+#pragma unroll
+    for (uint32_t k = 0; k < BAM_CHUNK_WAVES; k++) before += wave_sums[k];
+    for (uint32_t k = 0; k < pieces; k++) {
+        const uint32_t at = k * BAM_CHUNK_WAVES + bam::first(w);
+        const uint64_t first = (bam::first(p0) + at) * BAM_WAVE_ELEMS;
+        if (first > n) break;
+        bam::u64x2_t x[BAM_WAVE_ROWS];
+        if (!read_rows_resident(view, first, n, x)) { scan_gives_up(finished, call, host_left); break; }
+        uint64_t carry = before + bam::bcast(pieces_before, at);
+        /* entry e is the sum of the elements before element e, the last one, n, the total */
+#pragma unroll
+        for (uint32_t r = 0; r < BAM_WAVE_ROWS; r++) {
+            const uint64_t pair = x[r].x + x[r].y, incl = bam::wave_running_sum(pair), sum = carry + (incl - pair);
+            carry += bam::bcast(incl, BAM_WAVE_SIZE - 1);
+            const uint64_t e = first + r * BAM_ROW_ELEMS + 2u * lane;
+            if (first + BAM_WAVE_ELEMS <= n + 1) *(bam::u64x2_t*)(result + e) = bam::u64x2_t{sum, sum + x[r].x};
+            else {
+                if (e <= n) result[e] = sum;
+                if (e + 1 <= n) result[e + 1] = sum + x[r].x;
+            }
+        }
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        bam_stat_shard_t* const sh = view.r->shard();
+        __hip_atomic_fetch_add(&sh->access_cnt, (unsigned long long)n_access, __ATOMIC_RELAXED, BAM_AGENT);
+        __hip_atomic_fetch_add(&sh->hit_cnt, (unsigned long long)n_access, __ATOMIC_RELAXED, BAM_AGENT);
+    }
+}
+
 /* one block: v[i] = v[0] + ... + v[i] in place (the reference calls cub::DeviceScan::InclusiveSum here, scan/main.cu:416-418) */
 __global__ void k_scan_block_totals(unsigned long long* v, uint64_t n)
 {
@@ -148,6 +386,74 @@ __global__ void k_scan_finalsum(const unsigned long long* scanned_totals, unsign
     if (idx + B < len) output[idx + B] += add;
 }
 
+/*
+ * Whether bam_reduce and bam_scan read what is resident first, without references: arrays of one range whose element 0 is
+ * the first of a page, with the elements asked for in no more pages than the cache has (otherwise some are missing for sure,
+ * and the kernels that can miss do it all), and no capture (the launches work in buffers that are kept between calls).
+ */
+bool resident_first(bam_array_t* a, uint64_t n_elems, hipStream_t st)
+{
+    if (!two_launches_ok(a)) return false;
+    const range_d_t<uint64_t>& r = a->a->h_ranges[0];
+    if (r.index_start || r.page_start_offset || n_elems > r.count || r.cache.page_size < 512) return false;
+    if ((n_elems * sizeof(uint64_t) + r.cache.page_size - 1) / r.cache.page_size > r.cache.n_pages) return false;
+    return !is_captured(st);
+}
+
+/*
+ * The accesses a reduction or scan of n elements counts with workgroups of `half` threads when all is resident: thread t of
+ * a workgroup reads elements t and t + half of its 2 half, one access each unless they lie on the same page.  In groups of
+ * 64 elements, which lie on one page and in one half; where the groups' places in a page and in a workgroup repeat, one
+ * period stands for all.
+ */
+uint64_t paired_accesses(uint64_t n, uint64_t half, uint64_t page_elems)
+{
+    const uint64_t b = half / 64, epg = page_elems / 64;
+    auto of_group = [&](uint64_t g) -> uint64_t {
+        if (g / b & 1 || g * 64 >= n) return 0;
+        const uint64_t e2 = (g + b) * 64;
+        return std::min<uint64_t>(64, n - g * 64) + (g / epg != (g + b) / epg && e2 < n ? std::min<uint64_t>(64, n - e2) : 0);
+    };
+    uint64_t period = 2 * b;
+    while (period % epg) period += 2 * b;
+    const uint64_t groups = (n + 63) / 64, whole = groups > b + 1 ? (groups - b - 1) / period : 0;      /* periods whose pairs are all complete */
+    uint64_t total = 0;
+    if (whole) { for (uint64_t g = 0; g < period; g++) total += of_group(g); total *= whole; }
+    for (uint64_t g = whole * period; g < groups; g++) total += of_group(g);
+    return total;
+}
+
+/* the scan of resident elements; false if some were not, and then the result is not written in full */
+bool scan_resident(bam_array_t* a, uint64_t n_elems, uint32_t block_size, uint64_t* d_result, hipStream_t st)
+{
+    BufferPtr host;
+    uint32_t call;
+    {
+        /* pieces per wave: as many as leave 2048 workgroups, eight at most (a chunk's pieces are looked after by the lanes of a
+         * wave); 2^26 elements 312 us, with 512 or 1024 workgroups at least 322, and with stretches of 2^24 elements, small
+         * enough for the last-level cache to hold them from the first launch to the second, 373.  n / 1024 + 1 pieces: entry n
+         * of the result is in the last */
+        const uint64_t n_pieces = n_elems / BAM_WAVE_ELEMS + 1;
+        uint32_t pieces = 1;
+        while (pieces < 8 && n_pieces / (BAM_CHUNK_WAVES * pieces * 2) >= 2048) pieces *= 2;
+        const uint64_t per_chunk = BAM_CHUNK_WAVES * pieces, n_chunks = (n_pieces + per_chunk - 1) / per_chunk;
+        const uint64_t n_access = paired_accesses(n_elems, block_size, a->a->h_ranges[0].cache.page_size / 8);
+        std::lock_guard<std::mutex> guard(a->scatter_mu);
+        bam_array::scatter_set* set = a->scatter_for(st, n_chunks * (per_chunk + 1) * sizeof(uint64_t), 0);
+        if (!set->host_words) set->host_words = createHostBuffer(64 * sizeof(uint32_t));
+        host = set->host_words;
+        call = set->next_call();
+        volatile uint32_t* left = (volatile uint32_t*)host.get() + call % 64;
+        uint64_t* piece_sums = (uint64_t*)set->notes.get(), *chunk_sums = piece_sums + n_chunks * per_chunk;
+        const dim3 grid((uint32_t)n_chunks), block(BAM_CHUNK_WAVES * BAM_WAVE_SIZE);
+        hipLaunchKernelGGL(k_scan_sums, grid, block, 0, st, a->a->d_array_ptr, n_elems, pieces, piece_sums, chunk_sums, set->finished(), call, left);
+        hipLaunchKernelGGL(k_scan_write, grid, block, 0, st, a->a->d_array_ptr, d_result, n_elems, pieces, piece_sums, chunk_sums, set->finished(), call, left, n_access);
+        hip_err_chk(hipGetLastError());
+    }
+    hip_err_chk(hipStreamSynchronize(st));
+    return ((volatile uint32_t*)host.get())[call % 64] != call;
+}
+
 } // namespace
 
 extern "C" {
@@ -172,8 +478,29 @@ int bam_reduce(bam_array_t* a, uint64_t n_elems, uint32_t block_size, uint64_t* 
     if (n_elems > a->a->adt.n_elems) return fail(EINVAL, "bam_reduce: more elements than the array holds");
     if (!n_elems) return 0;
     BAM_API_BEGIN
+    const uint64_t n_outputs = blocks_for(n_elems, 2ull * block_size);
+    /* two launches instead of one: 4 us more per call, made up for from here on (blocks of 64: 21 against 16 us at 2^16 elements;
+     * blocks of 256: 15 against 17 there, 17 both at 2^17, 20 against 17 at 2^18) */
+    if ((n_elems >= 1ull << 17 || n_outputs >= 512) && resident_first(a, n_elems, (hipStream_t)stream)) {
+        hipStream_t st = (hipStream_t)stream;
+        /* outputs per turn of a wave: as many as its rows hold, one at least (of more than eight rows, read in two goes) */
+        const uint32_t rows = block_size / BAM_WAVE_SIZE, per_note = rows < BAM_WAVE_ROWS ? BAM_WAVE_ROWS / rows : 1;
+        const uint64_t n_turns = (n_outputs + per_note - 1) / per_note;
+        std::lock_guard<std::mutex> guard(a->scatter_mu);
+        bam_array::scatter_set* set = a->scatter_for(st, n_turns, 0);
+        uint8_t* notes = (uint8_t*)set->notes.get();
+        const uint32_t call = set->next_call();
+        hipLaunchKernelGGL(k_reduce_resident, dim3((uint32_t)std::min<uint64_t>((n_turns + 3) / 4, 2048)), dim3(256), 0, st, a->a->d_array_ptr, (unsigned long long*)d_partials, n_elems,
+                           n_outputs, rows, per_note, notes, set->finished(), call, set->done());
+        const fetch_plan fp = make_fetch_plan(a, 1, block_size, 2ull * block_size, st, set->done());
+        const uint64_t at_a_time = 256ull * 1024 / block_size;                 /* sixteen waves per compute unit */
+        hipLaunchKernelGGL(k_reduce_rest, dim3((uint32_t)std::min<uint64_t>(n_outputs, at_a_time) + fp.blocks), dim3(block_size), 0, st, a->a->d_array_ptr, (unsigned long long*)d_partials,
+                           n_elems, n_outputs, per_note, notes, set->finished(), call, fp);
+        hip_err_chk(hipGetLastError());
+        return 0;
+    }
     const fetch_plan fp = make_fetch_plan(a, 1, block_size, 2ull * block_size, (hipStream_t)stream);
-    hipLaunchKernelGGL(k_reduce_ptr_pc, dim3(blocks_for(n_elems, 2ull * block_size) + fp.blocks), dim3(block_size), 0, (hipStream_t)stream,
+    hipLaunchKernelGGL(k_reduce_ptr_pc, dim3(n_outputs + fp.blocks), dim3(block_size), 0, (hipStream_t)stream,
                        a->a->d_array_ptr, (unsigned long long*)d_partials, n_elems, fp);
     hip_err_chk(hipGetLastError());
     BAM_API_END
@@ -186,6 +513,7 @@ int bam_scan(bam_array_t* a, uint64_t n_elems, uint32_t block_size, uint64_t* d_
     if (n_elems > a->a->adt.n_elems) return fail(EINVAL, "bam_scan: more elements than the array holds");
     BAM_API_BEGIN
     hipStream_t st = (hipStream_t)stream;
+    if (n_elems && (uintptr_t)d_result % 16 == 0 && resident_first(a, n_elems, st) && scan_resident(a, n_elems, block_size, d_result, st)) return 0;
     hip_err_chk(hipMemsetAsync(d_result, 0, sizeof(uint64_t), st));
     if (n_elems) {
         const uint64_t n_blocks = blocks_for(n_elems, 2ull * block_size);

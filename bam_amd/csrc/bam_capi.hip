@@ -59,17 +59,6 @@ __device__ __forceinline__ void fold_by_last_block(unsigned long long* partials,
     v = wave_sum(v);
     if (bam::lane() == 0 && v) atomicAdd(sum, (unsigned long long)v);
 }
-/* the word through which the first of two launches tells the second whether it left anything: the number of the call when it
- * did (the host counts the calls per array), so that nobody has to clear it */
-#define BAM_LEFT_WORD 96u
-/* by a whole wave that left something; the word is written only while it does not say so yet (thousands of waves storing to
- * one address take the device 12 ns a time, one after the other) */
-__device__ __forceinline__ void note_work_left(uint32_t* finished, const uint32_t call)
-{
-    if (bam::lane() == bam::first_lane(bam::active_mask()) && __hip_atomic_load(finished + BAM_LEFT_WORD, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != call)
-        __hip_atomic_store(finished + BAM_LEFT_WORD, call, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
 // ---- array benchmark (benchmarks/array/main.cu:43-65), with a checksum ----
 __global__ void k_array_read(array_d_t<uint64_t>* dr, uint64_t n_reqs, const uint64_t* assignment, uint64_t stride, uint64_t reqs_per_thread, unsigned long long* sum)
 {
@@ -1407,13 +1396,6 @@ int bam_array_stats(bam_array_t* a, uint64_t* out, int reset)
     BAM_API_END
 }
 
-/* whether the entry points that have a two-launch form may use it on this array: one range, reads of resident pages
- * without a reference switched on (the first launch reads that way) */
-static bool two_launches_ok(bam_array_t* a)
-{
-    return a->a->adt.n_ranges == 1 && a->a->h_ranges[0].cache.fast_reads != 0;
-}
-
 extern "C++" {
 namespace {
 /* whether a gather is better off as several launches than as one that can miss; they keep notes between launches, which a
@@ -1423,9 +1405,7 @@ bool scattered_launches_pay(bam_array_t* a, uint64_t n_reqs, hipStream_t st)
     if (!two_launches_ok(a)) return false;
     const range_d_t<uint64_t>& range = a->a->h_ranges[0];
     if (n_reqs < (range.page_count > range.cache.n_pages ? 1ull << 14 : 1ull << 20)) return false;
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(st, &cap) != hipSuccess) { (void)hipGetLastError(); return false; }
-    return cap == hipStreamCaptureStatusNone;
+    return !is_captured(st);
 }
 /*
  * Scattered reads in several launches: what is resident (k_array_read_n), then the rest.  Where the array is larger than

@@ -83,9 +83,12 @@ struct bam_array {
         BufferPtr words, notes, wanted;
         size_t notes_bytes = 0, wanted_bytes = 0;
         uint32_t calls = 0;
+        BufferPtr host_words;           /* [64] in host memory, one per call in turn: the number of a scan that found a page missing */
         unsigned long long* partials() { return (unsigned long long*)words.get(); }
         uint32_t* finished() { return (uint32_t*)(partials() + BAM_SUM_PARTIALS); }
         uint32_t next_call() { if (++calls == 0) calls = 1; return calls; }
+        /* the word the computing workgroups of a reduction count themselves off in for the fetching ones */
+        unsigned long long* done() { return (unsigned long long*)(finished() + 104); }
     };
     std::mutex scatter_mu;
     std::vector<std::unique_ptr<scatter_set>> scatter_sets;
@@ -156,6 +159,17 @@ __device__ __forceinline__ void block_accumulate(unsigned long long* partials, u
 {
     v = wave_sum(v);
     if (bam::lane() == 0 && v) atomicAdd(&partials[(blockIdx.x * 0x9E3779B1u) >> 20], (unsigned long long)v);
+}
+
+/* the word through which the first of two launches tells the second whether it left anything: the number of the call when it
+ * did (the host counts the calls per array), so that nobody has to clear it */
+#define BAM_LEFT_WORD 96u
+/* by a whole wave that left something; the word is written only while it does not say so yet (thousands of waves storing to
+ * one address take the device 12 ns a time, one after the other) */
+__device__ __forceinline__ void note_work_left(uint32_t* finished, const uint32_t call)
+{
+    if (bam::lane() == bam::first_lane(bam::active_mask()) && __hip_atomic_load(finished + BAM_LEFT_WORD, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != call)
+        __hip_atomic_store(finished + BAM_LEFT_WORD, call, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 /* a page that is not resident as far as one look at its state tells: what the read-ahead asks for (a page that is resident is
@@ -267,7 +281,7 @@ __device__ __forceinline__ void fetch_role(array_d_t<T>* const (&arrays)[N], con
  * (32768 pages on their way; measured on 1 GiB read from the store: 32 waves 18 GB/s, 64 waves 29, 256 waves 34-42, 512 waves
  * 37-44, none 9-11), fewer where a quarter of the cache is less than that; BAM_FETCH_WAVES in the environment overrides the
  * number (0: none); `done` is cleared on the stream */
-inline fetch_plan make_fetch_plan(bam_array_t* a, int n_arrays, uint32_t block_size, uint64_t elems_per_block, hipStream_t st)
+inline fetch_plan make_fetch_plan(bam_array_t* a, int n_arrays, uint32_t block_size, uint64_t elems_per_block, hipStream_t st, unsigned long long* cleared = nullptr)
 {
     fetch_plan fp{nullptr, 0, 1u << 18, 0, elems_per_block};
     if (a->a->adt.n_ranges != 1) return fp;
@@ -283,10 +297,25 @@ inline fetch_plan make_fetch_plan(bam_array_t* a, int n_arrays, uint32_t block_s
     const uint32_t waves_per_block = block_size / BAM_WAVE_SIZE;
     fp.blocks = (uint32_t)((waves + waves_per_block - 1) / waves_per_block);
     fp.lead_elems = budget_pages * (cache.page_size / sizeof(uint64_t));
+    if (cleared) { fp.done = cleared; return fp; }      /* a word that an earlier launch on the stream clears */
     if (!a->progress) a->progress = createBuffer(64, 0);
     fp.done = (unsigned long long*)a->progress.get();
     hip_err_chk(hipMemsetAsync(fp.done, 0, sizeof(unsigned long long), st));
     return fp;
+}
+
+/* whether the entry points that have a two-launch form may use it on this array: one range, reads of resident pages
+ * without a reference switched on (the first launch reads that way) */
+inline bool two_launches_ok(bam_array_t* a)
+{
+    return a->a->adt.n_ranges == 1 && a->a->h_ranges[0].cache.fast_reads != 0;
+}
+/* whether `st` is being captured (or cannot say): launches that keep notes for each other from call to call stay out of graphs */
+inline bool is_captured(hipStream_t st)
+{
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &cap) != hipSuccess) { (void)hipGetLastError(); return true; }
+    return cap != hipStreamCaptureStatusNone;
 }
 
 inline uint32_t blocks_for(uint64_t n, uint32_t bs) { return (uint32_t)((n + bs - 1) / bs); }

@@ -266,6 +266,45 @@ __device__ __forceinline__ void ld_payload_nt(const uint64_t* const (&p)[N], uin
 }
 
 /*
+ * Eight pieces of 16 bytes at eight addresses of the lane's own, loaded like the streaming words above: a wave that reads
+ * consecutive elements takes 1 KiB per load, two elements per lane.  Every address must be readable and a multiple of 16.
+ */
+typedef uint64_t u64x2_t __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ void ld_payload_stream8x2(const u64x2_t* const (&p)[8], u64x2_t (&x)[8])
+{
+    asm volatile("global_load_dwordx4 %0, %8, off sc1 nt\n\tglobal_load_dwordx4 %1, %9, off sc1 nt\n\t"
+                 "global_load_dwordx4 %2, %10, off sc1 nt\n\tglobal_load_dwordx4 %3, %11, off sc1 nt\n\t"
+                 "global_load_dwordx4 %4, %12, off sc1 nt\n\tglobal_load_dwordx4 %5, %13, off sc1 nt\n\t"
+                 "global_load_dwordx4 %6, %14, off sc1 nt\n\tglobal_load_dwordx4 %7, %15, off sc1 nt\n\ts_waitcnt vmcnt(0)"
+                 : "=&v"(x[0]), "=&v"(x[1]), "=&v"(x[2]), "=&v"(x[3]), "=&v"(x[4]), "=&v"(x[5]), "=&v"(x[6]), "=&v"(x[7])
+                 : "v"(p[0]), "v"(p[1]), "v"(p[2]), "v"(p[3]), "v"(p[4]), "v"(p[5]), "v"(p[6]), "v"(p[7]) : "memory");
+}
+
+/*
+ * Running sums over the 64 lanes of a wave (all active), lane l receiving the sum of the values of lanes 0 .. l: four
+ * shifts within the rows of sixteen lanes, then the last lane of a row broadcast to the row behind it and the last lane of
+ * the first two to the last two, all of them operand modifiers of the vector unit.  The same over ds_bpermute takes twelve
+ * trips through the LDS.
+ */
+template <int CTRL, int ROWS>
+__device__ __forceinline__ uint64_t dpp_or_zero(const uint64_t v)
+{
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)v, CTRL, ROWS, 0xf, false);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(v >> 32), CTRL, ROWS, 0xf, false);
+    return ((uint64_t)hi << 32) | lo;
+}
+__device__ __forceinline__ uint64_t wave_running_sum(uint64_t v)
+{
+    v += dpp_or_zero<0x111, 0xf>(v);
+    v += dpp_or_zero<0x112, 0xf>(v);
+    v += dpp_or_zero<0x114, 0xf>(v);
+    v += dpp_or_zero<0x118, 0xf>(v);
+    v += dpp_or_zero<0x142, 0xa>(v);
+    v += dpp_or_zero<0x143, 0xc>(v);
+    return v;
+}
+
+/*
  * Sixteen bytes per lane at system scope, for moving payload between a staging page in host memory and a cache slot.
  * The load is never served from a cache that remembers the staging page's last tenant, so nobody has to invalidate
  * caches after a completion; the store goes through to memory, so the wave that moved a page in can publish it after
