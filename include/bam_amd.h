@@ -261,7 +261,9 @@ int bam_cc_shaped(bam_array_t* edges, const uint64_t* d_offsets, uint64_t n_vert
 int bam_bfs_frontier(bam_array_t* edges, const uint64_t* d_offsets, uint64_t n_vertices, uint64_t src, uint32_t* d_labels,
                      uint32_t* iterations, void* stream);
 /* ---- CC (benchmarks/cc/main.cu:123-144 cc_compute, :595-617 kernel, host loop :1410-1425, 1515-1521) ----
- * Min-label propagation; d_labels[V] receives the smallest vertex id of each vertex's component. */
+ * d_labels[V] receives the smallest vertex id of each vertex's component of an undirected graph (both directions of every
+ * edge in the CSR).  Where the reference propagates labels, sweep after sweep over the edges, the edges are read once here
+ * and the trees of their ends joined, and a pass over the vertices settles the labels: *iterations = 2. */
 int bam_cc(bam_array_t* edges, const uint64_t* d_offsets, uint64_t n_vertices, uint64_t* d_labels,
            uint32_t coarse, uint32_t* iterations, void* stream);
 
