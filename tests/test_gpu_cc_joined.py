@@ -1,0 +1,50 @@
+"""Components from one reading of the edges: shapes whose trees are long, wide, or not there at all."""
+import numpy as np
+import pytest
+
+import oracle
+from test_gpu_parity import _dev, _graph_rig, _u64, bam  # noqa: F401  (bam is the module fixture)
+
+pytestmark = pytest.mark.gpu
+
+
+def _csr(n_v, u, v):
+    """both directions of every pair, ordered by vertex"""
+    src, dst = np.concatenate([u, v]), np.concatenate([v, u])
+    order = np.argsort(src, kind="stable")
+    off = np.zeros(n_v + 1, dtype=np.uint64)
+    off[1:] = np.cumsum(np.bincount(src, minlength=n_v))
+    return off, dst[order].astype(np.uint64)
+
+
+def _pairs(shape, n_v, rng):
+    at = np.arange(n_v, dtype=np.int64)
+    if shape == "path":                                   # every vertex hooks onto the one before it
+        return at[:-1], at[1:]
+    if shape == "scattered_path":
+        p = rng.permutation(n_v)
+        return p[:-1], p[1:]
+    if shape == "star":                                   # one list in pieces, every join on the same root, which is the largest vertex
+        return np.full(n_v - 1, n_v - 1, dtype=np.int64), at[:-1]
+    if shape == "loops_and_copies":                       # each vertex to itself, and pairs of neighbours three times over
+        even = at[: n_v // 2 * 2 : 2]
+        return np.concatenate([at, even, even, even]), np.concatenate([at, even + 1, even + 1, even + 1])
+    return at[:1], at[-1:]                                # one edge between the ends, all other vertices by themselves
+
+
+@pytest.mark.parametrize("by_page", [False, True])
+@pytest.mark.parametrize("shape", ["path", "scattered_path", "star", "loops_and_copies", "ends"])
+@pytest.mark.parametrize("n_v", [2, 65, 512, 513, 100003])
+def test_cc_labels_of_long_wide_and_empty_trees(bam, n_v, shape, by_page):
+    off, nb = _csr(n_v, *_pairs(shape, n_v, np.random.default_rng(n_v)))
+    ref, _ = oracle.cc_labels(off, nb)
+    r, a = _graph_rig(bam, nb, 256, n_queues=16, depth=256)
+    with r:
+        d_off = _dev(off)
+        for kept in (False, True, True):                  # without a plan, then with one: from the front and from the back
+            if kept:
+                a.set_graph(d_off)
+            lb, it = a.cc(d_off, by_page=by_page)
+            assert np.array_equal(_u64(lb), ref), kept
+            assert it >= 1
+        assert not r.c.aborted()
