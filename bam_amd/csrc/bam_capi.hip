@@ -426,6 +426,83 @@ __global__ void k_array_update(array_d_t<uint64_t>* dr, uint64_t n_reqs, const u
     if (old) old[tid] = before;
 }
 
+/* one addition the way that can miss, as a call: its registers stay out of the kernel below */
+__attribute__((noinline)) __device__ uint64_t update_call(const array_d_t<uint64_t>* dr, const uint64_t idx, const uint64_t val) { return dr->AtomicAdd(idx, val); }
+/*
+ * k_array_update<0> with several elements per lane (arrays of one range).  With one, every 64 elements wait for three
+ * atomics one after the other and for a release that writes the second-level cache back.  Here the references of all
+ * elements of a wave are taken side by side, one per page and round as in range_view::acquire, the elements of resident
+ * pages added to, and one release goes before all references are dropped.  Only then is the rest asked for the way that can
+ * miss, a round at a time: no wave waits holding references.  What bounds it now are the atomics, two on a page's descriptor
+ * and one on the element, which the device performs at the memory, some 20 G/s of them.
+ * 1000003 elements of a resident 256 MiB (us; one, two, four, eight per lane): scattered 204, 168, 152, 149; sorted 164, 104,
+ * 76, 62; in order 153, 83, 55, 28; on 64 elements 434, 425, 434, 439.  (References per run of neighbouring lanes instead of
+ * per page: scattered 149, on 64 elements 708.)
+ */
+#define BAM_UPDATES_PER_LANE 4
+__global__ __launch_bounds__(1024) void k_array_update_n(array_d_t<uint64_t>* dr, uint64_t n_reqs, const uint64_t* assignment, const uint64_t* values, uint64_t* old)
+{
+    constexpr int N = BAM_UPDATES_PER_LANE;
+    const uint32_t me = bam::lane();
+    const uint64_t first = (uint64_t)blockIdx.x * blockDim.x * N + threadIdx.x;
+    bam::range_view<uint64_t> v;
+    v.load(dr->d_ranges);
+    uint64_t val[N], sv[N];
+    size_t idx[N];
+    data_page_t* dp[N];
+    uint32_t in_page[N], refs[N], leader[N];              /* refs: the references the lane takes for all lanes on its page, 0 unless it is the first of them */
+    bool want[N], hit[N];
+#pragma unroll
+    for (int j = 0; j < N; j++) {
+        const uint64_t t = first + (uint64_t)j * blockDim.x;
+        want[j] = t < n_reqs;
+        idx[j] = want[j] ? assignment[t] : 0;
+        val[j] = want[j] ? values[t] : 0;
+    }
+#pragma unroll
+    for (int j = 0; j < N; j++) {
+        const bool inside = want[j] && idx[j] - v.index_start < v.index_end - v.index_start;
+        const uint64_t byte = inside ? v.byte_of(idx[j]) : 0;
+        dp[j] = v.pages + (byte >> v.page_size_log);
+        in_page[j] = (uint32_t)byte & (v.page_size - 1);
+        const uint64_t eq_mask = bam::match_any(inside ? (uint64_t)dp[j] : 0ull);
+        leader[j] = bam::first_lane(eq_mask);
+        refs[j] = inside && leader[j] == me ? bam::popc(eq_mask) : 0u;
+        hit[j] = inside;
+    }
+#pragma unroll
+    for (int j = 0; j < N; j++) {
+        sv[j] = 0;
+        if (refs[j]) sv[j] = __hip_atomic_fetch_add((uint64_t*)dp[j], (uint64_t)refs[j], __ATOMIC_RELAXED, BAM_AGENT);
+    }
+#pragma unroll
+    for (int j = 0; j < N; j++) {
+        const uint32_t s = (uint32_t)sv[j];
+        if (refs[j] && (s >> (CNT_SHIFT + 1)) == V_NB && (s & DIRTY) == 0) __hip_atomic_fetch_or(&dp[j]->state, DIRTY, __ATOMIC_RELAXED, BAM_AGENT);
+    }
+    uint64_t was[N];
+#pragma unroll
+    for (int j = 0; j < N; j++) {
+        const uint64_t w = bam::shfl(sv[j], leader[j]);
+        hit[j] = hit[j] && ((uint32_t)w >> (CNT_SHIFT + 1)) == V_NB;
+        was[j] = 0;
+        if (hit[j]) {
+            was[j] = atomicAdd((unsigned long long*)(v.base_addr + ((uint64_t)((uint32_t)(w >> 32) & BAM_SLOT_MASK) << v.page_size_log) + in_page[j]), (unsigned long long)val[j]);
+            v.account(true);
+        }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+#pragma unroll
+    for (int j = 0; j < N; j++)
+        if (refs[j]) __hip_atomic_fetch_add(&dp[j]->state, 0u - refs[j], __ATOMIC_RELAXED, BAM_AGENT);
+    v.template flush_stats_bits<3>();
+#pragma unroll
+    for (int j = 0; j < N; j++) {
+        if (want[j] && !hit[j]) was[j] = update_call(dr, idx[j], val[j]);
+        if (want[j] && old) old[first + (uint64_t)j * blockDim.x] = was[j];
+    }
+}
+
 /* lane l encodes the submission entry of command (cid + l) for block (lba + l) the way the miss path does (nvm_cmd_header,
  * nvm_cmd_data_ptr, nvm_cmd_rw_blks, and nvm_cmd_seal with ticket + l on top when asked): 64 entries of 16 dwords */
 __global__ void k_sqe_image(uint16_t cid, uint8_t opcode, uint32_t nsid, uint64_t prp1, uint64_t prp2, uint64_t lba, uint16_t n_blocks, int seal, uint32_t ticket,
@@ -1589,7 +1666,12 @@ int bam_array_update(bam_array_t* a, int api, uint64_t n_reqs, const uint64_t* d
     const dim3 grid(blocks_for(n_reqs, block_size)), block(block_size);
     hipStream_t st = (hipStream_t)stream;
     array_d_t<uint64_t>* d = a->a->d_array_ptr;
-    if (api == 0) hipLaunchKernelGGL(k_array_update<0>, grid, block, 0, st, d, n_reqs, d_assignment, d_values, d_old);
+    /* Several per lane: from where the waves left still fill the device (scattered, resident, one against four per lane: 16.6 and
+     * 19.7 us for 64000, 28.9 and 27.6 for 128000, 57.7 and 43.2 for 256000), and not where the array outgrows its cache, so
+     * that many of the elements miss (10^6 of them, first call: 0.67 s and 0.76 s). */
+    if (api == 0 && n_reqs >= 1ull << 17 && a->a->adt.n_ranges == 1 && a->a->h_ranges[0].page_count <= a->a->h_ranges[0].cache.n_pages)
+        hipLaunchKernelGGL(k_array_update_n, dim3(blocks_for(n_reqs, (uint64_t)block_size * BAM_UPDATES_PER_LANE)), block, 0, st, d, n_reqs, d_assignment, d_values, d_old);
+    else if (api == 0) hipLaunchKernelGGL(k_array_update<0>, grid, block, 0, st, d, n_reqs, d_assignment, d_values, d_old);
     else if (api == 1) hipLaunchKernelGGL(k_array_update<1>, grid, block, 0, st, d, n_reqs, d_assignment, d_values, d_old);
     else hipLaunchKernelGGL(k_array_update<2>, grid, block, 0, st, d, n_reqs, d_assignment, d_values, d_old);
     hip_err_chk(hipGetLastError());

@@ -346,7 +346,7 @@ class Array:
         """element assignment[t] += values[t] through AtomicAdd (api 0), an atomic on bam_ptr::memref (1) or ptr[i] += v (2);
         returns what each element held before (int64 tensor of bit patterns)."""
         n = assignment.numel()
-        old = torch.zeros(n, dtype=torch.int64, device=f"cuda:{self.device}")
+        old = torch.empty(n, dtype=torch.int64, device=f"cuda:{self.device}")
         _chk(self.L.bam_array_update(self.h, api, n, _ptr(assignment), _ptr(values), _ptr(old), block_size, _stream()), "bam_array_update")
         return old
 
