@@ -1555,6 +1555,9 @@ int bam_array_read_shaped(bam_array_t* a, uint64_t n_reqs, const uint64_t* d_ass
     if (!n_reqs) return 0;
     BAM_API_BEGIN
     hipStream_t st = (hipStream_t)stream;
+    /* a graph keeps the addresses it was recorded with and may be replayed beside other calls: it gets the shape that keeps no
+     * notes between launches (the same sum) */
+    if (shape == BAM_READ_TWO_LAUNCHES && is_captured(st)) shape = BAM_READ_FOUR_PER_THREAD;
     array_d_t<uint64_t>* d = a->a->d_array_ptr;
     unsigned long long* part = (unsigned long long*)a->partials.get();
     if (shape == BAM_READ_ONE_PER_THREAD) {

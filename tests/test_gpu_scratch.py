@@ -1,0 +1,56 @@
+"""What calls in several launches keep between them (bam_array_read, bam_array_gather, bam_reduce, bam_scan): graphs, streams, threads."""
+import ctypes
+
+import numpy as np
+import pytest
+
+import oracle
+from test_gpu_parity import Rig, SEED, bam, _dev, _u64  # noqa: F401  (bam is the module fixture)
+
+pytestmark = pytest.mark.gpu
+
+
+def _read_into(a, n, d_idx, out, shape=0):
+    import torch
+    st = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    idx, dst = ctypes.c_void_p(d_idx.data_ptr()), ctypes.c_void_p(out.data_ptr())
+    if shape:
+        assert a.L.bam_array_read_shaped(a.h, n, idx, shape, 8, 64, dst, st) == 0
+    else:
+        assert a.L.bam_array_read(a.h, n, idx, 0, 1, 64, dst, st) == 0
+
+
+@pytest.mark.parametrize("shape", [0, 3])
+@pytest.mark.parametrize("cache_pages", [4096, 4400])
+def test_captured_reads_hold_nothing_of_the_array(bam, cache_pages, shape):
+    """a read recorded into a graph and replayed after, and between, calls on more streams than an array keeps notes for and
+    larger calls on the stream it was recorded on; the array larger than its cache, and resident"""
+    import torch
+    pages, n = 4400, (1 << 16) + 77
+    words = oracle.store(SEED, 0, pages * 512)
+    rng = np.random.default_rng(3)
+    with Rig(bam, pages * 4096, n_queues=16, depth=256) as r:
+        a = r.array(pages * 512, 4096, cache_pages)
+        reqs = rng.integers(0, pages * 512, 4 * n).astype(np.uint64)
+        d, total = _dev(reqs), torch.zeros(1, dtype=torch.int64, device="cuda")
+        other = torch.zeros(1, dtype=torch.int64, device="cuda")
+        want = int(np.sum(words[reqs[:n].astype(np.int64)], dtype=np.uint64))
+        want_all = int(np.sum(words[reqs.astype(np.int64)], dtype=np.uint64))
+        a.read(n, d)
+        torch.cuda.synchronize()
+        graph, side = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+        with torch.cuda.graph(graph, stream=side):
+            _read_into(a, n, d, total, shape)
+        streams = [torch.cuda.Stream() for _ in range(7)] + [side]
+        for rep in range(3):
+            total.zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert int(total.item()) & (2 ** 64 - 1) == want, rep
+            for s in streams:
+                with torch.cuda.stream(s):
+                    other.zero_()
+                    _read_into(a, 4 * n, d, other)
+                torch.cuda.synchronize()
+                assert int(other.item()) & (2 ** 64 - 1) == want_all, rep
+        assert not r.c.aborted()
