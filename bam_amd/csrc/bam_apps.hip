@@ -423,7 +423,8 @@ uint64_t paired_accesses(uint64_t n, uint64_t half, uint64_t page_elems)
     return total;
 }
 
-/* the scan of resident elements; false if some were not, and then the result is not written in full */
+/* the scan of resident elements; false if some were not, and then the result is not written in full, or if there is no
+ * memory for the sums */
 bool scan_resident(bam_array_t* a, uint64_t n_elems, uint32_t block_size, uint64_t* d_result, hipStream_t st)
 {
     BufferPtr host;
@@ -438,8 +439,9 @@ bool scan_resident(bam_array_t* a, uint64_t n_elems, uint32_t block_size, uint64
         while (pieces < 8 && n_pieces / (BAM_CHUNK_WAVES * pieces * 2) >= 2048) pieces *= 2;
         const uint64_t per_chunk = BAM_CHUNK_WAVES * pieces, n_chunks = (n_pieces + per_chunk - 1) / per_chunk;
         const uint64_t n_access = paired_accesses(n_elems, block_size, a->a->h_ranges[0].cache.page_size / 8);
-        std::lock_guard<std::mutex> guard(a->scatter_mu);
-        bam_array::scatter_set* set = a->scatter_for(st, n_chunks * (per_chunk + 1) * sizeof(uint64_t), 0);
+        std::lock_guard<std::mutex> guard(a->scratch.mu);
+        scratch_set* set = scratch_for(a, st, n_chunks * (per_chunk + 1) * sizeof(uint64_t), 0);
+        if (!set) return false;
         if (!set->host_words) set->host_words = createHostBuffer(64 * sizeof(uint32_t));
         host = set->host_words;
         call = set->next_call();
@@ -486,18 +488,19 @@ int bam_reduce(bam_array_t* a, uint64_t n_elems, uint32_t block_size, uint64_t* 
         /* outputs per turn of a wave: as many as its rows hold, one at least (of more than eight rows, read in two goes) */
         const uint32_t rows = block_size / BAM_WAVE_SIZE, per_note = rows < BAM_WAVE_ROWS ? BAM_WAVE_ROWS / rows : 1;
         const uint64_t n_turns = (n_outputs + per_note - 1) / per_note;
-        std::lock_guard<std::mutex> guard(a->scatter_mu);
-        bam_array::scatter_set* set = a->scatter_for(st, n_turns, 0);
-        uint8_t* notes = (uint8_t*)set->notes.get();
-        const uint32_t call = set->next_call();
-        hipLaunchKernelGGL(k_reduce_resident, dim3((uint32_t)std::min<uint64_t>((n_turns + 3) / 4, 2048)), dim3(256), 0, st, a->a->d_array_ptr, (unsigned long long*)d_partials, n_elems,
-                           n_outputs, rows, per_note, notes, set->finished(), call, set->done());
-        const fetch_plan fp = make_fetch_plan(a, 1, block_size, 2ull * block_size, st, set->done());
-        const uint64_t at_a_time = 256ull * 1024 / block_size;                 /* sixteen waves per compute unit */
-        hipLaunchKernelGGL(k_reduce_rest, dim3((uint32_t)std::min<uint64_t>(n_outputs, at_a_time) + fp.blocks), dim3(block_size), 0, st, a->a->d_array_ptr, (unsigned long long*)d_partials,
-                           n_elems, n_outputs, per_note, notes, set->finished(), call, fp);
-        hip_err_chk(hipGetLastError());
-        return 0;
+        std::lock_guard<std::mutex> guard(a->scratch.mu);
+        if (scratch_set* set = scratch_for(a, st, n_turns, 0)) {
+            uint8_t* notes = (uint8_t*)set->notes.get();
+            const uint32_t call = set->next_call();
+            hipLaunchKernelGGL(k_reduce_resident, dim3((uint32_t)std::min<uint64_t>((n_turns + 3) / 4, 2048)), dim3(256), 0, st, a->a->d_array_ptr, (unsigned long long*)d_partials, n_elems,
+                               n_outputs, rows, per_note, notes, set->finished(), call, set->done());
+            const fetch_plan fp = make_fetch_plan(a, 1, block_size, 2ull * block_size, st, set->done());
+            const uint64_t at_a_time = 256ull * 1024 / block_size;             /* sixteen waves per compute unit */
+            hipLaunchKernelGGL(k_reduce_rest, dim3((uint32_t)std::min<uint64_t>(n_outputs, at_a_time) + fp.blocks), dim3(block_size), 0, st, a->a->d_array_ptr, (unsigned long long*)d_partials,
+                               n_elems, n_outputs, per_note, notes, set->finished(), call, fp);
+            hip_err_chk(hipGetLastError());
+            return 0;
+        }
     }
     const fetch_plan fp = make_fetch_plan(a, 1, block_size, 2ull * block_size, (hipStream_t)stream);
     hipLaunchKernelGGL(k_reduce_ptr_pc, dim3(n_outputs + fp.blocks), dim3(block_size), 0, (hipStream_t)stream,

@@ -1488,10 +1488,11 @@ bool scattered_launches_pay(bam_array_t* a, uint64_t n_reqs, hipStream_t st)
  * Scattered reads in several launches: what is resident (k_array_read_n), then the rest.  Where the array is larger than
  * its cache and there are enough requests for them to meet on pages, the rest goes page by page: the pages somebody waits
  * for are fetched, each once, in whole batches (k_fetch_wanted), and then the requests for them are read
- * (k_array_read_deferred), a stretch of the range at a time so that what is fetched is still there when it is read.
+ * (k_array_read_deferred), a stretch of the range at a time so that what is fetched is still there when it is read.  False,
+ * with nothing launched, where there is no memory for the notes.
  */
 template <bool GATHER>
-void scattered_reads(bam_array_t* a, uint64_t n_reqs, const uint64_t* d_assignment, uint32_t N, unsigned long long* sum, uint64_t* d_out, hipStream_t st)
+bool scattered_reads(bam_array_t* a, uint64_t n_reqs, const uint64_t* d_assignment, uint32_t N, unsigned long long* sum, uint64_t* d_out, hipStream_t st)
 {
     const range_d_t<uint64_t>& range = a->a->h_ranges[0];
     const uint64_t cache_pages = range.cache.n_pages, pages = range.page_count;
@@ -1507,8 +1508,9 @@ void scattered_reads(bam_array_t* a, uint64_t n_reqs, const uint64_t* d_assignme
      * for as many again */
     const bool by_page = pages > cache_pages && n_reqs >= pages / 2 && cache_pages >= 4096;
     const uint64_t wanted_bytes = by_page ? (pages + 511) / 512 * 512 : 0;
-    std::lock_guard<std::mutex> guard(a->scatter_mu);
-    bam_array::scatter_set* set = a->scatter_for(st, n_words * sizeof(uint64_t), wanted_bytes);
+    std::lock_guard<std::mutex> guard(a->scratch.mu);
+    scratch_set* set = scratch_for(a, st, n_words * sizeof(uint64_t), wanted_bytes);
+    if (!set) return false;
     uint64_t* missed = (uint64_t*)set->notes.get();
     uint8_t* wanted = by_page ? (uint8_t*)set->wanted.get() : nullptr;
     unsigned long long* part = set->partials();
@@ -1539,6 +1541,7 @@ void scattered_reads(bam_array_t* a, uint64_t n_reqs, const uint64_t* d_assignme
         hipLaunchKernelGGL(k_array_read_deferred<GATHER>, grid_d, block, 0, st, d, n_reqs, d_assignment, missed, n_words, words, p, q, part, sum, d_out, fin, call);
     }
     hip_err_chk(hipGetLastError());
+    return true;
 }
 } // namespace
 } // extern "C++"
@@ -1556,19 +1559,18 @@ int bam_array_read_shaped(bam_array_t* a, uint64_t n_reqs, const uint64_t* d_ass
     BAM_API_BEGIN
     hipStream_t st = (hipStream_t)stream;
     /* a graph keeps the addresses it was recorded with and may be replayed beside other calls: it gets the shape that keeps no
-     * notes between launches (the same sum) */
-    if (shape == BAM_READ_TWO_LAUNCHES && is_captured(st)) shape = BAM_READ_FOUR_PER_THREAD;
+     * notes between launches (the same sum), as does a call for whose notes there is no memory */
+    if (shape == BAM_READ_TWO_LAUNCHES && !is_captured(st) && scattered_reads<false>(a, n_reqs, d_assignment, reads_per_lane, (unsigned long long*)d_sum, nullptr, st)) return 0;
     array_d_t<uint64_t>* d = a->a->d_array_ptr;
     unsigned long long* part = (unsigned long long*)a->partials.get();
     if (shape == BAM_READ_ONE_PER_THREAD) {
         hipLaunchKernelGGL(k_array_read, dim3(blocks_for(n_reqs, block_size)), dim3(block_size), 0, st, d, n_reqs, d_assignment, (uint64_t)1, (uint64_t)1, part);
         hipLaunchKernelGGL(k_fold_partials, dim3(1), dim3(1024), 0, st, part, (unsigned long long*)d_sum);
-    } else if (shape == BAM_READ_FOUR_PER_THREAD) {
+    } else {
         const uint64_t threads = (n_reqs + BAM_READS_PER_LANE - 1) / BAM_READS_PER_LANE;
         hipLaunchKernelGGL(k_array_read_n_whole, dim3(blocks_for(threads, block_size)), dim3(block_size), 0, st, d, n_reqs, d_assignment, threads, part);
         hipLaunchKernelGGL(k_fold_partials, dim3(1), dim3(1024), 0, st, part, (unsigned long long*)d_sum);
-    } else
-        scattered_reads<false>(a, n_reqs, d_assignment, reads_per_lane, (unsigned long long*)d_sum, nullptr, st);
+    }
     hip_err_chk(hipGetLastError());
     BAM_API_END
 }
@@ -1604,10 +1606,7 @@ int bam_array_gather(bam_array_t* a, uint64_t n_reqs, const uint64_t* d_assignme
     if (!block_size || block_size % BAM_WAVE_SIZE || block_size > 1024) return fail(EINVAL, "bam_array_gather: block size must be a multiple of 64, at most 1024");
     if (!n_reqs) return 0;
     BAM_API_BEGIN
-    if (d_assignment && scattered_launches_pay(a, n_reqs, (hipStream_t)stream)) {
-        scattered_reads<true>(a, n_reqs, d_assignment, 8, nullptr, d_out, (hipStream_t)stream);
-        return 0;
-    }
+    if (d_assignment && scattered_launches_pay(a, n_reqs, (hipStream_t)stream) && scattered_reads<true>(a, n_reqs, d_assignment, 8, nullptr, d_out, (hipStream_t)stream)) return 0;
     hipLaunchKernelGGL(k_array_gather, dim3(blocks_for(n_reqs, block_size)), dim3(block_size), 0, (hipStream_t)stream,
                        a->a->d_array_ptr, n_reqs, d_assignment, stride, d_out);
     hip_err_chk(hipGetLastError());

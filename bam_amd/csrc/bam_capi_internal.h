@@ -24,6 +24,7 @@
 #include "nvmt.h"
 #include "page_cache.h"
 #include "bafs_ptr.h"
+#include "scratch_sets.h"
 
 // ---------------------------------------------------------------------------
 // error plumbing
@@ -58,8 +59,6 @@ struct bam_target {
 struct bam_ctrl { Controller* c; };
 struct bam_page_cache { page_cache_t* pc; Controller* ctrl; };      /* ctrl: the first controller of the cache */
 struct bam_range { range_t<uint64_t>* r; };
-#define BAM_SUM_PARTIALS 4096
-#define BAM_SCATTER_SETS 4
 struct bam_array {
     array_t<uint64_t>* a;
     BufferPtr partials, progress;       /* progress: the word the computing workgroups of vectoradd, reduction and scan count themselves off in */
@@ -69,55 +68,7 @@ struct bam_array {
     BufferPtr notes, finished;
     size_t notes_bytes = 0;
     uint32_t calls = 0;
-    /*
-     * What a call of scattered reads in several launches works in: the bits of the requests its first launch leaves, a byte
-     * per page of the range that somebody waits for (zero between calls), checksum shards and the count of finished
-     * workgroups.  One set per stream, because the launches of two calls on one stream run one after the other and those on
-     * two streams do not; the set is picked and its launches are queued under the mutex, so the calls of two threads on one
-     * stream do not mix.  At most BAM_SCATTER_SETS sets are kept: the one longest unused makes room (freeing waits for the
-     * device), and all go with the array.
-     */
-    struct scatter_set {
-        hipStream_t st = nullptr;
-        uint64_t used = 0;
-        BufferPtr words, notes, wanted;
-        size_t notes_bytes = 0, wanted_bytes = 0;
-        uint32_t calls = 0;
-        BufferPtr host_words;           /* [64] in host memory, one per call in turn: the number of a scan that found a page missing */
-        unsigned long long* partials() { return (unsigned long long*)words.get(); }
-        uint32_t* finished() { return (uint32_t*)(partials() + BAM_SUM_PARTIALS); }
-        uint32_t next_call() { if (++calls == 0) calls = 1; return calls; }
-        /* the word the computing workgroups of a reduction count themselves off in for the fetching ones */
-        unsigned long long* done() { return (unsigned long long*)(finished() + 104); }
-    };
-    std::mutex scatter_mu;
-    std::vector<std::unique_ptr<scatter_set>> scatter_sets;
-    uint64_t scatter_clock = 0;
-    /* with scatter_mu held */
-    scatter_set* scatter_for(hipStream_t st, size_t notes_bytes, size_t wanted_bytes)
-    {
-        scatter_set* s = nullptr;
-        for (auto& x : scatter_sets) if (x->st == st) s = x.get();
-        const bool grown = !s || notes_bytes > s->notes_bytes || wanted_bytes > s->wanted_bytes;
-        const relaxed_capture relaxed(grown);
-        if (!s) {
-            if (scatter_sets.size() >= BAM_SCATTER_SETS) {
-                size_t old = 0;
-                for (size_t i = 1; i < scatter_sets.size(); i++) if (scatter_sets[i]->used < scatter_sets[old]->used) old = i;
-                hip_err_chk(hipDeviceSynchronize());
-                scatter_sets.erase(scatter_sets.begin() + (ptrdiff_t)old);
-            }
-            scatter_sets.emplace_back(new scatter_set());
-            s = scatter_sets.back().get();
-            s->st = st;
-            s->words = createBuffer(BAM_SUM_PARTIALS * sizeof(uint64_t) + 512, 0);
-        }
-        s->used = ++scatter_clock;
-        if (notes_bytes > s->notes_bytes) { s->notes = createBuffer(notes_bytes, 0); s->notes_bytes = notes_bytes; }
-        if (wanted_bytes > s->wanted_bytes) { s->wanted = createBuffer(wanted_bytes, 0); s->wanted_bytes = wanted_bytes; }
-        if (grown) hip_err_chk(hipStreamSynchronize(0));        /* cleared on the null stream, which `st` need not wait for */
-        return s;
-    }
+    scratch_sets scratch;
     void* notes_for(size_t bytes)
     {
         if (bytes > notes_bytes) { notes = createBuffer(bytes, 0); notes_bytes = bytes; }
@@ -128,6 +79,23 @@ struct bam_array {
 };
 struct bam_range32 { range_t<uint32_t>* r; };
 struct bam_array32 { array_t<uint32_t>* a; BufferPtr partials; };      /* partials: [BAM_SUM_PARTIALS] checksum shards, zero between launches */
+
+/*
+ * The scratch of a call on `st`, with a->scratch.mu held; NULL where device memory is short: the call then takes a route that
+ * needs none.
+ */
+inline scratch_set* scratch_for(bam_array_t* a, hipStream_t st, size_t notes_bytes, size_t wanted_bytes)
+{
+    const relaxed_capture relaxed(true);
+    bool fresh = false;
+    auto alloc = [&](size_t bytes) -> BufferPtr {
+        fresh = true;
+        try { return createBuffer(bytes, 0); } catch (const std::exception&) { (void)hipGetLastError(); return nullptr; }
+    };
+    scratch_set* s = a->scratch.get(st, notes_bytes, wanted_bytes, alloc, [] { hip_err_chk(hipDeviceSynchronize()); });
+    if (fresh) hip_err_chk(hipStreamSynchronize(0));        /* cleared on the null stream, which `st` need not wait for */
+    return s;
+}
 
 // ---------------------------------------------------------------------------
 // device helpers

@@ -1,0 +1,81 @@
+// What the calls of one array that take several launches keep between the launches, and from call to call.  Host side only,
+// no HIP in here: the memory comes from the caller's allocator (tests/native/test_scratch.cpp hands in one of its own).
+#ifndef __BAM_SCRATCH_SETS_H__
+#define __BAM_SCRATCH_SETS_H__
+#include <cstddef>
+#include <cstdint>
+#include <memory>
+#include <mutex>
+#include <vector>
+
+#define BAM_SUM_PARTIALS 4096
+#define BAM_SCRATCH_SETS 4
+#define BAM_SCRATCH_WORDS_BYTES (BAM_SUM_PARTIALS * sizeof(uint64_t) + 512)
+
+/*
+ * The bits of the requests a first launch leaves, a byte per page of the range that somebody waits for (zero between calls),
+ * checksum shards and the count of finished workgroups.
+ */
+struct scratch_set {
+    void* stream = nullptr;
+    uint64_t used = 0;
+    std::shared_ptr<void> words, notes, wanted;
+    size_t notes_bytes = 0, wanted_bytes = 0;
+    uint32_t calls = 0;
+    std::shared_ptr<void> host_words;       /* [64] in host memory, one per call in turn: the number of a scan that found a page missing */
+    unsigned long long* partials() { return (unsigned long long*)words.get(); }
+    uint32_t* finished() { return (uint32_t*)(partials() + BAM_SUM_PARTIALS); }
+    uint32_t next_call() { if (++calls == 0) calls = 1; return calls; }
+    /* the word the computing workgroups of a reduction count themselves off in for the fetching ones */
+    unsigned long long* done() { return (unsigned long long*)(finished() + 104); }
+};
+
+/*
+ * One set per stream, because the launches of two calls on one stream run one after the other and those on two streams do
+ * not; the set is picked and its launches are queued under the mutex, so the calls of two threads on one stream do not mix.
+ * At most BAM_SCRATCH_SETS sets are kept: the one longest unused makes room, and all go with the array.
+ */
+struct scratch_sets {
+    std::mutex mu;
+    std::vector<std::unique_ptr<scratch_set>> sets;
+    uint64_t clock = 0;
+    /*
+     * The set of `stream` with at least these sizes, with `mu` held; NULL where the memory is refused, and then the caller
+     * takes a route that needs none.  alloc(bytes) gives zeroed memory or NULL; idle() returns when nothing queued so far
+     * still runs.  A set is entered once all of it is there, and a buffer changes place with a larger one that is there.
+     */
+    template <typename Alloc, typename Idle>
+    scratch_set* get(void* stream, size_t notes_bytes, size_t wanted_bytes, Alloc&& alloc, Idle&& idle)
+    {
+        scratch_set* s = nullptr;
+        for (auto& x : sets) if (x->stream == stream) s = x.get();
+        if (!s) {
+            std::unique_ptr<scratch_set> made(new scratch_set());
+            made->stream = stream;
+            if (!(made->words = alloc(BAM_SCRATCH_WORDS_BYTES))) return nullptr;
+            if (sets.size() >= BAM_SCRATCH_SETS) {
+                size_t old = 0;
+                for (size_t i = 1; i < sets.size(); i++) if (sets[i]->used < sets[old]->used) old = i;
+                idle();
+                sets.erase(sets.begin() + (ptrdiff_t)old);
+            }
+            sets.push_back(std::move(made));
+            s = sets.back().get();
+        }
+        s->used = ++clock;
+        return grown(s->notes, s->notes_bytes, notes_bytes, alloc) && grown(s->wanted, s->wanted_bytes, wanted_bytes, alloc) ? s : nullptr;
+    }
+
+private:
+    template <typename Alloc>
+    static bool grown(std::shared_ptr<void>& buf, size_t& have, size_t bytes, Alloc& alloc)
+    {
+        if (bytes <= have) return true;
+        std::shared_ptr<void> larger = alloc(bytes);
+        if (!larger) return false;
+        buf = larger;
+        have = bytes;
+        return true;
+    }
+};
+#endif /* __BAM_SCRATCH_SETS_H__ */

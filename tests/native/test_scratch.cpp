@@ -1,0 +1,54 @@
+// Checks of what calls in several launches keep between them (bam_amd/csrc/scratch_sets.h), with an allocator that can be made
+// to refuse.  No GPU.  Prints "ok <name>" per check; exit 0 = all passed.
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <map>
+#include "scratch_sets.h"
+
+static int failures = 0;
+#define CHECK(name, cond) do { if (cond) printf("ok %s\n", name); else { printf("FAIL %s (%s:%d)\n", name, __FILE__, __LINE__); failures++; } } while (0)
+
+struct Memory {
+    int allocs = 0, frees = 0, refuse_from = -1;
+    std::map<void*, size_t> live;
+    std::shared_ptr<void> operator()(size_t bytes)
+    {
+        if (refuse_from >= 0 && allocs >= refuse_from) return nullptr;
+        allocs++;
+        void* p = calloc(1, bytes);
+        live[p] = bytes;
+        return std::shared_ptr<void>(p, [this](void* q) { live.erase(q); frees++; free(q); });
+    }
+    bool holds(const std::shared_ptr<void>& b, size_t bytes) const { auto it = live.find(b.get()); return it != live.end() && it->second >= bytes; }
+};
+static void* stream(uintptr_t k) { return (void*)(0x1000 * k); }
+static bool whole(const Memory& m, scratch_set* s, size_t notes, size_t wanted)
+{
+    return s && m.holds(s->words, BAM_SCRATCH_WORDS_BYTES) && m.holds(s->notes, notes) && (!wanted || m.holds(s->wanted, wanted));
+}
+
+int main()
+{
+    auto idle = [] {};
+    /* a refusal at every place a call can meet one: the call gets nothing, and the next one a whole set */
+    for (int at = 0; at < 3; at++) {
+        Memory mem;
+        {
+            scratch_sets sets;
+            auto alloc = [&](size_t b) { return mem(b); };
+            mem.refuse_from = at;
+            scratch_set* s = sets.get(stream(1), 4096, 512, alloc, idle);
+            CHECK("refused: nothing", s == nullptr);
+            mem.refuse_from = -1;
+            s = sets.get(stream(1), 4096, 512, alloc, idle);
+            CHECK("then a whole set", whole(mem, s, 4096, 512));
+            mem.refuse_from = mem.allocs;
+            CHECK("a larger call is refused", sets.get(stream(1), 8192, 512, alloc, idle) == nullptr);
+            CHECK("and the smaller still has its set", sets.get(stream(1), 4096, 512, alloc, idle) == s && whole(mem, s, 4096, 512));
+        }
+        CHECK("all is given back", mem.live.empty() && mem.frees == mem.allocs);
+    }
+    printf(failures ? "FAILED\n" : "PASSED\n");
+    return failures != 0;
+}

@@ -18,6 +18,14 @@ def test_native_host_checks(tmp_path):
     assert len(oks) >= 40 and "PASSED" in r.stdout
 
 
+def test_scratch_between_launches(tmp_path):
+    exe = tmp_path / "test_scratch"
+    subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-I", os.path.join(ROOT, "bam_amd", "csrc"),
+                    os.path.join(ROOT, "tests", "native", "test_scratch.cpp"), "-o", str(exe), "-lpthread"], check=True)
+    r = subprocess.run([str(exe)], capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0 and "PASSED" in r.stdout, r.stdout + r.stderr
+
+
 def test_program_against_the_cpp_surface_builds():
     """bam_amd/examples/array_sum.hip uses Controller / page_cache_t / range_t / array_t / array_d_t / bam_ptr the way
     the reference's benchmarks do; it has to compile for gfx950 and link against the library (no GPU needed for that)"""
