@@ -92,7 +92,7 @@ inline scratch_set* scratch_for(bam_array_t* a, hipStream_t st, size_t notes_byt
         fresh = true;
         try { return createBuffer(bytes, 0); } catch (const std::exception&) { (void)hipGetLastError(); return nullptr; }
     };
-    scratch_set* s = a->scratch.get(st, notes_bytes, wanted_bytes, alloc, [] { hip_err_chk(hipDeviceSynchronize()); });
+    scratch_set* s = a->scratch.get(st, st == hipStreamPerThread ? scratch_thread_number() : 0, notes_bytes, wanted_bytes, alloc, [] { hip_err_chk(hipDeviceSynchronize()); });
     if (fresh) hip_err_chk(hipStreamSynchronize(0));        /* cleared on the null stream, which `st` need not wait for */
     return s;
 }

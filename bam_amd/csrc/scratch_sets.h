@@ -2,6 +2,7 @@
 // no HIP in here: the memory comes from the caller's allocator (tests/native/test_scratch.cpp hands in one of its own).
 #ifndef __BAM_SCRATCH_SETS_H__
 #define __BAM_SCRATCH_SETS_H__
+#include <atomic>
 #include <cstddef>
 #include <cstdint>
 #include <memory>
@@ -18,6 +19,7 @@
  */
 struct scratch_set {
     void* stream = nullptr;
+    uint64_t thread = 0;
     uint64_t used = 0;
     std::shared_ptr<void> words, notes, wanted;
     size_t notes_bytes = 0, wanted_bytes = 0;
@@ -30,9 +32,19 @@ struct scratch_set {
     unsigned long long* done() { return (unsigned long long*)(finished() + 104); }
 };
 
+/* a number of the calling thread's own, given out once in the life of the process (the number of a thread that has ended may
+ * not come back: its work may still run) */
+inline uint64_t scratch_thread_number()
+{
+    static std::atomic<uint64_t> last{0};
+    thread_local const uint64_t mine = ++last;
+    return mine;
+}
+
 /*
  * One set per stream, because the launches of two calls on one stream run one after the other and those on two streams do
  * not; the set is picked and its launches are queued under the mutex, so the calls of two threads on one stream do not mix.
+ * One handle, hipStreamPerThread, names another stream in each thread: its sets belong to the thread as well.
  * At most BAM_SCRATCH_SETS sets are kept: the one longest unused makes room, and all go with the array.
  */
 struct scratch_sets {
@@ -40,18 +52,19 @@ struct scratch_sets {
     std::vector<std::unique_ptr<scratch_set>> sets;
     uint64_t clock = 0;
     /*
-     * The set of `stream` with at least these sizes, with `mu` held; NULL where the memory is refused, and then the caller
+     * The set of `stream` (and of `thread`, 0 where the handle names one stream everywhere) with at least these sizes, with `mu` held; NULL where the memory is refused, and then the caller
      * takes a route that needs none.  alloc(bytes) gives zeroed memory or NULL; idle() returns when nothing queued so far
      * still runs.  A set is entered once all of it is there, and a buffer changes place with a larger one that is there.
      */
     template <typename Alloc, typename Idle>
-    scratch_set* get(void* stream, size_t notes_bytes, size_t wanted_bytes, Alloc&& alloc, Idle&& idle)
+    scratch_set* get(void* stream, uint64_t thread, size_t notes_bytes, size_t wanted_bytes, Alloc&& alloc, Idle&& idle)
     {
         scratch_set* s = nullptr;
-        for (auto& x : sets) if (x->stream == stream) s = x.get();
+        for (auto& x : sets) if (x->stream == stream && x->thread == thread) s = x.get();
         if (!s) {
             std::unique_ptr<scratch_set> made(new scratch_set());
             made->stream = stream;
+            made->thread = thread;
             if (!(made->words = alloc(BAM_SCRATCH_WORDS_BYTES))) return nullptr;
             if (sets.size() >= BAM_SCRATCH_SETS) {
                 size_t old = 0;

@@ -4,6 +4,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <map>
+#include <thread>
 #include "scratch_sets.h"
 
 static int failures = 0;
@@ -38,16 +39,35 @@ int main()
             scratch_sets sets;
             auto alloc = [&](size_t b) { return mem(b); };
             mem.refuse_from = at;
-            scratch_set* s = sets.get(stream(1), 4096, 512, alloc, idle);
+            scratch_set* s = sets.get(stream(1), 0, 4096, 512, alloc, idle);
             CHECK("refused: nothing", s == nullptr);
             mem.refuse_from = -1;
-            s = sets.get(stream(1), 4096, 512, alloc, idle);
+            s = sets.get(stream(1), 0, 4096, 512, alloc, idle);
             CHECK("then a whole set", whole(mem, s, 4096, 512));
             mem.refuse_from = mem.allocs;
-            CHECK("a larger call is refused", sets.get(stream(1), 8192, 512, alloc, idle) == nullptr);
-            CHECK("and the smaller still has its set", sets.get(stream(1), 4096, 512, alloc, idle) == s && whole(mem, s, 4096, 512));
+            CHECK("a larger call is refused", sets.get(stream(1), 0, 8192, 512, alloc, idle) == nullptr);
+            CHECK("and the smaller still has its set", sets.get(stream(1), 0, 4096, 512, alloc, idle) == s && whole(mem, s, 4096, 512));
         }
         CHECK("all is given back", mem.live.empty() && mem.frees == mem.allocs);
+    }
+    /* one handle that is another stream in each thread: two threads share nothing, each finds its own again */
+    {
+        Memory mem;
+        scratch_sets sets;
+        auto alloc = [&](size_t b) { return mem(b); };
+        scratch_set* got[2][2] = {};
+        uint64_t number[2] = {};
+        for (int k = 0; k < 2; k++)
+            std::thread([&] {
+                number[k] = scratch_thread_number();
+                for (int rep = 0; rep < 2; rep++) {
+                    std::lock_guard<std::mutex> guard(sets.mu);
+                    got[k][rep] = sets.get((void*)2, scratch_thread_number(), 1024, 512, alloc, idle);
+                }
+            }).join();
+        CHECK("threads have numbers of their own", number[0] != number[1] && number[0] && number[1]);
+        CHECK("each thread finds its set again", got[0][0] == got[0][1] && got[1][0] == got[1][1]);
+        CHECK("threads share no set", got[0][0] != got[1][0] && got[0][0]->notes != got[1][0]->notes && got[0][0]->words != got[1][0]->words && got[0][0]->wanted != got[1][0]->wanted);
     }
     printf(failures ? "FAILED\n" : "PASSED\n");
     return failures != 0;

@@ -54,3 +54,46 @@ def test_captured_reads_hold_nothing_of_the_array(bam, cache_pages, shape):
                 torch.cuda.synchronize()
                 assert int(other.item()) & (2 ** 64 - 1) == want_all, rep
         assert not r.c.aborted()
+
+
+def test_two_threads_on_the_stream_of_each_thread(bam):
+    """hipStreamPerThread is one handle and another stream in each thread: gathers, reductions and scans of two threads on one
+    array larger than its cache, and on one that fits, each thread with requests of its own"""
+    import threading
+    import torch
+    per_thread = ctypes.c_void_p(2)
+    n = (1 << 20) + 5
+    for pages, cache_pages in ((9000, 4096), (4096, 4096)):
+        n_elems = pages * 512
+        words = oracle.store(SEED, 0, n_elems)
+        with Rig(bam, pages * 4096, n_queues=16, depth=256) as r:
+            a = r.array(n_elems, 4096, cache_pages)
+            reqs = [np.random.default_rng(k).integers(0, n_elems, n).astype(np.uint64) for k in range(2)]
+            d = [_dev(x) for x in reqs]
+            outs = [[torch.zeros(n, dtype=torch.int64, device="cuda") for _ in range(3)] for _ in range(2)]
+            sums = [torch.zeros(n_elems // 128, dtype=torch.int64, device="cuda") for _ in range(2)]
+            runs = [torch.zeros(n_elems + 2, dtype=torch.int64, device="cuda") for _ in range(2)]
+            torch.cuda.synchronize()
+            rcs, start = [[], []], threading.Barrier(2)
+
+            def work(k):
+                torch.cuda.set_device(0)
+                start.wait()
+                for o in outs[k]:
+                    rcs[k].append(a.L.bam_array_gather(a.h, n, ctypes.c_void_p(d[k].data_ptr()), 0, 64, ctypes.c_void_p(o.data_ptr()), per_thread))
+                rcs[k].append(a.L.bam_reduce(a.h, n_elems - k, 64, ctypes.c_void_p(sums[k].data_ptr()), per_thread))
+                rcs[k].append(a.L.bam_scan(a.h, n_elems - k, 64, ctypes.c_void_p(runs[k].data_ptr()), per_thread))
+
+            threads = [threading.Thread(target=work, args=(k,)) for k in range(2)]
+            for t in threads:
+                t.start()
+            for t in threads:
+                t.join()
+            torch.cuda.synchronize()
+            assert rcs == [[0] * 5] * 2
+            for k in range(2):
+                for o in outs[k]:
+                    assert np.array_equal(_u64(o), words[reqs[k].astype(np.int64)]), (pages, k)
+                assert np.array_equal(_u64(sums[k]), oracle.reduce_blocks(words[:n_elems - k], 64)), (pages, k)
+                assert np.array_equal(_u64(runs[k])[:n_elems - k + 1], oracle.scan(words[:n_elems - k])), (pages, k)
+            assert not r.c.aborted()
