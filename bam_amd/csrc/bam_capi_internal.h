@@ -41,12 +41,11 @@ std::string& bam_err();            /* message of the last failure on the calling
 static inline int fail(int code, const char* msg) { g_err = msg; return code; }
 static inline int fail(int code, const std::string& msg) { g_err = msg; return code; }
 
-/* lets the calling thread allocate and synchronise while some other stream of the process is being captured */
+/* lets the calling thread allocate while some other stream of the process is being captured */
 struct relaxed_capture {
     hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
-    bool on;
-    explicit relaxed_capture(bool on_) : on(on_) { if (on) (void)hipThreadExchangeStreamCaptureMode(&mode); }
-    ~relaxed_capture() { if (on) (void)hipThreadExchangeStreamCaptureMode(&mode); }
+    relaxed_capture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+    ~relaxed_capture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
 };
 
 struct bam_target {
@@ -81,20 +80,20 @@ struct bam_range32 { range_t<uint32_t>* r; };
 struct bam_array32 { array_t<uint32_t>* a; BufferPtr partials; };      /* partials: [BAM_SUM_PARTIALS] checksum shards, zero between launches */
 
 /*
- * The scratch of a call on `st`, with a->scratch.mu held; NULL where device memory is short: the call then takes a route that
- * needs none.
+ * The scratch of a call on `st`, with a->scratch.mu held; NULL where device memory is short or too many streams have called:
+ * the call then takes a route that needs none.  Nothing here waits for the device.
  */
 inline scratch_set* scratch_for(bam_array_t* a, hipStream_t st, size_t notes_bytes, size_t wanted_bytes)
 {
-    const relaxed_capture relaxed(true);
-    bool fresh = false;
     auto alloc = [&](size_t bytes) -> BufferPtr {
-        fresh = true;
-        try { return createBuffer(bytes, 0); } catch (const std::exception&) { (void)hipGetLastError(); return nullptr; }
+        const relaxed_capture relaxed;
+        void* p = nullptr;
+        if (hipMalloc(&p, bytes) != hipSuccess) { (void)hipGetLastError(); return nullptr; }
+        BufferPtr b(p, [](void* q) { (void)hipFree(q); });
+        hip_err_chk(hipMemsetAsync(p, 0, bytes, st));       /* never on a stream that is being captured: those calls take no scratch */
+        return b;
     };
-    scratch_set* s = a->scratch.get(st, st == hipStreamPerThread ? scratch_thread_number() : 0, notes_bytes, wanted_bytes, alloc, [] { hip_err_chk(hipDeviceSynchronize()); });
-    if (fresh) hip_err_chk(hipStreamSynchronize(0));        /* cleared on the null stream, which `st` need not wait for */
-    return s;
+    return a->scratch.get(st, st == hipStreamPerThread ? scratch_thread_number() : 0, notes_bytes, wanted_bytes, alloc);
 }
 
 // ---------------------------------------------------------------------------

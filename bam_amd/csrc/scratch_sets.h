@@ -10,7 +10,7 @@
 #include <vector>
 
 #define BAM_SUM_PARTIALS 4096
-#define BAM_SCRATCH_SETS 4
+#define BAM_SCRATCH_SETS 64
 #define BAM_SCRATCH_WORDS_BYTES (BAM_SUM_PARTIALS * sizeof(uint64_t) + 512)
 
 /*
@@ -20,7 +20,6 @@
 struct scratch_set {
     void* stream = nullptr;
     uint64_t thread = 0;
-    uint64_t used = 0;
     std::shared_ptr<void> words, notes, wanted;
     size_t notes_bytes = 0, wanted_bytes = 0;
     uint32_t calls = 0;
@@ -45,49 +44,49 @@ inline uint64_t scratch_thread_number()
  * One set per stream, because the launches of two calls on one stream run one after the other and those on two streams do
  * not; the set is picked and its launches are queued under the mutex, so the calls of two threads on one stream do not mix.
  * One handle, hipStreamPerThread, names another stream in each thread: its sets belong to the thread as well.
- * At most BAM_SCRATCH_SETS sets are kept: the one longest unused makes room, and all go with the array.
+ * A set stays where it is until the array goes, and so does a buffer that a larger one has replaced (the larger one is twice
+ * its size or more, so that all of them together are no larger than the last): launches that use them may still be queued, and
+ * to wait for them would hold up every stream of the device.  BAM_SCRATCH_SETS bounds the sets; a stream for which none is left
+ * takes the routes that need none.
  */
 struct scratch_sets {
     std::mutex mu;
     std::vector<std::unique_ptr<scratch_set>> sets;
-    uint64_t clock = 0;
+    std::vector<std::shared_ptr<void>> replaced;
     /*
      * The set of `stream` (and of `thread`, 0 where the handle names one stream everywhere) with at least these sizes, with `mu` held; NULL where the memory is refused, and then the caller
-     * takes a route that needs none.  alloc(bytes) gives zeroed memory or NULL; idle() returns when nothing queued so far
-     * still runs.  A set is entered once all of it is there, and a buffer changes place with a larger one that is there.
+     * takes a route that needs none.  alloc(bytes) gives memory that is zero to what is queued on `stream` from now on, or NULL.
+     * A set is entered once all of it is there, and a buffer changes place with a larger one that is there.
      */
-    template <typename Alloc, typename Idle>
-    scratch_set* get(void* stream, uint64_t thread, size_t notes_bytes, size_t wanted_bytes, Alloc&& alloc, Idle&& idle)
+    template <typename Alloc>
+    scratch_set* get(void* stream, uint64_t thread, size_t notes_bytes, size_t wanted_bytes, Alloc&& alloc)
     {
         scratch_set* s = nullptr;
         for (auto& x : sets) if (x->stream == stream && x->thread == thread) s = x.get();
+        if (!s && sets.size() >= BAM_SCRATCH_SETS) return nullptr;
         if (!s) {
             std::unique_ptr<scratch_set> made(new scratch_set());
             made->stream = stream;
             made->thread = thread;
             if (!(made->words = alloc(BAM_SCRATCH_WORDS_BYTES))) return nullptr;
-            if (sets.size() >= BAM_SCRATCH_SETS) {
-                size_t old = 0;
-                for (size_t i = 1; i < sets.size(); i++) if (sets[i]->used < sets[old]->used) old = i;
-                idle();
-                sets.erase(sets.begin() + (ptrdiff_t)old);
-            }
             sets.push_back(std::move(made));
             s = sets.back().get();
         }
-        s->used = ++clock;
         return grown(s->notes, s->notes_bytes, notes_bytes, alloc) && grown(s->wanted, s->wanted_bytes, wanted_bytes, alloc) ? s : nullptr;
     }
 
 private:
     template <typename Alloc>
-    static bool grown(std::shared_ptr<void>& buf, size_t& have, size_t bytes, Alloc& alloc)
+    bool grown(std::shared_ptr<void>& buf, size_t& have, size_t bytes, Alloc& alloc)
     {
         if (bytes <= have) return true;
-        std::shared_ptr<void> larger = alloc(bytes);
+        size_t size = bytes < 2 * have ? 2 * have : bytes;
+        std::shared_ptr<void> larger = alloc(size);
+        if (!larger && size > bytes) larger = alloc(size = bytes);
         if (!larger) return false;
+        if (buf) replaced.push_back(buf);
         buf = larger;
-        have = bytes;
+        have = size;
         return true;
     }
 };

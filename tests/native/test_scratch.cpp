@@ -31,7 +31,6 @@ static bool whole(const Memory& m, scratch_set* s, size_t notes, size_t wanted)
 
 int main()
 {
-    auto idle = [] {};
     /* a refusal at every place a call can meet one: the call gets nothing, and the next one a whole set */
     for (int at = 0; at < 3; at++) {
         Memory mem;
@@ -39,14 +38,14 @@ int main()
             scratch_sets sets;
             auto alloc = [&](size_t b) { return mem(b); };
             mem.refuse_from = at;
-            scratch_set* s = sets.get(stream(1), 0, 4096, 512, alloc, idle);
+            scratch_set* s = sets.get(stream(1), 0, 4096, 512, alloc);
             CHECK("refused: nothing", s == nullptr);
             mem.refuse_from = -1;
-            s = sets.get(stream(1), 0, 4096, 512, alloc, idle);
+            s = sets.get(stream(1), 0, 4096, 512, alloc);
             CHECK("then a whole set", whole(mem, s, 4096, 512));
             mem.refuse_from = mem.allocs;
-            CHECK("a larger call is refused", sets.get(stream(1), 0, 8192, 512, alloc, idle) == nullptr);
-            CHECK("and the smaller still has its set", sets.get(stream(1), 0, 4096, 512, alloc, idle) == s && whole(mem, s, 4096, 512));
+            CHECK("a larger call is refused", sets.get(stream(1), 0, 8192, 512, alloc) == nullptr);
+            CHECK("and the smaller still has its set", sets.get(stream(1), 0, 4096, 512, alloc) == s && whole(mem, s, 4096, 512));
         }
         CHECK("all is given back", mem.live.empty() && mem.frees == mem.allocs);
     }
@@ -62,12 +61,40 @@ int main()
                 number[k] = scratch_thread_number();
                 for (int rep = 0; rep < 2; rep++) {
                     std::lock_guard<std::mutex> guard(sets.mu);
-                    got[k][rep] = sets.get((void*)2, scratch_thread_number(), 1024, 512, alloc, idle);
+                    got[k][rep] = sets.get((void*)2, scratch_thread_number(), 1024, 512, alloc);
                 }
             }).join();
         CHECK("threads have numbers of their own", number[0] != number[1] && number[0] && number[1]);
         CHECK("each thread finds its set again", got[0][0] == got[0][1] && got[1][0] == got[1][1]);
         CHECK("threads share no set", got[0][0] != got[1][0] && got[0][0]->notes != got[1][0]->notes && got[0][0]->words != got[1][0]->words && got[0][0]->wanted != got[1][0]->wanted);
+    }
+    /* streams by turns: after the first round nothing is allocated and nothing moves; a buffer that was replaced is still
+     * there (its launches may be queued); beyond the bound a stream gets nothing, and the others keep what they have */
+    {
+        Memory mem;
+        {
+            scratch_sets sets;
+            auto alloc = [&](size_t b) { return mem(b); };
+            std::shared_ptr<void> first[8];
+            for (uintptr_t k = 0; k < 8; k++) first[k] = sets.get(stream(k + 1), 0, 1000 + k, 512, alloc)->notes;
+            const int allocs = mem.allocs;
+            bool same = true;
+            for (int rep = 0; rep < 3; rep++)
+                for (uintptr_t k = 0; k < 8; k++) same &= sets.get(stream(k + 1), 0, 1000, 512, alloc)->notes == first[k];
+            CHECK("eight streams by turns allocate once", same && mem.allocs == allocs && mem.frees == 0);
+            void* const before = first[0].get();
+            first[0].reset();
+            scratch_set* s = sets.get(stream(1), 0, 1001, 512, alloc);
+            CHECK("a larger buffer is twice the size, the smaller one stays", whole(mem, s, 2000, 512) && s->notes.get() != before && mem.live.count(before) && mem.frees == 0);
+            mem.refuse_from = mem.allocs;
+            CHECK("refused: the set keeps what it has", sets.get(stream(1), 0, 5000, 512, alloc) == nullptr && sets.get(stream(1), 0, 2000, 512, alloc) == s);
+            mem.refuse_from = -1;
+            for (uintptr_t k = 8; k < BAM_SCRATCH_SETS; k++) sets.get(stream(k + 1), 0, 64, 0, alloc);
+            const int full = mem.allocs;
+            CHECK("no set beyond the bound", sets.get(stream(BAM_SCRATCH_SETS + 1), 0, 64, 0, alloc) == nullptr && mem.allocs == full);
+            CHECK("the others keep theirs", sets.get(stream(1), 0, 64, 0, alloc) == s && sets.get(stream(BAM_SCRATCH_SETS), 0, 64, 0, alloc) && mem.frees == 0);
+        }
+        CHECK("all is given back", mem.live.empty());
     }
     printf(failures ? "FAILED\n" : "PASSED\n");
     return failures != 0;

@@ -97,3 +97,40 @@ def test_two_threads_on_the_stream_of_each_thread(bam):
                 assert np.array_equal(_u64(sums[k]), oracle.reduce_blocks(words[:n_elems - k], 64)), (pages, k)
                 assert np.array_equal(_u64(runs[k])[:n_elems - k + 1], oracle.scan(words[:n_elems - k])), (pages, k)
             assert not r.c.aborted()
+
+
+def test_many_streams_by_turns(bam):
+    """gathers and reductions on seventy streams by turns, more than sets of scratch are kept for: a second round allocates
+    nothing, and every result is right"""
+    import torch
+    pages = 4400
+    n_elems = pages * 512
+    words = oracle.store(SEED, 0, n_elems)
+    with Rig(bam, pages * 4096, n_queues=16, depth=256) as r:
+        a = r.array(n_elems, 4096, pages)
+        d = [_dev(np.random.default_rng(k).integers(0, n_elems, (1 << 20) + k).astype(np.uint64)) for k in range(8)]
+        torch.cuda.synchronize()
+        made = (ctypes.c_void_p * 70)()
+        hip = ctypes.CDLL("libamdhip64.so.7")
+        for k in range(70):
+            assert hip.hipStreamCreateWithFlags(ctypes.byref(made, 8 * k), 1) == 0
+        sums = torch.zeros((70, n_elems // 128), dtype=torch.int64, device="cuda")
+        outs = [torch.zeros(x.numel(), dtype=torch.int64, device="cuda") for x in d]
+        torch.cuda.synchronize()
+        for rep in range(2):
+            for k in range(70):
+                st = ctypes.c_void_p(made[k])
+                assert a.L.bam_array_gather(a.h, d[k % 8].numel(), ctypes.c_void_p(d[k % 8].data_ptr()), 0, 64, ctypes.c_void_p(outs[k % 8].data_ptr()), st) == 0
+                assert a.L.bam_reduce(a.h, n_elems, 64, ctypes.c_void_p(sums[k].data_ptr()), st) == 0
+            if rep == 0:
+                torch.cuda.synchronize()
+                free = torch.cuda.mem_get_info()[0]
+        torch.cuda.synchronize()
+        assert torch.cuda.mem_get_info()[0] == free
+        want = oracle.reduce_blocks(words, 64)
+        assert np.array_equal(_u64(sums), np.broadcast_to(want, (70, len(want))))
+        for x, o in zip(d, outs):
+            assert np.array_equal(_u64(o), words[x.cpu().numpy()])
+        for k in range(70):
+            assert hip.hipStreamDestroy(ctypes.c_void_p(made[k])) == 0
+        assert not r.c.aborted()
