@@ -1441,6 +1441,7 @@ int bam_array_create(bam_array_t** out, uint64_t n_elems, uint64_t disk_start_of
     std::vector<range_t<uint64_t>*> rs;
     for (uint32_t i = 0; i < n_ranges; i++) rs.push_back(ranges[i]->r);
     *out = new bam_array{new array_t<uint64_t>(n_elems, disk_start_offset, rs, device), createBuffer(BAM_SUM_PARTIALS * sizeof(uint64_t), device)};
+    (*out)->device = (int)device;
     BAM_API_END
 }
 

@@ -68,6 +68,7 @@ struct bam_array {
     size_t notes_bytes = 0;
     uint32_t calls = 0;
     scratch_sets scratch;
+    int device = 0;                     /* where the array lives, and its scratch with it */
     void* notes_for(size_t bytes)
     {
         if (bytes > notes_bytes) { notes = createBuffer(bytes, 0); notes_bytes = bytes; }
@@ -81,17 +82,26 @@ struct bam_array32 { array_t<uint32_t>* a; BufferPtr partials; };      /* partia
 
 /*
  * The scratch of a call on `st`, with a->scratch.mu held; NULL where device memory is short or too many streams have called:
- * the call then takes a route that needs none.  Nothing here waits for the device.
+ * the call then takes a route that needs none.  It lies on the array's device, and the caller's current device stays as it is.
+ * Nothing here waits, unless those two differ and memory has to be cleared.
  */
 inline scratch_set* scratch_for(bam_array_t* a, hipStream_t st, size_t notes_bytes, size_t wanted_bytes)
 {
     auto alloc = [&](size_t bytes) -> BufferPtr {
         const relaxed_capture relaxed;
+        int current = a->device;
+        (void)hipGetDevice(&current);
+        const bool elsewhere = current != a->device;
         void* p = nullptr;
-        if (hipMalloc(&p, bytes) != hipSuccess) { (void)hipGetLastError(); return nullptr; }
-        BufferPtr b(p, [](void* q) { (void)hipFree(q); });
-        hip_err_chk(hipMemsetAsync(p, 0, bytes, st));       /* never on a stream that is being captured: those calls take no scratch */
-        return b;
+        if (elsewhere && hipSetDevice(a->device) != hipSuccess) { (void)hipGetLastError(); return nullptr; }
+        hipError_t e = hipMalloc(&p, bytes);
+        /* never on a stream that is being captured: those calls take no scratch.  `st` may be the null stream of the caller's
+         * device, which does not wait for this one's */
+        if (e == hipSuccess) e = elsewhere ? hipMemset(p, 0, bytes) : hipMemsetAsync(p, 0, bytes, st);
+        if (e == hipSuccess && elsewhere) e = hipStreamSynchronize(0);
+        if (elsewhere) (void)hipSetDevice(current);
+        if (e != hipSuccess) { (void)hipGetLastError(); if (p) (void)hipFree(p); return nullptr; }
+        return BufferPtr(p, [](void* q) { (void)hipFree(q); });
     };
     return a->scratch.get(st, st == hipStreamPerThread ? scratch_thread_number() : 0, notes_bytes, wanted_bytes, alloc);
 }
