@@ -266,6 +266,7 @@ __global__ void k_scan_ptr_pc(array_d_t<uint64_t>* da, unsigned long long* outpu
  * A page that is not resident: the wave tells the second launch and the host, which then runs the kernels that can miss.
  */
 #define BAM_CHUNK_WAVES 8u
+#define BAM_COUNTED_WORD 98u      /* of the scratch's words: the call whose accesses were counted */
 __device__ __forceinline__ void scan_gives_up(uint32_t* finished, const uint32_t call, volatile uint32_t* host_left)
 {
     if (bam::lane() == 0 && __hip_atomic_load(finished + BAM_LEFT_WORD, __ATOMIC_RELAXED, BAM_AGENT) != call &&
@@ -352,7 +353,17 @@ __global__ __launch_bounds__(BAM_CHUNK_WAVES * BAM_WAVE_SIZE) void k_scan_write(
         bam_stat_shard_t* const sh = view.r->shard();
         __hip_atomic_fetch_add(&sh->access_cnt, (unsigned long long)n_access, __ATOMIC_RELAXED, BAM_AGENT);
         __hip_atomic_fetch_add(&sh->hit_cnt, (unsigned long long)n_access, __ATOMIC_RELAXED, BAM_AGENT);
+        finished[BAM_COUNTED_WORD] = call;
     }
+}
+/* behind a k_scan_write of which some wave gave up: the kernels that can miss count the whole scan, so what its first
+ * workgroup counted (it does not wait for the others) is taken off again */
+__global__ void k_scan_uncount(array_d_t<uint64_t>* da, const uint32_t* finished, const uint32_t call, const uint64_t n_access)
+{
+    if (finished[BAM_COUNTED_WORD] != call) return;
+    bam_stat_shard_t* const sh = da->d_ranges->shard();
+    __hip_atomic_fetch_add(&sh->access_cnt, 0ull - n_access, __ATOMIC_RELAXED, BAM_AGENT);
+    __hip_atomic_fetch_add(&sh->hit_cnt, 0ull - n_access, __ATOMIC_RELAXED, BAM_AGENT);
 }
 
 /* one block: v[i] = v[0] + ... + v[i] in place (the reference calls cub::DeviceScan::InclusiveSum here, scan/main.cu:416-418) */
@@ -423,12 +434,53 @@ uint64_t paired_accesses(uint64_t n, uint64_t half, uint64_t page_elems)
     return total;
 }
 
+/*
+ * A word in host memory that the device can write, one call's own for as long as it lasts: a scan waits for its result, and
+ * finds there whether it is whole.  Page-locked memory takes far longer to get than a scan does, so the words are kept for the
+ * next call, whichever array or thread makes it; there are as many as calls were ever waiting at a time, in steps of 64.  A
+ * word that launches may still write (the wait failed) is not given back.  `at` is NULL where no memory is to be had.
+ */
+struct host_word {
+    volatile uint32_t* at = nullptr;
+    bool idle = true;
+    host_word()
+    {
+        pool& p = shared();
+        std::lock_guard<std::mutex> guard(p.mu);
+        if (p.free.empty()) {
+            const relaxed_capture relaxed;
+            void* mem = nullptr;
+            if (hipHostMalloc(&mem, 64 * sizeof(uint32_t), hipHostMallocMapped | hipHostMallocPortable) != hipSuccess) { (void)hipGetLastError(); return; }
+            for (uint32_t k = 0; k < 64; k++) p.free.push_back((volatile uint32_t*)mem + k);
+        }
+        at = p.free.back();
+        p.free.pop_back();
+        *at = 0;                    /* never the number of a call */
+    }
+    ~host_word()
+    {
+        if (!at || !idle) return;
+        pool& p = shared();
+        std::lock_guard<std::mutex> guard(p.mu);
+        p.free.push_back(at);
+    }
+    host_word(const host_word&) = delete;
+    host_word& operator=(const host_word&) = delete;
+
+private:
+    struct pool { std::mutex mu; std::vector<volatile uint32_t*> free; };
+    static pool& shared() { static pool* p = new pool(); return *p; }      /* never taken down: the runtime may be gone by then */
+};
+
 /* the scan of resident elements; false if some were not, and then the result is not written in full, or if there is no
  * memory for the sums */
 bool scan_resident(bam_array_t* a, uint64_t n_elems, uint32_t block_size, uint64_t* d_result, hipStream_t st)
 {
-    BufferPtr host;
+    host_word left;
+    if (!left.at) return false;
     uint32_t call;
+    uint32_t* finished;
+    const uint64_t n_access = paired_accesses(n_elems, block_size, a->a->h_ranges[0].cache.page_size / 8);
     {
         /* pieces per wave: as many as leave 2048 workgroups, eight at most (a chunk's pieces are looked after by the lanes of a
          * wave); 2^26 elements 312 us, with 512 or 1024 workgroups at least 322, and with stretches of 2^24 elements, small
@@ -438,22 +490,24 @@ bool scan_resident(bam_array_t* a, uint64_t n_elems, uint32_t block_size, uint64
         uint32_t pieces = 1;
         while (pieces < 8 && n_pieces / (BAM_CHUNK_WAVES * pieces * 2) >= 2048) pieces *= 2;
         const uint64_t per_chunk = BAM_CHUNK_WAVES * pieces, n_chunks = (n_pieces + per_chunk - 1) / per_chunk;
-        const uint64_t n_access = paired_accesses(n_elems, block_size, a->a->h_ranges[0].cache.page_size / 8);
         std::lock_guard<std::mutex> guard(a->scratch.mu);
         scratch_set* set = scratch_for(a, st, n_chunks * (per_chunk + 1) * sizeof(uint64_t), 0);
         if (!set) return false;
-        if (!set->host_words) set->host_words = createHostBuffer(64 * sizeof(uint32_t));
-        host = set->host_words;
         call = set->next_call();
-        volatile uint32_t* left = (volatile uint32_t*)host.get() + call % 64;
+        finished = set->finished();
         uint64_t* piece_sums = (uint64_t*)set->notes.get(), *chunk_sums = piece_sums + n_chunks * per_chunk;
         const dim3 grid((uint32_t)n_chunks), block(BAM_CHUNK_WAVES * BAM_WAVE_SIZE);
-        hipLaunchKernelGGL(k_scan_sums, grid, block, 0, st, a->a->d_array_ptr, n_elems, pieces, piece_sums, chunk_sums, set->finished(), call, left);
-        hipLaunchKernelGGL(k_scan_write, grid, block, 0, st, a->a->d_array_ptr, d_result, n_elems, pieces, piece_sums, chunk_sums, set->finished(), call, left, n_access);
+        hipLaunchKernelGGL(k_scan_sums, grid, block, 0, st, a->a->d_array_ptr, n_elems, pieces, piece_sums, chunk_sums, finished, call, left.at);
+        hipLaunchKernelGGL(k_scan_write, grid, block, 0, st, a->a->d_array_ptr, d_result, n_elems, pieces, piece_sums, chunk_sums, finished, call, left.at, n_access);
         hip_err_chk(hipGetLastError());
     }
-    hip_err_chk(hipStreamSynchronize(st));
-    return ((volatile uint32_t*)host.get())[call % 64] != call;
+    const hipError_t e = hipStreamSynchronize(st);
+    left.idle = e == hipSuccess;
+    hip_err_chk(e);
+    if (*left.at != call) return true;
+    hipLaunchKernelGGL(k_scan_uncount, dim3(1), dim3(1), 0, st, a->a->d_array_ptr, finished, call, n_access);
+    hip_err_chk(hipGetLastError());
+    return false;
 }
 
 } // namespace

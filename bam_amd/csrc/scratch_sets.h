@@ -23,7 +23,6 @@ struct scratch_set {
     std::shared_ptr<void> words, notes, wanted;
     size_t notes_bytes = 0, wanted_bytes = 0;
     uint32_t calls = 0;
-    std::shared_ptr<void> host_words;       /* [64] in host memory, one per call in turn: the number of a scan that found a page missing */
     unsigned long long* partials() { return (unsigned long long*)words.get(); }
     uint32_t* finished() { return (uint32_t*)(partials() + BAM_SUM_PARTIALS); }
     uint32_t next_call() { if (++calls == 0) calls = 1; return calls; }

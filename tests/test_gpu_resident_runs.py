@@ -78,3 +78,45 @@ def test_runs_on_several_streams_and_results_at_odd_addresses(bam):
         assert a.L.bam_scan(a.h, n, 256, ctypes.c_void_p(out.data_ptr() + 8), None) == 0
         torch.cuda.synchronize()
         assert np.array_equal(_u64(out[1:]), oracle.scan(vals)) and not r.c.aborted()
+
+
+def test_scans_while_another_array_evicts(bam):
+    """pages leave before, between and during the launches of a scan: another array of the same cache is gathered from on a second
+    stream, a different while after the scan is queued each time.  Every scan is right, and counts what it reads once, whichever
+    kernels end up doing it"""
+    import torch
+    from bam_amd import Array, PageCache, Range
+    pages, other = 65536, 65536
+    n, n_b = pages * 512 - 3, other * 512
+    n_access = _accesses(n, 64, 512)
+    with Rig(bam, (pages + other) * 4096, n_queues=16, depth=256) as r:
+        pc = PageCache(4096, pages + 8192, 0, r.c)
+        ra, rb = Range(0, n, 0, pages, 0, 4096, pc, 0), Range(0, n_b, pages, other, 0, 4096, pc, 0)
+        a, b = Array(n, 0, [ra], 0), Array(n_b, pages * 4096, [rb], 0)
+        want = torch.from_numpy(oracle.scan(oracle.store(SEED, 0, n)).view(np.int64)).cuda()
+        side = torch.cuda.Stream()
+        ids = [torch.arange(64, dtype=torch.int64, device="cuda") * 512 + k * 32768 for k in range(other // 64)]
+        for k in range(128):                        # the slots lie by turns, so that a page that comes back soon pushes out one of the other array
+            a.gather(512, torch.arange(512, dtype=torch.int64, device="cuda") * 512 + k * 262144)
+            b.gather(64, ids[k])
+        torch.cuda.synchronize()
+        began, ended = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        began.record()
+        torch.cuda._sleep(1 << 20)
+        ended.record()
+        torch.cuda.synchronize()
+        per_us = (1 << 20) / (began.elapsed_time(ended) * 1e3)
+        for rep in range(80):
+            for _ in range(50):                     # until all of it is resident (what comes back pushes others out, for a while)
+                a.stats()
+                a.reduce(n, 256)
+                if not a.stats()["read_io_cnt"]:
+                    break
+            with torch.cuda.stream(side):
+                torch.cuda._sleep(int(per_us * 5 * rep))
+                b.gather(64, ids[(128 + rep) % len(ids)])
+            assert torch.equal(a.scan(n, 64), want), rep
+            st = a.stats()
+            assert st["access_cnt"] == n_access, (rep, st)
+        assert not r.c.aborted()
+        a.close(); b.close(); ra.close(); rb.close(); pc.close()
