@@ -3,6 +3,8 @@
 // follow the reference's benchmark kernels (cited per kernel); lane arithmetic is for 64-wide waves.
 #include "bam_capi_internal.h"
 
+#include <atomic>
+
 namespace {
 
 /* the per-vertex kernels (the group walk below) are held to the registers of this many waves per SIMD: left alone the
@@ -588,9 +590,9 @@ __global__ void k_cc_settle(unsigned long long* comp, uint64_t vertex_count)
 }
 
 __global__ __launch_bounds__(128) BAM_GRAPH_KERNEL_WAVES void k_cc_coalesce_coarse_ptr_pc(array_d_t<uint64_t>* da, uint64_t vertex_count, const uint64_t* vertexList, unsigned long long* comp,
-                                                                  uint64_t coarse, const heavy_piece_t* heavy, uint64_t n_heavy, unsigned long long* next_work, uint32_t sweep)
+                                                                  uint64_t coarse, const heavy_piece_t* heavy, uint64_t n_heavy, unsigned long long* next_work, bool backwards)
 {
-    walk_vertex_groups(da, vertexList, vertex_count, coarse, heavy, n_heavy, next_work, (sweep & 1u) != 0,
+    walk_vertex_groups(da, vertexList, vertex_count, coarse, heavy, n_heavy, next_work, backwards,
                        [&](uint64_t) { return true; },
                        [&](uint64_t v, uint64_t next, uint64_t) { cc_join(comp, v, next); });
 }
@@ -706,10 +708,18 @@ __global__ __launch_bounds__(64) void k_bfs_by_page(array_d_t<uint64_t>* da, uin
     if (any) *changed = 1;
 }
 
-__global__ __launch_bounds__(64) void k_cc_by_page(array_d_t<uint64_t>* da, const uint64_t* offsets, const uint64_t* first, uint64_t n_edges, uint32_t ppw, uint32_t sweep,
+__global__ __launch_bounds__(64) void k_cc_sweep_by_page(array_d_t<uint64_t>* da, bool* curr_visit, bool* next_visit, const uint64_t* offsets,
+                                                          const uint64_t* first, uint64_t n_edges, uint32_t ppw, unsigned long long* comp, bool* changed)
+{
+    graph_by_page(da, offsets, first, n_edges, ppw, false,
+                  [&](uint64_t v) { return curr_visit[v]; },
+                  [&](uint64_t src, uint64_t next, uint64_t) { cc_compute(src, comp, next, next_visit, changed); });
+}
+
+__global__ __launch_bounds__(64) void k_cc_by_page(array_d_t<uint64_t>* da, const uint64_t* offsets, const uint64_t* first, uint64_t n_edges, uint32_t ppw, bool backwards,
                                                     unsigned long long* comp)
 {
-    graph_by_page(da, offsets, first, n_edges, ppw, (sweep & 1u) != 0,
+    graph_by_page(da, offsets, first, n_edges, ppw, backwards,
                   [&](uint64_t) { return true; },
                   [&](uint64_t src, uint64_t next, uint64_t) { cc_join(comp, src, next); });
 }
@@ -837,7 +847,13 @@ struct graph_plan {
     uint64_t n_pieces = 0;
     uint64_t group = 512;                    /* vertices handed to a wave at a time */
     uint64_t resident = 0;                   /* waves a sweep runs */
-    uint32_t cc_sweeps = 0;                  /* calls that read all edges run forwards and backwards by turns: what the last one left in the cache is what the next asks for first */
+    bool all_cached = false;                 /* the cache has a slot for every page of the edge array */
+    std::atomic<uint32_t> cc_calls{0};
+    /* Where some edges are on the store, calls that read all of them run forwards and backwards by turns: what the last one left
+     * in the cache is what the next asks for first (2^22 vertices, a quarter cached: 7.4 ms along the pages, 8.4 always
+     * forwards).  Where all are cached always forwards: from the back, chains grow long, each vertex hooked by the one before
+     * it (2^19 vertices: 0.3 and 2.5 ms along the pages, 1.46 and 1.80 per vertex) */
+    bool cc_backwards() { return !all_cached && (cc_calls++ & 1u) != 0; }
     by_page_plan bp;
     bool bp_built = false;
     BufferPtr bytes_a, bytes_b, floats_a, floats_b, words_a;      /* per-vertex buffers: flags, PageRank's delta and residual, SSSP's new costs */
@@ -861,6 +877,8 @@ struct graph_plan {
         /* every lane of a running wave may hold a page of its own (its bam_ptr keeps the last one it read): more waves
          * than the cache has pages for would wait for slots that only they can give back */
         uint64_t cache_pages = edges->a->adt.n_ranges ? edges->a->h_ranges[0].cache.n_pages : 0;
+        all_cached = true;
+        for (uint64_t k = 0; k < edges->a->adt.n_ranges; k++) all_cached &= edges->a->h_ranges[k].page_count <= edges->a->h_ranges[k].cache.n_pages;
         if (other_cache_pages && other_cache_pages < cache_pages) cache_pages = other_cache_pages;
         if (cache_pages && resident > cache_pages / BAM_WAVE_SIZE) resident = cache_pages / BAM_WAVE_SIZE;
         if (resident < 2) resident = 2;
@@ -1152,7 +1170,7 @@ int bam_cc(bam_array_t* edges, const uint64_t* d_offsets, uint64_t n_vertices, u
     unsigned long long* comp = (unsigned long long*)d_labels;
     hipLaunchKernelGGL(k_iota, dim3(blocks_for(n_vertices, 256)), dim3(256), 0, st, comp, n_vertices);
     hipLaunchKernelGGL(k_cc_coalesce_coarse_ptr_pc, dim3(pl->blocks(n_vertices, group)), dim3(128), 0, st, edges->a->d_array_ptr, n_vertices, d_offsets, comp, group,
-                       pl->pieces, pl->n_pieces, pl->next_work(), pl->cc_sweeps++);
+                       pl->pieces, pl->n_pieces, pl->next_work(), pl->cc_backwards());
     hipLaunchKernelGGL(k_cc_settle, dim3(blocks_for(n_vertices, 256)), dim3(256), 0, st, comp, n_vertices);
     hip_err_chk(hipGetLastError());
     pl->level_end(st);
@@ -1197,13 +1215,41 @@ int bam_cc_by_page(bam_array_t* edges, const uint64_t* d_offsets, uint64_t n_ver
     if (int rc = pl->by_page(edges, st)) return rc;
     unsigned long long* comp = (unsigned long long*)d_labels;
     hipLaunchKernelGGL(k_iota, dim3(blocks_for(n_vertices, 256)), dim3(256), 0, st, comp, n_vertices);
-    if (pl->bp.n_pages)
-        hipLaunchKernelGGL(k_cc_by_page, dim3(pl->bp.blocks), dim3(BAM_WAVE_SIZE), 0, st, edges->a->d_array_ptr, d_offsets, (const uint64_t*)pl->bp.first.get(), pl->bp.n_edges, pl->bp.ppw,
-                           pl->cc_sweeps++, comp);
-    hipLaunchKernelGGL(k_cc_settle, dim3(blocks_for(n_vertices, 256)), dim3(256), 0, st, comp, n_vertices);
-    hip_err_chk(hipGetLastError());
-    pl->level_end(st);
-    if (iterations) *iterations = 2;
+    uint32_t iter = 0;
+    bool changed = true;
+    /*
+     * With every edge cached a sweep of label propagation costs 40 to 60 us up to 2^22 entries, and a reading that joins as much
+     * as its longest chain of loads and exchanges that failed: sweeps / joins in us for 0.03, 0.13, 0.26, 0.5, 1, 2.1, 4.2, 8.4
+     * million entries of a uniform random graph 116 / 78, 140 / 111, 164 / 164, 183 / 250, 219 / 253, 308 / 376, 413 / 336,
+     * 735 / 430; of a power-law graph of 0.1, 0.5, 1.9, 7.7, 15 million 105 / 83, 142 / 186, 197 / 337, 437 / 434, 886 / 691.
+     * A graph that is long rather than wide would take a sweep per step: after six the edges are joined, from the labels as they
+     * are, each of which names a smaller vertex of the component or the vertex itself.
+     */
+    if (pl->bp.n_pages && pl->all_cached && pl->bp.n_edges > (1ull << 17) && pl->bp.n_edges < (1ull << 22)) {
+        bool* curr = (bool*)graph_plan::sized(pl->bytes_a, n_vertices);
+        bool* next = (bool*)graph_plan::sized(pl->bytes_b, n_vertices);
+        hip_err_chk(hipMemsetAsync(curr, 0x01, n_vertices, st));
+        hip_err_chk(hipMemsetAsync(next, 0x00, n_vertices, st));
+        while (changed && iter < 6) {
+            hipLaunchKernelGGL(k_cc_sweep_by_page, dim3(pl->bp.blocks), dim3(BAM_WAVE_SIZE), 0, st, edges->a->d_array_ptr, curr, next, d_offsets,
+                               (const uint64_t*)pl->bp.first.get(), pl->bp.n_edges, pl->bp.ppw, comp, (bool*)pl->changed);
+            hip_err_chk(hipGetLastError());
+            hip_err_chk(hipMemsetAsync(curr, 0x00, n_vertices, st));
+            std::swap(curr, next);
+            iter++;
+            changed = pl->level_end(st);
+        }
+    }
+    if (changed) {
+        if (pl->bp.n_pages)
+            hipLaunchKernelGGL(k_cc_by_page, dim3(pl->bp.blocks), dim3(BAM_WAVE_SIZE), 0, st, edges->a->d_array_ptr, d_offsets, (const uint64_t*)pl->bp.first.get(), pl->bp.n_edges, pl->bp.ppw,
+                               pl->cc_backwards(), comp);
+        hipLaunchKernelGGL(k_cc_settle, dim3(blocks_for(n_vertices, 256)), dim3(256), 0, st, comp, n_vertices);
+        hip_err_chk(hipGetLastError());
+        pl->level_end(st);
+        iter += 2;
+    }
+    if (iterations) *iterations = iter;
     BAM_API_END
 }
 

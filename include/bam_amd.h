@@ -264,7 +264,10 @@ int bam_bfs_frontier(bam_array_t* edges, const uint64_t* d_offsets, uint64_t n_v
 /* ---- CC (benchmarks/cc/main.cu:123-144 cc_compute, :595-617 kernel, host loop :1410-1425, 1515-1521) ----
  * d_labels[V] receives the smallest vertex id of each vertex's component of an undirected graph (both directions of every
  * edge in the CSR).  Where the reference propagates labels, sweep after sweep over the edges, the edges are read once here
- * and the trees of their ends joined, and a pass over the vertices settles the labels: *iterations = 2. */
+ * and the trees of their ends joined, and a pass over the vertices settles the labels; bam_cc_by_page propagates labels first
+ * where all edges are cached and sweeps are quicker.  *iterations: the passes made, over the edges and over the vertices.
+ * (Of a CSR that holds one direction of some edges, joining gives the components of the graph with both; propagation leaves
+ * there what the order of its updates happens to give.) */
 int bam_cc(bam_array_t* edges, const uint64_t* d_offsets, uint64_t n_vertices, uint64_t* d_labels,
            uint32_t coarse, uint32_t* iterations, void* stream);
 

@@ -48,3 +48,30 @@ def test_cc_labels_of_long_wide_and_empty_trees(bam, n_v, shape, by_page):
             assert np.array_equal(_u64(lb), ref), kept
             assert it >= 1
         assert not r.c.aborted()
+
+
+# all edges cached, around the numbers of entries between which labels are propagated along the pages (2^17, 2^22): a wide graph,
+# which a few sweeps settle, and paths, which they do not
+@pytest.mark.parametrize("shape", ["wide", "path", "scattered_path", "star"])
+@pytest.mark.parametrize("n_pairs", [(1 << 16) - 1, 1 << 16, (1 << 16) + 1, 300001, (1 << 21) - 1, 1 << 21])
+def test_cc_labels_where_all_edges_are_cached(bam, n_pairs, shape):
+    rng = np.random.default_rng(n_pairs)
+    n_v = n_pairs // 4 if shape == "wide" else n_pairs + 1
+    u, v = (rng.integers(0, n_v, n_pairs), rng.integers(0, n_v, n_pairs)) if shape == "wide" else _pairs(shape, n_v, rng)
+    off, nb = _csr(n_v, u, v)
+    ref, _ = oracle.cc_labels(off, nb)
+    pages = (len(nb) + 511) // 512
+    sweeps = 1 << 17 < len(nb) < 1 << 22
+    r, a = _graph_rig(bam, nb, max(128, pages), n_queues=16, depth=256)
+    with r:
+        d_off = _dev(off)
+        for kept in (False, True, True):
+            if kept:
+                a.set_graph(d_off)
+            for by_page in (True, False):
+                lb, it = a.cc(d_off, by_page=by_page)
+                assert np.array_equal(_u64(lb), ref), (kept, by_page)
+                # joined: a pass over the edges and one over the vertices; propagated: until a sweep changes nothing, six at most
+                assert it == 2 if not (by_page and sweeps) else 2 <= it <= 6 or it == 8, (it, by_page)
+                assert not (by_page and sweeps and shape == "scattered_path") or it == 8
+        assert a.stats()["read_io_cnt"] == pages and not r.c.aborted()
