@@ -1476,13 +1476,41 @@ int bam_array_stats(bam_array_t* a, uint64_t* out, int reset)
 
 extern "C++" {
 namespace {
-/* whether a gather is better off as several launches than as one that can miss; they keep notes between launches, which a
- * stream under capture must not (the graph may be replayed beside other calls) */
+/* the requests the kernels that can miss have on their way at a time: sixteen waves on each of 256 compute units */
+#define BAM_REQS_AT_A_TIME (1ull << 18)
+/*
+ * Whether what is missing is fetched page by page: arrays larger than their cache, with a request for every other page or more
+ * (below that nearly every request has its page to itself, and the requests by themselves make whole batches), and a cache
+ * that takes 64 pages from each of 32 waves and has room for as many again.  Where all requests are on their way together,
+ * only if the pages missing are far more than the cache holds and are asked for often (request by request / page by page, ms:
+ * 2^24 elements behind half of them, 2^16 to 2^18 requests 1.4 / 1.7 to 1.6 / 1.8; behind a quarter 2^16 requests 3.0 / 3.8, 2^17
+ * 7.7 / 4.6; 2^26 elements behind a quarter 2^17 requests 5.2 / 5.7, 2^18 11.3 / 7.6).  Beyond that always: 2^19 requests,
+ * half cached: 2^24 elements 1.77 / 1.77, 2^26 6.7 / 5.4, 2^28 13.4 / 13.9, 2^22 requests 25 / 20; a quarter cached 32 / 4.5,
+ * 20.7 / 8.3, 22 / 20.
+ */
+bool page_by_page(const range_d_t<uint64_t>& range, uint64_t n_reqs)
+{
+    const uint64_t pages = range.page_count, cache_pages = range.cache.n_pages;
+    if (pages <= cache_pages || n_reqs < pages / 2 || cache_pages < 4096) return false;
+    return pages > 2 * cache_pages ? n_reqs >= BAM_REQS_AT_A_TIME || n_reqs >= 4 * pages : n_reqs > BAM_REQS_AT_A_TIME;
+}
+/*
+ * Whether a gather is better off as several launches than as one that can miss; they keep notes between launches, which a
+ * stream under capture must not (the graph may be replayed beside other calls).
+ *   Arrays larger than their cache: while all requests are on their way together, those on one page share its fetch, and one
+ * launch is as good or better (2^26 elements behind a quarter of them, one / two launches / page by page: 2^17 requests 5.1 / 5.2 / 5.6
+ * ms; 2^24 elements, 2^16 requests, all in cache 11 / 37 / 37 us); beyond, a page has left again when the next request for it
+ * starts (3 * 2^17 requests 18.7 / 16.1 / 8.0 ms, 2^19 26.8 / 20.6 / 8.3).
+ *   Arrays that fit: two launches from 2^21 requests on, where the last-level cache holds little of the array (2^27 elements,
+ * one / two launches: 2^20 requests 38 / 40 us, 2^21 70 / 68, 2^24 518 / 465; 2^26 elements 64 / 68 and 477 / 464; 2^24
+ * elements 55 / 66 and 375 / 451: there the look at the descriptor after the element is not hidden).
+ */
 bool scattered_launches_pay(bam_array_t* a, uint64_t n_reqs, hipStream_t st)
 {
     if (!two_launches_ok(a)) return false;
     const range_d_t<uint64_t>& range = a->a->h_ranges[0];
-    if (n_reqs < (range.page_count > range.cache.n_pages ? 1ull << 14 : 1ull << 20)) return false;
+    if (range.page_count > range.cache.n_pages) { if (n_reqs <= BAM_REQS_AT_A_TIME && !page_by_page(range, n_reqs)) return false; }
+    else if (n_reqs < 1ull << 21 || range.page_count * range.cache.page_size <= 512ull << 20) return false;
     return !is_captured(st);
 }
 /*
@@ -1504,10 +1532,7 @@ bool scattered_reads(bam_array_t* a, uint64_t n_reqs, const uint64_t* d_assignme
     while (rounds < 32 && n_reqs / ((uint64_t)N * rounds * 2 * 256) >= 16384) rounds *= 2;
     const uint64_t per_thread = (uint64_t)N * rounds;
     const uint64_t n_words = (n_reqs + BAM_WAVE_SIZE - 1) / BAM_WAVE_SIZE, n_waves = (n_words + per_thread - 1) / per_thread;
-    /* page by page: with a request for every other page or more (below that nearly every request has its page to itself, and
-     * the requests by themselves make whole batches), and a cache that takes 64 pages from each of 32 waves and has room
-     * for as many again */
-    const bool by_page = pages > cache_pages && n_reqs >= pages / 2 && cache_pages >= 4096;
+    const bool by_page = page_by_page(range, n_reqs);
     const uint64_t wanted_bytes = by_page ? (pages + 511) / 512 * 512 : 0;
     std::lock_guard<std::mutex> guard(a->scratch.mu);
     scratch_set* set = scratch_for(a, st, n_words * sizeof(uint64_t), wanted_bytes);
@@ -1530,9 +1555,11 @@ bool scattered_reads(bam_array_t* a, uint64_t n_reqs, const uint64_t* d_assignme
     const uint64_t n_chunks = (n_words + words - 1) / words;
     const uint64_t waves = n_chunks < 16384 ? n_chunks : 16384;
     const dim3 grid_d(blocks_for(waves * BAM_WAVE_SIZE, 256));
-    /* stretches of which at most three quarters of the cache can be wanted (all of it is when the requests are spread evenly) */
-    const uint64_t room = cache_pages - cache_pages / 4, most = pages < n_reqs ? pages : n_reqs;
-    const uint64_t stretches = by_page ? (most + room - 1) / room : 1;
+    /* stretches of which no more can be wanted than the cache holds (all of it is when the requests are spread evenly).  Each
+     * ends with a batch that is waited for, and two where one would do cost more than pages that are fetched and leave unread:
+     * with three quarters of the cache to a stretch 2^20 reads of 2^24 elements behind half of them took 2.35 ms, now 1.81 */
+    const uint64_t most = pages < n_reqs ? pages : n_reqs;
+    const uint64_t stretches = by_page ? (most + cache_pages - 1) / cache_pages : 1;
     const uint64_t step = ((pages + stretches - 1) / stretches + 511) / 512 * 512;
     const uint64_t f_waves = std::min<uint64_t>(BAM_FETCH_PAGE_WAVES, cache_pages / (2 * BAM_WAVE_SIZE));
     for (uint64_t p = 0; p < pages; p += step) {

@@ -114,7 +114,7 @@ int bam_array_read(bam_array_t* a, uint64_t n_reqs, const uint64_t* d_assignment
  *   BAM_READ_TWO_LAUNCHES     a first launch reads what is resident, reads_per_lane (1, 2, 4, 8) requests per thread, with a
  *                             kernel that cannot miss (no call, no stack, a fraction of the registers) and notes the rest;
  *                             a second launch reads the rest, 64 requests to a wave whatever the share of misses was.
- *                             Where the array is larger than its cache and there is a request for every other page or more,
+ *                             Where the array is larger than its cache and there are many requests for a page that is missing,
  *                             the rest goes page by page: launches that fetch the pages somebody waits for, each once, in
  *                             batches of 64 commands, alternate with launches that read the requests for them.  Arrays of
  *                             one range only (EINVAL otherwise); on a stream that is being captured the
@@ -129,8 +129,8 @@ int bam_array_read_shaped(bam_array_t* a, uint64_t n_reqs, const uint64_t* d_ass
                           uint64_t* d_sum, void* stream);
 /* the same requests with the values handed out: d_out[t] = element d_assignment[t] (or t * stride); what a kernel of the
  * reference's benchmark would hold in its register after array_d_t::operator[] (benchmarks/array/main.cu:57).  Launches of
- * 2^20 requests and more, 2^14 where the array is larger than its cache, run as BAM_READ_TWO_LAUNCHES does (arrays of one
- * range, streams that are not being captured) */
+ * more than 2^18 requests where the array is larger than its cache, and of 2^21 and more where it is larger than 512 MiB, run as
+ * BAM_READ_TWO_LAUNCHES does (arrays of one range, streams that are not being captured) */
 int bam_array_gather(bam_array_t* a, uint64_t n_reqs, const uint64_t* d_assignment, uint64_t stride, uint32_t block_size, uint64_t* d_out, void* stream);
 /* The read pattern of bam_array_read (one thread per request, element d_assignment[t] or t * span) through the other
  * access routes of array_d_t (include/page_cache.h:1240-1716, 414-485): api 1 get_raw/release_raw, 2 get_page_gid +

@@ -8,14 +8,25 @@ from test_gpu_parity import Rig, SEED, bam, _dev, _u64  # noqa: F401  (bam is th
 pytestmark = pytest.mark.gpu
 
 
+IN_FLIGHT = 1 << 18        # requests that are on their way together in a launch that can miss
+
+
+def _page_by_page(pages, cache_pages, n):
+    if pages <= cache_pages or 2 * n < pages - 1 or cache_pages < 4096:
+        return False
+    return n >= IN_FLIGHT or n >= 4 * pages if pages > 2 * cache_pages else n > IN_FLIGHT
+
+
 # pages of data and of cache: everything resident; just below and at the smallest cache that is fetched for page by page, one
-# stretch and several; requests around the sizes where the shape of the launch changes, and fewer than a request per two pages
+# stretch and several; requests around the numbers where the shape of the launch changes, and fewer than a request per two pages
 @pytest.mark.parametrize("pages,cache_pages,n", [(4096, 4096, (1 << 20) + 1), (4100, 4095, 1 << 14), (4100, 4096, (1 << 14) - 1), (4100, 4096, (1 << 14) + 77),
-                                                 (12289, 4096, 100003), (12289, 5000, (1 << 20) - 1), (40000, 4096, 19999), (40000, 4096, 20001)])
+                                                 (12289, 4096, 100003), (12289, 5000, (1 << 20) - 1), (40000, 4096, 19999), (40000, 4096, 20001),
+                                                 (4100, 4095, IN_FLIGHT + 1), (4100, 4096, IN_FLIGHT), (4100, 4096, IN_FLIGHT + 1), (8192, 4096, IN_FLIGHT), (8193, 4096, 4 * 8193 - 1),
+                                                 (8193, 4096, 4 * 8193), (70000, 8192, IN_FLIGHT - 1), (70000, 8192, IN_FLIGHT), (70000, 8192, IN_FLIGHT + 65)])
 def test_scattered_reads_element_by_element(bam, pages, cache_pages, n):
     """Every element of a gather and the sum of the same requests, twice (the second call finds what the first left behind),
     with a few requests outside the array (they read as 0 and are not counted) and a skewed half; every request inside is
-    counted once and misses cover the reads from the store."""
+    counted once and misses cover the reads from the store.  Page by page each page asked for is read once, cold or not."""
     n_elems = pages * 512 - 37
     words = oracle.store(SEED, 0, n_elems)
     rng = np.random.default_rng(n)
@@ -28,9 +39,12 @@ def test_scattered_reads_element_by_element(bam, pages, cache_pages, n):
         inside = idx < n_elems
         want = np.where(inside, words[np.where(inside, idx, 0).astype(np.int64)], 0).astype(np.uint64)
         d_idx = _dev(idx)
+        asked = len(np.unique(idx[inside] // 512))
         for rep in range(2):
             assert np.array_equal(_u64(a.gather(n, d_idx)), want), rep
             st = a.stats()
+            if _page_by_page(pages, cache_pages, n):
+                assert st["read_io_cnt"] == asked if rep == 0 else st["read_io_cnt"] <= asked, (st, asked)
             assert st["access_cnt"] == inside.sum() and st["hit_cnt"] + st["miss_cnt"] == st["access_cnt"], st
             assert st["read_io_cnt"] <= st["miss_cnt"] or rep == 0, st
             assert a.read(n, d_idx) == int(np.sum(want, dtype=np.uint64)), rep
@@ -40,6 +54,55 @@ def test_scattered_reads_element_by_element(bam, pages, cache_pages, n):
             a.gather(n, d_idx)
             assert a.stats()["hit_cnt"] == inside.sum()
         assert not r.c.aborted() and r.c.info()["error_completions"] == 0
+
+
+@pytest.mark.parametrize("page", [512, 4096, 8192, 65536])
+@pytest.mark.parametrize("first,offset", [(0, 0), (1000, 0), (0, 24), (777, 504)])
+def test_scattered_reads_of_ranges_that_begin_inside_a_page(bam, page, first, offset):
+    """other page sizes, ranges whose first element is not the array's first and does not start a page; resident, and larger than the
+    cache, requests in front of the range and behind it among them (they read as 0)"""
+    from bam_amd import Array, PageCache, Range
+    per = page // 8
+    pages, n = 9001, IN_FLIGHT + 77
+    n_elems = (pages * page - offset) // 8 - 3
+    if page == 65536:
+        pages, n_elems = 4500, 4500 * per - offset // 8 - 3
+    words = oracle.store(SEED, 3 * per + offset // 8, n_elems)
+    rng = np.random.default_rng(page + first)
+    idx = (rng.integers(0, n_elems, n) + first).astype(np.uint64)
+    idx[rng.integers(0, n, 6)] = np.array([first - 1 if first else (1 << 64) - 1, 0 if first else n_elems, first + n_elems, first + n_elems + 1, 1 << 40, (1 << 64) - 1], dtype=np.uint64)
+    at = idx - np.uint64(first)
+    inside = at < n_elems
+    want = np.where(inside, words[np.where(inside, at, 0).astype(np.int64)], 0).astype(np.uint64)
+    for cache_pages in (4096, pages):
+        with Rig(bam, (pages + 4) * page // 65536 * 65536 + 65536, n_queues=16, depth=256) as r:
+            pc = PageCache(page, cache_pages, 0, r.c)
+            rg = Range(first, first + n_elems, 3, pages, offset, page, pc, 0)
+            a = Array(first + n_elems, 0, [rg], 0)
+            d_idx = _dev(idx)
+            for rep in range(2):
+                assert np.array_equal(_u64(a.gather(n, d_idx)), want), (cache_pages, rep)
+                assert a.stats()["access_cnt"] == inside.sum()
+                assert a.read(n, d_idx) == int(np.sum(want, dtype=np.uint64)), (cache_pages, rep)
+                assert a.stats()["access_cnt"] == inside.sum()
+            assert not r.c.aborted()
+            a.close(); rg.close(); pc.close()
+
+
+def test_gathers_from_a_large_resident_array(bam):
+    """more than the last-level cache holds, around the number of requests from which they run in two launches; some pages missing"""
+    pages = (1 << 17) + 1
+    n_elems = pages * 512 - 5
+    words = oracle.store(SEED, 0, n_elems)
+    idx = np.random.default_rng(9).integers(0, n_elems, (1 << 21) + 1).astype(np.uint64)
+    d = _dev(idx)
+    want = words[idx.astype(np.int64)]
+    with Rig(bam, pages * 4096, n_queues=16, depth=256) as r:
+        a = r.array(n_elems, 4096, pages)
+        for n in ((1 << 21) + 1, (1 << 21) - 1, 1 << 21):
+            assert np.array_equal(_u64(a.gather(n, d)), want[:n]), n
+            assert a.stats()["access_cnt"] == n
+        assert not r.c.aborted()
 
 
 def test_gathers_on_several_streams_of_one_array(bam):
