@@ -30,27 +30,33 @@ __global__ __launch_bounds__(64) void k_vectoradd_ptr_pc(array_d_t<uint64_t>* da
 }
 
 // ---- reduction (benchmarks/reduction/main.cu:166-195 kernel_reduce_baseline_ptr_pc): output[b] = sum of the 2 x blockDim elements of block b ----
-/* one output; by all threads of the workgroup */
-__device__ __forceinline__ void reduce_output(array_d_t<uint64_t>* da, unsigned long long* output, const uint64_t len, const uint64_t bid, uint64_t* wave_total)
+/* output `bid` by `half` consecutive threads of the workgroup (a multiple of 64; each such group its own output, or none: take =
+ * false); all threads of the workgroup come in */
+__device__ __forceinline__ void reduce_output(array_d_t<uint64_t>* da, unsigned long long* output, const uint64_t len, const uint64_t bid, const uint32_t half, const bool take, uint64_t* wave_total)
 {
-    const uint64_t tid = threadIdx.x, start = 2ull * blockDim.x * bid;
+    const uint64_t tid = threadIdx.x % half, start = 2ull * half * bid;
+    const uint32_t w = threadIdx.x / BAM_WAVE_SIZE;
     uint64_t v = 0;
-    {
+    if (take) {
         bam_ptr<uint64_t> in_ptr(da);
         const bam_ptr<uint64_t>& input = in_ptr;
-        /* a workgroup reads 2 x blockDim consecutive elements: its waves' first elements */
+        /* a group reads 2 x half consecutive elements: its waves' first elements */
         const uint64_t first = start + tid - tid % BAM_WAVE_SIZE;
         if (first < len) touch_ahead(da, first, len);
-        if (first + blockDim.x < len) touch_ahead(da, first + blockDim.x, len);
+        if (first + half < len) touch_ahead(da, first + half, len);
         if (start + tid < len) v = input[start + tid];
-        if (blockDim.x + start + tid < len) v += input[blockDim.x + start + tid];
+        if (half + start + tid < len) v += input[half + start + tid];
     }
     v = wave_sum(v);
-    if (bam::lane() == 0) wave_total[tid / BAM_WAVE_SIZE] = v;
+    if (half == BAM_WAVE_SIZE) {                /* a wave's own output: nothing to wait for */
+        if (tid == 0 && take) output[bid] = v;
+        return;
+    }
+    if (bam::lane() == 0) wave_total[w] = v;
     __syncthreads();
     if (tid < BAM_WAVE_SIZE) {
-        v = wave_sum(tid < blockDim.x / BAM_WAVE_SIZE ? wave_total[tid] : 0);
-        if (tid == 0) output[bid] = v;
+        v = wave_sum(tid < half / BAM_WAVE_SIZE ? wave_total[w + tid] : 0);
+        if (tid == 0 && take) output[bid] = v;
     }
 }
 
@@ -63,32 +69,37 @@ __global__ void k_reduce_ptr_pc(array_d_t<uint64_t>* da, unsigned long long* out
         return;
     }
     const uint64_t bid = blockIdx.x - (fp.done ? fp.blocks : 0u);
-    reduce_output(da, output, len, bid, wave_total);
+    reduce_output(da, output, len, bid, blockDim.x, true, wave_total);
     if (fp.done && threadIdx.x == 0) __hip_atomic_fetch_add(fp.done, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 /*
- * The outputs k_reduce_resident left, by as many workgroups as the device holds at a time: what is resident was summed
- * there, and a grid with a workgroup per output would take longer to find nothing to do (131072 workgroups) than that
- * kernel takes.  notes[k] covers `per_note` consecutive outputs.
+ * The outputs k_reduce_resident left, by at most 32768 waves: what is resident was summed there, and a grid with a workgroup
+ * per output takes as long to find nothing to do as that kernel takes (2^24 elements, blocks of 64, all resident: 71 us a call,
+ * 47 with 32768 workgroups of a wave, 42 with 8192 of four).  So small outputs are taken `blockDim / half` to a workgroup.
+ * notes[k] covers `per_note` consecutive outputs.  Bound by the store where all is missing (2^24 elements, blocks of 64: 8.7 ms
+ * in one launch of a workgroup per output, 7.7 here; with 4096 waves 11).  The word that says whether anything was left is read as an ordinary
+ * load, and is on another line than *done: read past the caches by every wave, on the line the workgroups count themselves off
+ * in, it cost some 12 ns a wave, one after the other (2^22 elements in workgroups of a wave: 2.35 ms, as here 1.9).
  */
-__global__ void k_reduce_rest(array_d_t<uint64_t>* da, unsigned long long* output, uint64_t len, uint64_t n_outputs, uint32_t per_note, const uint8_t* notes,
+#define BAM_REST_WAVES 32768u
+__global__ void k_reduce_rest(array_d_t<uint64_t>* da, unsigned long long* output, uint64_t len, uint64_t n_outputs, uint32_t half, uint32_t per_note, const uint8_t* notes,
                               const uint32_t* finished, uint32_t call, const fetch_plan fp)
 {
     __shared__ uint64_t wave_total[1024 / BAM_WAVE_SIZE];
-    if (__hip_atomic_load(finished + BAM_LEFT_WORD, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != call) return;      /* nothing was left */
+    if (finished[BAM_LEFT_WORD] != call) return;      /* nothing was left */
     const uint32_t fetching = fp.done ? fp.blocks : 0u;
     if (blockIdx.x < fetching) {
         array_d_t<uint64_t>* const arrays[1] = {da};
         fetch_role(arrays, len, fp);
         return;
     }
-    for (uint64_t bid = blockIdx.x - fetching; bid < n_outputs; bid += gridDim.x - fetching) {
-        if (notes[bid / per_note]) {
-            reduce_output(da, output, len, bid, wave_total);
-            __syncthreads();
-        }
-        if (fp.done && threadIdx.x == 0) __hip_atomic_fetch_add(fp.done, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const uint32_t groups = blockDim.x / half;
+    for (uint64_t b0 = (uint64_t)(blockIdx.x - fetching) * groups; b0 < n_outputs; b0 += (uint64_t)(gridDim.x - fetching) * groups) {
+        const uint64_t bid = b0 + threadIdx.x / half;
+        reduce_output(da, output, len, bid, half, bid < n_outputs && notes[bid / per_note] != 0, wave_total);
+        if (half > BAM_WAVE_SIZE) __syncthreads();
+        if (fp.done && threadIdx.x % half == 0) __hip_atomic_fetch_add(fp.done, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
 }
 
@@ -548,10 +559,11 @@ int bam_reduce(bam_array_t* a, uint64_t n_elems, uint32_t block_size, uint64_t* 
             const uint32_t call = set->next_call();
             hipLaunchKernelGGL(k_reduce_resident, dim3((uint32_t)std::min<uint64_t>((n_turns + 3) / 4, 2048)), dim3(256), 0, st, a->a->d_array_ptr, (unsigned long long*)d_partials, n_elems,
                                n_outputs, rows, per_note, notes, set->finished(), call, set->done());
-            const fetch_plan fp = make_fetch_plan(a, 1, block_size, 2ull * block_size, st, set->done());
-            const uint64_t at_a_time = 256ull * 1024 / block_size;             /* sixteen waves per compute unit */
-            hipLaunchKernelGGL(k_reduce_rest, dim3((uint32_t)std::min<uint64_t>(n_outputs, at_a_time) + fp.blocks), dim3(block_size), 0, st, a->a->d_array_ptr, (unsigned long long*)d_partials,
-                               n_elems, n_outputs, per_note, notes, set->finished(), call, fp);
+            const uint32_t groups = block_size <= 128 ? 256 / block_size : 1, threads = groups * block_size;
+            const fetch_plan fp = make_fetch_plan(a, 1, threads, 2ull * block_size, st, set->done());
+            const uint64_t at_a_time = (uint64_t)BAM_REST_WAVES * BAM_WAVE_SIZE / threads;
+            hipLaunchKernelGGL(k_reduce_rest, dim3((uint32_t)std::min<uint64_t>((n_outputs + groups - 1) / groups, at_a_time) + fp.blocks), dim3(threads), 0, st, a->a->d_array_ptr,
+                               (unsigned long long*)d_partials, n_elems, n_outputs, block_size, per_note, notes, set->finished(), call, fp);
             hip_err_chk(hipGetLastError());
             return 0;
         }

@@ -11,7 +11,7 @@
 
 #define BAM_SUM_PARTIALS 4096
 #define BAM_SCRATCH_SETS 64
-#define BAM_SCRATCH_WORDS_BYTES (BAM_SUM_PARTIALS * sizeof(uint64_t) + 512)
+#define BAM_SCRATCH_WORDS_BYTES (BAM_SUM_PARTIALS * sizeof(uint64_t) + 1024)
 
 /*
  * The bits of the requests a first launch leaves, a byte per page of the range that somebody waits for (zero between calls),
@@ -26,8 +26,8 @@ struct scratch_set {
     unsigned long long* partials() { return (unsigned long long*)words.get(); }
     uint32_t* finished() { return (uint32_t*)(partials() + BAM_SUM_PARTIALS); }
     uint32_t next_call() { if (++calls == 0) calls = 1; return calls; }
-    /* the word the computing workgroups of a reduction count themselves off in for the fetching ones */
-    unsigned long long* done() { return (unsigned long long*)(finished() + 104); }
+    /* the word the computing workgroups of a reduction count themselves off in for the fetching ones, on a line of its own */
+    unsigned long long* done() { return (unsigned long long*)(finished() + 128); }
 };
 
 /* a number of the calling thread's own, given out once in the life of the process (the number of a thread that has ended may
