@@ -274,7 +274,8 @@ __global__ void k_scan_ptr_pc(array_d_t<uint64_t>* da, unsigned long long* outpu
  * through bam_ptr with a pass over the result to add the block totals; 2^20: 27 against 73).  One pass in which a workgroup waits
  * for the sums of the ones before it reads the array once, but took 350 us there and 92 for 2^22: the number of the next
  * tile, drawn from one word, costs the device 20 ns each, and a workgroup's registers sit idle for the 12 us it waits.
- * A page that is not resident: the wave tells the second launch and the host, which then runs the kernels that can miss.
+ * A page that is not resident: the wave tells the second launch and the host, which then runs the kernels that can miss
+ * (host_left[0] names the call if the first launch gave up, [1] if the second did).
  */
 #define BAM_CHUNK_WAVES 8u
 #define BAM_COUNTED_WORD 98u      /* of the scratch's words: the call whose accesses were counted */
@@ -345,7 +346,7 @@ __global__ __launch_bounds__(BAM_CHUNK_WAVES * BAM_WAVE_SIZE) void k_scan_write(
         const uint64_t first = (bam::first(p0) + at) * BAM_WAVE_ELEMS;
         if (first > n) break;
         bam::u64x2_t x[BAM_WAVE_ROWS];
-        if (!read_rows_resident(view, first, n, x)) { scan_gives_up(finished, call, host_left); break; }
+        if (!read_rows_resident(view, first, n, x)) { scan_gives_up(finished, call, host_left + 1); break; }
         uint64_t carry = before + bam::bcast(pieces_before, at);
         /* entry e is the sum of the elements before element e, the last one, n, the total */
 #pragma unroll
@@ -446,10 +447,10 @@ uint64_t paired_accesses(uint64_t n, uint64_t half, uint64_t page_elems)
 }
 
 /*
- * A word in host memory that the device can write, one call's own for as long as it lasts: a scan waits for its result, and
+ * Two words in host memory that the device can write, one call's own for as long as it lasts: a scan waits for its result, and
  * finds there whether it is whole.  Page-locked memory takes far longer to get than a scan does, so the words are kept for the
- * next call, whichever array or thread makes it; there are as many as calls were ever waiting at a time, in steps of 64.  A
- * word that launches may still write (the wait failed) is not given back.  `at` is NULL where no memory is to be had.
+ * next call, whichever array or thread makes it; there are as many as calls were ever waiting at a time, in steps of 32.
+ * Words that launches may still write (the wait failed) are not given back.  `at` is NULL where no memory is to be had.
  */
 struct host_word {
     volatile uint32_t* at = nullptr;
@@ -462,11 +463,11 @@ struct host_word {
             const relaxed_capture relaxed;
             void* mem = nullptr;
             if (hipHostMalloc(&mem, 64 * sizeof(uint32_t), hipHostMallocMapped | hipHostMallocPortable) != hipSuccess) { (void)hipGetLastError(); return; }
-            for (uint32_t k = 0; k < 64; k++) p.free.push_back((volatile uint32_t*)mem + k);
+            for (uint32_t k = 0; k < 64; k += 2) p.free.push_back((volatile uint32_t*)mem + k);
         }
         at = p.free.back();
         p.free.pop_back();
-        *at = 0;                    /* never the number of a call */
+        at[0] = at[1] = 0;          /* never the number of a call */
     }
     ~host_word()
     {
@@ -515,8 +516,8 @@ bool scan_resident(bam_array_t* a, uint64_t n_elems, uint32_t block_size, uint64
     const hipError_t e = hipStreamSynchronize(st);
     left.idle = e == hipSuccess;
     hip_err_chk(e);
-    if (*left.at != call) return true;
-    hipLaunchKernelGGL(k_scan_uncount, dim3(1), dim3(1), 0, st, a->a->d_array_ptr, finished, call, n_access);
+    if (left.at[0] != call && left.at[1] != call) return true;
+    if (left.at[1] == call) hipLaunchKernelGGL(k_scan_uncount, dim3(1), dim3(1), 0, st, a->a->d_array_ptr, finished, call, n_access);
     hip_err_chk(hipGetLastError());
     return false;
 }
@@ -582,19 +583,33 @@ int bam_scan(bam_array_t* a, uint64_t n_elems, uint32_t block_size, uint64_t* d_
     if (n_elems > a->a->adt.n_elems) return fail(EINVAL, "bam_scan: more elements than the array holds");
     BAM_API_BEGIN
     hipStream_t st = (hipStream_t)stream;
-    if (n_elems && (uintptr_t)d_result % 16 == 0 && resident_first(a, n_elems, st) && scan_resident(a, n_elems, block_size, d_result, st)) return 0;
+    const bool kept = n_elems && (uintptr_t)d_result % 16 == 0 && resident_first(a, n_elems, st);
+    if (kept && scan_resident(a, n_elems, block_size, d_result, st)) return 0;
     hip_err_chk(hipMemsetAsync(d_result, 0, sizeof(uint64_t), st));
     if (n_elems) {
         const uint64_t n_blocks = blocks_for(n_elems, 2ull * block_size);
-        BufferPtr totals = createBuffer(n_blocks * sizeof(uint64_t), 0);
+        /* the block totals: in the scratch of a call that has just looked for resident pages, else in memory of their own */
+        BufferPtr own;
+        unsigned long long* totals = nullptr;
+        std::unique_lock<std::mutex> guard(a->scratch.mu, std::defer_lock);
+        if (kept) {
+            guard.lock();
+            if (scratch_set* set = scratch_for(a, st, n_blocks * sizeof(uint64_t), 0)) totals = (unsigned long long*)set->notes.get();
+            else guard.unlock();
+        }
+        if (!totals) {
+            own = createBuffer(n_blocks * sizeof(uint64_t), 0);
+            totals = (unsigned long long*)own.get();
+        }
         unsigned long long* out = (unsigned long long*)d_result + 1;
         const size_t lds = (2 * block_size + 1024 / BAM_WAVE_SIZE) * sizeof(uint64_t);
         const fetch_plan fp = make_fetch_plan(a, 1, block_size, 2ull * block_size, st);
-        hipLaunchKernelGGL(k_scan_ptr_pc, dim3(n_blocks + fp.blocks), dim3(block_size), lds, st, a->a->d_array_ptr, out, (unsigned long long*)totals.get(), n_elems, fp);
-        hipLaunchKernelGGL(k_scan_block_totals, dim3(1), dim3(1024), 0, st, (unsigned long long*)totals.get(), n_blocks);
-        hipLaunchKernelGGL(k_scan_finalsum, dim3(n_blocks), dim3(block_size), 0, st, (const unsigned long long*)totals.get(), out, n_elems);
+        hipLaunchKernelGGL(k_scan_ptr_pc, dim3(n_blocks + fp.blocks), dim3(block_size), lds, st, a->a->d_array_ptr, out, totals, n_elems, fp);
+        hipLaunchKernelGGL(k_scan_block_totals, dim3(1), dim3(1024), 0, st, totals, n_blocks);
+        hipLaunchKernelGGL(k_scan_finalsum, dim3(n_blocks), dim3(block_size), 0, st, totals, out, n_elems);
         hip_err_chk(hipGetLastError());
-        hip_err_chk(hipStreamSynchronize(st));         /* `totals` is released on return */
+        if (guard.owns_lock()) guard.unlock();
+        hip_err_chk(hipStreamSynchronize(st));         /* `own` is released on return */
     }
     BAM_API_END
 }
