@@ -235,15 +235,15 @@ __global__ __launch_bounds__(256) void k_fetch_wanted(array_d_t<uint64_t>* dr, u
  * the requests up in LDS, index and all, and reads them four per lane side by side as far as they are resident
  * (k_fetch_wanted has just brought their pages in, where it ran), what is not one after the other, 64 to a wave: whatever
  * the share of misses, the batches of commands that go to the store are whole waves' worth.  The bits of what was read are
- * cleared.  All of them count as misses: the first launch looked and did not find their page.  The last workgroup to finish
- * adds the checksum of these reads to the first launch's.  When the first launch left nothing (it says so in a word of its
- * own) this one ends at once.
+ * cleared.  Where pages were fetched for them (`fetched`) those that find theirs count as misses: the first launch looked and did
+ * not find it.  Otherwise each counts by what it finds now.  The last workgroup to finish adds the checksum of these reads to
+ * the first launch's.  When the first launch left nothing (it says so in a word of its own) this one ends at once.
  */
 #define BAM_DEFER_MAX_WORDS 16u
 template <bool GATHER>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_array_read_deferred(array_d_t<uint64_t>* dr, uint64_t n_reqs, const uint64_t* __restrict__ assignment, uint64_t* missed,
-                                                             uint64_t n_words, uint32_t words, uint64_t page_first, uint64_t page_last, unsigned long long* partials, unsigned long long* sum,
-                                                             uint64_t* out_list, uint32_t* finished, uint32_t call)
+                                                             uint64_t n_words, uint32_t words, uint64_t page_first, uint64_t page_last, bool fetched, unsigned long long* partials,
+                                                             unsigned long long* sum, uint64_t* out_list, uint32_t* finished, uint32_t call)
 {
     __shared__ uint64_t list[256 / BAM_WAVE_SIZE][BAM_DEFER_MAX_WORDS * BAM_WAVE_SIZE];      /* index of the request's element */
     __shared__ uint16_t ids[256 / BAM_WAVE_SIZE][BAM_DEFER_MAX_WORDS * BAM_WAVE_SIZE];       /* which request of the chunk it is */
@@ -303,7 +303,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
     }
-    view.n_hit = 0;
+    if (fetched) view.n_hit = 0;
     view.flush_stats();
     if constexpr (!GATHER) {
         if (bam::ballot(any)) block_accumulate(partials, v);
@@ -1566,7 +1566,7 @@ bool scattered_reads(bam_array_t* a, uint64_t n_reqs, const uint64_t* d_assignme
         const uint64_t q = p + step < pages ? p + step : pages;
         if (by_page)
             hipLaunchKernelGGL(k_fetch_wanted, dim3(blocks_for(f_waves * BAM_WAVE_SIZE, 256)), block, 0, st, d, (uint64_t*)wanted, p, q, fin, call);
-        hipLaunchKernelGGL(k_array_read_deferred<GATHER>, grid_d, block, 0, st, d, n_reqs, d_assignment, missed, n_words, words, p, q, part, sum, d_out, fin, call);
+        hipLaunchKernelGGL(k_array_read_deferred<GATHER>, grid_d, block, 0, st, d, n_reqs, d_assignment, missed, n_words, words, p, q, by_page, part, sum, d_out, fin, call);
     }
     hip_err_chk(hipGetLastError());
     return true;

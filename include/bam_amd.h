@@ -118,8 +118,8 @@ int bam_array_read(bam_array_t* a, uint64_t n_reqs, const uint64_t* d_assignment
  *                             the rest goes page by page: launches that fetch the pages somebody waits for, each once, in
  *                             batches of 64 commands, alternate with launches that read the requests for them.  Arrays of
  *                             one range only (EINVAL otherwise); on a stream that is being captured the
- *                             call runs as BAM_READ_FOUR_PER_THREAD.  A request that did not find its page in the first launch
- *                             counts as a miss.
+ *                             call runs as BAM_READ_FOUR_PER_THREAD.  A request whose page these launches
+ *                             fetched counts as a miss, any other by what it finds when it is read.
  * bam_array_read picks BAM_READ_TWO_LAUNCHES with eight reads per lane for launches of 2^16 requests and more where the array
  * allows it (BAM_READ_FOUR_PER_THREAD where not) and BAM_READ_ONE_PER_THREAD below that. */
 #define BAM_READ_ONE_PER_THREAD  1

@@ -89,6 +89,23 @@ def test_scattered_reads_of_ranges_that_begin_inside_a_page(bam, page, first, of
             a.close(); rg.close(); pc.close()
 
 
+def test_counters_of_reads_in_two_launches(bam):
+    """requests that the first launch leaves count by what they find in the second: of 2^22 for one page that is on the store, those
+    looked at once it is there are hits, in several times as many waves as the device holds; page by page none is"""
+    n = 1 << 22
+    for pages, cache_pages, by_page in ((600, 512, False), (4200, 4096, True)):
+        with Rig(bam, pages * 4096, n_queues=16, depth=256) as r:
+            a = r.array(pages * 512, 4096, cache_pages)
+            assert _page_by_page(pages, cache_pages, n) == by_page
+            idx = np.random.default_rng(4).integers(5 * 512, 6 * 512, n).astype(np.uint64)
+            assert a.read(n, _dev(idx)) == int(np.sum(oracle.store(SEED, 0, 6 * 512)[idx.astype(np.int64)], dtype=np.uint64))
+            st = a.stats()
+            assert st["access_cnt"] == n and st["hit_cnt"] + st["miss_cnt"] == n and st["read_io_cnt"] == 1, st
+            assert st["hit_cnt"] == 0 if by_page else st["hit_cnt"] > n // 2, st
+            a.read(n, _dev(idx))
+            assert a.stats()["hit_cnt"] == n and not r.c.aborted()
+
+
 def test_gathers_from_a_large_resident_array(bam):
     """more than the last-level cache holds, around the number of requests from which they run in two launches; some pages missing"""
     pages = (1 << 17) + 1
