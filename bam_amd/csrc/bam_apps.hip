@@ -425,24 +425,26 @@ bool resident_first(bam_array_t* a, uint64_t n_elems, hipStream_t st)
 
 /*
  * The accesses a reduction or scan of n elements counts with workgroups of `half` threads when all is resident: thread t of
- * a workgroup reads elements t and t + half of its 2 half, one access each unless they lie on the same page.  In groups of
- * 64 elements, which lie on one page and in one half; where the groups' places in a page and in a workgroup repeat, one
- * period stands for all.
+ * a workgroup reads elements t and t + half of its 2 half, one access each unless they lie on the same page.  The second
+ * elements on another page than their first are those within `half` behind a page boundary; where boundaries lie in a
+ * workgroup repeats, and one period stands for all that are complete.
  */
 uint64_t paired_accesses(uint64_t n, uint64_t half, uint64_t page_elems)
 {
-    const uint64_t b = half / 64, epg = page_elems / 64;
-    auto of_group = [&](uint64_t g) -> uint64_t {
-        if (g / b & 1 || g * 64 >= n) return 0;
-        const uint64_t e2 = (g + b) * 64;
-        return std::min<uint64_t>(64, n - g * 64) + (g / epg != (g + b) / epg && e2 < n ? std::min<uint64_t>(64, n - e2) : 0);
+    if (half >= page_elems) return n;
+    auto behind = [&](uint64_t boundary) {
+        const uint64_t in_half = boundary % half, lo = boundary / half & 1 ? boundary : boundary + half - in_half, hi = boundary / half & 1 ? boundary + half - in_half : boundary + half;
+        return std::min(hi, n) - std::min(lo, n);
     };
-    uint64_t period = 2 * b;
-    while (period % epg) period += 2 * b;
-    const uint64_t groups = (n + 63) / 64, whole = groups > b + 1 ? (groups - b - 1) / period : 0;      /* periods whose pairs are all complete */
-    uint64_t total = 0;
-    if (whole) { for (uint64_t g = 0; g < period; g++) total += of_group(g); total *= whole; }
-    for (uint64_t g = whole * period; g < groups; g++) total += of_group(g);
+    uint64_t total = n / (2 * half) * half + std::min(half, n % (2 * half)), period = 1;
+    while (period * page_elems % (2 * half)) period++;
+    const uint64_t complete = n > half ? (n - half) / page_elems / period * period : 0;
+    if (complete) {
+        uint64_t one = 0;
+        for (uint64_t k = 1; k <= period; k++) one += behind(k * page_elems);
+        total += one * (complete / period);
+    }
+    for (uint64_t k = complete + 1; k * page_elems < n; k++) total += behind(k * page_elems);
     return total;
 }
 
