@@ -123,7 +123,7 @@ def test_gathers_from_a_large_resident_array(bam):
 
 
 def test_gathers_on_several_streams_of_one_array(bam):
-    """Six streams (more than the sets of notes an array keeps) gather from one array at once, each its own requests."""
+    """Six streams gather from one array at once, page by page, each its own requests and with notes of its own."""
     import torch
     pages, n = 9000, 60001
     n_elems = pages * 512

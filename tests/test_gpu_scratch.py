@@ -23,8 +23,8 @@ def _read_into(a, n, d_idx, out, shape=0):
 @pytest.mark.parametrize("shape", [0, 3])
 @pytest.mark.parametrize("cache_pages", [4096, 4400])
 def test_captured_reads_hold_nothing_of_the_array(bam, cache_pages, shape):
-    """a read recorded into a graph and replayed after, and between, calls on more streams than an array keeps notes for and
-    larger calls on the stream it was recorded on; the array larger than its cache, and resident"""
+    """a read recorded into a graph and replayed after, and between, larger calls on the stream it was recorded on and on seven
+    others; the array larger than its cache, and resident"""
     import torch
     pages, n = 4400, (1 << 16) + 77
     words = oracle.store(SEED, 0, pages * 512)
@@ -100,8 +100,8 @@ def test_two_threads_on_the_stream_of_each_thread(bam):
 
 
 def test_many_streams_by_turns(bam):
-    """gathers and reductions on seventy streams by turns, more than sets of scratch are kept for: a second round allocates
-    nothing, and every result is right"""
+    """reductions on seventy streams by turns, more than sets of scratch are kept for, with gathers that need none between them: a
+    second round allocates nothing, and every result is right"""
     import torch
     pages = 4400
     n_elems = pages * 512
