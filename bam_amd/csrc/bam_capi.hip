@@ -1484,15 +1484,31 @@ namespace {
  * that takes 64 pages from each of 32 waves and has room for as many again.  Where all requests are on their way together,
  * only if the pages missing are far more than the cache holds and are asked for often (request by request / page by page, ms:
  * 2^24 elements behind half of them, 2^16 to 2^18 requests 1.4 / 1.7 to 1.6 / 1.8; behind a quarter 2^16 requests 3.0 / 3.8, 2^17
- * 7.7 / 4.6; 2^26 elements behind a quarter 2^17 requests 5.2 / 5.7, 2^18 11.3 / 7.6).  Beyond that always: 2^19 requests,
- * half cached: 2^24 elements 1.77 / 1.77, 2^26 6.7 / 5.4, 2^28 13.4 / 13.9, 2^22 requests 25 / 20; a quarter cached 32 / 4.5,
- * 20.7 / 8.3, 22 / 20.
+ * 7.7 / 4.6; 2^26 elements behind a quarter 2^17 requests 5.2 / 5.7, 2^18 11.3 / 7.6).
+ *   Beyond that always where the cache holds less than two fifths (2^19 requests, a quarter cached, 2^24, 2^26, 2^28 elements: 32 / 4.5,
+ * 20.7 / 8.3, 22 / 20), and otherwise where many pages are missing: a stretch ends with a batch that is waited for, and with few
+ * missing the requests of two launches bring them in before pages are short (reads, two launches / page by page, ms, 2^18, 2^19,
+ * 2^20, 2^22 of them; pages behind a cache of so many: 8192 / 4096 0.79 1.35, 0.80 1.32, 1.18 1.36, 1.28 1.46; 16384 / 8192 1.05
+ * 1.39, 1.05 1.36, 1.34 1.41, 1.45 1.50; 32768 / 24576 1.02 1.50, 1.10 1.53, 1.05 1.50, 1.37 1.58; 32768 / 16384 1.65 1.73, 1.73 1.69,
+ * 1.79 1.68, 1.95 1.79; 65536 / 49152 1.65 1.78, 1.93 1.93, 1.77 2.00, 1.95 2.10; 65536 / 40960 2.35 2.54, 2.68 2.54, 2.46 2.52, 2.57 2.58;
+ * 65536 / 32768 2.88 2.77, 3.31 2.82, 3.19 2.72, 3.31 2.82; 131072 / 98304 1.90 1.54, 4.16 2.77, 3.37 3.02, 3.22 3.27).
+ *   Between two fifths and half there are three stretches, 2.4 to 2.8 ms for few pages, and two launches get slower with the requests
+ * and with what the array has beyond twice the cache (the same for 2^17, 2^18, 2^19, 2^22; 8232 / 4096 0.61 2.45, 0.78 2.57, 1.00
+ * 2.43, 2.42 2.54; 9216 / 4096 0.75 2.41, 0.94 2.40, 1.93 2.41, 9.57 2.57; 10240 / 4096 1.21 2.44, 1.48 2.51, 3.97 2.49, 27 2.6; 18432 / 8192
+ * 1.15 2.47, 1.33 2.56, 2.71 2.56, 13.8 2.6; 20480 / 8192 2.54 2.56, 2.68 2.55, 6.91 2.64, 41 2.7; 40960 / 16384, 2^18 on, 5.46 2.91, 10.9 3.0;
+ * 65863 / 32768 2.99 3.44, 3.72 3.45; 73728 / 32768 3.48 4.01, 5.80 3.84; 131727 / 65536 4.21 4.22, 6.53 5.50).
  */
 bool page_by_page(const range_d_t<uint64_t>& range, uint64_t n_reqs)
 {
     const uint64_t pages = range.page_count, cache_pages = range.cache.n_pages;
     if (pages <= cache_pages || n_reqs < pages / 2 || cache_pages < 4096) return false;
-    return pages > 2 * cache_pages ? n_reqs >= BAM_REQS_AT_A_TIME || n_reqs >= 4 * pages : n_reqs > BAM_REQS_AT_A_TIME;
+    const uint64_t missing = pages - cache_pages;
+    if (2 * pages > 5 * cache_pages) return n_reqs >= BAM_REQS_AT_A_TIME || n_reqs >= 4 * pages;
+    if (pages > 2 * cache_pages) {
+        const uint64_t beyond = (n_reqs >> 17) * (pages - 2 * cache_pages);
+        return missing >= 24576 ? n_reqs >= 3ull << 17 || beyond >= cache_pages : beyond > cache_pages;
+    }
+    return n_reqs > BAM_REQS_AT_A_TIME && missing >= (pages == 2 * cache_pages ? 16384 : 24576);
 }
 /*
  * Whether a gather is better off as several launches than as one that can miss; they keep notes between launches, which a

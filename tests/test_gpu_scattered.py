@@ -14,7 +14,12 @@ IN_FLIGHT = 1 << 18        # requests that are on their way together in a launch
 def _page_by_page(pages, cache_pages, n):
     if pages <= cache_pages or 2 * n < pages - 1 or cache_pages < 4096:
         return False
-    return n >= IN_FLIGHT or n >= 4 * pages if pages > 2 * cache_pages else n > IN_FLIGHT
+    if 2 * pages > 5 * cache_pages:
+        return n >= IN_FLIGHT or n >= 4 * pages
+    if pages > 2 * cache_pages:
+        beyond = (n >> 17) * (pages - 2 * cache_pages)
+        return n >= 3 << 17 or beyond >= cache_pages if pages - cache_pages >= 24576 else beyond > cache_pages
+    return n > IN_FLIGHT and pages - cache_pages >= (16384 if pages == 2 * cache_pages else 24576)
 
 
 # pages of data and of cache: everything resident; just below and at the smallest cache that is fetched for page by page, one
@@ -22,7 +27,10 @@ def _page_by_page(pages, cache_pages, n):
 @pytest.mark.parametrize("pages,cache_pages,n", [(4096, 4096, (1 << 20) + 1), (4100, 4095, 1 << 14), (4100, 4096, (1 << 14) - 1), (4100, 4096, (1 << 14) + 77),
                                                  (12289, 4096, 100003), (12289, 5000, (1 << 20) - 1), (40000, 4096, 19999), (40000, 4096, 20001),
                                                  (4100, 4095, IN_FLIGHT + 1), (4100, 4096, IN_FLIGHT), (4100, 4096, IN_FLIGHT + 1), (8192, 4096, IN_FLIGHT), (8193, 4096, 4 * 8193 - 1),
-                                                 (8193, 4096, 4 * 8193), (70000, 8192, IN_FLIGHT - 1), (70000, 8192, IN_FLIGHT), (70000, 8192, IN_FLIGHT + 65)])
+                                                 (8193, 4096, 4 * 8193), (70000, 8192, IN_FLIGHT - 1), (70000, 8192, IN_FLIGHT), (70000, 8192, IN_FLIGHT + 65),
+                                                 (8193, 4096, IN_FLIGHT + 1), (10240, 4096, (1 << 17) * 3 - 1), (10240, 4096, (1 << 17) * 3), (10241, 4096, IN_FLIGHT - 1), (10241, 4096, IN_FLIGHT), (32766, 16383, IN_FLIGHT + 1), (32768, 16384, IN_FLIGHT), (32768, 16384, IN_FLIGHT + 1),
+                                                 (57344, 32769, IN_FLIGHT + 1), (57344, 32768, IN_FLIGHT + 1),
+                                                 (40960, 16384, IN_FLIGHT - 1), (40960, 16384, IN_FLIGHT), (40000, 15424, 3 << 17)])
 def test_scattered_reads_element_by_element(bam, pages, cache_pages, n):
     """Every element of a gather and the sum of the same requests, twice (the second call finds what the first left behind),
     with a few requests outside the array (they read as 0 and are not counted) and a skewed half; every request inside is
@@ -63,7 +71,7 @@ def test_scattered_reads_of_ranges_that_begin_inside_a_page(bam, page, first, of
     cache, requests in front of the range and behind it among them (they read as 0)"""
     from bam_amd import Array, PageCache, Range
     per = page // 8
-    pages, n = 9001, IN_FLIGHT + 77
+    pages, n = 10300, IN_FLIGHT + 77
     n_elems = (pages * page - offset) // 8 - 3
     if page == 65536:
         pages, n_elems = 4500, 4500 * per - offset // 8 - 3
@@ -93,7 +101,7 @@ def test_counters_of_reads_in_two_launches(bam):
     """requests that the first launch leaves count by what they find in the second: of 2^22 for one page that is on the store, those
     looked at once it is there are hits, in several times as many waves as the device holds; page by page none is"""
     n = 1 << 22
-    for pages, cache_pages, by_page in ((600, 512, False), (4200, 4096, True)):
+    for pages, cache_pages, by_page in ((600, 512, False), (4200, 4096, False), (10300, 4096, True)):
         with Rig(bam, pages * 4096, n_queues=16, depth=256) as r:
             a = r.array(pages * 512, 4096, cache_pages)
             assert _page_by_page(pages, cache_pages, n) == by_page
@@ -125,7 +133,7 @@ def test_gathers_from_a_large_resident_array(bam):
 def test_gathers_on_several_streams_of_one_array(bam):
     """Six streams gather from one array at once, page by page, each its own requests and with notes of its own."""
     import torch
-    pages, n = 9000, 60001
+    pages, n = 10300, 60001
     n_elems = pages * 512
     words = oracle.store(SEED, 0, n_elems)
     rng = np.random.default_rng(5)
