@@ -567,11 +567,9 @@ __device__ __forceinline__ unsigned long long cc_root(unsigned long long* comp, 
     }
     return v;
 }
-__device__ __forceinline__ void cc_join(unsigned long long* comp, const uint64_t a, const uint64_t b)
+/* the trees that u and v are in */
+__device__ __forceinline__ void cc_join_trees(unsigned long long* comp, unsigned long long u, unsigned long long v)
 {
-    /* most edges join what is joined already, and once the chains are short both ends name the same vertex: two loads side by side */
-    unsigned long long u = bam::ld_relaxed(comp + a), v = bam::ld_relaxed(comp + b);
-    if (u == v) return;
     u = cc_root(comp, u); v = cc_root(comp, v);
     while (u != v) {
         if (u < v) { const unsigned long long t = u; u = v; v = t; }
@@ -579,6 +577,12 @@ __device__ __forceinline__ void cc_join(unsigned long long* comp, const uint64_t
         if (was == u) break;
         u = cc_root(comp, was);
     }
+}
+__device__ __forceinline__ void cc_join(unsigned long long* comp, const uint64_t a, const uint64_t b)
+{
+    /* most edges join what is joined already, and once the chains are short both ends name the same vertex: two loads side by side */
+    const unsigned long long u = bam::ld_relaxed(comp + a), v = bam::ld_relaxed(comp + b);
+    if (u != v) cc_join_trees(comp, u, v);
 }
 __global__ void k_cc_settle(unsigned long long* comp, uint64_t vertex_count)
 {
@@ -627,7 +631,8 @@ __global__ void k_page_first_vertex(const uint64_t* offsets, uint64_t n_vertices
 }
 
 /*
- * One wave, `ppw` consecutive pages of the edge array per trip (lane l looks after page l of the trip), trips
+ * For PageRank, and for BFS and components where a page is smaller than 4 KiB or larger than 64 (else k_along_resident):
+ * one wave, `ppw` consecutive pages of the edge array per trip (lane l looks after page l of the trip), trips
  * handed out wave by wave along the array.  A page is wanted when one of its vertices is active; the wanted pages
  * of a trip are taken with one acquire, so their misses go to the store as one batch of commands, and the whole
  * wave then walks the active vertices of each page, 64 edges at a time, before the references are dropped.
@@ -724,6 +729,318 @@ __global__ __launch_bounds__(64) void k_cc_by_page(array_d_t<uint64_t>* da, cons
                   [&](uint64_t src, uint64_t next, uint64_t) { cc_join(comp, src, next); });
 }
 
+// ---- BFS / CC along the edge array, what is resident first ----
+/*
+ * A reading of the edge array in two launches.  The first visits the pages that are wanted and resident, and lists the
+ * wanted ones that are not; the second fetches those in batches of up to 64 commands and visits them.  Front to back,
+ * whatever is resident, a sweep over an array larger than its cache pushes out what it has not reached yet: of 27 800
+ * cached and wanted pages of 118 000 (2^21 vertices, a power-law graph) it found 1 000.  The list also makes every batch
+ * but the last a whole one whichever pages are wanted, where a wave that looks after a run of neighbouring pages sends as many
+ * commands as the cache has pages for each wave (seven there, 9 M pages/s; batches of 64 reach 13).
+ *
+ * Both launches take a segment at a time: 512 entries, eight rows of 64, one per lane and row, all loaded before any is
+ * used; which entries are to be visited, and for which vertex, is worked out in LDS while they are on their way.  The
+ * pages are referenced meanwhile (a take and a drop per page and wave; a page is 512 entries).
+ * Bound by the store where edges are missing: BFS of that graph 19.2 -> 10.9 ms (175 000 -> 124 000 page reads, 11.6 M a second),
+ * with 2^18 vertices 4.8 -> 1.8; components of 2^22 vertices, 8 entries each, half cached, 4.7 -> 3.8.  All cached, by the
+ * trips to memory a wave makes one after the other: BFS of 2^20 vertices 1.65 -> 0.47 ms, components of 2^22 1.55 -> 1.2.
+ */
+#define BAM_SEG_ROWS 8u
+#define BAM_SEG_EDGES (BAM_SEG_ROWS * BAM_WAVE_SIZE)
+#define BAM_TRIP_SEGS 16u
+#define BAM_TRIP_WAVES 4u                       /* waves to a workgroup of the first launch: they share an add to the list */
+struct along_t {
+    const uint64_t* offsets;
+    const uint64_t* first;                      /* [n_segs + 1] the vertex whose list holds the segment's first entry */
+    uint64_t n_edges, n_pages, n_segs;
+    uint32_t seg_log;                           /* log2 of the segments in a page, at most that of BAM_TRIP_SEGS */
+    uint32_t trip_segs;                         /* segments a wave of the first launch looks after: whole pages, BAM_TRIP_SEGS at most */
+    uint32_t* missing;                          /* [n_pages] the pages the first launch leaves to the second */
+    unsigned long long* n_missing;              /* zero between sweeps, like the next one */
+    unsigned long long* next_chunk;             /* of the list, for the waves of the second launch */
+    uint64_t* ahead;                            /* [n_segs * BAM_SEG_ROWS] a bit per entry (bfs_along) */
+    unsigned long long* flags;                  /* [2] what the sweep tells the host */
+};
+/* written and read by the lanes of one wave, which runs its LDS operations in order */
+__device__ __forceinline__ void wave_lds_fence()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+__device__ __forceinline__ void raise_flag(unsigned long long* flag, const bool mine)
+{
+    const uint64_t m = bam::ballot(mine);
+    if (m && bam::lane() == bam::first_lane(m) && bam::ld_relaxed(flag) == 0) bam::st_relaxed(flag, 1ull);
+}
+
+/*
+ * One level of BFS.  AHEAD: the entries of vertices found on this very level are visited along with those of the level
+ * itself where their page is at hand anyway; the neighbours they find are two levels on, as far as is known (somebody nearer
+ * may still be looking at them, hence the minimum), and are not visited from before the next level, when their labels are
+ * settled.  A bit per entry says that it has been visited ahead of its level, so that the next one does not bring the page in for
+ * it: 43 300 page reads instead of 34 200 without it on a 2^19-vertex power-law graph, a quarter of the edges cached.  The bits of
+ * a segment are those of the last sweep that visited it: of older levels' entries nobody asks.
+ */
+template <bool AHEAD>
+struct bfs_along {
+    uint32_t* label;
+    uint32_t level;
+    static constexpr uint64_t most_blocks = 1ull << 31;
+    struct lds_t { unsigned long long now[BAM_TRIP_SEGS * BAM_SEG_ROWS], next[AHEAD ? BAM_TRIP_SEGS * BAM_SEG_ROWS : 1]; };
+
+    static __device__ __forceinline__ void mark(unsigned long long* bits, const uint32_t a, const uint32_t b, const bool mine)      /* entries [a, b), b > a where mine */
+    {
+        const uint32_t lane = bam::lane(), wa = a / BAM_WAVE_SIZE, wb = mine ? (b - 1) / BAM_WAVE_SIZE : wa;
+        const bool wide = mine && wb - wa >= 4;
+        if (mine && !wide)
+            for (uint32_t w = wa; w <= wb; w++)
+                atomicOr(bits + w, (w == wa ? ~0ull << (a % BAM_WAVE_SIZE) : ~0ull) & (w == wb ? ~0ull >> (63 - (b - 1) % BAM_WAVE_SIZE) : ~0ull));
+        for (uint64_t m = bam::ballot(wide); m; m &= m - 1) {
+            const uint32_t j = bam::first_lane(m), ja = bam::bcast(a, j), jb = bam::bcast(b, j) - 1;
+            for (uint32_t w = ja / BAM_WAVE_SIZE + lane; w <= jb / BAM_WAVE_SIZE; w += BAM_WAVE_SIZE)
+                atomicOr(bits + w, (w == ja / BAM_WAVE_SIZE ? ~0ull << (ja % BAM_WAVE_SIZE) : ~0ull) & (w == jb / BAM_WAVE_SIZE ? ~0ull >> (63 - jb % BAM_WAVE_SIZE) : ~0ull));
+        }
+    }
+    /* which of the n_segs segments from seg0 on are wanted; s is ready for visit() of any of them */
+    __device__ __forceinline__ uint32_t prepare(const along_t& g, lds_t& s, const uint64_t seg0, const uint32_t n_segs) const
+    {
+        const uint32_t lane = bam::lane(), n_words = n_segs * BAM_SEG_ROWS;
+        wave_lds_fence();                       /* what was read there before has been read */
+        for (uint32_t w = lane; w < n_words; w += BAM_WAVE_SIZE) { s.now[w] = 0; if (AHEAD) s.next[w] = 0; }
+        wave_lds_fence();
+        const uint64_t e0 = seg0 * BAM_SEG_EDGES, e1 = e0 + n_segs * BAM_SEG_EDGES < g.n_edges ? e0 + n_segs * BAM_SEG_EDGES : g.n_edges;
+        const uint64_t v_last = g.first[seg0 + n_segs];
+        for (uint64_t vbase = g.first[seg0]; vbase <= v_last; vbase += 4 * BAM_WAVE_SIZE) {
+            /* four vertices to a lane at a time: most sweeps find few or none of their level, and are the trips of these loads */
+            uint32_t l[4];
+#pragma unroll
+            for (uint32_t q = 0; q < 4; q++) { const uint64_t v = vbase + q * BAM_WAVE_SIZE + lane; l[q] = v <= v_last ? bam::ld_relaxed(label + v) : MYINFINITY; }
+#pragma unroll
+            for (uint32_t q = 0; q < 4; q++) {
+                const uint64_t v = vbase + q * BAM_WAVE_SIZE + lane;
+                bool mine = l[q] == level || (AHEAD && l[q] == level + 1);
+                if (!bam::ballot(mine)) continue;
+                uint64_t es = 0, ee = 0;
+                if (mine) { es = g.offsets[v]; ee = g.offsets[v + 1]; }
+                if (es < e0) es = e0;
+                if (ee > e1) ee = e1;
+                mine = mine && ee > es;
+                const uint32_t a = (uint32_t)(es - e0), b = (uint32_t)(ee - e0);
+                mark(s.now, a, b, mine && l[q] == level);
+                if (AHEAD) mark(s.next, a, b, mine && l[q] != level);
+            }
+        }
+        wave_lds_fence();
+        uint64_t any = 0;                       /* bit k: word 64 q + k of turn q is not empty; a segment is a byte of it */
+        uint32_t wanted = 0;
+        for (uint32_t w0 = 0; w0 < n_words; w0 += BAM_WAVE_SIZE) {
+            const uint32_t w = w0 + lane;
+            unsigned long long now = w < n_words ? s.now[w] : 0ull;
+            if constexpr (AHEAD) {
+                const unsigned long long next = w < n_words ? s.next[w] : 0ull;
+                if (now | next) {
+                    const unsigned long long seen = g.ahead[seg0 * BAM_SEG_ROWS + w];
+                    now &= ~seen;
+                    s.now[w] = now;
+                    s.next[w] = next & ~seen;
+                }
+            }
+            any = bam::ballot(now != 0);
+            for (uint32_t k = 0; k < BAM_WAVE_SIZE / BAM_SEG_ROWS; k++)
+                if ((any >> (k * BAM_SEG_ROWS)) & ((1u << BAM_SEG_ROWS) - 1u)) wanted |= 1u << (w0 / BAM_SEG_ROWS + k);
+        }
+        wave_lds_fence();
+        return wanted;
+    }
+    /* the entries of the segment, the k-th of those prepared: lane l holds entry 64 r + l in id[r] */
+    __device__ __forceinline__ void visit(const along_t& g, lds_t& s, const uint64_t seg, const uint32_t k, const uint64_t (&id)[BAM_SEG_ROWS], bool& found, bool& found_ahead) const
+    {
+        const uint32_t lane = bam::lane();
+        uint32_t have[BAM_SEG_ROWS];
+        unsigned long long all[BAM_SEG_ROWS], next[BAM_SEG_ROWS];
+#pragma unroll
+        for (uint32_t r = 0; r < BAM_SEG_ROWS; r++) {
+            next[r] = AHEAD ? bam::first((uint64_t)s.next[k * BAM_SEG_ROWS + r]) : 0ull;
+            all[r] = bam::first((uint64_t)s.now[k * BAM_SEG_ROWS + r]) | next[r];
+            have[r] = 0;
+            if ((all[r] >> lane) & 1) have[r] = bam::ld_relaxed(label + id[r]);
+        }
+#pragma unroll
+        for (uint32_t r = 0; r < BAM_SEG_ROWS; r++) {
+            const bool on = AHEAD && ((next[r] >> lane) & 1);
+            const uint32_t to = level + 1u + (on ? 1u : 0u);
+            if (have[r] > to) {                 /* (zero where the lane has nothing to visit) */
+                if (AHEAD) __hip_atomic_fetch_min(label + id[r], to, __ATOMIC_RELAXED, BAM_AGENT);
+                else bam::st_relaxed(label + id[r], to);
+                found |= !on; found_ahead |= on;
+            }
+        }
+        if (AHEAD && lane < BAM_SEG_ROWS) g.ahead[seg * BAM_SEG_ROWS + lane] = s.next[k * BAM_SEG_ROWS + lane];
+    }
+};
+
+/* connected components: every entry is visited once, with the vertex whose list it is in */
+struct cc_along {
+    unsigned long long* comp;
+    /* chains grow with the edges that are joined at a time: 2^22 vertices, all cached, 2.6 ms with 16384 waves, 1.45 with 4096, 1.48
+     * with 2048, 1.6 with 1024 */
+    static constexpr uint64_t most_blocks = 4096 / BAM_TRIP_WAVES;
+    struct lds_t { unsigned long long starts[BAM_SEG_ROWS]; uint32_t vertex[BAM_SEG_EDGES]; };      /* where lists begin; whose, from the segment's first vertex on */
+    __device__ __forceinline__ uint32_t prepare(const along_t&, lds_t&, const uint64_t, const uint32_t n_segs) const { return (1u << n_segs) - 1u; }
+    __device__ __forceinline__ void visit(const along_t& g, lds_t& s, const uint64_t seg, const uint32_t, const uint64_t (&id)[BAM_SEG_ROWS], bool&, bool&) const
+    {
+        const uint32_t lane = bam::lane();
+        const uint64_t e0 = seg * BAM_SEG_EDGES, e1 = e0 + BAM_SEG_EDGES < g.n_edges ? e0 + BAM_SEG_EDGES : g.n_edges;
+        const uint64_t v0 = g.first[seg], v_last = g.first[seg + 1];
+        wave_lds_fence();
+        if (lane < BAM_SEG_ROWS) s.starts[lane] = lane ? 0ull : 1ull;
+        if (lane == 0) s.vertex[0] = 0;
+        wave_lds_fence();
+        for (uint64_t vbase = v0 + 1; vbase <= v_last; vbase += BAM_WAVE_SIZE) {
+            const uint64_t v = vbase + lane;
+            uint64_t es = 0, ee = 0;
+            if (v <= v_last) { es = g.offsets[v]; ee = g.offsets[v + 1]; }
+            if (ee > es && es >= e0 && es < e1) {
+                const uint32_t a = (uint32_t)(es - e0);
+                s.vertex[a] = (uint32_t)(v - v0);
+                atomicOr(s.starts + a / BAM_WAVE_SIZE, 1ull << (a % BAM_WAVE_SIZE));
+            }
+        }
+        wave_lds_fence();
+        uint32_t begin = 0;                     /* the last list that begins before the row */
+        unsigned long long u[BAM_SEG_ROWS], w[BAM_SEG_ROWS];
+        /* most entries join what is joined already, and once the chains are short both ends name the same vertex: the loads
+         * of all rows side by side.  A word read a while ago still names an ancestor. */
+#pragma unroll
+        for (uint32_t r = 0; r < BAM_SEG_ROWS; r++) {
+            const uint64_t m = bam::first((uint64_t)s.starts[r]), below = m & (~0ull >> (63 - lane));
+            const uint64_t src = v0 + s.vertex[below ? r * BAM_WAVE_SIZE + 63u - (uint32_t)__builtin_clzll(below) : begin];
+            if (m) begin = r * BAM_WAVE_SIZE + 63u - (uint32_t)__builtin_clzll(m);
+            u[r] = w[r] = 0;
+            if (e0 + r * BAM_WAVE_SIZE + lane < e1) { u[r] = bam::ld_relaxed(comp + src); w[r] = bam::ld_relaxed(comp + id[r]); }
+        }
+#pragma unroll
+        for (uint32_t r = 0; r < BAM_SEG_ROWS; r++) {
+            /* the rows before may have joined these two (or given what they name a parent): all cached, 1.56 -> 1.45 ms */
+            if (r && u[r] != w[r]) { u[r] = bam::ld_relaxed(comp + u[r]); w[r] = bam::ld_relaxed(comp + w[r]); }
+            if (u[r] != w[r]) cc_join_trees(comp, u[r], w[r]);
+        }
+    }
+};
+
+/* a workgroup takes trips of 16 segments at most, a wave each, until there are none left */
+template <typename A>
+__global__ __launch_bounds__(BAM_TRIP_WAVES * BAM_WAVE_SIZE) void k_along_resident(array_d_t<uint64_t>* da, const along_t g, const A algo)
+{
+    __shared__ typename A::lds_t lds[BAM_TRIP_WAVES];
+    __shared__ uint32_t left[BAM_TRIP_WAVES];
+    __shared__ unsigned long long base;
+    const uint32_t lane = bam::lane(), w_in_block = bam::first(threadIdx.x / BAM_WAVE_SIZE);
+    typename A::lds_t& s = lds[w_in_block];
+    bam::range_view<uint64_t> view;
+    view.load(da->d_ranges);
+    bool found = false, found_ahead = false;
+    for (uint64_t blk = blockIdx.x; blk * BAM_TRIP_WAVES * g.trip_segs < g.n_segs; blk += gridDim.x) {
+        const uint64_t trip = blk * BAM_TRIP_WAVES + w_in_block, seg0 = trip * g.trip_segs;
+        const uint64_t p0 = seg0 >> g.seg_log;
+        bool miss = false;
+        if (seg0 < g.n_segs) {
+            const uint32_t n_segs = (uint32_t)(g.n_segs - seg0 < g.trip_segs ? g.n_segs - seg0 : g.trip_segs);
+            const uint32_t wanted = algo.prepare(g, s, seg0, n_segs);
+            /* lane j: the trip's j-th page */
+            const uint32_t per = 1u << g.seg_log;
+            const bool want = lane < (g.trip_segs >> g.seg_log) && ((wanted >> (lane << g.seg_log)) & ((1u << per) - 1u)) != 0;
+            data_page_t* const dp = view.pages + (view.pso >> view.page_size_log) + p0 + (want ? lane : 0);
+            uint64_t sv = 0;
+            uint32_t slot = 0;
+            bool have = false;
+            if (want && ((bam::ld_relaxed(&dp->state)) >> (CNT_SHIFT + 1)) == V_NB) {
+                have = bam_try_hit(dp, 1, false, sv, slot);
+                if (!have) __hip_atomic_fetch_add(&dp->state, 0u - 1u, __ATOMIC_RELAXED, BAM_AGENT);      /* it went in between: not waited for here */
+            }
+            miss = want && !have;
+            view.n_access += have ? 1u : 0u;
+            view.n_hit = view.n_access;
+            for (uint64_t m = bam::ballot(have); m; m &= m - 1) {
+                const uint32_t j = bam::first_lane(m);
+                const uint64_t* payload = (const uint64_t*)view.slot_addr(bam::bcast(slot, j)) + lane;
+                for (uint32_t k = j << g.seg_log; k < (j + 1) << g.seg_log; k++) {
+                    if (!((wanted >> k) & 1)) continue;
+                    const uint64_t* const at = payload + (k & (per - 1u)) * BAM_SEG_EDGES;
+                    uint64_t id[BAM_SEG_ROWS];
+#pragma unroll
+                    for (uint32_t r = 0; r < BAM_SEG_ROWS; r++) id[r] = bam::ld_payload(at + r * BAM_WAVE_SIZE);
+                    algo.visit(g, s, seg0 + k, k, id, found, found_ahead);
+                }
+            }
+            if (have) bam_release_refs(dp, 1, false);
+        }
+        const uint64_t mm = bam::ballot(miss);
+        if (lane == 0) left[w_in_block] = bam::popc(mm);
+        __syncthreads();
+        uint32_t before = 0, total = 0;
+#pragma unroll
+        for (uint32_t k = 0; k < BAM_TRIP_WAVES; k++) { if (k < w_in_block) before += left[k]; total += left[k]; }
+        if (threadIdx.x == 0 && total) base = __hip_atomic_fetch_add(g.n_missing, (unsigned long long)total, __ATOMIC_RELAXED, BAM_AGENT);
+        __syncthreads();
+        if (miss) g.missing[base + before + bam::popc(mm & bam::lanes_below(lane))] = (uint32_t)(p0 + lane);
+    }
+    view.flush_stats();
+    raise_flag(g.flags, found);
+    raise_flag(g.flags + 1, found_ahead);
+}
+
+/* a wave holds at most `chunk` pages at a time; the launch keeps waves x chunk under half the cache */
+template <typename A>
+__global__ __launch_bounds__(BAM_WAVE_SIZE) void k_along_missing(array_d_t<uint64_t>* da, const along_t g, const A algo, const uint32_t chunk)
+{
+    __shared__ typename A::lds_t s;
+    const uint64_t n = *g.n_missing;
+    if (!n) return;
+    const uint32_t lane = bam::lane();
+    bam::range_view<uint64_t> view;
+    view.load(da->d_ranges);
+    view.place = BAM_PLACE_PULLED;
+    const uint64_t pso_pages = view.pso >> view.page_size_log;
+    bool found = false, found_ahead = false;
+    for (;;) {
+        uint64_t c = 0;
+        if (lane == 0) c = __hip_atomic_fetch_add(g.next_chunk, 1ull, __ATOMIC_RELAXED, BAM_AGENT) * chunk;
+        c = bam::bcast(c, 0);
+        if (c >= n) break;
+        const bool want = lane < chunk && c + lane < n;
+        const uint64_t p = g.missing[want ? c + lane : c];
+        uint32_t slot = BAM_NO_SLOT;
+        auto keep = [&](uint32_t s_) { slot = s_; return false; };
+        view.acquire_helped(p + pso_pages, want, false, keep, keep);
+        /* a page whose wait was given up (the controller is marked aborted) has no slot and is not visited */
+        for (uint64_t m = bam::ballot(want && slot != BAM_NO_SLOT); m; m &= m - 1) {
+            const uint32_t j = bam::first_lane(m);
+            const uint64_t seg0 = bam::bcast(p, j) << g.seg_log;
+            const uint64_t* payload = (const uint64_t*)view.slot_addr(bam::bcast(slot, j)) + lane;
+            for (uint32_t k = 0; k < 1u << g.seg_log && seg0 + k < g.n_segs; k++) {
+                uint64_t id[BAM_SEG_ROWS];
+#pragma unroll
+                for (uint32_t r = 0; r < BAM_SEG_ROWS; r++) id[r] = bam::ld_payload(payload + k * BAM_SEG_EDGES + r * BAM_WAVE_SIZE);
+                if (algo.prepare(g, s, seg0 + k, 1)) algo.visit(g, s, seg0 + k, 0, id, found, found_ahead);
+            }
+        }
+        if (want) view.release(p + pso_pages, false);
+    }
+    raise_flag(g.flags, found);
+    raise_flag(g.flags + 1, found_ahead);
+    view.flush_stats();
+}
+
+/* whether any vertex has this label */
+__global__ void k_any_label(const uint32_t* label, const uint64_t n, const uint32_t which, unsigned long long* flag)
+{
+    bool any = false;
+    for (uint64_t v = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; v < n; v += (uint64_t)gridDim.x * blockDim.x) any |= label[v] == which;
+    raise_flag(flag, any);
+}
+
 // ---- PageRank by residual pushes (benchmarks/pagerank/main.cu:107-115 initialize, :252-273 kernel_coalesce_pc, :412-421 update) ----
 __global__ void k_pr_initialize(bool* label, float* delta, float* residual, float* value, const uint64_t vertex_count, const uint64_t* vertexList, float alpha)
 {
@@ -806,10 +1123,12 @@ __global__ void k_sssp_update(bool* label, uint32_t* costList, const uint32_t* n
     }
 }
 
-__global__ void k_iota(unsigned long long* p, uint64_t n)
+/* every vertex by itself, and an empty list of missing pages for the reading behind it (NULL: none) */
+__global__ void k_iota(unsigned long long* p, uint64_t n, unsigned long long* n_missing, unsigned long long* next_chunk)
 {
     const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) p[i] = i;
+    if (i == 0 && n_missing) *n_missing = *next_chunk = 0;
 }
 
 } // namespace
@@ -817,17 +1136,22 @@ __global__ void k_iota(unsigned long long* p, uint64_t n)
 extern "C" {
 
 namespace {
+#define BAM_ALONG_WAVES 512u            /* waves that fetch what is missing, at most: as many as keep the store busy (k_fetch_wanted) */
 /* launch shape of the by-page graph kernels: pages per wave trip and number of waves, so that what the waves hold
  * at any time stays under half of the cache */
 struct by_page_plan { uint64_t n_edges = 0, n_pages = 0; uint32_t epp = 0, ppw = 0, blocks = 0; BufferPtr first; };
 
 /* the end of a level: the device's `changed` word goes to the host through pinned memory, and it and the counter the next
  * sweep takes its work from start the next level at zero.  One small launch instead of two copies and a fill. */
-__global__ void k_level_end(uint64_t* changed, unsigned long long* next_work, volatile uint64_t* host_flag)
+#define BAM_PLAN_WORDS 128u             /* words of a plan: [0] pieces, [1] next piece of work, [2] changed; the others, written by many waves, on lines of their own */
+#define BAM_PLAN_FLAGS 16u              /* along_t::flags */
+#define BAM_PLAN_MISSING 32u            /* along_t::n_missing */
+#define BAM_PLAN_CHUNK 48u              /* along_t::next_chunk */
+__global__ void k_level_end(unsigned long long* words, volatile uint64_t* host_flag)
 {
-    *host_flag = *changed;
-    *changed = 0;
-    *next_work = 0;
+    host_flag[0] = words[2] | words[BAM_PLAN_FLAGS];
+    host_flag[1] = words[BAM_PLAN_FLAGS + 1];
+    words[1] = words[2] = words[BAM_PLAN_FLAGS] = words[BAM_PLAN_FLAGS + 1] = words[BAM_PLAN_MISSING] = words[BAM_PLAN_CHUNK] = 0;
 }
 
 /*
@@ -856,6 +1180,8 @@ struct graph_plan {
     bool cc_backwards() { return !all_cached && (cc_calls++ & 1u) != 0; }
     by_page_plan bp;
     bool bp_built = false;
+    along_t along{};                         /* n_segs = 0: the array or its pages do not qualify */
+    uint32_t along_waves = 0, along_chunk = 0;
     BufferPtr bytes_a, bytes_b, floats_a, floats_b, words_a;      /* per-vertex buffers: flags, PageRank's delta and residual, SSSP's new costs */
     BufferPtr queue_a, queue_b, queue_bits, queue_totals;         /* bam_bfs_frontier: the two queues, the bit map that puts a queue in order and its counts per 4096 vertices */
 
@@ -864,7 +1190,7 @@ struct graph_plan {
         offsets = d_offsets; n_vertices = nv; n_edges = edges->a->adt.n_elems;
         const uint64_t cap = 2 * (n_edges / BAM_HEAVY_EDGES) + 1;
         buf = createBuffer(cap * sizeof(heavy_piece_t), 0);
-        words = createBuffer(64, 0);
+        words = createBuffer(BAM_PLAN_WORDS * sizeof(unsigned long long), 0);
         host_words = createHostBuffer(64);
         pieces = (heavy_piece_t*)buf.get();
         count = (unsigned long long*)words.get();
@@ -882,7 +1208,7 @@ struct graph_plan {
         if (other_cache_pages && other_cache_pages < cache_pages) cache_pages = other_cache_pages;
         if (cache_pages && resident > cache_pages / BAM_WAVE_SIZE) resident = cache_pages / BAM_WAVE_SIZE;
         if (resident < 2) resident = 2;
-        hip_err_chk(hipMemsetAsync(words.get(), 0, 64, st));
+        hip_err_chk(hipMemsetAsync(words.get(), 0, BAM_PLAN_WORDS * sizeof(unsigned long long), st));
         hipLaunchKernelGGL(k_heavy_pieces, dim3(blocks_for(n_vertices, 256)), dim3(256), 0, st, d_offsets, n_vertices, pieces, count);
         hip_err_chk(hipGetLastError());
         unsigned long long n = 0;
@@ -901,7 +1227,7 @@ struct graph_plan {
     /* between sweeps `changed` and the work counter are zero; true if the sweep just queued on `st` changed anything */
     bool level_end(hipStream_t st)
     {
-        hipLaunchKernelGGL(k_level_end, dim3(1), dim3(1), 0, st, changed, count + 1, host_flag);
+        hipLaunchKernelGGL(k_level_end, dim3(1), dim3(1), 0, st, count, host_flag);
         hip_err_chk(hipGetLastError());
         hip_err_chk(hipStreamSynchronize(st));
         return *host_flag != 0;
@@ -936,12 +1262,85 @@ int graph_plan::by_page(bam_array_t* edges, hipStream_t st)
     if (waves > trips) waves = trips;
     pl.ppw = (uint32_t)ppw;
     pl.blocks = (uint32_t)waves;                               /* one wave per workgroup */
-    pl.first = createBuffer((pl.n_pages + 1) * sizeof(uint64_t), dev);
+    const uint64_t segs_per_page = r.cache.page_size / (BAM_SEG_EDGES * 8);
+    const bool in_segs = segs_per_page && segs_per_page <= BAM_TRIP_SEGS && pl.n_pages && pl.n_pages <= 0xFFFFFFFFull;
+    const uint64_t n_segs = in_segs ? (pl.n_edges + BAM_SEG_EDGES - 1) / BAM_SEG_EDGES : 0;
+    /* one allocation: the first vertices of the pages, of the segments where those are not the pages, the bits (only where some
+     * edges are on the store are there sweeps to spare), the list of missing pages */
+    const uint64_t seg_words = segs_per_page > 1 && in_segs ? n_segs + 1 : 0, bit_words = all_cached ? 0 : n_segs * BAM_SEG_ROWS;
+    pl.first = createBuffer((pl.n_pages + 1 + seg_words + bit_words) * sizeof(uint64_t) + (in_segs ? pl.n_pages * sizeof(uint32_t) : 0), dev);
     hipLaunchKernelGGL(k_page_first_vertex, dim3(blocks_for(pl.n_pages + 1, 256)), dim3(256), 0, st, offsets, n_vertices, (uint64_t)pl.epp, pl.n_pages,
                        (uint64_t*)pl.first.get());
+    if (in_segs) {
+        uint64_t* const seg_first = (uint64_t*)pl.first.get() + (seg_words ? pl.n_pages + 1 : 0);
+        uint64_t* const bits = (uint64_t*)pl.first.get() + pl.n_pages + 1 + seg_words;
+        along.offsets = offsets; along.n_edges = pl.n_edges; along.n_pages = pl.n_pages; along.n_segs = n_segs;
+        along.seg_log = (uint32_t)__builtin_ctzll(segs_per_page);
+        along.trip_segs = (uint32_t)segs_per_page;
+        /* a wave's share as small as leaves 16384 waves or more (2^20 vertices, all cached, BFS: 0.47 ms, with 8192 0.50, 4096 0.56, 2048 0.70) */
+        while (along.trip_segs < BAM_TRIP_SEGS && n_segs / along.trip_segs >= 32768) along.trip_segs *= 2;
+        along.first = seg_first;
+        if (seg_words)
+            hipLaunchKernelGGL(k_page_first_vertex, dim3(blocks_for(n_segs + 1, 256)), dim3(256), 0, st, offsets, n_vertices, (uint64_t)BAM_SEG_EDGES, n_segs, seg_first);
+        along.ahead = bit_words ? bits : nullptr;
+        along.missing = (uint32_t*)(bits + bit_words);
+        along.n_missing = count + BAM_PLAN_MISSING;
+        along.next_chunk = count + BAM_PLAN_CHUNK;
+        along.flags = count + BAM_PLAN_FLAGS;
+        /* as many waves as leave each a batch worth sending (pages a wave, ms: 29 500 cached, BFS of 2^21 vertices 64 11.8, 32 11.4, 16
+         * 11.6, 8 11.9; 7 500, 2^19 16 3.18, 8 3.11, 4 3.27; 3 700, 2^18 16 1.89, 8 1.73, 4 1.79; 2 048, 2^16 16 0.88, 8 0.72, 4 0.62, 2 0.70) */
+        along_chunk = 32;
+        while (along_chunk > 4 && budget / along_chunk < 256) along_chunk /= 2;
+        along_waves = (uint32_t)std::min<uint64_t>(BAM_ALONG_WAVES, std::max<uint64_t>(1, budget / along_chunk));
+        if (along_chunk > budget) along_chunk = (uint32_t)budget;
+    }
     hip_err_chk(hipGetLastError());
     bp_built = true;
     return 0;
+}
+
+extern "C++" {
+/* one reading of the edge array, or of what the algorithm wants of it */
+template <typename A>
+void along_sweep(bam_array_t* edges, const graph_plan* pl, const A& algo, hipStream_t st)
+{
+    const uint64_t trips = (pl->along.n_segs + pl->along.trip_segs - 1) / pl->along.trip_segs;
+    const uint32_t blocks = (uint32_t)std::min<uint64_t>(A::most_blocks, (trips + BAM_TRIP_WAVES - 1) / BAM_TRIP_WAVES);
+    hipLaunchKernelGGL(k_along_resident<A>, dim3(blocks), dim3(BAM_TRIP_WAVES * BAM_WAVE_SIZE), 0, st, edges->a->d_array_ptr, pl->along, algo);
+    hipLaunchKernelGGL(k_along_missing<A>, dim3(pl->along_waves), dim3(BAM_WAVE_SIZE), 0, st, edges->a->d_array_ptr, pl->along, algo, pl->along_chunk);
+    hip_err_chk(hipGetLastError());
+}
+}
+
+/* all levels from labels of which the source's is set; the number of levels there are */
+uint32_t bfs_along_levels(bam_array_t* edges, graph_plan* pl, uint32_t* d_labels, hipStream_t st)
+{
+    const bool ahead = pl->along.ahead != nullptr;
+    if (ahead) hip_err_chk(hipMemsetAsync(pl->along.ahead, 0, pl->along.n_segs * BAM_SEG_ROWS * sizeof(uint64_t), st));
+    /* whether this level has vertices for sure, and whether the next two may */
+    bool sure = true, next = false;
+    uint32_t level = 0;
+    for (;; level++) {
+        if (ahead) along_sweep(edges, pl, bfs_along<true>{d_labels, level}, st);
+        else along_sweep(edges, pl, bfs_along<false>{d_labels, level}, st);
+        const bool found = pl->level_end(st), found_ahead = pl->host_flag[1] != 0;
+        if (!found && !next) break;
+        sure = found;
+        next = found_ahead;
+    }
+    if (sure) return level + 1;
+    /* the last sweep was for vertices that a sweep ahead of their level had found; a nearer one may have found them since */
+    hipLaunchKernelGGL(k_any_label, dim3(1024), dim3(256), 0, st, d_labels, pl->n_vertices, level, pl->along.flags);
+    return pl->level_end(st) ? level + 1 : level;
+}
+
+/* one reading of the edges that joins the trees of their ends.  In one launch where all are cached and few: 2^15 entries take 80 us, in two 88 */
+void cc_read_edges(bam_array_t* edges, graph_plan* pl, unsigned long long* comp, hipStream_t st)
+{
+    if (pl->along.n_segs && !(pl->all_cached && pl->bp.n_edges <= 1ull << 17)) along_sweep(edges, pl, cc_along{comp}, st);
+    else if (pl->bp.n_pages)
+        hipLaunchKernelGGL(k_cc_by_page, dim3(pl->bp.blocks), dim3(BAM_WAVE_SIZE), 0, st, edges->a->d_array_ptr, pl->offsets, (const uint64_t*)pl->bp.first.get(), pl->bp.n_edges, pl->bp.ppw,
+                           pl->cc_backwards(), comp);
 }
 
 /* the plan bam_array_set_graph made for this graph, or one made now in `local` that lives for the call */
@@ -1076,7 +1475,7 @@ int bam_cc_shaped(bam_array_t* edges, const uint64_t* d_offsets, uint64_t n_vert
     const shaped_launch sl = shape_of(shape, n_vertices, coarse, stride, edges->a->adt.n_ranges ? edges->a->h_ranges[0].cache.n_pages : 0);
     bool* curr = (bool*)graph_plan::sized(pl->bytes_a, n_vertices);
     bool* next = (bool*)graph_plan::sized(pl->bytes_b, n_vertices);
-    hipLaunchKernelGGL(k_iota, dim3(blocks_for(n_vertices, 256)), dim3(256), 0, st, (unsigned long long*)d_labels, n_vertices);
+    hipLaunchKernelGGL(k_iota, dim3(blocks_for(n_vertices, 256)), dim3(256), 0, st, (unsigned long long*)d_labels, n_vertices, (unsigned long long*)nullptr, (unsigned long long*)nullptr);
     hip_err_chk(hipMemsetAsync(curr, 0x01, n_vertices, st));
     hip_err_chk(hipMemsetAsync(next, 0x00, n_vertices, st));
     uint32_t iter = 0;
@@ -1168,7 +1567,7 @@ int bam_cc(bam_array_t* edges, const uint64_t* d_offsets, uint64_t n_vertices, u
     graph_plan* pl = plan_for(edges, d_offsets, n_vertices, 0, st, local);
     const uint64_t group = coarse > 512 ? coarse : 512;
     unsigned long long* comp = (unsigned long long*)d_labels;
-    hipLaunchKernelGGL(k_iota, dim3(blocks_for(n_vertices, 256)), dim3(256), 0, st, comp, n_vertices);
+    hipLaunchKernelGGL(k_iota, dim3(blocks_for(n_vertices, 256)), dim3(256), 0, st, comp, n_vertices, pl->along.n_missing, pl->along.next_chunk);
     hipLaunchKernelGGL(k_cc_coalesce_coarse_ptr_pc, dim3(pl->blocks(n_vertices, group)), dim3(128), 0, st, edges->a->d_array_ptr, n_vertices, d_offsets, comp, group,
                        pl->pieces, pl->n_pieces, pl->next_work(), pl->cc_backwards());
     hipLaunchKernelGGL(k_cc_settle, dim3(blocks_for(n_vertices, 256)), dim3(256), 0, st, comp, n_vertices);
@@ -1190,6 +1589,11 @@ int bam_bfs_by_page(bam_array_t* edges, const uint64_t* d_offsets, uint64_t n_ve
     if (int rc = pl->by_page(edges, st)) return rc;
     hip_err_chk(hipMemsetAsync(d_labels, 0xFF, n_vertices * sizeof(uint32_t), st));
     hip_err_chk(hipMemsetAsync(d_labels + src, 0, sizeof(uint32_t), st));
+    if (pl->along.n_segs) {
+        const uint32_t iter = bfs_along_levels(edges, pl, d_labels, st);
+        if (iterations) *iterations = iter;
+        return 0;
+    }
     uint32_t level = 0, iter = 0;
     bool changed;
     do {
@@ -1214,7 +1618,7 @@ int bam_cc_by_page(bam_array_t* edges, const uint64_t* d_offsets, uint64_t n_ver
     graph_plan* pl = plan_for(edges, d_offsets, n_vertices, 0, st, local);
     if (int rc = pl->by_page(edges, st)) return rc;
     unsigned long long* comp = (unsigned long long*)d_labels;
-    hipLaunchKernelGGL(k_iota, dim3(blocks_for(n_vertices, 256)), dim3(256), 0, st, comp, n_vertices);
+    hipLaunchKernelGGL(k_iota, dim3(blocks_for(n_vertices, 256)), dim3(256), 0, st, comp, n_vertices, pl->along.n_missing, pl->along.next_chunk);
     uint32_t iter = 0;
     bool changed = true;
     /*
@@ -1241,12 +1645,10 @@ int bam_cc_by_page(bam_array_t* edges, const uint64_t* d_offsets, uint64_t n_ver
         }
     }
     if (changed) {
-        if (pl->bp.n_pages)
-            hipLaunchKernelGGL(k_cc_by_page, dim3(pl->bp.blocks), dim3(BAM_WAVE_SIZE), 0, st, edges->a->d_array_ptr, d_offsets, (const uint64_t*)pl->bp.first.get(), pl->bp.n_edges, pl->bp.ppw,
-                               pl->cc_backwards(), comp);
+        cc_read_edges(edges, pl, comp, st);
         hipLaunchKernelGGL(k_cc_settle, dim3(blocks_for(n_vertices, 256)), dim3(256), 0, st, comp, n_vertices);
         hip_err_chk(hipGetLastError());
-        pl->level_end(st);
+        hip_err_chk(hipStreamSynchronize(st));
         iter += 2;
     }
     if (iterations) *iterations = iter;

@@ -1,0 +1,99 @@
+"""BFS and components along the edge array in two launches, what is resident first: numbers of entries at the edges of rows,
+segments and of a wave's share, lists that cross pages, vertices without lists, and levels found ahead of their sweep."""
+import numpy as np
+import pytest
+
+import oracle
+from test_gpu_parity import SEED, Rig, _dev, _u64, bam  # noqa: F401  (bam is the module fixture)
+
+pytestmark = pytest.mark.gpu
+
+KINDS = [{"by_page": True}]
+
+
+def _rig(bam, nb, page, cache_pages):
+    pad = (-len(nb)) % (page // 8)
+    r = Rig(bam, (len(nb) + pad) * 8, backing=True, n_queues=16, depth=256, stage_bytes=max(4096, min(page, 8192)))
+    r.backing(len(nb) + pad)[:len(nb)] = nb
+    return r, r.array(len(nb), page, cache_pages)
+
+
+def _check_bfs(r, a, off, nb, sources):
+    d_off = _dev(off)
+    for kept in (False, True):
+        if kept:
+            a.set_graph(d_off)
+        for src in sources:
+            want, want_it = oracle.bfs_levels(off, nb, int(src))
+            for kw in KINDS:
+                lv, it = a.bfs(d_off, int(src), **kw)
+                assert np.array_equal(lv.cpu().numpy().view(np.uint32), want) and it == want_it, (kept, src, kw, it, want_it)
+    assert not r.c.aborted()
+
+
+# a directed graph with lists of 0 to `most` entries: one below, at and one above a row, a segment, two, sixteen of them
+@pytest.mark.parametrize("n_edges", [1, 63, 64, 65, 511, 512, 513, 1025, 8191, 8192, 8193, 33333])
+@pytest.mark.parametrize("page,cache_pages", [(4096, 2), (4096, 9), (4096, 1024), (512, 40), (8192, 5), (16384, 3), (65536, 2)])
+def test_levels_of_directed_graphs_of_all_lengths(bam, n_edges, page, cache_pages):
+    rng = np.random.default_rng(n_edges + page + cache_pages)
+    most = 1500 if n_edges > 9000 else 40
+    deg = []
+    while sum(deg) < n_edges:
+        deg.append(0 if rng.random() < 0.3 else int(rng.integers(1, most)))
+    deg = np.array([0, 0] + deg + [0])                     # the first vertices and the last have no list
+    deg[np.nonzero(deg)[0][-1]] -= deg.sum() - n_edges
+    n_v = len(deg)
+    off = np.concatenate([[0], np.cumsum(deg)]).astype(np.uint64)
+    # mostly to vertices nearby, so that there are several levels
+    owner = np.repeat(np.arange(n_v), deg)
+    nb = ((owner + rng.integers(-3, 8, n_edges)) % n_v).astype(np.uint64)
+    r, a = _rig(bam, nb, page, cache_pages)
+    with r:
+        _check_bfs(r, a, off, nb, [0, int(np.nonzero(deg)[0][0]), int(rng.integers(0, n_v))])
+
+
+@pytest.mark.parametrize("page,cache_pages", [(4096, 30), (4096, 500), (8192, 30), (65536, 4)])
+def test_labels_and_levels_of_a_random_graph(bam, page, cache_pages):
+    for off, nb in (oracle.rmat_csr(SEED, 13), oracle.uniform_csr(SEED, 30011, 50021)):
+        r, a = _rig(bam, nb, page, cache_pages)
+        with r:
+            _check_bfs(r, a, off, nb, oracle.bfs_sources(SEED, off, 2))
+            want, _ = oracle.cc_labels(off, nb)
+            for kept in (True, True, False):
+                if not kept:
+                    a.set_graph(None)
+                for by_page in (False, True):
+                    lb, _ = a.cc(_dev(off), by_page=by_page)
+                    assert np.array_equal(_u64(lb), want), (kept, by_page)
+            assert not r.c.aborted()
+
+
+def test_a_vertex_found_two_levels_ahead_and_then_nearer(bam):
+    """Twelve pages behind eight, read front to back by one wave.  Page 1: vertex 1 (level 1) finds vertex 3 (level 2).  Page 2 is
+    there for vertex 2 (level 1) and holds the list of vertex 3, which finds vertex 9 ahead, as of level 3.  Page 3: vertex 4
+    (level 1) has it next to itself.  There is no level 3, and the sweep that looks for one must not count."""
+    lists = {0: [1, 2, 4], 1: [3], 2: [5], 3: [9], 4: [9]}
+    place = {0: 0, 1: 512, 2: 1024, 3: 1024 + 300, 4: 1536}
+    n_edges, n_v = 12 * 512, 20
+    order = [0, 10, 1, 11, 2, 12, 3, 13, 4, 14]            # 10, ... fill the pages up; nobody leads to them
+    at, off_of, nb = 0, {}, np.full(n_edges, 15, dtype=np.uint64)
+    for k, v in enumerate(order):
+        off_of[v] = at
+        if v in lists:
+            assert at == place[v]
+            nb[at:at + len(lists[v])] = lists[v]
+            at += len(lists[v])
+        else:
+            at = place[order[k + 1]] if k + 1 < len(order) else n_edges
+    # vertices are numbered along the array
+    rank = {v: k for k, v in enumerate(order)}
+    rank.update({v: len(order) + k for k, v in enumerate(x for x in range(n_v) if x not in rank)})
+    off = np.full(n_v + 1, n_edges, dtype=np.uint64)
+    for k, v in enumerate(order):
+        off[k] = off_of[v]
+    nb = np.array([rank[int(x)] for x in nb], dtype=np.uint64)
+    want, want_it = oracle.bfs_levels(off, nb, rank[0])
+    assert want_it == 3 and want[rank[9]] == 2 and want[rank[3]] == 2
+    r, a = _rig(bam, nb, 4096, 8)
+    with r:
+        _check_bfs(r, a, off, nb, [rank[0]] * 3)
