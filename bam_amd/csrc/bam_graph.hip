@@ -1233,6 +1233,7 @@ struct graph_plan {
         return *host_flag != 0;
     }
     int by_page(bam_array_t* edges, hipStream_t st);
+    bool along_edges(bam_array_t* edges, hipStream_t st);
     static void* sized(BufferPtr& b, uint64_t bytes) { if (!b) b = createBuffer(bytes ? bytes : 8, 0); return b.get(); }
 };
 
@@ -1297,6 +1298,21 @@ int graph_plan::by_page(bam_array_t* edges, hipStream_t st)
     hip_err_chk(hipGetLastError());
     bp_built = true;
     return 0;
+}
+
+/*
+ * Whether BFS and components of an array are read along its pages, whichever entry point asks for them: the array has one
+ * range that begins on a page boundary, and pages the two launches take.  Per vertex, and over a queue of vertices, the same
+ * levels took 2.9 ms (2^20 vertices, all cached; 0.47 along the pages), 10.4 and 13.6 ms (2^18, a quarter cached; 1.8), 0.72
+ * and 1.27 (2^12; 0.12; without a plan made for the graph 0.80 and 1.44, 0.25).
+ */
+bool graph_plan::along_edges(bam_array_t* edges, hipStream_t st)
+{
+    if (!bp_built && edges->a->adt.n_ranges == 1) {
+        const range_d_t<uint64_t>& r = edges->a->h_ranges[0];
+        if (r.index_start == 0 && r.page_start_offset % r.cache.page_size == 0 && r.cache.n_pages >= 2) by_page(edges, st);
+    }
+    return along.n_segs != 0;
 }
 
 extern "C++" {
@@ -1391,11 +1407,16 @@ int bam_bfs(bam_array_t* edges, const uint64_t* d_offsets, uint64_t n_vertices, 
     hipStream_t st = (hipStream_t)stream;
     std::unique_ptr<graph_plan> local;
     graph_plan* pl = plan_for(edges, d_offsets, n_vertices, 0, st, local);
+    hip_err_chk(hipMemsetAsync(d_labels, 0xFF, n_vertices * sizeof(uint32_t), st));
+    hip_err_chk(hipMemsetAsync(d_labels + src, 0, sizeof(uint32_t), st));
+    if (pl->along_edges(edges, st)) {
+        const uint32_t levels = bfs_along_levels(edges, pl, d_labels, st);
+        if (iterations) *iterations = levels;
+        return 0;
+    }
     /* a group's lists are asked for as one batch of commands: a few hundred vertices make that batch large enough for the
      * store path, and keep the one word all waves take their work from out of the way */
     const uint64_t group = coarse > 512 ? coarse : 512;
-    hip_err_chk(hipMemsetAsync(d_labels, 0xFF, n_vertices * sizeof(uint32_t), st));
-    hip_err_chk(hipMemsetAsync(d_labels + src, 0, sizeof(uint32_t), st));
     const uint32_t threads = 128;
     uint32_t level = 0, iter = 0;
     bool changed;
@@ -1511,6 +1532,13 @@ int bam_bfs_frontier(bam_array_t* edges, const uint64_t* d_offsets, uint64_t n_v
     hipStream_t st = (hipStream_t)stream;
     std::unique_ptr<graph_plan> local;
     graph_plan* pl = plan_for(edges, d_offsets, n_vertices, 0, st, local);
+    if (pl->along_edges(edges, st)) {
+        hip_err_chk(hipMemsetAsync(d_labels, 0xFF, n_vertices * sizeof(uint32_t), st));
+        hip_err_chk(hipMemsetAsync(d_labels + src, 0, sizeof(uint32_t), st));
+        const uint32_t levels = bfs_along_levels(edges, pl, d_labels, st);
+        if (iterations) *iterations = levels;
+        return 0;
+    }
     /* two queues of at most every vertex once (benchmarks/bfs/main.cu:1489-1492); the size of the next one is the reference's `changed`.
      * They, and what puts a queue in order, belong to the plan: with bam_array_set_graph nothing is allocated here */
     uint32_t* curr = (uint32_t*)graph_plan::sized(pl->queue_a, n_vertices * sizeof(uint32_t));
@@ -1567,12 +1595,16 @@ int bam_cc(bam_array_t* edges, const uint64_t* d_offsets, uint64_t n_vertices, u
     graph_plan* pl = plan_for(edges, d_offsets, n_vertices, 0, st, local);
     const uint64_t group = coarse > 512 ? coarse : 512;
     unsigned long long* comp = (unsigned long long*)d_labels;
+    const bool along = pl->along_edges(edges, st);
     hipLaunchKernelGGL(k_iota, dim3(blocks_for(n_vertices, 256)), dim3(256), 0, st, comp, n_vertices, pl->along.n_missing, pl->along.next_chunk);
-    hipLaunchKernelGGL(k_cc_coalesce_coarse_ptr_pc, dim3(pl->blocks(n_vertices, group)), dim3(128), 0, st, edges->a->d_array_ptr, n_vertices, d_offsets, comp, group,
+    if (along) cc_read_edges(edges, pl, comp, st);
+    else
+        hipLaunchKernelGGL(k_cc_coalesce_coarse_ptr_pc, dim3(pl->blocks(n_vertices, group)), dim3(128), 0, st, edges->a->d_array_ptr, n_vertices, d_offsets, comp, group,
                        pl->pieces, pl->n_pieces, pl->next_work(), pl->cc_backwards());
     hipLaunchKernelGGL(k_cc_settle, dim3(blocks_for(n_vertices, 256)), dim3(256), 0, st, comp, n_vertices);
     hip_err_chk(hipGetLastError());
-    pl->level_end(st);
+    if (along) { hip_err_chk(hipStreamSynchronize(st)); }
+    else pl->level_end(st);
     if (iterations) *iterations = 2;
     BAM_API_END
 }

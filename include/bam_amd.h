@@ -227,6 +227,8 @@ int bam_array_set_graph(bam_array_t* edges, const uint64_t* d_offsets, uint64_t 
 /* ---- BFS (benchmarks/bfs/main.cu:658-689 kernel_coalesce_coarse_ptr_pc, host loop :1557-1566, 1577-1736) ----
  * Level-synchronous BFS from src: d_offsets[V+1] in device memory, neighbour ids read through the array,
  * d_labels[V] receives the level of every vertex (0xFFFFFFFF = unreachable).  *iterations = levels swept.
+ * Where the array has one range that begins on a page boundary, and pages of 4 to 64 KiB, the edges are read along their pages
+ * (bam_bfs_by_page), which is quicker whatever the graph; the same for bam_bfs_frontier and bam_cc.  Otherwise:
  * The vertices are handed out in groups of max(coarse, 512) to as many waves as the device holds.  A wave first
  * touches the pages that hold the lists of its group's active vertices (what is not resident comes in as one batch of
  * commands), then reads the lists of 64 vertices at a time through bam_ptr, 64 entries per step across list ends.
@@ -274,9 +276,11 @@ int bam_cc(bam_array_t* edges, const uint64_t* d_offsets, uint64_t n_vertices, u
 /* ---- the same two traversals, laid out along the edge array instead of along the vertices ----
  * The reference's page-tiled variant (benchmarks/bfs/main.cu:1074-1140 kernel_optimized_ptr_pc, with the table of the
  * first vertex of every page built by kernel_first_vertex_step1/2, :122-181; the same in benchmarks/cc): one warp per
- * page of the edge array, which it walks vertex by vertex.  Here a wave takes a run of up to 64 consecutive pages,
- * acquires those that hold edges of active vertices with one call (their misses reach the store as one batch of
- * commands) and relaxes those vertices' edges from the resident pages; the table is built by binary search.
+ * page of the edge array, which it walks vertex by vertex.  Here a sweep is two launches: the pages that hold edges of active
+ * vertices and are resident are visited, the others listed, and then fetched in batches and visited; the table is built
+ * by binary search.  Where some edges are on the store, edges of the next level's vertices are visited along with a level's
+ * own where their page is there anyway, and their pages need not come in for them again.  (Pages smaller than 4 KiB or larger
+ * than 64: a wave takes a run of up to 64 consecutive pages, and acquires those that hold edges of active vertices with one call.)
  * Same inputs, same outputs as bam_bfs / bam_cc (levels and labels are unique, so they are bit-identical).
  * The array must consist of one range that starts on a page boundary. */
 int bam_bfs_by_page(bam_array_t* edges, const uint64_t* d_offsets, uint64_t n_vertices, uint64_t src, uint32_t* d_labels,

@@ -8,7 +8,7 @@ from test_gpu_parity import SEED, Rig, _dev, _u64, bam  # noqa: F401  (bam is th
 
 pytestmark = pytest.mark.gpu
 
-KINDS = [{"by_page": True}]
+KINDS = [{"by_page": True}, {"coarse": 64}, {"frontier": True}]
 
 
 def _rig(bam, nb, page, cache_pages):
