@@ -29,6 +29,237 @@ __global__ __launch_bounds__(64) void k_vectoradd_ptr_pc(array_d_t<uint64_t>* da
     if (fp.done && threadIdx.x == 0) __hip_atomic_fetch_add(fp.done, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+/*
+ * The same sums a page at a time, for arrays whose pages are 4 or 8 KiB and fit a staging page.  A wave holds up to 16 or 32
+ * pages of A and of B, loads them in 16-byte pieces and writes the sums, past the caches, straight to where they go:
+ *  - into the slot of C's page where that is resident;
+ *  - where it is not, and the three arrays are larger than the cache, to the store: into the staging pages of a batch of write
+ *    commands.  Read by read, a page of C would come in only to be written over, push out a page of A or B, and be pushed out
+ *    in turn, a command at a time, by whoever needs its slot.  The page's descriptor is BUSY until its write has completed, as
+ *    under an evictor, so nobody brings the old content in meanwhile.
+ * First the pages of which A and B are resident (k_vectoradd_resident), so that what a call left in the cache is there for the
+ * next one, then the others in batches (k_vectoradd_missing).  What neither could do (C's page was being loaded or evicted, a
+ * command failed) is left to k_vectoradd_rest.
+ * Bound by the store: 10^7 elements, a cache of half their pages: 39 000 + 19 500 page reads and as many writes, 11.4 ms;
+ * here XXX.
+ */
+struct vadd_t {
+    array_d_t<uint64_t>* a;
+    array_d_t<uint64_t>* b;
+    array_d_t<uint64_t>* c;
+    uint64_t n_elems, n_full;                   /* pages that the elements fill */
+    uint32_t past_cache;                        /* C's pages that are not resident go to the store */
+    uint8_t* done;                              /* [n_full] pages that are finished */
+    uint32_t* list;                             /* [n_full] pages left to the second launch */
+    unsigned long long* n_list;                 /* zero between calls, like the next one */
+    unsigned long long* next_chunk;
+    uint32_t* finished;
+    uint32_t call;
+};
+#define BAM_VADD_PAGES 32u                      /* pages of C a wave of the first launch looks after */
+
+/* the place of a page of C for the lane to write its sums to, taken in one of the two ways above */
+struct vadd_dest { data_page_t* dp; uint8_t* at; bool in_place, claimed; };
+__device__ __forceinline__ vadd_dest vadd_take(const bam::range_view<uint64_t>& view, const uint64_t page, const bool has, const bool past_cache)
+{
+    vadd_dest d{view.pages + (has ? page : 0), nullptr, false, false};
+    if (!has) return d;
+    const uint32_t st = bam::ld_relaxed(&d.dp->state) >> (CNT_SHIFT + 1);
+    if (st == V_NB) {
+        uint64_t sv;
+        uint32_t slot = 0;
+        d.in_place = bam_try_hit(d.dp, 1, true, sv, slot);
+        if (d.in_place) d.at = view.slot_addr(slot);
+        else __hip_atomic_fetch_add(&d.dp->state, 0u - 1u, __ATOMIC_RELAXED, BAM_AGENT);
+    } else if (st == NV_NB && past_cache) {
+        const uint32_t o = __hip_atomic_fetch_or(&d.dp->state, BUSY, __ATOMIC_RELAXED, BAM_AGENT);
+        if ((o & BUSY) == 0) {
+            if ((o >> (CNT_SHIFT + 1)) == NV_NB) d.claimed = true;
+            else __hip_atomic_fetch_and(&d.dp->state, DISABLE_BUSY_MASK, __ATOMIC_RELAXED, BAM_AGENT);      /* it came in meanwhile */
+        }
+    }
+    return d;
+}
+
+/* by the whole wave: the sums of the lanes' pages (payload of A at pa, of B at pb) to their places, which are given back; true for the lanes whose sums are there */
+__device__ __forceinline__ bool vadd_pages(const bam::range_view<uint64_t>& view, const uint64_t page, vadd_dest d, const uint8_t* pa, const uint8_t* pb)
+{
+    using bam::u64x2_t;
+    const uint32_t lane = bam::lane();
+    page_cache_d_t* const cache = &view.r->cache;
+    Controller* const ctl = cache->d_ctrls[0];
+    QueuePair* const qp = ctl->d_qps + bam::first(bam::wave_slot_hash() % ctl->n_qps);
+    /* more commands than half the queue's slots go through it in rounds */
+    const uint32_t step = qp->sq.qs >> 1 ? qp->sq.qs >> 1 : 1u;
+    uint64_t todo = bam::ballot(d.claimed);
+    bool ok = false, pending = d.in_place;
+    do {
+        const bool mine = ((todo >> lane) & 1) != 0 && bam::rank_in(todo) < step;
+        uint32_t ticket = 0, id = 0;
+        if (mine) {
+            ticket = bam::sq_reserve_group(&qp->sq);
+            id = ticket & qp->sq.qs_minus_1;
+            d.at = qp->stage + (size_t)id * qp->stage_stride;
+        }
+        for (uint64_t m = bam::ballot(mine || pending); m; m &= m - 1) {
+            const uint32_t j = bam::first_lane(m);
+            const uint8_t* qa = (const uint8_t*)bam::bcast((uint64_t)pa, j) + lane * 16u;
+            const uint8_t* qb = (const uint8_t*)bam::bcast((uint64_t)pb, j) + lane * 16u;
+            uint8_t* to = (uint8_t*)bam::bcast((uint64_t)d.at, j) + lane * 16u;
+            for (uint32_t o = 0; o < view.page_size; o += 4096u) {
+                const u64x2_t* p[8];
+                u64x2_t x[8];
+#pragma unroll
+                for (uint32_t r = 0; r < 4; r++) { p[r] = (const u64x2_t*)(qa + o + r * 1024u); p[r + 4] = (const u64x2_t*)(qb + o + r * 1024u); }
+                bam::ld_payload_stream8x2(p, x);
+#pragma unroll
+                for (uint32_t r = 0; r < 4; r++) {
+                    const u64x2_t sum = {x[r].x + x[r + 4].x, x[r].y + x[r + 4].y};
+                    bam::st16_sys(to + o + r * 1024u, __builtin_bit_cast(bam::u32x4_t, sum));
+                }
+            }
+        }
+        bam::wait_stores();                     /* in memory, or in the staging pages, before anybody is told */
+        if (mine) {
+            const uint64_t stage = qp->stage_ioaddr + (uint64_t)id * qp->stage_stride;
+            nvm_cmd_t cmd;
+#pragma unroll
+            for (int i = 0; i < 16; i++) cmd.dword[i] = 0;
+            nvm_cmd_header(&cmd, (uint16_t)id, NVM_IO_WRITE, qp->nvmNamespace);
+            nvm_cmd_data_ptr(&cmd, stage, view.page_size > qp->pageSize ? stage + qp->pageSize : 0);
+            nvm_cmd_rw_blks(&cmd, view.r->get_backing_page(page) * cache->n_blocks_per_page, (uint16_t)cache->n_blocks_per_page);
+            bam::sq_submit_group(&qp->sq, &cmd, ticket);
+            ok = bam::cq_wait_group(&qp->cq, &qp->sq, id);
+            bam::sq_release_group(&qp->sq, id);
+        }
+        pending = false;
+        todo &= ~bam::ballot(mine);
+    } while (todo);
+    if (d.claimed) __hip_atomic_fetch_and(&d.dp->state, DISABLE_BUSY_MASK, __ATOMIC_RELAXED, BAM_AGENT);
+    if (d.in_place) bam_release_refs(d.dp, 1, false);         /* written through: nothing to make visible */
+    return d.in_place || (d.claimed && ok);
+}
+
+/* the accesses of `pages` pages, an element each, as the bam_ptrs of k_vectoradd_ptr_pc count them; all lanes */
+__device__ __forceinline__ void vadd_account(bam::range_view<uint64_t>& view, const uint32_t pages, const uint32_t hits)
+{
+    view.n_access = pages * (view.page_size / (8u * BAM_WAVE_SIZE));
+    view.n_hit = hits * (view.page_size / (8u * BAM_WAVE_SIZE));
+    view.flush_stats();
+}
+
+/* elements [first, last) of one page, through bam_ptr; the whole wave */
+__device__ __forceinline__ void vadd_elements(const vadd_t& g, const uint64_t first, const uint64_t last)
+{
+    for (uint64_t e = first + bam::lane(); e < last; e += BAM_WAVE_SIZE) {
+        bam_ptr<uint64_t> Aptr(g.a);
+        bam_ptr<uint64_t> Bptr(g.b);
+        bam_ptr<uint64_t> Cptr(g.c);
+        const bam_ptr<uint64_t>& A = Aptr;
+        const bam_ptr<uint64_t>& B = Bptr;
+        Cptr[e] = A[e] + B[e];
+    }
+}
+
+__global__ __launch_bounds__(BAM_WAVE_SIZE) void k_vectoradd_resident(const vadd_t g)
+{
+    const uint32_t lane = bam::lane();
+    bam::range_view<uint64_t> va, vb, vc;
+    va.load(g.a->d_ranges);
+    const uint64_t per_page = va.page_size / 8;
+    if (blockIdx.x == gridDim.x - 1) {          /* what is behind the last full page */
+        if (g.n_full * per_page < g.n_elems) vadd_elements(g, g.n_full * per_page, g.n_elems);
+        return;
+    }
+    vb.load(g.b->d_ranges);
+    vc.load(g.c->d_ranges);
+    const uint64_t i = (uint64_t)blockIdx.x * BAM_VADD_PAGES + lane;
+    const bool mine = lane < BAM_VADD_PAGES && i < g.n_full;
+    data_page_t* const da = va.pages + (va.pso >> va.page_size_log) + (mine ? i : 0);
+    data_page_t* const db = vb.pages + (vb.pso >> vb.page_size_log) + (mine ? i : 0);
+    bool has = false;
+    uint32_t slot_a = 0, slot_b = 0;
+    if (mine && bam::ld_relaxed(&da->state) >> (CNT_SHIFT + 1) == V_NB && bam::ld_relaxed(&db->state) >> (CNT_SHIFT + 1) == V_NB) {
+        uint64_t sv;
+        if (bam_try_hit(da, 1, false, sv, slot_a)) {
+            has = bam_try_hit(db, 1, false, sv, slot_b);
+            if (!has) __hip_atomic_fetch_add(&db->state, 0u - 1u, __ATOMIC_RELAXED, BAM_AGENT);
+        }
+        if (!has) __hip_atomic_fetch_add(&da->state, 0u - 1u, __ATOMIC_RELAXED, BAM_AGENT);
+    }
+    const uint64_t page_c = (vc.pso >> vc.page_size_log) + i;
+    vadd_dest d = vadd_take(vc, page_c, has, g.past_cache != 0);
+    const uint32_t pages = bam::popc(bam::ballot(d.in_place || d.claimed)), placed = bam::popc(bam::ballot(d.in_place));
+    bool took = false;
+    if (pages) took = vadd_pages(vc, page_c, d, va.slot_addr(slot_a), vb.slot_addr(slot_b));
+    if (has) { bam_release_refs(da, 1, false); bam_release_refs(db, 1, false); }
+    if (mine) g.done[i] = took ? 1 : 0;
+    const uint64_t left = bam::ballot(mine && !took);
+    if (left) {
+        uint64_t at = 0;
+        if (lane == 0) at = __hip_atomic_fetch_add(g.n_list, (unsigned long long)bam::popc(left), __ATOMIC_RELAXED, BAM_AGENT);
+        at = bam::bcast(at, 0);
+        if (mine && !took) g.list[at + bam::popc(left & bam::lanes_below(lane))] = (uint32_t)i;
+    }
+    if (!pages) return;
+    vadd_account(va, pages, pages);
+    vadd_account(vb, pages, pages);
+    vadd_account(vc, pages, placed);
+}
+
+/* a wave holds at most 3 x `chunk` pages at a time; the launch keeps what all hold under half the cache */
+__global__ __launch_bounds__(BAM_WAVE_SIZE) void k_vectoradd_missing(const vadd_t g, const uint32_t chunk)
+{
+    const uint64_t n = *g.n_list;
+    if (!n) return;
+    const uint32_t lane = bam::lane();
+    bam::range_view<uint64_t> va, vb, vc;
+    va.load(g.a->d_ranges);
+    vb.load(g.b->d_ranges);
+    vc.load(g.c->d_ranges);
+    va.place = vb.place = vc.place = BAM_PLACE_PULLED;
+    const uint64_t pso_a = va.pso >> va.page_size_log, pso_b = vb.pso >> vb.page_size_log, pso_c = vc.pso >> vc.page_size_log;
+    bool any_left = false;
+    uint32_t pages = 0, placed = 0;
+    for (;;) {
+        uint64_t k = 0;
+        if (lane == 0) k = __hip_atomic_fetch_add(g.next_chunk, 1ull, __ATOMIC_RELAXED, BAM_AGENT) * chunk;
+        k = bam::bcast(k, 0);
+        if (k >= n) break;
+        const bool want = lane < chunk && k + lane < n;
+        const uint64_t i = g.list[want ? k + lane : k];
+        uint32_t slot_a = BAM_NO_SLOT, slot_b = BAM_NO_SLOT;
+        auto keep_a = [&](uint32_t s_) { slot_a = s_; return false; };
+        auto keep_b = [&](uint32_t s_) { slot_b = s_; return false; };
+        auto touch = [](uint32_t) { return true; };
+        va.acquire_helped(pso_a + i, want, false, keep_a, keep_a);
+        vb.acquire_helped(pso_b + i, want, false, keep_b, keep_b);
+        if (!g.past_cache) vc.acquire_helped(pso_c + i, want, false, touch, touch);
+        const bool has = want && slot_a != BAM_NO_SLOT && slot_b != BAM_NO_SLOT;
+        vadd_dest d = vadd_take(vc, pso_c + i, has, g.past_cache != 0);
+        pages += bam::popc(bam::ballot(d.in_place || d.claimed));
+        placed += bam::popc(bam::ballot(d.in_place));
+        bool took = false;
+        if (bam::ballot(d.in_place || d.claimed)) took = vadd_pages(vc, pso_c + i, d, va.slot_addr(has ? slot_a : 0), vb.slot_addr(has ? slot_b : 0));
+        if (want) { va.release(pso_a + i, false); vb.release(pso_b + i, false); }
+        if (took) g.done[i] = 1;
+        any_left |= want && !took;
+    }
+    if (bam::ballot(any_left)) note_work_left(g.finished, g.call);
+    vadd_account(va, pages, 0);
+    vadd_account(vb, pages, 0);
+    vadd_account(vc, pages, placed);
+}
+
+__global__ __launch_bounds__(BAM_WAVE_SIZE) void k_vectoradd_rest(const vadd_t g)
+{
+    if (blockIdx.x == 0 && threadIdx.x == 0) *g.n_list = *g.next_chunk = 0;
+    if (g.finished[BAM_LEFT_WORD] != g.call) return;
+    const uint64_t per_page = g.a->d_ranges[0].cache.page_size / 8;
+    for (uint64_t i = blockIdx.x; i < g.n_full; i += gridDim.x)
+        if (!g.done[i]) vadd_elements(g, i * per_page, (i + 1) * per_page);
+}
+
 // ---- reduction (benchmarks/reduction/main.cu:166-195 kernel_reduce_baseline_ptr_pc): output[b] = sum of the 2 x blockDim elements of block b ----
 /* output `bid` by `half` consecutive threads of the workgroup (a multiple of 64; each such group its own output, or none: take =
  * false); all threads of the workgroup come in */
@@ -486,6 +717,44 @@ private:
     static pool& shared() { static pool* p = new pool(); return *p; }      /* never taken down: the runtime may be gone by then */
 };
 
+/*
+ * Whole pages of the three arrays (k_vectoradd_resident); false, with nothing launched, where they do not lend themselves to it:
+ * arrays of one range whose element 0 is the first of a page, behind one cache of pages that fit a staging page, one
+ * controller, no capture (the launches keep notes for each other), memory for the notes.
+ */
+bool vectoradd_by_page(bam_array_t* a, bam_array_t* b, bam_array_t* c, uint64_t n_elems, hipStream_t st)
+{
+    uint64_t pages = 0;
+    bam_array_t* const all[3] = {a, b, c};
+    const page_cache_d_t* cache = nullptr;
+    for (int k = 0; k < 3; k++) {
+        if (all[k]->a->adt.n_ranges != 1) return false;
+        const range_d_t<uint64_t>& r = all[k]->a->h_ranges[0];
+        if (r.index_start || r.page_start_offset % r.cache.page_size || n_elems > r.count) return false;
+        if (cache && cache->base_addr != r.cache.base_addr) return false;
+        cache = &r.cache;
+        pages += (n_elems * sizeof(uint64_t) + r.cache.page_size - 1) / r.cache.page_size;
+    }
+    if (cache->n_ctrls != 1 || (cache->page_size != 4096 && cache->page_size != 8192) || cache->page_size > cache->stage_bytes) return false;
+    const uint64_t n_full = n_elems * sizeof(uint64_t) / cache->page_size;
+    if (!n_full || n_full > 0xFFFFFFFFull || is_captured(st)) return false;
+    uint32_t chunk = 16;
+    const uint64_t budget = cache->n_pages / 2;
+    while (chunk > 4 && budget / (3 * chunk) < 256) chunk /= 2;
+    const uint64_t waves = budget / (3 * chunk);
+    if (!waves) return false;
+    std::lock_guard<std::mutex> guard(c->scratch.mu);
+    scratch_set* set = scratch_for(c, st, n_full * (sizeof(uint32_t) + 1), 0);
+    if (!set) return false;
+    vadd_t g{a->a->d_array_ptr, b->a->d_array_ptr, c->a->d_array_ptr, n_elems, n_full, pages > cache->n_pages ? 1u : 0u, (uint8_t*)set->notes.get() + n_full * sizeof(uint32_t),
+             (uint32_t*)set->notes.get(), set->listed(), set->next_chunk(), set->finished(), set->next_call()};
+    hipLaunchKernelGGL(k_vectoradd_resident, dim3((uint32_t)((n_full + BAM_VADD_PAGES - 1) / BAM_VADD_PAGES) + 1), dim3(BAM_WAVE_SIZE), 0, st, g);
+    hipLaunchKernelGGL(k_vectoradd_missing, dim3((uint32_t)std::min<uint64_t>(waves, (n_full + chunk - 1) / chunk)), dim3(BAM_WAVE_SIZE), 0, st, g, chunk);
+    hipLaunchKernelGGL(k_vectoradd_rest, dim3((uint32_t)std::min<uint64_t>(n_full, std::min<uint64_t>(4096, cache->n_pages / 8))), dim3(BAM_WAVE_SIZE), 0, st, g);      /* a wave holds a page of each array */
+    hip_err_chk(hipGetLastError());
+    return true;
+}
+
 /* the scan of resident elements; false if some were not, and then the result is not written in full, or if there is no
  * memory for the sums */
 bool scan_resident(bam_array_t* a, uint64_t n_elems, uint32_t block_size, uint64_t* d_result, hipStream_t st)
@@ -534,6 +803,7 @@ int bam_vectoradd(bam_array_t* a, bam_array_t* b, bam_array_t* c, uint64_t n_ele
     if (n_elems > a->a->adt.n_elems || n_elems > b->a->adt.n_elems || n_elems > c->a->adt.n_elems) return fail(EINVAL, "bam_vectoradd: more elements than the arrays hold");
     if (!n_elems) return 0;
     BAM_API_BEGIN
+    if (vectoradd_by_page(a, b, c, n_elems, (hipStream_t)stream)) return 0;
     const fetch_plan fp = make_fetch_plan(a, 3, 64, 64, (hipStream_t)stream);
     hipLaunchKernelGGL(k_vectoradd_ptr_pc, dim3(blocks_for(n_elems, 64) + fp.blocks), dim3(64), 0, (hipStream_t)stream,
                        a->a->d_array_ptr, b->a->d_array_ptr, n_elems, c->a->d_array_ptr, fp);

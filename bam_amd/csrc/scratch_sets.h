@@ -28,6 +28,9 @@ struct scratch_set {
     uint32_t next_call() { if (++calls == 0) calls = 1; return calls; }
     /* the word the computing workgroups of a reduction count themselves off in for the fetching ones, on a line of its own */
     unsigned long long* done() { return (unsigned long long*)(finished() + 128); }
+    /* how many pages a first launch has listed for the second, and which of them comes next: zero between calls, a line each */
+    unsigned long long* listed() { return (unsigned long long*)(finished() + 160); }
+    unsigned long long* next_chunk() { return (unsigned long long*)(finished() + 192); }
 };
 
 /* a number of the calling thread's own, given out once in the life of the process (the number of a thread that has ended may

@@ -141,6 +141,7 @@ struct page_cache_d_t {
     uint32_t direct_limit;           /* not 0: instead of that share, a read batch of the miss path goes direct while fewer than this many directly placed commands are in flight on the whole cache (*direct_gauge) */
     uint32_t* direct_gauge;
     uint32_t direct_share_raw;       /* the same for reads through read_data / access_data (raw block I/O into slots the caller names) */
+    uint32_t stage_bytes;            /* size of a staging page; 0 without staging */
     uint64_t* prp2;                  /* [n_pages] second page or PRP list when page_size > controller page */
     uint64_t ctrl_page_size;
     uint64_t range_cap;
@@ -2115,6 +2116,7 @@ struct page_cache_t {
         pdt.prof = ctrl.prof;
 
         const bool staged = ctrl.n_qps && ctrl.h_qps[0]->stage != nullptr;
+        pdt.stage_bytes = staged ? ctrl.h_qps[0]->stage_stride : 0;
         const uint64_t cache_size = ps * np;
         pdt.direct_share = 3;        /* measured best on the random-gather workload: 12.1M 4 KiB reads/s against 11.4M all staged, 10.4M all direct */
         if (const char* e = getenv("BAM_DIRECT_SHARE")) pdt.direct_share = (uint32_t)atoi(e);
