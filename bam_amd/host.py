@@ -15,6 +15,8 @@ import torch
 
 from . import _lib
 
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None) if hasattr(torch._C, "_cuda_getDevice") else None
+
 c_u64, c_u32, c_vp = ctypes.c_uint64, ctypes.c_uint32, ctypes.c_void_p
 MASK64 = (1 << 64) - 1
 
@@ -42,6 +44,10 @@ def _ptr(t):
 
 
 def _stream():
+    """The handle of the current stream.  Read from torch's binding, once the device is up: the Stream object that
+    torch.cuda.current_stream() makes around it took 2.9 of the 8.4 us of a gather of a thousand elements, this takes 0.3."""
+    if _raw_stream is not None and torch.cuda.is_initialized():
+        return c_vp(_raw_stream(torch._C._cuda_getDevice()))
     return c_vp(torch.cuda.current_stream().cuda_stream)
 
 

@@ -288,8 +288,11 @@ int bam_bfs_by_page(bam_array_t* edges, const uint64_t* d_offsets, uint64_t n_ve
 int bam_cc_by_page(bam_array_t* edges, const uint64_t* d_offsets, uint64_t n_vertices, uint64_t* d_labels, uint32_t* iterations, void* stream);
 
 /* ---- vectoradd (benchmarks/vectoradd/main.cu:102-117 kernel_baseline_ptr_pc) ----
- * c[i] = a[i] + b[i] for i < n_elems, one thread per element, all three arrays read and written through bam_ptr; the
- * results reach the store when their pages are evicted or the cache is flushed (bam_page_cache_flush).
+ * c[i] = a[i] + b[i] for i < n_elems; the results reach the store when their pages are evicted or the cache is flushed
+ * (bam_page_cache_flush), or in the call itself.  Whole pages where the arrays allow it (one range each that begins on a page boundary,
+ * one cache of 4 or 8 KiB pages with staging pages as large, one controller): pages of a and b that are resident first, the
+ * others in batches, and, where the three arrays are larger than the cache, results whose page is not resident written straight to
+ * the store.  Otherwise one thread per element, all three arrays read and written through bam_ptr.
  * In this kernel, in bam_reduce, bam_scan and in bam_array_read without an assignment, consecutive threads read
  * consecutive (or evenly spaced) elements: the first wave of every window of up to 64 pages touches a window further
  * on, one page per lane, so that the store is asked for pages in batches of a window and not one page per wave
