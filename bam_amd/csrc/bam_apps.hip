@@ -499,94 +499,111 @@ __global__ void k_scan_ptr_pc(array_d_t<uint64_t>* da, unsigned long long* outpu
 }
 
 /*
- * The scan of elements that are resident, in two launches: the sums of all pieces of 1024 elements and of all chunks of
- * 8 x `pieces` pieces, and then, chunk by chunk, what comes before the chunk, before each of its pieces, and the running
- * sums.  The first launch reads the array, the second reads it again and writes the result; no workgroup waits for another.
- * Bound by HBM: 16 bytes per element at least, 24 here (2^26 elements: 312 us with the wait at the end, 5 TB/s of what is moved; 4690
- * through bam_ptr with a pass over the result to add the block totals; 2^20: 27 against 73).  One pass in which a workgroup waits
- * for the sums of the ones before it reads the array once, but took 350 us there and 92 for 2^22: the number of the next
- * tile, drawn from one word, costs the device 20 ns each, and a workgroup's registers sit idle for the 12 us it waits.
- * A page that is not resident: the wave tells the second launch and the host, which then runs the kernels that can miss
- * (host_left[0] names the call if the first launch gave up, [1] if the second did).
+ * The scan of elements that are resident, in one reading.  A workgroup holds a tile of 16384 elements in registers, tells the
+ * others its sum, adds up what lies before it and writes the running sums.  What lies before: the tiles' sums, back to the nearest
+ * tile that has told the sum of everything up to its end; a wave looks at 64 of them at a time.
+ *   Tiles are taken in the order the workgroups are started in, which is that of their numbers on each cluster of compute
+ * units, so the tile somebody waits for is running or will be next where it is to run; a wait that lasts longer than a second
+ * is given up all the same.  (The number of the next tile, drawn from one word, would cost the device 20 ns a tile.)
+ *   A word of a tile is 32 bits of a sum and the number of the call: it says by itself whether it has been written, and nothing
+ * has to be cleared or ordered.
+ *   Bound by HBM: 16 bytes per element.  2^26 elements: 314 -> 245 us a call (4.4 TB/s; a copy of as much on this device 4.9), 2^25
+ * 171 -> 130, 2^22 45 -> 34, 2^16 30 -> 27, 4099 28 -> 22, against two launches of which the first added up and the second
+ * read the elements again.  While a tile waits another has to load: two of 16 waves fit a compute unit with 64 registers a lane
+ * (four are spilled); with 68, one, 272 us; tiles of 8 waves, three to a compute unit, 293 (twice as many sums to look back over).
+ *   A page that is not resident: the wave tells the other workgroups and the host, which then runs the kernels that can miss.
  */
-#define BAM_CHUNK_WAVES 8u
+#define BAM_TILE_WAVES 16u
+#define BAM_TILE_ELEMS (BAM_TILE_WAVES * BAM_WAVE_ELEMS)
 #define BAM_COUNTED_WORD 98u      /* of the scratch's words: the call whose accesses were counted */
 __device__ __forceinline__ void scan_gives_up(uint32_t* finished, const uint32_t call, volatile uint32_t* host_left)
 {
     if (bam::lane() == 0 && __hip_atomic_load(finished + BAM_LEFT_WORD, __ATOMIC_RELAXED, BAM_AGENT) != call &&
         __hip_atomic_exchange(finished + BAM_LEFT_WORD, call, __ATOMIC_RELAXED, BAM_AGENT) != call) *host_left = call;
 }
-__global__ __launch_bounds__(BAM_CHUNK_WAVES * BAM_WAVE_SIZE) void k_scan_sums(array_d_t<uint64_t>* da, const uint64_t n, const uint32_t pieces, uint64_t* piece_sums,
-                                                                               uint64_t* chunk_sums, uint32_t* finished, const uint32_t call, volatile uint32_t* host_left)
+/* [0, 1] the tile's sum, [2, 3] the sum of all elements up to its end */
+struct scan_tile_t { uint64_t word[4]; };
+__device__ __forceinline__ void scan_tell(uint64_t* word, const uint64_t sum, const uint32_t call)
 {
-    __shared__ uint64_t wave_sums[BAM_CHUNK_WAVES];
-    const uint32_t lane = bam::lane(), w = threadIdx.x / BAM_WAVE_SIZE;
-    const uint64_t chunk = blockIdx.x, p0 = bam::first(chunk * BAM_CHUNK_WAVES * pieces + w);
-    bam::range_view<uint64_t> view;
-    view.load(da->d_ranges);
-    uint64_t total = 0;
-    bool missing = false;
-    for (uint32_t k = 0; k < pieces; k++) {
-        const uint64_t piece = p0 + k * BAM_CHUNK_WAVES;
-        bam::u64x2_t x[BAM_WAVE_ROWS];
-        if (!read_rows_resident(view, piece * BAM_WAVE_ELEMS, n, x)) { missing = true; break; }
-        uint64_t v = 0;
-#pragma unroll
-        for (uint32_t r = 0; r < BAM_WAVE_ROWS; r++) v += x[r].x + x[r].y;
-        v = bam::wave_running_sum(v);
-        if (lane == BAM_WAVE_SIZE - 1) piece_sums[piece] = v;
-        total += v;
-    }
-    if (missing) scan_gives_up(finished, call, host_left);
-    if (lane == BAM_WAVE_SIZE - 1) wave_sums[w] = total;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        uint64_t v = 0;
-#pragma unroll
-        for (uint32_t k = 0; k < BAM_CHUNK_WAVES; k++) v += wave_sums[k];
-        chunk_sums[chunk] = v;
+    bam::st_relaxed(word, ((uint64_t)call << 32) | (uint32_t)sum);
+    bam::st_relaxed(word + 1, ((uint64_t)call << 32) | (uint32_t)(sum >> 32));
+}
+/* by a whole wave: the sum of everything before tile `tile` */
+__device__ __forceinline__ uint64_t scan_look_back(const scan_tile_t* tiles, const uint64_t tile, const uint32_t call, uint32_t* finished, volatile uint32_t* host_left)
+{
+    const uint32_t lane = bam::lane();
+    uint64_t acc = 0, t0 = 0;
+    for (uint64_t end = tile;; end -= BAM_WAVE_SIZE) {
+        /* lane l: tile end - 1 - l; before the first there is nothing, known for sure */
+        const bool there = lane < end;
+        const scan_tile_t* const at = tiles + (there ? end - 1 - lane : 0);
+        uint64_t sum = 0;
+        bool known = !there, all = !there;
+        for (uint32_t looks = 1;; looks++) {
+            if (!known || !all) {
+                const uint64_t a0 = bam::ld_relaxed(&at->word[0]), a1 = bam::ld_relaxed(&at->word[1]), b0 = bam::ld_relaxed(&at->word[2]), b1 = bam::ld_relaxed(&at->word[3]);
+                if ((uint32_t)(b0 >> 32) == call && (uint32_t)(b1 >> 32) == call) { sum = (b1 << 32) | (uint32_t)b0; known = all = true; }
+                else if ((uint32_t)(a0 >> 32) == call && (uint32_t)(a1 >> 32) == call) { sum = (a1 << 32) | (uint32_t)a0; known = true; }
+            }
+            const uint64_t m = bam::ballot(all);
+            const uint64_t need = m ? (m & (0ull - m)) | ((m & (0ull - m)) - 1) : ~0ull;      /* up to the nearest that has it all */
+            if ((bam::ballot(known) & need) == need) {
+                acc += wave_sum((need >> lane) & 1 ? sum : 0);
+                if (m) return acc;
+                break;
+            }
+            __builtin_amdgcn_s_sleep(1);
+            if ((looks & 1023u) == 0) {
+                const uint64_t now = wall_clock64();
+                if (!t0) t0 = now;
+                else if (now - t0 > 100000000ull) { scan_gives_up(finished, call, host_left); return acc; }
+            }
+        }
     }
 }
-
 /* n_access: what the scan counts, as the kernels that can miss count it */
-__global__ __launch_bounds__(BAM_CHUNK_WAVES * BAM_WAVE_SIZE) void k_scan_write(array_d_t<uint64_t>* da, uint64_t* result, const uint64_t n, const uint32_t pieces,
-                                                                                const uint64_t* piece_sums, const uint64_t* chunk_sums, uint32_t* finished, const uint32_t call,
-                                                                                volatile uint32_t* host_left, const uint64_t n_access)
+__global__ __launch_bounds__(BAM_TILE_WAVES * BAM_WAVE_SIZE) __attribute__((amdgpu_waves_per_eu(8))) void k_scan_tiles(array_d_t<uint64_t>* da, uint64_t* result, const uint64_t n, scan_tile_t* tiles, uint32_t* finished,
+                                                                               const uint32_t call, volatile uint32_t* host_left, const uint64_t n_access)
 {
-    __shared__ uint64_t wave_sums[BAM_CHUNK_WAVES];
-    const uint32_t lane = bam::lane(), w = threadIdx.x / BAM_WAVE_SIZE;
+    __shared__ uint64_t wave_sums[BAM_TILE_WAVES], before_s;
+    const uint32_t lane = bam::lane(), w = bam::first(threadIdx.x / BAM_WAVE_SIZE);
     bam::range_view<uint64_t> view;
     view.load(da->d_ranges);
-    if (__hip_atomic_load(finished + BAM_LEFT_WORD, __ATOMIC_RELAXED, BAM_AGENT) == call) {
-        if (blockIdx.x == 0 && threadIdx.x == 0) *host_left = call;
-        return;
-    }
-    const uint64_t chunk = blockIdx.x, p0 = chunk * BAM_CHUNK_WAVES * pieces;
-    uint64_t before = 0;
-    for (uint64_t c = threadIdx.x; c < chunk; c += BAM_CHUNK_WAVES * BAM_WAVE_SIZE) before += chunk_sums[c];
-    /* lane l: the sum of the chunk's l-th piece (there are at most 64); the sums of pieces behind the last element are 0 */
-    const uint64_t mine = lane < BAM_CHUNK_WAVES * pieces ? piece_sums[p0 + lane] : 0;
-    const uint64_t pieces_before = bam::wave_running_sum(mine) - mine;
-    before = bam::wave_running_sum(before);
-    if (lane == BAM_WAVE_SIZE - 1) wave_sums[w] = before;
-    __syncthreads();
-    before = 0;
+    const uint64_t tile = blockIdx.x, first = tile * BAM_TILE_ELEMS + w * BAM_WAVE_ELEMS;
+    /* once somebody has given up the result is not wanted: the tile is told as it is */
+    const bool given_up = __hip_atomic_load(finished + BAM_LEFT_WORD, __ATOMIC_RELAXED, BAM_AGENT) == call;
+    bam::u64x2_t x[BAM_WAVE_ROWS];
+    if (given_up || !read_rows_resident(view, first, n, x)) {
+        if (!given_up) scan_gives_up(finished, call, host_left);
 #pragma unroll
-    for (uint32_t k = 0; k < BAM_CHUNK_WAVES; k++) before += wave_sums[k];
-    for (uint32_t k = 0; k < pieces; k++) {
-        const uint32_t at = k * BAM_CHUNK_WAVES + bam::first(w);
-        const uint64_t first = (bam::first(p0) + at) * BAM_WAVE_ELEMS;
-        if (first > n) break;
-        bam::u64x2_t x[BAM_WAVE_ROWS];
-        if (!read_rows_resident(view, first, n, x)) { scan_gives_up(finished, call, host_left + 1); break; }
-        uint64_t carry = before + bam::bcast(pieces_before, at);
+        for (uint32_t r = 0; r < BAM_WAVE_ROWS; r++) x[r] = bam::u64x2_t{0, 0};
+    }
+    uint64_t v = 0;
+#pragma unroll
+    for (uint32_t r = 0; r < BAM_WAVE_ROWS; r++) v += x[r].x + x[r].y;
+    v = wave_sum(v);
+    if (lane == 0) wave_sums[w] = v;
+    __syncthreads();
+    if (w == 0) {
+        uint64_t total = 0;
+#pragma unroll
+        for (uint32_t k = 0; k < BAM_TILE_WAVES; k++) total += wave_sums[k];
+        if (lane == 0 && tile) scan_tell(tiles[tile].word, total, call);
+        const uint64_t before = tile ? scan_look_back(tiles, tile, call, finished, host_left) : 0;
+        if (lane == 0) { scan_tell(tiles[tile].word + 2, before + total, call); before_s = before; }
+    }
+    __syncthreads();
+    if (!given_up && first <= n) {
+        uint64_t carry = before_s;
+#pragma unroll
+        for (uint32_t k = 0; k < BAM_TILE_WAVES; k++) carry += k < w ? wave_sums[k] : 0;
         /* entry e is the sum of the elements before element e, the last one, n, the total */
 #pragma unroll
         for (uint32_t r = 0; r < BAM_WAVE_ROWS; r++) {
             const uint64_t pair = x[r].x + x[r].y, incl = bam::wave_running_sum(pair), sum = carry + (incl - pair);
             carry += bam::bcast(incl, BAM_WAVE_SIZE - 1);
             const uint64_t e = first + r * BAM_ROW_ELEMS + 2u * lane;
-            if (first + BAM_WAVE_ELEMS <= n + 1) *(bam::u64x2_t*)(result + e) = bam::u64x2_t{sum, sum + x[r].x};
+            if (first + BAM_WAVE_ELEMS <= n + 1) __builtin_nontemporal_store(bam::u64x2_t{sum, sum + x[r].x}, (bam::u64x2_t*)(result + e));
             else {
                 if (e <= n) result[e] = sum;
                 if (e + 1 <= n) result[e + 1] = sum + x[r].x;
@@ -600,7 +617,7 @@ __global__ __launch_bounds__(BAM_CHUNK_WAVES * BAM_WAVE_SIZE) void k_scan_write(
         finished[BAM_COUNTED_WORD] = call;
     }
 }
-/* behind a k_scan_write of which some wave gave up: the kernels that can miss count the whole scan, so what its first
+/* behind a k_scan_tiles of which some wave gave up: the kernels that can miss count the whole scan, so what its first
  * workgroup counted (it does not wait for the others) is taken off again */
 __global__ void k_scan_uncount(array_d_t<uint64_t>* da, const uint32_t* finished, const uint32_t call, const uint64_t n_access)
 {
@@ -681,9 +698,9 @@ uint64_t paired_accesses(uint64_t n, uint64_t half, uint64_t page_elems)
 }
 
 /*
- * Two words in host memory that the device can write, one call's own for as long as it lasts: a scan waits for its result, and
+ * A word in host memory that the device can write, one call's own for as long as it lasts: a scan waits for its result, and
  * finds there whether it is whole.  Page-locked memory takes far longer to get than a scan does, so the words are kept for the
- * next call, whichever array or thread makes it; there are as many as calls were ever waiting at a time, in steps of 32.
+ * next call, whichever array or thread makes it; there are as many as calls were ever waiting at a time, in steps of 64.
  * Words that launches may still write (the wait failed) are not given back.  `at` is NULL where no memory is to be had.
  */
 struct host_word {
@@ -697,11 +714,11 @@ struct host_word {
             const relaxed_capture relaxed;
             void* mem = nullptr;
             if (hipHostMalloc(&mem, 64 * sizeof(uint32_t), hipHostMallocMapped | hipHostMallocPortable) != hipSuccess) { (void)hipGetLastError(); return; }
-            for (uint32_t k = 0; k < 64; k += 2) p.free.push_back((volatile uint32_t*)mem + k);
+            for (uint32_t k = 0; k < 64; k++) p.free.push_back((volatile uint32_t*)mem + k);
         }
         at = p.free.back();
         p.free.pop_back();
-        at[0] = at[1] = 0;          /* never the number of a call */
+        at[0] = 0;                  /* never the number of a call */
     }
     ~host_word()
     {
@@ -766,30 +783,21 @@ bool scan_resident(bam_array_t* a, uint64_t n_elems, uint32_t block_size, uint64
     uint32_t* finished;
     const uint64_t n_access = paired_accesses(n_elems, block_size, a->a->h_ranges[0].cache.page_size / 8);
     {
-        /* pieces per wave: as many as leave 2048 workgroups, eight at most (a chunk's pieces are looked after by the lanes of a
-         * wave); 2^26 elements 312 us, with 512 or 1024 workgroups at least 322, and with stretches of 2^24 elements, small
-         * enough for the last-level cache to hold them from the first launch to the second, 373.  n / 1024 + 1 pieces: entry n
-         * of the result is in the last */
-        const uint64_t n_pieces = n_elems / BAM_WAVE_ELEMS + 1;
-        uint32_t pieces = 1;
-        while (pieces < 8 && n_pieces / (BAM_CHUNK_WAVES * pieces * 2) >= 2048) pieces *= 2;
-        const uint64_t per_chunk = BAM_CHUNK_WAVES * pieces, n_chunks = (n_pieces + per_chunk - 1) / per_chunk;
+        const uint64_t n_tiles = n_elems / BAM_TILE_ELEMS + 1;          /* entry n of the result is in the last */
         std::lock_guard<std::mutex> guard(a->scratch.mu);
-        scratch_set* set = scratch_for(a, st, n_chunks * (per_chunk + 1) * sizeof(uint64_t), 0);
+        scratch_set* set = scratch_for(a, st, 0, 0, n_tiles * sizeof(scan_tile_t));
         if (!set) return false;
         call = set->next_call();
         finished = set->finished();
-        uint64_t* piece_sums = (uint64_t*)set->notes.get(), *chunk_sums = piece_sums + n_chunks * per_chunk;
-        const dim3 grid((uint32_t)n_chunks), block(BAM_CHUNK_WAVES * BAM_WAVE_SIZE);
-        hipLaunchKernelGGL(k_scan_sums, grid, block, 0, st, a->a->d_array_ptr, n_elems, pieces, piece_sums, chunk_sums, finished, call, left.at);
-        hipLaunchKernelGGL(k_scan_write, grid, block, 0, st, a->a->d_array_ptr, d_result, n_elems, pieces, piece_sums, chunk_sums, finished, call, left.at, n_access);
+        hipLaunchKernelGGL(k_scan_tiles, dim3((uint32_t)n_tiles), dim3(BAM_TILE_WAVES * BAM_WAVE_SIZE), 0, st, a->a->d_array_ptr, d_result, n_elems, (scan_tile_t*)set->tiles.get(), finished, call,
+                           left.at, n_access);
         hip_err_chk(hipGetLastError());
     }
     const hipError_t e = hipStreamSynchronize(st);
     left.idle = e == hipSuccess;
     hip_err_chk(e);
-    if (left.at[0] != call && left.at[1] != call) return true;
-    if (left.at[1] == call) hipLaunchKernelGGL(k_scan_uncount, dim3(1), dim3(1), 0, st, a->a->d_array_ptr, finished, call, n_access);
+    if (left.at[0] != call) return true;
+    hipLaunchKernelGGL(k_scan_uncount, dim3(1), dim3(1), 0, st, a->a->d_array_ptr, finished, call, n_access);
     hip_err_chk(hipGetLastError());
     return false;
 }

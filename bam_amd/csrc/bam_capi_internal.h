@@ -85,7 +85,7 @@ struct bam_array32 { array_t<uint32_t>* a; BufferPtr partials; };      /* partia
  * the call then takes a route that needs none.  It lies on the array's device, and the caller's current device stays as it is.
  * Nothing here waits, unless those two differ and memory has to be cleared.
  */
-inline scratch_set* scratch_for(bam_array_t* a, hipStream_t st, size_t notes_bytes, size_t wanted_bytes)
+inline scratch_set* scratch_for(bam_array_t* a, hipStream_t st, size_t notes_bytes, size_t wanted_bytes, size_t tiles_bytes = 0)
 {
     auto alloc = [&](size_t bytes) -> BufferPtr {
         const relaxed_capture relaxed;
@@ -103,7 +103,7 @@ inline scratch_set* scratch_for(bam_array_t* a, hipStream_t st, size_t notes_byt
         if (e != hipSuccess) { (void)hipGetLastError(); if (p) (void)hipFree(p); return nullptr; }
         return BufferPtr(p, [](void* q) { (void)hipFree(q); });
     };
-    return a->scratch.get(st, st == hipStreamPerThread ? scratch_thread_number() : 0, notes_bytes, wanted_bytes, alloc);
+    return a->scratch.get(st, st == hipStreamPerThread ? scratch_thread_number() : 0, notes_bytes, wanted_bytes, alloc, tiles_bytes);
 }
 
 // ---------------------------------------------------------------------------

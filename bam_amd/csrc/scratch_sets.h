@@ -15,13 +15,14 @@
 
 /*
  * The bits of the requests a first launch leaves, a byte per page of the range that somebody waits for (zero between calls),
- * checksum shards and the count of finished workgroups.
+ * what the tiles of a scan tell each other (words that carry the number of their call), checksum shards and the count of finished
+ * workgroups.
  */
 struct scratch_set {
     void* stream = nullptr;
     uint64_t thread = 0;
-    std::shared_ptr<void> words, notes, wanted;
-    size_t notes_bytes = 0, wanted_bytes = 0;
+    std::shared_ptr<void> words, notes, wanted, tiles;
+    size_t notes_bytes = 0, wanted_bytes = 0, tiles_bytes = 0;
     uint32_t calls = 0;
     unsigned long long* partials() { return (unsigned long long*)words.get(); }
     uint32_t* finished() { return (uint32_t*)(partials() + BAM_SUM_PARTIALS); }
@@ -61,7 +62,7 @@ struct scratch_sets {
      * A set is entered once all of it is there, and a buffer changes place with a larger one that is there.
      */
     template <typename Alloc>
-    scratch_set* get(void* stream, uint64_t thread, size_t notes_bytes, size_t wanted_bytes, Alloc&& alloc)
+    scratch_set* get(void* stream, uint64_t thread, size_t notes_bytes, size_t wanted_bytes, Alloc&& alloc, size_t tiles_bytes = 0)
     {
         scratch_set* s = nullptr;
         for (auto& x : sets) if (x->stream == stream && x->thread == thread) s = x.get();
@@ -74,7 +75,8 @@ struct scratch_sets {
             sets.push_back(std::move(made));
             s = sets.back().get();
         }
-        return grown(s->notes, s->notes_bytes, notes_bytes, alloc) && grown(s->wanted, s->wanted_bytes, wanted_bytes, alloc) ? s : nullptr;
+        return grown(s->notes, s->notes_bytes, notes_bytes, alloc) && grown(s->wanted, s->wanted_bytes, wanted_bytes, alloc) &&
+               grown(s->tiles, s->tiles_bytes, tiles_bytes, alloc) ? s : nullptr;
     }
 
 private:

@@ -16,10 +16,11 @@ def _accesses(n, half, page_elems):
     return len(e) + int(((e2 < n) & (e // page_elems != e2 // page_elems)).sum())
 
 
-# around a row (128), a wave (1024), a tile (2048 and, from 2^22 on, 8192), a page and an output; page sizes on both sides of a row
+# around a row (128), a wave (1024), a tile of a scan (16384), 64 of them, a page and an output; page sizes on both sides of a row
 @pytest.mark.parametrize("page", [512, 4096, 8192, 65536])
 @pytest.mark.parametrize("n,block", [(1, 64), (127, 64), (128, 64), (129, 192), (1023, 128), (1024, 512), (2047, 256), (2048, 256), (2049, 1024),
-                                     (65537, 64), (65537, 320), (300001, 576), (300001, 960), ((1 << 22) - 1, 256), (1 << 22, 64), ((1 << 22) + 8193, 1024)])
+                                     (65537, 64), (65537, 320), (300001, 576), (300001, 960), ((1 << 22) - 1, 256), (1 << 22, 64), ((1 << 22) + 8193, 1024),
+                                     (16383, 64), (16384, 64), (16385, 128), (64 * 16384 - 1, 64), (64 * 16384, 256), (65 * 16384, 256), (65 * 16384 + 1, 512)])
 def test_resident_runs_element_by_element(bam, page, n, block):
     per = page // 8
     pages = (n + per - 1) // per
