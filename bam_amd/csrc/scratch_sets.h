@@ -23,7 +23,7 @@ struct scratch_set {
     uint64_t thread = 0;
     std::shared_ptr<void> words, notes, wanted, tiles;
     size_t notes_bytes = 0, wanted_bytes = 0, tiles_bytes = 0;
-    uint32_t calls = 0;
+    uint32_t calls = 0, updates = 0;
     unsigned long long* partials() { return (unsigned long long*)words.get(); }
     uint32_t* finished() { return (uint32_t*)(partials() + BAM_SUM_PARTIALS); }
     uint32_t next_call() { if (++calls == 0) calls = 1; return calls; }
@@ -32,6 +32,8 @@ struct scratch_set {
     /* how many pages a first launch has listed for the second, and which of them comes next: zero between calls, a line each */
     unsigned long long* listed() { return (unsigned long long*)(finished() + 160); }
     unsigned long long* next_chunk() { return (unsigned long long*)(finished() + 192); }
+    /* how many updates a slice has left for its last launch, by turns: the one's word is cleared by the other */
+    unsigned long long* left_over(uint32_t which) { return (unsigned long long*)(finished() + (which ? 240 : 224)); }
 };
 
 /* a number of the calling thread's own, given out once in the life of the process (the number of a thread that has ended may

@@ -1,0 +1,64 @@
+"""bam_array_update dealt out to bins of pages: numbers of requests around where that begins and around a slice, numbers of pages around
+a bin's and around what 512 bins hold one each, all pages resident, none and some, requests scattered, in order and on few pages."""
+import ctypes
+
+import numpy as np
+import pytest
+
+import oracle
+from test_gpu_parity import Rig, SEED, _check_add_chains, _dev, _u64, bam  # noqa: F401  (bam is the module fixture)
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("api,n", [(0, 1 << 18), (0, (1 << 18) + 4095), (1, 1 << 17), (2, (1 << 17) + 1), (0, (1 << 20) - 1), (2, 1 << 20), (1, (1 << 20) + 1), (0, (2 << 20) + 77)])
+@pytest.mark.parametrize("page,spare,warm", [(4096, 3, 1.0), (4096, 3, 0.0), (512, 1, 0.5), (8192, 40000, 1.0)])
+@pytest.mark.parametrize("kind", ["scattered", "in_order"])
+def test_updates_without_repeats(bam, api, n, page, spare, warm, kind):
+    per = page // 8
+    n_elems = n + spare * 7 + 5
+    pages = (n_elems + per - 1) // per
+    rng = np.random.default_rng(n + api)
+    with Rig(bam, pages * page, backing=True, n_queues=16, depth=256, stage_bytes=max(4096, page)) as r:
+        x0 = r.backing(n_elems).copy()
+        a = r.array(n_elems, page, pages)
+        if warm:
+            a.gather(max(1, int(pages * warm)), None, stride=per)
+        idx = (rng.permutation(n_elems)[:n] if kind == "scattered" else np.arange(n) + 5).astype(np.uint64)
+        vals = rng.integers(1, 1 << 63, n).astype(np.uint64)
+        outside = rng.integers(0, n, 3)
+        idx[outside] = np.array([n_elems, 1 << 40, (1 << 64) - 1], dtype=np.uint64)
+        inside = idx < n_elems
+        model = x0.copy()
+        for rep in range(2):                                  # the second call finds everything resident, and the counts cleared
+            a.stats()
+            old = _u64(a.update(api, _dev(idx), _dev(vals), block_size=64))
+            st = a.stats()
+            assert np.array_equal(old[inside], model[idx[inside].astype(np.int64)]) and (api or not old[~inside].any()), rep
+            model[idx[inside].astype(np.int64)] += vals[inside]
+            assert api or st["access_cnt"] == inside.sum(), st
+            assert rep == 0 and warm < 1 or st["read_io_cnt"] == 0, st
+        r.objs[0][2].flush()
+        assert np.array_equal(r.backing(n_elems), model) and not r.c.aborted()
+
+
+@pytest.mark.parametrize("span", [1, 64, 512, 3 * 4096, 40 * 512])
+@pytest.mark.parametrize("pages", [1, 511, 512, 513, 1025, 1300])
+def test_updates_that_meet(bam, pages, span):
+    n, n_elems = (1 << 18) + 333, pages * 512 - 1
+    rng = np.random.default_rng(pages + span)
+    with Rig(bam, pages * 4096, backing=True, n_queues=8, depth=256) as r:
+        x0 = r.backing(n_elems).copy()
+        a = r.array(n_elems, 4096, pages)
+        idx = (rng.integers(0, n_elems) + rng.integers(0, span, n)).astype(np.uint64) % np.uint64(n_elems)
+        vals = rng.integers(1, 1 << 20, n).astype(np.uint64)
+        old = _u64(a.update(0, _dev(idx), _dev(vals)))
+        model = x0.copy()
+        np.add.at(model, idx.astype(np.int64), vals)
+        _check_add_chains(x0, idx, vals, old, model)
+        # and without a place for what the elements held
+        d_idx, d_vals = _dev(idx), _dev(vals)
+        assert a.L.bam_array_update(a.h, 1, n, ctypes.c_void_p(d_idx.data_ptr()), ctypes.c_void_p(d_vals.data_ptr()), None, 64, None) == 0
+        np.add.at(model, idx.astype(np.int64), vals)
+        r.objs[0][2].flush()
+        assert np.array_equal(r.backing(n_elems), model) and not r.c.aborted()
