@@ -759,7 +759,10 @@ struct along_t {
     unsigned long long* n_missing;              /* zero between sweeps, like the next one */
     unsigned long long* next_chunk;             /* of the list, for the waves of the second launch */
     uint64_t* ahead;                            /* [n_segs * BAM_SEG_ROWS] a bit per entry (bfs_along) */
-    unsigned long long* flags;                  /* [2] what the sweep tells the host */
+    unsigned long long* flags;                  /* [2] what the sweep tells the host, and the sweeps queued behind it */
+    /* the sweep is made if it is sure to be wanted, or if one of these words, NULL or an earlier sweep's, says so */
+    uint32_t sure;
+    const unsigned long long* gate[2];
 };
 /* written and read by the lanes of one wave, which runs its LDS operations in order */
 __device__ __forceinline__ void wave_lds_fence()
@@ -933,6 +936,7 @@ struct cc_along {
 template <typename A>
 __global__ __launch_bounds__(BAM_TRIP_WAVES * BAM_WAVE_SIZE) void k_along_resident(array_d_t<uint64_t>* da, const along_t g, const A algo)
 {
+    if (!g.sure && !(g.gate[0] && *g.gate[0]) && !(g.gate[1] && *g.gate[1])) return;
     __shared__ typename A::lds_t lds[BAM_TRIP_WAVES];
     __shared__ uint32_t left[BAM_TRIP_WAVES];
     __shared__ unsigned long long base;
@@ -1143,15 +1147,26 @@ struct by_page_plan { uint64_t n_edges = 0, n_pages = 0; uint32_t epp = 0, ppw =
 
 /* the end of a level: the device's `changed` word goes to the host through pinned memory, and it and the counter the next
  * sweep takes its work from start the next level at zero.  One small launch instead of two copies and a fill. */
-#define BAM_PLAN_WORDS 128u             /* words of a plan: [0] pieces, [1] next piece of work, [2] changed; the others, written by many waves, on lines of their own */
-#define BAM_PLAN_FLAGS 16u              /* along_t::flags */
-#define BAM_PLAN_MISSING 32u            /* along_t::n_missing */
-#define BAM_PLAN_CHUNK 48u              /* along_t::next_chunk */
+/* words of a plan: [0] pieces, [1] next piece of work, [2] changed; then, written by many waves and on lines of their own, the words
+ * of along_t for each of the sweeps that are queued before the host looks */
+#define BAM_PLAN_SWEEPS 6u
+#define BAM_PLAN_WORDS (16u + BAM_PLAN_SWEEPS * 48u)
+#define BAM_PLAN_FLAGS(k) (16u + (k) * 48u)          /* along_t::flags of sweep k, */
+#define BAM_PLAN_MISSING(k) (32u + (k) * 48u)        /* n_missing, */
+#define BAM_PLAN_CHUNK(k) (48u + (k) * 48u)          /* next_chunk */
 __global__ void k_level_end(unsigned long long* words, volatile uint64_t* host_flag)
 {
-    host_flag[0] = words[2] | words[BAM_PLAN_FLAGS];
-    host_flag[1] = words[BAM_PLAN_FLAGS + 1];
-    words[1] = words[2] = words[BAM_PLAN_FLAGS] = words[BAM_PLAN_FLAGS + 1] = words[BAM_PLAN_MISSING] = words[BAM_PLAN_CHUNK] = 0;
+    *host_flag = words[2];
+    words[1] = words[2] = 0;
+}
+/* the end of the sweeps along the edges that were queued: two flags of each to the host; one wave */
+__global__ void k_sweeps_end(unsigned long long* words, volatile uint64_t* host_flags)
+{
+    const uint32_t k = threadIdx.x;
+    if (k >= BAM_PLAN_SWEEPS) return;
+    host_flags[2 * k] = words[BAM_PLAN_FLAGS(k)];
+    host_flags[2 * k + 1] = words[BAM_PLAN_FLAGS(k) + 1];
+    words[BAM_PLAN_FLAGS(k)] = words[BAM_PLAN_FLAGS(k) + 1] = words[BAM_PLAN_MISSING(k)] = words[BAM_PLAN_CHUNK(k)] = 0;
 }
 
 /*
@@ -1191,7 +1206,7 @@ struct graph_plan {
         const uint64_t cap = 2 * (n_edges / BAM_HEAVY_EDGES) + 1;
         buf = createBuffer(cap * sizeof(heavy_piece_t), 0);
         words = createBuffer(BAM_PLAN_WORDS * sizeof(unsigned long long), 0);
-        host_words = createHostBuffer(64);
+        host_words = createHostBuffer(2 * BAM_PLAN_SWEEPS * sizeof(uint64_t));
         pieces = (heavy_piece_t*)buf.get();
         count = (unsigned long long*)words.get();
         changed = (uint64_t*)words.get() + 2;
@@ -1231,6 +1246,13 @@ struct graph_plan {
         hip_err_chk(hipGetLastError());
         hip_err_chk(hipStreamSynchronize(st));
         return *host_flag != 0;
+    }
+    /* the same for the sweeps along the edges: host_flag[2 k], [2 k + 1] are what sweep k found */
+    void sweeps_end(hipStream_t st)
+    {
+        hipLaunchKernelGGL(k_sweeps_end, dim3(1), dim3(BAM_WAVE_SIZE), 0, st, count, host_flag);
+        hip_err_chk(hipGetLastError());
+        hip_err_chk(hipStreamSynchronize(st));
     }
     int by_page(bam_array_t* edges, hipStream_t st);
     bool along_edges(bam_array_t* edges, hipStream_t st);
@@ -1285,9 +1307,10 @@ int graph_plan::by_page(bam_array_t* edges, hipStream_t st)
             hipLaunchKernelGGL(k_page_first_vertex, dim3(blocks_for(n_segs + 1, 256)), dim3(256), 0, st, offsets, n_vertices, (uint64_t)BAM_SEG_EDGES, n_segs, seg_first);
         along.ahead = bit_words ? bits : nullptr;
         along.missing = (uint32_t*)(bits + bit_words);
-        along.n_missing = count + BAM_PLAN_MISSING;
-        along.next_chunk = count + BAM_PLAN_CHUNK;
-        along.flags = count + BAM_PLAN_FLAGS;
+        along.n_missing = count + BAM_PLAN_MISSING(0);
+        along.next_chunk = count + BAM_PLAN_CHUNK(0);
+        along.flags = count + BAM_PLAN_FLAGS(0);
+        along.sure = 1;
         /* as many waves as leave each a batch worth sending (pages a wave, ms: 29 500 cached, BFS of 2^21 vertices 64 11.8, 32 11.4, 16
          * 11.6, 8 11.9; 7 500, 2^19 16 3.18, 8 3.11, 4 3.27; 3 700, 2^18 16 1.89, 8 1.73, 4 1.79; 2 048, 2^16 16 0.88, 8 0.72, 4 0.62, 2 0.70) */
         along_chunk = 32;
@@ -1316,44 +1339,60 @@ bool graph_plan::along_edges(bam_array_t* edges, hipStream_t st)
 }
 
 extern "C++" {
-/* one reading of the edge array, or of what the algorithm wants of it */
+/* one reading of the edge array, or of what the algorithm wants of it, with the words g names */
 template <typename A>
-void along_sweep(bam_array_t* edges, const graph_plan* pl, const A& algo, hipStream_t st)
+void along_sweep(bam_array_t* edges, const graph_plan* pl, const along_t& g, const A& algo, hipStream_t st)
 {
-    const uint64_t trips = (pl->along.n_segs + pl->along.trip_segs - 1) / pl->along.trip_segs;
+    const uint64_t trips = (g.n_segs + g.trip_segs - 1) / g.trip_segs;
     const uint32_t blocks = (uint32_t)std::min<uint64_t>(A::most_blocks, (trips + BAM_TRIP_WAVES - 1) / BAM_TRIP_WAVES);
-    hipLaunchKernelGGL(k_along_resident<A>, dim3(blocks), dim3(BAM_TRIP_WAVES * BAM_WAVE_SIZE), 0, st, edges->a->d_array_ptr, pl->along, algo);
-    hipLaunchKernelGGL(k_along_missing<A>, dim3(pl->along_waves), dim3(BAM_WAVE_SIZE), 0, st, edges->a->d_array_ptr, pl->along, algo, pl->along_chunk);
+    hipLaunchKernelGGL(k_along_resident<A>, dim3(blocks), dim3(BAM_TRIP_WAVES * BAM_WAVE_SIZE), 0, st, edges->a->d_array_ptr, g, algo);
+    hipLaunchKernelGGL(k_along_missing<A>, dim3(pl->along_waves), dim3(BAM_WAVE_SIZE), 0, st, edges->a->d_array_ptr, g, algo, pl->along_chunk);
     hip_err_chk(hipGetLastError());
 }
 }
 
-/* all levels from labels of which the source's is set; the number of levels there are */
+/*
+ * All levels from labels of which the source's is set; the number of levels there are.  BAM_PLAN_SWEEPS sweeps are queued before
+ * the host looks, each made only if the ones before found vertices for it: with a look after every level that look was most of a
+ * small graph's time (all cached, 2^12 vertices, 5 levels: 118 -> 74 us; 2^16, 6: 197 -> 137; 2^20, 6: 479 -> 418; three sweeps at a time
+ * 88, 150, 433, eight 84, 146, 424).
+ */
 uint32_t bfs_along_levels(bam_array_t* edges, graph_plan* pl, uint32_t* d_labels, hipStream_t st)
 {
     const bool ahead = pl->along.ahead != nullptr;
     if (ahead) hip_err_chk(hipMemsetAsync(pl->along.ahead, 0, pl->along.n_segs * BAM_SEG_ROWS * sizeof(uint64_t), st));
-    /* whether this level has vertices for sure, and whether the next two may */
+    unsigned long long* const words = pl->count;
+    /* a level has vertices for sure if the sweep before found some; it may have some if the one before that found some ahead */
     bool sure = true, next = false;
-    uint32_t level = 0;
-    for (;; level++) {
-        if (ahead) along_sweep(edges, pl, bfs_along<true>{d_labels, level}, st);
-        else along_sweep(edges, pl, bfs_along<false>{d_labels, level}, st);
-        const bool found = pl->level_end(st), found_ahead = pl->host_flag[1] != 0;
-        if (!found && !next) break;
-        sure = found;
-        next = found_ahead;
+    for (uint32_t base = 0;; base += BAM_PLAN_SWEEPS) {
+        for (uint32_t k = 0; k < BAM_PLAN_SWEEPS; k++) {
+            along_t g = pl->along;
+            g.flags = words + BAM_PLAN_FLAGS(k);
+            g.n_missing = words + BAM_PLAN_MISSING(k);
+            g.next_chunk = words + BAM_PLAN_CHUNK(k);
+            g.sure = k == 0 || (k == 1 && next);
+            g.gate[0] = k ? words + BAM_PLAN_FLAGS(k - 1) : nullptr;
+            g.gate[1] = k > 1 ? words + BAM_PLAN_FLAGS(k - 2) + 1 : nullptr;
+            if (ahead) along_sweep(edges, pl, g, bfs_along<true>{d_labels, base + k}, st);
+            else along_sweep(edges, pl, g, bfs_along<false>{d_labels, base + k}, st);
+        }
+        pl->sweeps_end(st);
+        for (uint32_t k = 0; k < BAM_PLAN_SWEEPS; k++) {
+            const bool found = pl->host_flag[2 * k] != 0, found_ahead = pl->host_flag[2 * k + 1] != 0;
+            if (found || next) { sure = found; next = found_ahead; continue; }
+            if (sure) return base + k + 1;
+            /* the last sweep was for vertices that a sweep ahead of their level had found; a nearer one may have found them since */
+            hipLaunchKernelGGL(k_any_label, dim3(1024), dim3(256), 0, st, d_labels, pl->n_vertices, base + k, words + BAM_PLAN_FLAGS(0));
+            pl->sweeps_end(st);
+            return pl->host_flag[0] ? base + k + 1 : base + k;
+        }
     }
-    if (sure) return level + 1;
-    /* the last sweep was for vertices that a sweep ahead of their level had found; a nearer one may have found them since */
-    hipLaunchKernelGGL(k_any_label, dim3(1024), dim3(256), 0, st, d_labels, pl->n_vertices, level, pl->along.flags);
-    return pl->level_end(st) ? level + 1 : level;
 }
 
 /* one reading of the edges that joins the trees of their ends.  In one launch where all are cached and few: 2^15 entries take 80 us, in two 88 */
 void cc_read_edges(bam_array_t* edges, graph_plan* pl, unsigned long long* comp, hipStream_t st)
 {
-    if (pl->along.n_segs && !(pl->all_cached && pl->bp.n_edges <= 1ull << 17)) along_sweep(edges, pl, cc_along{comp}, st);
+    if (pl->along.n_segs && !(pl->all_cached && pl->bp.n_edges <= 1ull << 17)) along_sweep(edges, pl, pl->along, cc_along{comp}, st);
     else if (pl->bp.n_pages)
         hipLaunchKernelGGL(k_cc_by_page, dim3(pl->bp.blocks), dim3(BAM_WAVE_SIZE), 0, st, edges->a->d_array_ptr, pl->offsets, (const uint64_t*)pl->bp.first.get(), pl->bp.n_edges, pl->bp.ppw,
                            pl->cc_backwards(), comp);

@@ -68,6 +68,20 @@ def test_labels_and_levels_of_a_random_graph(bam, page, cache_pages):
             assert not r.c.aborted()
 
 
+@pytest.mark.parametrize("n_levels", [1, 2, 5, 6, 7, 11, 12, 13, 19])
+@pytest.mark.parametrize("entries,cache_pages", [(1, 64), (700, 6)])
+def test_as_many_levels_as_are_queued_at_a_time(bam, n_levels, entries, cache_pages):
+    """a path, one vertex a level: around the number of sweeps between two looks of the host, all edges cached and most of them not
+    (every list holds its one neighbour `entries` times)"""
+    off = np.concatenate([np.arange(n_levels) * entries, [(n_levels - 1) * entries], [(n_levels - 1) * entries]]).astype(np.uint64)[: n_levels + 1]
+    nb = np.repeat(np.arange(1, max(n_levels, 2)), entries).astype(np.uint64)[: max(1, (n_levels - 1) * entries)]
+    if n_levels == 1:
+        off, nb = np.array([0, 0, 1], dtype=np.uint64), np.zeros(1, dtype=np.uint64)      # the source has no list
+    r, a = _rig(bam, nb, 4096, cache_pages)
+    with r:
+        _check_bfs(r, a, off, nb, [0])
+
+
 def test_a_vertex_found_two_levels_ahead_and_then_nearer(bam):
     """Twelve pages behind eight, read front to back by one wave.  Page 1: vertex 1 (level 1) finds vertex 3 (level 2).  Page 2 is
     there for vertex 2 (level 1) and holds the list of vertex 3, which finds vertex 9 ahead, as of level 3.  Page 3: vertex 4
