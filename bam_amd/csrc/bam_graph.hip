@@ -584,9 +584,11 @@ __device__ __forceinline__ void cc_join(unsigned long long* comp, const uint64_t
     const unsigned long long u = bam::ld_relaxed(comp + a), v = bam::ld_relaxed(comp + b);
     if (u != v) cc_join_trees(comp, u, v);
 }
-__global__ void k_cc_settle(unsigned long long* comp, uint64_t vertex_count)
+/* n_missing, next_chunk: along_t's, of the reading before, which are zero between sweeps (NULL: it had none) */
+__global__ void k_cc_settle(unsigned long long* comp, uint64_t vertex_count, unsigned long long* n_missing, unsigned long long* next_chunk)
 {
     const uint64_t v = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (v == 0 && n_missing) *n_missing = *next_chunk = 0;
     if (v >= vertex_count) return;
     unsigned long long r = v;
     for (unsigned long long up = bam::ld_relaxed(comp + r); up != r; up = bam::ld_relaxed(comp + r)) r = up;
@@ -1127,12 +1129,10 @@ __global__ void k_sssp_update(bool* label, uint32_t* costList, const uint32_t* n
     }
 }
 
-/* every vertex by itself, and an empty list of missing pages for the reading behind it (NULL: none) */
-__global__ void k_iota(unsigned long long* p, uint64_t n, unsigned long long* n_missing, unsigned long long* next_chunk)
+__global__ void k_iota(unsigned long long* p, uint64_t n)
 {
     const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) p[i] = i;
-    if (i == 0 && n_missing) *n_missing = *next_chunk = 0;
 }
 
 } // namespace
@@ -1535,7 +1535,7 @@ int bam_cc_shaped(bam_array_t* edges, const uint64_t* d_offsets, uint64_t n_vert
     const shaped_launch sl = shape_of(shape, n_vertices, coarse, stride, edges->a->adt.n_ranges ? edges->a->h_ranges[0].cache.n_pages : 0);
     bool* curr = (bool*)graph_plan::sized(pl->bytes_a, n_vertices);
     bool* next = (bool*)graph_plan::sized(pl->bytes_b, n_vertices);
-    hipLaunchKernelGGL(k_iota, dim3(blocks_for(n_vertices, 256)), dim3(256), 0, st, (unsigned long long*)d_labels, n_vertices, (unsigned long long*)nullptr, (unsigned long long*)nullptr);
+    hipLaunchKernelGGL(k_iota, dim3(blocks_for(n_vertices, 256)), dim3(256), 0, st, (unsigned long long*)d_labels, n_vertices);
     hip_err_chk(hipMemsetAsync(curr, 0x01, n_vertices, st));
     hip_err_chk(hipMemsetAsync(next, 0x00, n_vertices, st));
     uint32_t iter = 0;
@@ -1635,12 +1635,12 @@ int bam_cc(bam_array_t* edges, const uint64_t* d_offsets, uint64_t n_vertices, u
     const uint64_t group = coarse > 512 ? coarse : 512;
     unsigned long long* comp = (unsigned long long*)d_labels;
     const bool along = pl->along_edges(edges, st);
-    hipLaunchKernelGGL(k_iota, dim3(blocks_for(n_vertices, 256)), dim3(256), 0, st, comp, n_vertices, pl->along.n_missing, pl->along.next_chunk);
+    hipLaunchKernelGGL(k_iota, dim3(blocks_for(n_vertices, 256)), dim3(256), 0, st, comp, n_vertices);
     if (along) cc_read_edges(edges, pl, comp, st);
     else
         hipLaunchKernelGGL(k_cc_coalesce_coarse_ptr_pc, dim3(pl->blocks(n_vertices, group)), dim3(128), 0, st, edges->a->d_array_ptr, n_vertices, d_offsets, comp, group,
                        pl->pieces, pl->n_pieces, pl->next_work(), pl->cc_backwards());
-    hipLaunchKernelGGL(k_cc_settle, dim3(blocks_for(n_vertices, 256)), dim3(256), 0, st, comp, n_vertices);
+    hipLaunchKernelGGL(k_cc_settle, dim3(blocks_for(n_vertices, 256)), dim3(256), 0, st, comp, n_vertices, pl->along.n_missing, pl->along.next_chunk);
     hip_err_chk(hipGetLastError());
     if (along) { hip_err_chk(hipStreamSynchronize(st)); }
     else pl->level_end(st);
@@ -1689,7 +1689,7 @@ int bam_cc_by_page(bam_array_t* edges, const uint64_t* d_offsets, uint64_t n_ver
     graph_plan* pl = plan_for(edges, d_offsets, n_vertices, 0, st, local);
     if (int rc = pl->by_page(edges, st)) return rc;
     unsigned long long* comp = (unsigned long long*)d_labels;
-    hipLaunchKernelGGL(k_iota, dim3(blocks_for(n_vertices, 256)), dim3(256), 0, st, comp, n_vertices, pl->along.n_missing, pl->along.next_chunk);
+    hipLaunchKernelGGL(k_iota, dim3(blocks_for(n_vertices, 256)), dim3(256), 0, st, comp, n_vertices);
     uint32_t iter = 0;
     bool changed = true;
     /*
@@ -1717,7 +1717,7 @@ int bam_cc_by_page(bam_array_t* edges, const uint64_t* d_offsets, uint64_t n_ver
     }
     if (changed) {
         cc_read_edges(edges, pl, comp, st);
-        hipLaunchKernelGGL(k_cc_settle, dim3(blocks_for(n_vertices, 256)), dim3(256), 0, st, comp, n_vertices);
+        hipLaunchKernelGGL(k_cc_settle, dim3(blocks_for(n_vertices, 256)), dim3(256), 0, st, comp, n_vertices, pl->along.n_missing, pl->along.next_chunk);
         hip_err_chk(hipGetLastError());
         hip_err_chk(hipStreamSynchronize(st));
         iter += 2;

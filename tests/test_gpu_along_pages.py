@@ -82,6 +82,25 @@ def test_as_many_levels_as_are_queued_at_a_time(bam, n_levels, entries, cache_pa
         _check_bfs(r, a, off, nb, [0])
 
 
+@pytest.mark.parametrize("by_page", [False, True])
+def test_levels_after_components_with_one_plan(bam, by_page):
+    """the list of missing pages is empty again when a call ends, whichever call comes next"""
+    off, nb = oracle.uniform_csr(SEED, 20011, 60007)
+    src = int(oracle.bfs_sources(SEED, off, 1)[0])
+    want, want_it = oracle.bfs_levels(off, nb, src)
+    labels, _ = oracle.cc_labels(off, nb)
+    r, a = _rig(bam, nb, 4096, 24)
+    with r:
+        d_off = _dev(off)
+        a.set_graph(d_off)
+        for _ in range(3):
+            lb, _ = a.cc(d_off, by_page=by_page)
+            assert np.array_equal(_u64(lb), labels)
+            lv, it = a.bfs(d_off, src, by_page=by_page)
+            assert np.array_equal(lv.cpu().numpy().view(np.uint32), want) and it == want_it
+        assert not r.c.aborted()
+
+
 def test_a_vertex_found_two_levels_ahead_and_then_nearer(bam):
     """Twelve pages behind eight, read front to back by one wave.  Page 1: vertex 1 (level 1) finds vertex 3 (level 2).  Page 2 is
     there for vertex 2 (level 1) and holds the list of vertex 3, which finds vertex 9 ahead, as of level 3.  Page 3: vertex 4
