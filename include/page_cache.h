@@ -85,11 +85,13 @@ enum data_dist_t { REPLICATE = 0, STRIPE = 1 };
  * load up to direct_limit; AHEAD: the wave fetches for others that compute meanwhile, up to direct_limit_ahead; PULLED:
  * the wave has nothing else to do and nobody computes beside it, so it pulls all of it from the staging pages itself
  * (waves that only fetch, alone on the device: 262144 pages in 19.9 ms = 13.2 M pages/s all pulled; 20.7 ms with at most
- * 1024 commands placed by the controller, 22.9 with 8192: what the controller pushes takes it ten times as long)
+ * 1024 commands placed by the controller, 22.9 with 8192: what the controller pushes takes it ten times as long); AGAIN: the
+ * same, into slots that the wave names (find_slot, range_view::again).
  */
 #define BAM_PLACE_NORMAL 0u
 #define BAM_PLACE_AHEAD  1u
 #define BAM_PLACE_PULLED 2u
+#define BAM_PLACE_AGAIN  3u
 
 #define BAM_TOKEN_SLOTS 4096u
 #define BAM_STAT_SHARDS 4096
@@ -166,7 +168,7 @@ struct page_cache_d_t {
     uint32_t spin_limit;
 
     __forceinline__ __device__ cache_page_t* get_cache_page(const uint32_t page) const { return &cache_pages[page]; }
-    __forceinline__ __device__ uint32_t find_slot(uint64_t address, uint64_t range_id, const uint32_t queue_);
+    __forceinline__ __device__ uint32_t find_slot(uint64_t address, uint64_t range_id, const uint32_t queue_, uint32_t again = 0xffffffffu);
     __forceinline__ __device__ bool spin_giveup(bam::spin_t& s) const { return bam::spin_giveup(guard, spin_limit, s); }
 };
 
@@ -437,7 +439,7 @@ inline __device__ void read_begin(page_cache_d_t* pc, QueuePair* qp, const uint6
         bam::for_each_group((uint64_t)qp, (uint64_t)pc, [&](uint64_t q, uint64_t c) {
             bam::for_each_chunk(((QueuePair*)q)->sq.qs >> 1, [&]() {
                 ok = bam::io_group((page_cache_d_t*)c, (QueuePair*)q, starting_lba, (uint32_t)n_blocks, pc_entry, NVM_IO_READ,
-                                   place == BAM_PLACE_PULLED ? 0u : ((page_cache_d_t*)c)->direct_share);
+                                   place >= BAM_PLACE_PULLED ? 0u : ((page_cache_d_t*)c)->direct_share);
             });
         });
         return;
@@ -445,8 +447,8 @@ inline __device__ void read_begin(page_cache_d_t* pc, QueuePair* qp, const uint6
     QueuePair* cur = (QueuePair*)bam::first((uint64_t)qp);
     page_cache_d_t* cpc = (page_cache_d_t*)bam::first((uint64_t)pc);
     uint32_t pos;
-    uint32_t gauged = place == BAM_PLACE_PULLED ? 0u : place == BAM_PLACE_AHEAD ? 2u : 1u;
-    cid = bam::io_submit_group(cpc, cur, starting_lba, (uint32_t)n_blocks, pc_entry, NVM_IO_READ, stage, pos, place == BAM_PLACE_PULLED ? 0u : cpc->direct_share, gauged);
+    uint32_t gauged = place >= BAM_PLACE_PULLED ? 0u : place == BAM_PLACE_AHEAD ? 2u : 1u;
+    cid = bam::io_submit_group(cpc, cur, starting_lba, (uint32_t)n_blocks, pc_entry, NVM_IO_READ, stage, pos, place >= BAM_PLACE_PULLED ? 0u : cpc->direct_share, gauged);
 #ifdef BAM_PROFILE
     const uint64_t pt2 = wall_clock64();
 #endif
@@ -535,9 +537,12 @@ inline __device__ void poll_async(QueuePair* qp, uint16_t cid, uint16_t sq_pos)
  * slots and returns BAM_NO_SLOT: its caller then lets the lanes that did get
  * a slot finish their loads before trying again, so that waves never wait for
  * slots while sitting on slots other waves wait for.
+ *   `again` is a slot the caller would rather have than one the hand takes from another page of the same range (BAM_NO_SLOT:
+ * none): what is free or holds another range's page goes first, so that a cache fills and follows what it is used for.  It is
+ * taken under the same conditions, and once; then the hand.
  */
 __forceinline__ __device__
-uint32_t page_cache_d_t::find_slot(uint64_t address, uint64_t range_id, const uint32_t queue_)
+uint32_t page_cache_d_t::find_slot(uint64_t address, uint64_t range_id, const uint32_t queue_, uint32_t again)
 {
     using namespace bam;
     const uint64_t global_address = (address << n_ranges_bits) | range_id;
@@ -553,7 +558,12 @@ uint32_t page_cache_d_t::find_slot(uint64_t address, uint64_t range_id, const ui
             uint32_t base = 0;
             if (lane() == ld) base = __hip_atomic_fetch_add(page_ticket, popc(need), __ATOMIC_RELAXED, BAM_AGENT);
             base = bcast(base, ld);
-            const uint32_t p = (uint32_t)((base + rank_in(need)) % n_pages);
+            uint32_t p = (uint32_t)((base + rank_in(need)) % n_pages);
+            if (again != BAM_NO_SLOT) {
+                const uint64_t at_hand = ld_relaxed(&cache_pages[p].page_translation);
+                if ((uint32_t)(at_hand >> BAM_TAKE_SHIFT) == UNLOCKED && (at_hand & n_ranges_mask) == range_id) p = again;
+                again = BAM_NO_SLOT;
+            }
             cache_page_t* cp = &cache_pages[p];
             const uint64_t w = __hip_atomic_fetch_or(&cp->page_translation, (uint64_t)LOCKED << BAM_TAKE_SHIFT, __ATOMIC_RELAXED, BAM_AGENT);
             const uint32_t v = (uint32_t)(w >> BAM_TAKE_SHIFT);
@@ -777,7 +787,7 @@ bool range_d_t<T>::slow_step(const size_t pg, const bool write, const uint32_t q
 #ifdef BAM_PROFILE
         const uint64_t pf0 = wall_clock64();
 #endif
-        found = cache.find_slot(pg, range_id, queue);
+        found = cache.find_slot(pg, range_id, queue, place == BAM_PLACE_AGAIN ? slot : BAM_NO_SLOT);
 #ifdef BAM_PROFILE
         if (cache.prof && bam::lane() == bam::first_lane(bam::active_mask())) { atomicAdd(&cache.prof[6], wall_clock64() - pf0); atomicAdd(&cache.prof[7], 1ull); atomicAdd(&cache.prof[8], (unsigned long long)bam::popc(bam::active_mask())); }
 #endif
@@ -946,6 +956,7 @@ struct range_view {
     uint32_t page_size_log, page_size;
     uint32_t n_access = 0, n_hit = 0;   /* this lane's accesses since the last flush_stats() */
     uint32_t place = BAM_PLACE_NORMAL;  /* waves that only fetch say so: BAM_PLACE_AHEAD, BAM_PLACE_PULLED */
+    uint32_t again = 0;                 /* BAM_PLACE_AGAIN: the lane's slot, see find_slot; otherwise not looked at */
 
     __forceinline__ __device__ void load(range_d_t<T>* r_)
     {
@@ -1041,7 +1052,7 @@ struct range_view {
         const uint32_t master = first_lane(eq_mask), count = popc(eq_mask);
         const bool dirty = (ballot(write) & eq_mask) != 0;
         uint64_t sv = 0, pack = 0;
-        uint32_t slot = 0;
+        uint32_t slot = again;
         if (master == me && (!HELPERS || take)) { const bool h = bam_try_hit(dp, count, dirty, sv, slot); pack = (uint64_t)slot | ((uint64_t)h << 63); }
         pack = shfl(pack, master);
         if (__builtin_expect((pack >> 63) != 0, 1)) {          /* resident: the path to keep lean; register spills, if any, belong in the other branch */

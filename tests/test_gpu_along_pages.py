@@ -130,3 +130,38 @@ def test_a_vertex_found_two_levels_ahead_and_then_nearer(bam):
     r, a = _rig(bam, nb, 4096, 8)
     with r:
         _check_bfs(r, a, off, nb, [rank[0]] * 3)
+
+
+@pytest.mark.parametrize("page,share", [(4096, 2), (4096, 3), (4096, 60), (8192, 4)])
+def test_levels_where_a_sweep_brings_in_more_than_the_cache_holds(bam, page, share):
+    """slots used again for the next chunk: a cache that is empty, then full of another array's changed pages, then of the
+    edges; nobody's elements suffer, and the other array's go to the store"""
+    off, nb = oracle.rmat_csr(SEED, 14)
+    per = page // 8
+    pages = (len(nb) + per - 1) // per
+    cache_pages = max(3, pages // share)
+    src = int(oracle.bfs_sources(SEED, off, 1)[0])
+    want, want_it = oracle.bfs_levels(off, nb, src)
+    n_b = cache_pages * per - 5
+    with Rig(bam, (pages + cache_pages) * page, backing=True, n_queues=16, depth=256, stage_bytes=page) as r:
+        store = r.backing((pages + cache_pages) * per)
+        store[:] = oracle.store(SEED, 0, len(store))
+        store[:len(nb)] = nb
+        pc = bam.PageCache(page, cache_pages, 0, r.c)
+        rs = [bam.Range(0, len(nb), 0, pages, 0, page, pc, 0), bam.Range(0, n_b, pages, cache_pages, 0, page, pc, 0)]
+        a, b = bam.Array(len(nb), 0, [rs[0]], 0), bam.Array(n_b, pages * page, [rs[1]], 0)
+        d_off = _dev(off)
+        a.set_graph(d_off)
+        new = np.random.default_rng(page + share).integers(0, 1 << 62, n_b, dtype=np.int64).astype(np.uint64)
+        for others in (False, True, False):
+            if others:
+                b.write(n_b, _dev(new))
+            for _ in range(2):
+                lv, it = a.bfs(d_off, src, by_page=True)
+                assert np.array_equal(lv.cpu().numpy().view(np.uint32), want) and it == want_it, others
+        assert np.array_equal(_u64(a.gather(len(nb))), nb) and np.array_equal(_u64(b.gather(n_b)), new)
+        pc.flush()
+        assert np.array_equal(store[pages * per:pages * per + n_b], new) and np.array_equal(store[:len(nb)], nb)
+        assert not r.c.aborted()
+        for x in (a, b, rs[0], rs[1], pc):
+            x.close()
