@@ -743,8 +743,8 @@ __global__ __launch_bounds__(64) void k_cc_by_page(array_d_t<uint64_t>* da, cons
  * Both launches take a segment at a time: 512 entries, eight rows of 64, one per lane and row, all loaded before any is
  * used; which entries are to be visited, and for which vertex, is worked out in LDS while they are on their way.  The
  * pages are referenced meanwhile (a take and a drop per page and wave; a page is 512 entries).
- * Bound by the store where edges are missing: BFS of that graph 19.2 -> 10.9 ms (175 000 -> 124 000 page reads, 11.6 M a second),
- * with 2^18 vertices 4.8 -> 1.8; components of 2^22 vertices, 8 entries each, half cached, 4.7 -> 3.8.  All cached, by the
+ * Bound by the store where edges are missing: BFS of that graph 19.2 -> 10.9 ms (175 000 -> 124 000 page reads, 11.6 M a second), and 9.0
+ * (98 000) with the slots used again; with 2^18 vertices 4.8 -> 1.6; components of 2^22 vertices, 8 entries each, half cached, 4.7 -> 3.8.  All cached, by the
  * trips to memory a wave makes one after the other: BFS of 2^20 vertices 1.65 -> 0.47 ms, components of 2^22 1.55 -> 1.2.
  */
 #define BAM_SEG_ROWS 8u

@@ -21,7 +21,7 @@ second over the timed steps.  On the same JSON line:
                 interconnect to the GPU, both measured in this run; the
                 ceiling is the slower of the two
   block         raw block benchmark (2^22 reads, 128 queue pairs x 1024)
-  bfs           RMAT-24 BFS through the page cache (with --bfs-scale): the edge-page kernel and the reference-shaped one
+  bfs           RMAT-24 BFS through the page cache (with --bfs-scale): by its three entry points
   cc            connected components of a 2^26-vertex uniform graph, 16 GiB of edges behind an 8 GiB cache (with --cc-logv)
 
 Everything is checked against the closed-form oracle while it is measured.
@@ -452,9 +452,8 @@ def main():
             refs += list(ex.map(lambda x: oracle.bfs_levels(off_h, nb_u, int(x)), srcs[1:]))
         log("[bench] bfs oracle: %d sources, %.1fs" % (len(refs), time.time() - t1))
         legs = {}
-        # the edge-page kernel on every source; the reference-shaped kernel (a wave per vertex, bam_ptr per element) on the first two
-        # (64 vertices per wave: consecutive vertices share pages, so the more vertices a wave has, the more distinct pages are asked for at a time)
-        # and the kernel that walks a queue of the level's vertices, sorted between levels
+        # bam_bfs_by_page on every source, bam_bfs and bam_bfs_frontier on the first few: this array (one range that starts on a page,
+        # 4 KiB pages) all three read along its pages
         for name, by_page, n_src, coarse in (("by_page", True, len(srcs), 1), ("per_vertex_bam_ptr", False, min(4, len(srcs)), 64),
                                              ("queue_of_vertices", False, min(4, len(srcs)), 0)):
             tot_ms, tot_edges, levels_ok, iters = 0.0, 0, True, []
@@ -539,20 +538,19 @@ def main():
                 break
             ref = new
         assert torch.equal(ref, lb) and not ctrl.aborted(), "CC labels differ from the fixed point"
-        # the reference's per-vertex kernel (edge lists through bam_ptr) on the same graph, starting on what the sweeps above left in the cache
+        # bam_cc on the same graph, starting on what the call above left in the cache (it reads this array along its pages as well)
         a2, b2 = event(), event()
         L.bam_event_record(a2, stream)
         lb2, it2 = ac.cc(off, coarse=64)
         L.bam_event_record(b2, stream)
         ms2 = elapsed_ms(a2, b2)
         st2 = ac.stats()
-        assert torch.equal(ref, lb2) and not ctrl.aborted(), "CC labels of the per-vertex kernel differ from the fixed point"
+        assert torch.equal(ref, lb2) and not ctrl.aborted(), "CC labels of bam_cc differ from the fixed point"
         by_page = {"ms": ms, "iterations": it, "GTEPS": n_e / ms / 1e6, "read_ios": st["read_io_cnt"], "MIOPS": st["read_io_cnt"] / ms / 1e3,
                    "frac_of_ceiling": st["read_io_cnt"] / ms * 1e3 / ceiling}
         per_vertex = {"coarse": 64, "ms": ms2, "iterations": it2, "GTEPS": n_e / ms2 / 1e6, "read_ios": st2["read_io_cnt"], "MIOPS": st2["read_io_cnt"] / ms2 / 1e3,
                       "frac_of_ceiling": st2["read_io_cnt"] / ms2 * 1e3 / ceiling}
-        # the headline of the leg is the faster of the two kernels; both are reported (the per-vertex one starts on what the
-        # by-page one left in the cache)
+        # the headline of the leg is the faster of the two; both are reported (the second starts on what the first left in the cache)
         lead, lead_name = (by_page, "by_page") if ms <= ms2 else (per_vertex, "per_vertex_bam_ptr")
         cc = {"log2_vertices": args.cc_logv, "edges": n_e, "cache_pages": cache_pages, "ms": lead["ms"], "iterations": lead["iterations"],
               "GTEPS": lead["GTEPS"], "read_ios": lead["read_ios"], "MIOPS": lead["MIOPS"], "frac_of_ceiling": lead["frac_of_ceiling"],
