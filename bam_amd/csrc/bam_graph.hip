@@ -752,9 +752,10 @@ __global__ __launch_bounds__(64) void k_cc_by_page(array_d_t<uint64_t>* da, cons
 #define BAM_TRIP_SEGS 16u
 #define BAM_TRIP_WAVES 4u                       /* waves to a workgroup of the first launch: they share an add to the list */
 struct along_t {
-    const uint64_t* offsets;
+    const uint64_t* offsets;                    /* [n_vertices + 1] */
+    uint64_t n_vertices;
     const uint64_t* first;                      /* [n_segs + 1] the vertex whose list holds the segment's first entry */
-    uint64_t n_edges, n_pages, n_segs;
+    uint64_t n_edges, n_pages, n_segs;          /* of the array, which may hold more than the lists */
     uint32_t seg_log;                           /* log2 of the segments in a page, at most that of BAM_TRIP_SEGS */
     uint32_t trip_segs;                         /* segments a wave of the first launch looks after: whole pages, BAM_TRIP_SEGS at most */
     uint32_t* missing;                          /* [n_pages] the pages the first launch leaves to the second */
@@ -886,7 +887,8 @@ struct bfs_along {
     }
 };
 
-/* connected components: every entry is visited once, with the vertex whose list it is in */
+/* connected components: every entry of a list is visited once, with the vertex whose list it is in.  What the array holds before
+ * the first list and behind the last is nobody's neighbour, and need not be the number of a vertex. */
 struct cc_along {
     unsigned long long* comp;
     /* chains grow with the edges that are joined at a time: 2^22 vertices, all cached, 2.6 ms with 16384 waves, 1.45 with 4096, 1.48
@@ -894,11 +896,19 @@ struct cc_along {
     static constexpr uint64_t most_blocks = 4096 / BAM_TRIP_WAVES;
     static constexpr bool again = false;       /* every page once */
     struct lds_t { unsigned long long starts[BAM_SEG_ROWS]; uint32_t vertex[BAM_SEG_EDGES]; };      /* where lists begin; whose, from the segment's first vertex on */
-    __device__ __forceinline__ uint32_t prepare(const along_t&, lds_t&, const uint64_t, const uint32_t n_segs) const { return (1u << n_segs) - 1u; }
+    __device__ __forceinline__ uint32_t prepare(const along_t& g, lds_t&, const uint64_t seg0, const uint32_t n_segs) const
+    {
+        const uint64_t begin = g.offsets[0], end = g.offsets[g.n_vertices];
+        uint32_t wanted = 0;
+        for (uint32_t k = 0; k < n_segs; k++)
+            if ((seg0 + k) * BAM_SEG_EDGES < end && (seg0 + k + 1) * BAM_SEG_EDGES > begin) wanted |= 1u << k;
+        return wanted;
+    }
     __device__ __forceinline__ void visit(const along_t& g, lds_t& s, const uint64_t seg, const uint32_t, const uint64_t (&id)[BAM_SEG_ROWS], bool&, bool&) const
     {
         const uint32_t lane = bam::lane();
-        const uint64_t e0 = seg * BAM_SEG_EDGES, e1 = e0 + BAM_SEG_EDGES < g.n_edges ? e0 + BAM_SEG_EDGES : g.n_edges;
+        const uint64_t e0 = seg * BAM_SEG_EDGES, begin_all = g.offsets[0], end_all = g.offsets[g.n_vertices];
+        const uint64_t e1 = e0 + BAM_SEG_EDGES < end_all ? e0 + BAM_SEG_EDGES : end_all;
         const uint64_t v0 = g.first[seg], v_last = g.first[seg + 1];
         wave_lds_fence();
         if (lane < BAM_SEG_ROWS) s.starts[lane] = lane ? 0ull : 1ull;
@@ -925,7 +935,8 @@ struct cc_along {
             const uint64_t src = v0 + s.vertex[below ? r * BAM_WAVE_SIZE + 63u - (uint32_t)__builtin_clzll(below) : begin];
             if (m) begin = r * BAM_WAVE_SIZE + 63u - (uint32_t)__builtin_clzll(m);
             u[r] = w[r] = 0;
-            if (e0 + r * BAM_WAVE_SIZE + lane < e1) { u[r] = bam::ld_relaxed(comp + src); w[r] = bam::ld_relaxed(comp + id[r]); }
+            const uint64_t e = e0 + r * BAM_WAVE_SIZE + lane;
+            if (e >= begin_all && e < e1) { u[r] = bam::ld_relaxed(comp + src); w[r] = bam::ld_relaxed(comp + id[r]); }
         }
 #pragma unroll
         for (uint32_t r = 0; r < BAM_SEG_ROWS; r++) {
@@ -1311,7 +1322,7 @@ int graph_plan::by_page(bam_array_t* edges, hipStream_t st)
     if (in_segs) {
         uint64_t* const seg_first = (uint64_t*)pl.first.get() + (seg_words ? pl.n_pages + 1 : 0);
         uint64_t* const bits = (uint64_t*)pl.first.get() + pl.n_pages + 1 + seg_words;
-        along.offsets = offsets; along.n_edges = pl.n_edges; along.n_pages = pl.n_pages; along.n_segs = n_segs;
+        along.offsets = offsets; along.n_vertices = n_vertices; along.n_edges = pl.n_edges; along.n_pages = pl.n_pages; along.n_segs = n_segs;
         along.seg_log = (uint32_t)__builtin_ctzll(segs_per_page);
         along.trip_segs = (uint32_t)segs_per_page;
         /* a wave's share as small as leaves 16384 waves or more (2^20 vertices, all cached, BFS: 0.47 ms, with 8192 0.50, 4096 0.56, 2048 0.70) */

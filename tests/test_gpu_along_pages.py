@@ -68,6 +68,47 @@ def test_labels_and_levels_of_a_random_graph(bam, page, cache_pages):
             assert not r.c.aborted()
 
 
+def _two_halves(n_v, n_e):
+    """two random graphs side by side, no edge between them"""
+    (oa, na), (ob, nb) = oracle.uniform_csr(SEED, n_v, n_e), oracle.uniform_csr(SEED + 1, n_v, n_e)
+    return np.concatenate([oa, ob[1:] + oa[-1]]), np.concatenate([na, nb + np.uint64(n_v)])
+
+
+# around a row, a segment and a page of 4 KiB, and several of them; the largest graph is one that bam_cc_by_page reads in this way though all of it is cached
+@pytest.mark.parametrize("before,behind,filler,n_v,n_e,share", [
+    (b, a, f, 9001, 40009, s) for b, a in ((0, 1), (0, 64), (0, 512), (0, 5000), (1, 0), (64, 0), (512, 0), (1500, 0), (700, 1300))
+    for f in ("zeros", "vertices") for s in (1, 2)] + [(700, 1300, "vertices", 150001, 1100003, 1)])
+def test_entries_that_are_in_no_list(bam, before, behind, filler, n_v, n_e, share):
+    """an array longer than the lists of its graph: what lies before the first list and behind the last is nobody's neighbour"""
+    off, nb = _two_halves(n_v, n_e)
+    want, _ = oracle.cc_labels(off, nb)
+    assert want[n_v] == n_v
+    src = int(oracle.bfs_sources(SEED, off, 1)[0])
+    levels, n_levels = oracle.bfs_levels(off, nb, src)
+    rng = np.random.default_rng(before + behind)
+
+    def fill(n):
+        return np.zeros(n, dtype=np.uint64) if filler == "zeros" else rng.integers(0, 2 * n_v, n).astype(np.uint64)
+
+    nb = np.concatenate([fill(before), nb, fill(behind)])
+    off = off + np.uint64(before)
+    if before and filler == "zeros":
+        nb[:before] = n_v                      # (entries before the first list would be the first vertex's)
+    r, a = _rig(bam, nb, 4096, (len(nb) + 511) // 512 // share + 1)
+    with r:
+        d_off = _dev(off)
+        for kept in (False, True):
+            if kept:
+                a.set_graph(d_off)
+            for by_page in (False, True):
+                lb, _ = a.cc(d_off, by_page=by_page)
+                assert np.array_equal(_u64(lb), want), (kept, by_page)
+            for kw in KINDS:
+                lv, it = a.bfs(d_off, src, **kw)
+                assert np.array_equal(lv.cpu().numpy().view(np.uint32), levels) and it == n_levels, (kept, kw)
+        assert not r.c.aborted()
+
+
 @pytest.mark.parametrize("n_levels", [1, 2, 5, 6, 7, 11, 12, 13, 19])
 @pytest.mark.parametrize("entries,cache_pages", [(1, 64), (700, 6)])
 def test_as_many_levels_as_are_queued_at_a_time(bam, n_levels, entries, cache_pages):
