@@ -781,6 +781,32 @@ __device__ __forceinline__ void raise_flag(unsigned long long* flag, const bool 
 }
 
 /*
+ * Whose lists the entries of a segment are in, found from the entries, where the vertices between its first and its last list are too
+ * many to be gone over: a run of vertices without lists lies in one segment whatever its length, and one wave has it.  (2^17 entries,
+ * half of them among the first vertices of 2^26 and half among the last: BFS, 8 levels, 867 ms gone over, 0.28 looked up, 1.06 over
+ * queues of vertices.)  The owner of entry e0 + 64 r + lane, r = r0 and r0 + 1, is v0 + at[r - r0]: the last of the vertices
+ * v0 .. v0 + span whose list begins there or before; only of use for entries of [offsets[0], offsets[V]).  Two searches side by side:
+ * four took 20 registers more, which every other sweep would pay for.
+ *   From how many vertices to a segment on: entries scattered over 2^13, 2^14, 2^15, 2^16 vertices a segment, levels (gone over 256 at a
+ * time) 95, 140, 236, 571 us and looked up 135, 213, 314, 428; joins (64 at a time) 223, 408, 715, 1273 and 198, 329, 527, 838, with 2^12
+ * the same.
+ */
+#define BAM_SEG_SPAN_LEVELS 32768u
+#define BAM_SEG_SPAN_JOINS 4096u
+__device__ __forceinline__ void segment_owners(const uint64_t* offsets, const uint64_t v0, const uint64_t span, const uint64_t e0, const uint32_t r0, uint64_t (&at)[2])
+{
+    const uint64_t* const from = offsets + v0;
+    const uint64_t e = e0 + r0 * BAM_WAVE_SIZE + bam::lane();
+#pragma unroll
+    for (uint32_t r = 0; r < 2; r++) at[r] = 0;
+#pragma unroll 1
+    for (uint64_t len = span + 1; len > 1; len -= len / 2)
+#pragma unroll
+        for (uint32_t r = 0; r < 2; r++)
+            if (from[at[r] + len / 2] <= e + r * BAM_WAVE_SIZE) at[r] += len / 2;
+}
+
+/*
  * One level of BFS.  AHEAD: the entries of vertices found on this very level are visited along with those of the level
  * itself where their page is at hand anyway; the neighbours they find are two levels on, as far as is known (somebody nearer
  * may still be looking at them, hence the minimum), and are not visited from before the next level, when their labels are
@@ -818,7 +844,24 @@ struct bfs_along {
         wave_lds_fence();
         const uint64_t e0 = seg0 * BAM_SEG_EDGES, e1 = e0 + n_segs * BAM_SEG_EDGES < g.n_edges ? e0 + n_segs * BAM_SEG_EDGES : g.n_edges;
         const uint64_t v_last = g.first[seg0 + n_segs];
-        for (uint64_t vbase = g.first[seg0]; vbase <= v_last; vbase += 4 * BAM_WAVE_SIZE) {
+        const uint64_t v_first = g.first[seg0];
+        const bool few_lists = v_last - v_first > (uint64_t)n_segs * BAM_SEG_SPAN_LEVELS;
+        if (few_lists) {
+#pragma unroll 1
+            for (uint32_t r0 = 0; r0 < n_words; r0 += 2) {
+                const uint64_t seg = seg0 + r0 / BAM_SEG_ROWS, v0 = g.first[seg];
+                uint64_t at[2];
+                segment_owners(g.offsets, v0, g.first[seg + 1] - v0, e0, r0, at);
+#pragma unroll
+                for (uint32_t r = 0; r < 2; r++) {
+                    const uint64_t e = e0 + (r0 + r) * BAM_WAVE_SIZE + lane;
+                    const uint32_t l = e >= g.offsets[0] && e < g.offsets[g.n_vertices] ? bam::ld_relaxed(label + v0 + at[r]) : MYINFINITY;
+                    const uint64_t now = bam::ballot(l == level), next = AHEAD ? bam::ballot(l == level + 1) : 0ull;
+                    if (lane == 0) { s.now[r0 + r] = now; if (AHEAD) s.next[r0 + r] = next; }
+                }
+            }
+        }
+        for (uint64_t vbase = few_lists ? v_last + 1 : v_first; vbase <= v_last; vbase += 4 * BAM_WAVE_SIZE) {
             /* four vertices to a lane at a time: most sweeps find few or none of their level, and are the trips of these loads */
             uint32_t l[4];
 #pragma unroll
@@ -911,10 +954,19 @@ struct cc_along {
         const uint64_t e1 = e0 + BAM_SEG_EDGES < end_all ? e0 + BAM_SEG_EDGES : end_all;
         const uint64_t v0 = g.first[seg], v_last = g.first[seg + 1];
         wave_lds_fence();
-        if (lane < BAM_SEG_ROWS) s.starts[lane] = lane ? 0ull : 1ull;
+        const bool few_lists = v_last - v0 > BAM_SEG_SPAN_JOINS;      /* every entry is taken for the beginning of its list */
+        if (lane < BAM_SEG_ROWS) s.starts[lane] = few_lists ? ~0ull : lane ? 0ull : 1ull;
         if (lane == 0) s.vertex[0] = 0;
         wave_lds_fence();
-        for (uint64_t vbase = v0 + 1; vbase <= v_last; vbase += BAM_WAVE_SIZE) {
+        if (few_lists)
+#pragma unroll 1
+            for (uint32_t r0 = 0; r0 < BAM_SEG_ROWS; r0 += 2) {
+                uint64_t at[2];
+                segment_owners(g.offsets, v0, v_last - v0, e0, r0, at);
+#pragma unroll
+                for (uint32_t r = 0; r < 2; r++) s.vertex[(r0 + r) * BAM_WAVE_SIZE + lane] = (uint32_t)at[r];
+            }
+        for (uint64_t vbase = few_lists ? v_last + 1 : v0 + 1; vbase <= v_last; vbase += BAM_WAVE_SIZE) {
             const uint64_t v = vbase + lane;
             uint64_t es = 0, ee = 0;
             if (v <= v_last) { es = g.offsets[v]; ee = g.offsets[v + 1]; }
@@ -1311,7 +1363,7 @@ int graph_plan::by_page(bam_array_t* edges, hipStream_t st)
     pl.ppw = (uint32_t)ppw;
     pl.blocks = (uint32_t)waves;                               /* one wave per workgroup */
     const uint64_t segs_per_page = r.cache.page_size / (BAM_SEG_EDGES * 8);
-    const bool in_segs = segs_per_page && segs_per_page <= BAM_TRIP_SEGS && pl.n_pages && pl.n_pages <= 0xFFFFFFFFull;
+    const bool in_segs = segs_per_page && segs_per_page <= BAM_TRIP_SEGS && pl.n_pages && pl.n_pages <= 0xFFFFFFFFull && n_vertices <= 1ull << 32;
     const uint64_t n_segs = in_segs ? (pl.n_edges + BAM_SEG_EDGES - 1) / BAM_SEG_EDGES : 0;
     /* one allocation: the first vertices of the pages, of the segments where those are not the pages, the bits (only where some
      * edges are on the store are there sweeps to spare), the list of missing pages */
@@ -1417,10 +1469,11 @@ uint32_t bfs_along_levels(bam_array_t* edges, graph_plan* pl, uint32_t* d_labels
     }
 }
 
-/* one reading of the edges that joins the trees of their ends.  In one launch where all are cached and few: 2^15 entries take 80 us, in two 88 */
+/* one reading of the edges that joins the trees of their ends.  In one launch where all are cached and few: 2^15 entries take 80 us, in two
+ * 88; but that one goes over the vertices between the lists of a page, so not where there may be many */
 void cc_read_edges(bam_array_t* edges, graph_plan* pl, unsigned long long* comp, hipStream_t st)
 {
-    if (pl->along.n_segs && !(pl->all_cached && pl->bp.n_edges <= 1ull << 17)) along_sweep(edges, pl, pl->along, cc_along{comp}, st);
+    if (pl->along.n_segs && !(pl->all_cached && pl->bp.n_edges <= 1ull << 17 && pl->n_vertices <= pl->bp.n_edges / 4)) along_sweep(edges, pl, pl->along, cc_along{comp}, st);
     else if (pl->bp.n_pages)
         hipLaunchKernelGGL(k_cc_by_page, dim3(pl->bp.blocks), dim3(BAM_WAVE_SIZE), 0, st, edges->a->d_array_ptr, pl->offsets, (const uint64_t*)pl->bp.first.get(), pl->bp.n_edges, pl->bp.ppw,
                            pl->cc_backwards(), comp);

@@ -109,6 +109,71 @@ def test_entries_that_are_in_no_list(bam, before, behind, filler, n_v, n_e, shar
         assert not r.c.aborted()
 
 
+# vertices without lists before, between and behind those that have some: around the spans from which owners of entries are looked up
+@pytest.mark.parametrize("page,share", [(4096, 1), (4096, 4), (8192, 2), (65536, 2)])
+@pytest.mark.parametrize("run,scattered", [(4094, 1), (4095, 1), (4096, 1), (32766, 1), (32767, 1), (32768, 1), (70001, 1), (540000, 1), (40, 4099), (3, 70000)])
+def test_long_runs_of_vertices_without_lists(bam, page, share, run, scattered):
+    """a random graph on some of the vertices: a run of `run` others after the first third of them, another before the first and
+    behind the last, and every `scattered`-th vertex of the last eighth of them"""
+    n = 4001
+    off, nb = oracle.uniform_csr(SEED, n, 24007 if page < 65536 else 90001)
+    place = np.arange(n, dtype=np.int64) + run                # where vertex v of that graph is
+    place[n // 3:] += run
+    place[n - n // 8:] += np.arange(n // 8) * min(scattered - 1, 4000000 // n)
+    n_v = int(place[-1]) + 1 + run
+    deg = np.zeros(n_v, dtype=np.uint64)
+    deg[place] = off[1:] - off[:-1]
+    sources = [int(x) for x in oracle.bfs_sources(SEED, off, 2)]
+    want = []
+    for src in sources:
+        lv, it = oracle.bfs_levels(off, nb, src)
+        all_levels = np.full(n_v, 0xFFFFFFFF, dtype=np.uint32)
+        all_levels[place] = lv
+        want.append((all_levels, it))
+    comp, _ = oracle.cc_labels(off, nb)
+    labels = np.arange(n_v, dtype=np.uint64)
+    labels[place] = place[comp.astype(np.int64)].astype(np.uint64)      # (the order of the vertices is the same)
+    off, nb = np.concatenate([[0], np.cumsum(deg)]).astype(np.uint64), place[nb.astype(np.int64)].astype(np.uint64)
+    r, a = _rig(bam, nb, page, max(2, (len(nb) * 8 + page - 1) // page // share))
+    with r:
+        d_off = _dev(off)
+        a.set_graph(d_off)
+        for kw in KINDS:
+            for src, (lv_want, it_want) in zip(sources, want):
+                lv, it = a.bfs(d_off, int(place[src]), **kw)
+                assert np.array_equal(lv.cpu().numpy().view(np.uint32), lv_want) and it == it_want, kw
+        for by_page in (False, True):
+            lb, _ = a.cc(d_off, by_page=by_page)
+            assert np.array_equal(_u64(lb), labels), by_page
+        assert not r.c.aborted()
+
+
+def test_a_run_of_vertices_without_lists_is_not_gone_over(bam):
+    """2^24 of them in the middle: one wave went over them on every level, 200 ms a call (and 1 ms vertex by vertex)"""
+    import time
+    import torch
+    n, run = 4001, 1 << 24
+    off, nb = oracle.uniform_csr(SEED, n, 24007)
+    place = np.arange(n, dtype=np.int64)
+    place[n // 2:] += run
+    deg = np.zeros(n + run, dtype=np.uint64)
+    deg[place] = off[1:] - off[:-1]
+    r, a = _rig(bam, nb, 4096, 200)
+    with r:
+        d_off = _dev(np.concatenate([[0], np.cumsum(deg)]).astype(np.uint64))
+        r.backing(len(nb))[:] = place[nb.astype(np.int64)]
+        a.set_graph(d_off)
+        for call in (lambda: a.bfs(d_off, int(place[int(nb[0])]), frontier=True), lambda: a.bfs(d_off, int(place[int(nb[0])]), coarse=64), lambda: a.cc(d_off)):
+            took = []
+            for _ in range(4):
+                torch.cuda.synchronize()
+                t = time.perf_counter()
+                call()
+                torch.cuda.synchronize()
+                took.append(time.perf_counter() - t)
+            assert min(took) < 0.04, took
+
+
 @pytest.mark.parametrize("n_levels", [1, 2, 5, 6, 7, 11, 12, 13, 19])
 @pytest.mark.parametrize("entries,cache_pages", [(1, 64), (700, 6)])
 def test_as_many_levels_as_are_queued_at_a_time(bam, n_levels, entries, cache_pages):
