@@ -763,6 +763,7 @@ struct along_t {
     unsigned long long* next_chunk;             /* of the list, for the waves of the second launch */
     uint64_t* ahead;                            /* [n_segs * BAM_SEG_ROWS] a bit per entry (bfs_along) */
     unsigned long long* flags;                  /* [2] what the sweep tells the host, and the sweeps queued behind it */
+    bool stretches;
     /* the sweep is made if it is sure to be wanted, or if one of these words, NULL or an earlier sweep's, says so */
     uint32_t sure;
     const unsigned long long* gate[2];
@@ -818,7 +819,7 @@ template <bool AHEAD>
 struct bfs_along {
     uint32_t* label;
     uint32_t level;
-    static constexpr uint64_t most_blocks = 1ull << 31;
+    static constexpr bool joins = false;
     static constexpr bool again = AHEAD;       /* a page that is visited on one level is likely to be wanted on the next */
     struct lds_t { unsigned long long now[BAM_TRIP_SEGS * BAM_SEG_ROWS], next[AHEAD ? BAM_TRIP_SEGS * BAM_SEG_ROWS : 1]; };
 
@@ -934,9 +935,7 @@ struct bfs_along {
  * the first list and behind the last is nobody's neighbour, and need not be the number of a vertex. */
 struct cc_along {
     unsigned long long* comp;
-    /* chains grow with the edges that are joined at a time: 2^22 vertices, all cached, 2.6 ms with 16384 waves, 1.45 with 4096, 1.48
-     * with 2048, 1.6 with 1024 */
-    static constexpr uint64_t most_blocks = 4096 / BAM_TRIP_WAVES;
+    static constexpr bool joins = true;
     static constexpr bool again = false;       /* every page once */
     struct lds_t { unsigned long long starts[BAM_SEG_ROWS]; uint32_t vertex[BAM_SEG_EDGES]; };      /* where lists begin; whose, from the segment's first vertex on */
     __device__ __forceinline__ uint32_t prepare(const along_t& g, lds_t&, const uint64_t seg0, const uint32_t n_segs) const
@@ -1012,7 +1011,11 @@ __global__ __launch_bounds__(BAM_TRIP_WAVES * BAM_WAVE_SIZE) void k_along_reside
     bam::range_view<uint64_t> view;
     view.load(da->d_ranges);
     bool found = false, found_ahead = false;
-    for (uint64_t blk = blockIdx.x; blk * BAM_TRIP_WAVES * g.trip_segs < g.n_segs; blk += gridDim.x) {
+    /* trips by turns, or, of joins, a stretch of them each (along_sweep) */
+    const uint64_t n_blk = (g.n_segs + BAM_TRIP_WAVES * g.trip_segs - 1) / (BAM_TRIP_WAVES * g.trip_segs);
+    const uint64_t per = A::joins && g.stretches ? (n_blk + gridDim.x - 1) / gridDim.x : 1, step = A::joins && g.stretches ? 1 : gridDim.x;
+    const uint64_t blk_end = A::joins && g.stretches && (blockIdx.x + 1) * per < n_blk ? (blockIdx.x + 1) * per : n_blk;
+    for (uint64_t blk = blockIdx.x * per; blk < blk_end; blk += step) {
         const uint64_t trip = blk * BAM_TRIP_WAVES + w_in_block, seg0 = trip * g.trip_segs;
         const uint64_t p0 = seg0 >> g.seg_log;
         bool miss = false;
@@ -1419,13 +1422,24 @@ bool graph_plan::along_edges(bam_array_t* edges, hipStream_t st)
 }
 
 extern "C++" {
-/* one reading of the edge array, or of what the algorithm wants of it, with the words g names */
+/*
+ * One reading of the edge array, or of what the algorithm wants of it, with the words g names.
+ * Joins: chains grow with the entries that are joined at a time (2^22 vertices, all cached, 2.6 ms with 16384 waves), and where they meet.
+ * Where all edges are cached, and make four turns or more, each of the workgroups that are there at a time, three on a compute unit, has a
+ * stretch of the array: on a graph of neighbours side by side grow along the array, and waves that take its next pieces by turns hook them
+ * to each other as they grow.  By turns with two workgroups on a unit, and stretches, ms: grids of 512 x 8192, 4096 x 4096 and 8192 x 8192
+ * 2.8, 13.2, 49 and 0.64, 2.9, 7.1; paths of 2^22 and 2^24 1.6, 5.3 and 1.3, 5.1; uniform, 2^22 and 2^24 vertices 1.45, 5.0 and 1.22, 4.9;
+ * a power-law graph of 2^20 0.65 and 0.55.
+ * Where some are on the store, those that are not often lie together, and stretches would leave the most of them to few: a quarter of 2^22
+ * vertices' cached 5.6 by turns, 6.2 in stretches; a half 4.1 and 4.2 (4.4 and more by turns with three workgroups on a unit, hence the LDS).
+ */
 template <typename A>
-void along_sweep(bam_array_t* edges, const graph_plan* pl, const along_t& g, const A& algo, hipStream_t st)
+void along_sweep(bam_array_t* edges, const graph_plan* pl, along_t g, const A& algo, hipStream_t st)
 {
-    const uint64_t trips = (g.n_segs + g.trip_segs - 1) / g.trip_segs;
-    const uint32_t blocks = (uint32_t)std::min<uint64_t>(A::most_blocks, (trips + BAM_TRIP_WAVES - 1) / BAM_TRIP_WAVES);
-    hipLaunchKernelGGL(k_along_resident<A>, dim3(blocks), dim3(BAM_TRIP_WAVES * BAM_WAVE_SIZE), 0, st, edges->a->d_array_ptr, g, algo);
+    const uint64_t n_blk = (g.n_segs + BAM_TRIP_WAVES * g.trip_segs - 1) / (BAM_TRIP_WAVES * g.trip_segs);
+    g.stretches = A::joins && pl->all_cached && n_blk >= 4 * 768;
+    const uint32_t blocks = (uint32_t)std::min<uint64_t>(!A::joins ? 1ull << 31 : g.stretches ? 768 : 1024, n_blk);
+    hipLaunchKernelGGL(k_along_resident<A>, dim3(blocks), dim3(BAM_TRIP_WAVES * BAM_WAVE_SIZE), A::joins && !g.stretches ? 48u << 10 : 0, st, edges->a->d_array_ptr, g, algo);
     hipLaunchKernelGGL(k_along_missing<A>, dim3(pl->along_waves), dim3(BAM_WAVE_SIZE), 0, st, edges->a->d_array_ptr, g, algo, pl->along_chunk, pl->along_again_waves);
     hip_err_chk(hipGetLastError());
 }

@@ -109,6 +109,36 @@ def test_entries_that_are_in_no_list(bam, before, behind, filler, n_v, n_e, shar
         assert not r.c.aborted()
 
 
+# 4 x 768 workgroups' turns of four pages of 512 entries, one turn fewer, an entry and a segment more: by turns and in stretches
+@pytest.mark.parametrize("n_edges", [3071 * 2048, 3071 * 2048 + 1, 3071 * 2048 + 513, 3840 * 2048 - 1, 3840 * 2048 + 1])
+def test_labels_where_each_workgroup_has_a_stretch(bam, n_edges):
+    """paths of 1 to 5000 vertices one after the other, all edges cached"""
+    rng = np.random.default_rng(n_edges)
+    n_v = n_edges // 2 + 9000
+    first = np.zeros(n_v, dtype=bool)
+    first[np.cumsum(rng.integers(1, 5000, n_v // 500)) % n_v] = True
+    first[0] = True
+    linked = ~first[1:]                                        # v and v + 1
+    linked[np.cumsum(linked) * 2 > n_edges] = False
+    deg = np.zeros(n_v, dtype=np.int64)
+    deg[:-1] += linked
+    deg[1:] += linked
+    v = np.arange(n_v, dtype=np.int64)
+    nb = np.stack([v - 1, v + 1], axis=1).reshape(-1)[np.stack([np.concatenate([[False], linked]), np.concatenate([linked, [False]])], axis=1).reshape(-1)]
+    labels = np.maximum.accumulate(np.where(np.concatenate([[True], ~linked]), v, 0)).astype(np.uint64)
+    off = np.concatenate([[0], np.cumsum(deg)]).astype(np.uint64)
+    assert n_edges - 5000 < len(nb) <= n_edges
+    nb = np.concatenate([nb, np.zeros(n_edges - len(nb), dtype=np.int64)]).astype(np.uint64)
+    r, a = _rig(bam, nb, 4096, (n_edges + 511) // 512)
+    with r:
+        d_off = _dev(off)
+        a.set_graph(d_off)
+        for by_page in (False, True, False):
+            lb, _ = a.cc(d_off, by_page=by_page)
+            assert np.array_equal(_u64(lb), labels), by_page
+        assert not r.c.aborted()
+
+
 # vertices without lists before, between and behind those that have some: around the spans from which owners of entries are looked up
 @pytest.mark.parametrize("page,share", [(4096, 1), (4096, 4), (8192, 2), (65536, 2)])
 @pytest.mark.parametrize("run,scattered", [(4094, 1), (4095, 1), (4096, 1), (32766, 1), (32767, 1), (32768, 1), (70001, 1), (540000, 1), (40, 4099), (3, 70000)])
