@@ -1,6 +1,7 @@
 // Graph kernels of the C-ABI library: BFS (per vertex, over queues of vertices, by edge page), connected components,
 // PageRank and SSSP over CSR graphs whose neighbour ids (and weights) are read through the page cache.  Kernel shapes
 // follow the reference's benchmark kernels (cited per kernel); lane arithmetic is for 64-wide waves.
+#include "along_tables.h"
 #include "bam_capi_internal.h"
 
 #include <atomic>
@@ -1275,7 +1276,8 @@ struct graph_plan {
     bool cc_backwards() { return !all_cached && (cc_calls++ & 1u) != 0; }
     by_page_plan bp;
     bool bp_built = false;
-    along_t along{};                         /* n_segs = 0: the array or its pages do not qualify */
+    along_t along{};                         /* n_segs = 0: the array or its pages do not qualify, or there is no memory for the tables */
+    along_tables along_mem;
     uint32_t along_waves = 0, along_chunk = 0, along_again_waves = 0;
     BufferPtr bytes_a, bytes_b, floats_a, floats_b, words_a;      /* per-vertex buffers: flags, PageRank's delta and residual, SSSP's new costs */
     BufferPtr queue_a, queue_b, queue_bits, queue_totals;         /* bam_bfs_frontier: the two queues, the bit map that puts a queue in order and its counts per 4096 vertices */
@@ -1334,12 +1336,24 @@ struct graph_plan {
         hip_err_chk(hipGetLastError());
         hip_err_chk(hipStreamSynchronize(st));
     }
-    int by_page(bam_array_t* edges, hipStream_t st);
-    bool along_edges(bam_array_t* edges, hipStream_t st);
+    int by_page(bam_array_t* edges, hipStream_t st, bool can_do_without = false);
+    bool along_edges(bam_array_t* edges, hipStream_t st, bool levels);
     static void* sized(BufferPtr& b, uint64_t bytes) { if (!b) b = createBuffer(bytes ? bytes : 8, 0); return b.get(); }
 };
 
-int graph_plan::by_page(bam_array_t* edges, hipStream_t st)
+extern "C++" {
+/* device memory, or NULL where it is refused */
+BufferPtr spare_buffer(size_t bytes, int dev)
+{
+    void* p = nullptr;
+    hip_err_chk(hipSetDevice(dev));
+    if (hipMalloc(&p, bytes) != hipSuccess) { (void)hipGetLastError(); return nullptr; }
+    return BufferPtr(p, [](void* q) { (void)hipFree(q); });
+}
+}
+
+/* not 0, with nothing changed, where the array does not qualify, or, if the caller can do without, where memory is refused */
+int graph_plan::by_page(bam_array_t* edges, hipStream_t st, const bool can_do_without)
 {
     if (bp_built) return 0;
     by_page_plan& pl = bp;
@@ -1365,18 +1379,43 @@ int graph_plan::by_page(bam_array_t* edges, hipStream_t st)
     if (waves > trips) waves = trips;
     pl.ppw = (uint32_t)ppw;
     pl.blocks = (uint32_t)waves;                               /* one wave per workgroup */
-    const uint64_t segs_per_page = r.cache.page_size / (BAM_SEG_EDGES * 8);
-    const bool in_segs = segs_per_page && segs_per_page <= BAM_TRIP_SEGS && pl.n_pages && pl.n_pages <= 0xFFFFFFFFull && n_vertices <= 1ull << 32;
-    const uint64_t n_segs = in_segs ? (pl.n_edges + BAM_SEG_EDGES - 1) / BAM_SEG_EDGES : 0;
-    /* one allocation: the first vertices of the pages, of the segments where those are not the pages, the bits (only where some
-     * edges are on the store are there sweeps to spare), the list of missing pages */
-    const uint64_t seg_words = segs_per_page > 1 && in_segs ? n_segs + 1 : 0, bit_words = all_cached ? 0 : n_segs * BAM_SEG_ROWS;
-    pl.first = createBuffer((pl.n_pages + 1 + seg_words + bit_words) * sizeof(uint64_t) + (in_segs ? pl.n_pages * sizeof(uint32_t) : 0), dev);
+    if (can_do_without) {
+        if (!(pl.first = spare_buffer((pl.n_pages + 1) * sizeof(uint64_t), dev))) return ENOMEM;
+    } else
+        pl.first = createBuffer((pl.n_pages + 1) * sizeof(uint64_t), dev);
     hipLaunchKernelGGL(k_page_first_vertex, dim3(blocks_for(pl.n_pages + 1, 256)), dim3(256), 0, st, offsets, n_vertices, (uint64_t)pl.epp, pl.n_pages,
                        (uint64_t*)pl.first.get());
-    if (in_segs) {
-        uint64_t* const seg_first = (uint64_t*)pl.first.get() + (seg_words ? pl.n_pages + 1 : 0);
-        uint64_t* const bits = (uint64_t*)pl.first.get() + pl.n_pages + 1 + seg_words;
+    hip_err_chk(hipGetLastError());
+    bp_built = true;
+    return 0;
+}
+
+/*
+ * Whether BFS and components of an array are read along its pages, whichever entry point asks for them: the array has one
+ * range that begins on a page boundary, and pages the two launches take.  Per vertex, and over a queue of vertices, the same
+ * levels took 2.9 ms (2^20 vertices, all cached; 0.47 along the pages), 10.4 and 13.6 ms (2^18, a quarter cached; 1.8), 0.72
+ * and 1.27 (2^12; 0.12; without a plan made for the graph 0.80 and 1.44, 0.25).
+ */
+bool graph_plan::along_edges(bam_array_t* edges, hipStream_t st, const bool levels)
+{
+    if (edges->a->adt.n_ranges != 1) return false;
+    const range_d_t<uint64_t>& r = edges->a->h_ranges[0];
+    if (r.index_start != 0 || r.page_start_offset % r.cache.page_size || r.cache.n_pages < 2) return false;
+    if (by_page(edges, st, true)) return false;
+    by_page_plan& pl = bp;
+    const uint64_t segs_per_page = r.cache.page_size / (BAM_SEG_EDGES * 8);
+    if (!segs_per_page || segs_per_page > BAM_TRIP_SEGS || !pl.n_pages || pl.n_pages > 0xFFFFFFFFull || n_vertices > 1ull << 32 || pl.n_edges > r.count) return false;
+    /* the first vertices of the segments where those are not the pages, the list of missing pages; and the bits, only where some edges
+     * are on the store: there are no sweeps to spare otherwise */
+    const uint64_t n_segs = (pl.n_edges + BAM_SEG_EDGES - 1) / BAM_SEG_EDGES, seg_words = segs_per_page > 1 ? n_segs + 1 : 0;
+    int dev = 0;
+    hip_err_chk(hipGetDevice(&dev));
+    if (!along_mem.get(seg_words * sizeof(uint64_t) + pl.n_pages * sizeof(uint32_t), levels && !all_cached ? n_segs * BAM_SEG_ROWS * sizeof(uint64_t) : 0,
+                       [&](size_t bytes) { return spare_buffer(bytes, dev); })) return false;
+    along.ahead = (uint64_t*)along_mem.bits.get();
+    if (!along.n_segs) {
+        const uint64_t budget = r.cache.n_pages / 2;           /* pages all waves together may hold */
+        uint64_t* const seg_first = seg_words ? (uint64_t*)along_mem.tables.get() : (uint64_t*)pl.first.get();
         along.offsets = offsets; along.n_vertices = n_vertices; along.n_edges = pl.n_edges; along.n_pages = pl.n_pages; along.n_segs = n_segs;
         along.seg_log = (uint32_t)__builtin_ctzll(segs_per_page);
         along.trip_segs = (uint32_t)segs_per_page;
@@ -1385,8 +1424,7 @@ int graph_plan::by_page(bam_array_t* edges, hipStream_t st)
         along.first = seg_first;
         if (seg_words)
             hipLaunchKernelGGL(k_page_first_vertex, dim3(blocks_for(n_segs + 1, 256)), dim3(256), 0, st, offsets, n_vertices, (uint64_t)BAM_SEG_EDGES, n_segs, seg_first);
-        along.ahead = bit_words ? bits : nullptr;
-        along.missing = (uint32_t*)(bits + bit_words);
+        along.missing = (uint32_t*)((uint64_t*)along_mem.tables.get() + seg_words);
         along.n_missing = count + BAM_PLAN_MISSING(0);
         along.next_chunk = count + BAM_PLAN_CHUNK(0);
         along.flags = count + BAM_PLAN_FLAGS(0);
@@ -1400,25 +1438,9 @@ int graph_plan::by_page(bam_array_t* edges, hipStream_t st)
         /* 128 of them where they reuse their slots; 1024 pages on their way all the same (2^18 vertices, 3 700 cached, chunks of 4: 256 waves 1.59
          * ms, 128 1.93, all 469 1.58; the hand alone 1.76) */
         along_again_waves = std::min(along_waves, std::max(128u, 1024u / along_chunk));
+        hip_err_chk(hipGetLastError());
     }
-    hip_err_chk(hipGetLastError());
-    bp_built = true;
-    return 0;
-}
-
-/*
- * Whether BFS and components of an array are read along its pages, whichever entry point asks for them: the array has one
- * range that begins on a page boundary, and pages the two launches take.  Per vertex, and over a queue of vertices, the same
- * levels took 2.9 ms (2^20 vertices, all cached; 0.47 along the pages), 10.4 and 13.6 ms (2^18, a quarter cached; 1.8), 0.72
- * and 1.27 (2^12; 0.12; without a plan made for the graph 0.80 and 1.44, 0.25).
- */
-bool graph_plan::along_edges(bam_array_t* edges, hipStream_t st)
-{
-    if (!bp_built && edges->a->adt.n_ranges == 1) {
-        const range_d_t<uint64_t>& r = edges->a->h_ranges[0];
-        if (r.index_start == 0 && r.page_start_offset % r.cache.page_size == 0 && r.cache.n_pages >= 2) by_page(edges, st);
-    }
-    return along.n_segs != 0;
+    return true;
 }
 
 extern "C++" {
@@ -1517,10 +1539,11 @@ int bam_array_set_graph(bam_array_t* edges, const uint64_t* d_offsets, uint64_t 
         const range_d_t<uint64_t>& r = edges->a->h_ranges[0];
         if (r.index_start == 0 && r.page_start_offset % r.cache.page_size == 0 && r.cache.n_pages >= 2) p->by_page(edges, st);
     }
+    const bool along = p->along_edges(edges, st, true);
     /* the per-vertex buffers the sweeps use, so that no later call has to allocate */
     graph_plan::sized(p->bytes_a, n_vertices); graph_plan::sized(p->bytes_b, n_vertices);
     graph_plan::sized(p->floats_a, n_vertices * sizeof(float)); graph_plan::sized(p->floats_b, n_vertices * sizeof(float));
-    if (n_vertices <= 0xFFFFFFFFull) {
+    if (n_vertices <= 0xFFFFFFFFull && !along) {
         /* bam_bfs_frontier's queues and what puts them in order */
         const uint64_t n_words = (n_vertices + 63) / 64;
         graph_plan::sized(p->queue_a, n_vertices * sizeof(uint32_t)); graph_plan::sized(p->queue_b, n_vertices * sizeof(uint32_t));
@@ -1543,7 +1566,7 @@ int bam_bfs(bam_array_t* edges, const uint64_t* d_offsets, uint64_t n_vertices, 
     graph_plan* pl = plan_for(edges, d_offsets, n_vertices, 0, st, local);
     hip_err_chk(hipMemsetAsync(d_labels, 0xFF, n_vertices * sizeof(uint32_t), st));
     hip_err_chk(hipMemsetAsync(d_labels + src, 0, sizeof(uint32_t), st));
-    if (pl->along_edges(edges, st)) {
+    if (pl->along_edges(edges, st, true)) {
         const uint32_t levels = bfs_along_levels(edges, pl, d_labels, st);
         if (iterations) *iterations = levels;
         return 0;
@@ -1666,7 +1689,7 @@ int bam_bfs_frontier(bam_array_t* edges, const uint64_t* d_offsets, uint64_t n_v
     hipStream_t st = (hipStream_t)stream;
     std::unique_ptr<graph_plan> local;
     graph_plan* pl = plan_for(edges, d_offsets, n_vertices, 0, st, local);
-    if (pl->along_edges(edges, st)) {
+    if (pl->along_edges(edges, st, true)) {
         hip_err_chk(hipMemsetAsync(d_labels, 0xFF, n_vertices * sizeof(uint32_t), st));
         hip_err_chk(hipMemsetAsync(d_labels + src, 0, sizeof(uint32_t), st));
         const uint32_t levels = bfs_along_levels(edges, pl, d_labels, st);
@@ -1729,7 +1752,7 @@ int bam_cc(bam_array_t* edges, const uint64_t* d_offsets, uint64_t n_vertices, u
     graph_plan* pl = plan_for(edges, d_offsets, n_vertices, 0, st, local);
     const uint64_t group = coarse > 512 ? coarse : 512;
     unsigned long long* comp = (unsigned long long*)d_labels;
-    const bool along = pl->along_edges(edges, st);
+    const bool along = pl->along_edges(edges, st, false);
     hipLaunchKernelGGL(k_iota, dim3(blocks_for(n_vertices, 256)), dim3(256), 0, st, comp, n_vertices);
     if (along) cc_read_edges(edges, pl, comp, st);
     else
@@ -1755,7 +1778,7 @@ int bam_bfs_by_page(bam_array_t* edges, const uint64_t* d_offsets, uint64_t n_ve
     if (int rc = pl->by_page(edges, st)) return rc;
     hip_err_chk(hipMemsetAsync(d_labels, 0xFF, n_vertices * sizeof(uint32_t), st));
     hip_err_chk(hipMemsetAsync(d_labels + src, 0, sizeof(uint32_t), st));
-    if (pl->along.n_segs) {
+    if (pl->along_edges(edges, st, true)) {
         const uint32_t iter = bfs_along_levels(edges, pl, d_labels, st);
         if (iterations) *iterations = iter;
         return 0;
@@ -1783,6 +1806,7 @@ int bam_cc_by_page(bam_array_t* edges, const uint64_t* d_offsets, uint64_t n_ver
     std::unique_ptr<graph_plan> local;
     graph_plan* pl = plan_for(edges, d_offsets, n_vertices, 0, st, local);
     if (int rc = pl->by_page(edges, st)) return rc;
+    pl->along_edges(edges, st, false);
     unsigned long long* comp = (unsigned long long*)d_labels;
     hipLaunchKernelGGL(k_iota, dim3(blocks_for(n_vertices, 256)), dim3(256), 0, st, comp, n_vertices);
     uint32_t iter = 0;

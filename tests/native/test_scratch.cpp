@@ -5,6 +5,7 @@
 #include <cstring>
 #include <map>
 #include <thread>
+#include "along_tables.h"
 #include "scratch_sets.h"
 
 static int failures = 0;
@@ -93,6 +94,24 @@ int main()
             const int full = mem.allocs;
             CHECK("no set beyond the bound", sets.get(stream(BAM_SCRATCH_SETS + 1), 0, 64, 0, alloc) == nullptr && mem.allocs == full);
             CHECK("the others keep theirs", sets.get(stream(1), 0, 64, 0, alloc) == s && sets.get(stream(BAM_SCRATCH_SETS), 0, 64, 0, alloc) && mem.frees == 0);
+        }
+        CHECK("all is given back", mem.live.empty());
+    }
+    /* the tables of readings along the edge pages: refused, the call goes another way; the bits refused, it goes without them; nothing
+     * is asked for that nobody wants, and nothing twice */
+    {
+        Memory mem;
+        {
+            along_tables t;
+            auto alloc = [&](size_t b) { return mem(b); };
+            mem.refuse_from = 0;
+            CHECK("tables refused", !t.get(4096, 512, alloc) && !t.tables && !t.bits);
+            mem.refuse_from = 1;
+            CHECK("bits refused", t.get(4096, 512, alloc) && mem.holds(t.tables, 4096) && !t.bits);
+            CHECK("components want none", t.get(4096, 0, alloc) && !t.bits && mem.allocs == 1);
+            mem.refuse_from = -1;
+            CHECK("a later call gets them", t.get(4096, 512, alloc) && mem.holds(t.bits, 512) && mem.allocs == 2);
+            CHECK("once", t.get(4096, 512, alloc) && t.get(4096, 0, alloc) && mem.allocs == 2 && mem.frees == 0);
         }
         CHECK("all is given back", mem.live.empty());
     }
