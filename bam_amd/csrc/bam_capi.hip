@@ -1895,9 +1895,13 @@ extern "C++" {
 namespace {
 /*
  * Updates dealt out to bins of pages (k_update_deal), in slices of 2^20 requests; false, with nothing launched, where it does not
- * pay or there is no memory for the bins.  The three routes to an element add the same (the third asks for indices that differ).
+ * pay or the memory for the bins is not there.  The three routes to an element add the same (the third asks for indices that differ).
+ *   That memory takes 70 us to get, more than the bins save a call of few requests: one that does not find it goes element by element
+ * and leaves in bytes_later what there should be for the next one, which is allocated behind the launch, while that runs.  First
+ * call of an array, element by element and with the memory got first, us: AtomicAdd 2^18 97 and 135, 2^19 136 and 158, 3 x 2^18 184 and 187,
+ * 10^6 235 and 205; memref 2^17 71 and 124, 2^18 106 and 137, 2^19 161 and 158; += 2^17 93 and 125, 3 x 2^16 118 and 130, 2^18 159 and 130.
  */
-bool updates_by_bins(bam_array_t* a, int api, uint64_t n_reqs, const uint64_t* d_assignment, const uint64_t* d_values, uint64_t* d_old, hipStream_t st)
+bool updates_by_bins(bam_array_t* a, int api, uint64_t n_reqs, const uint64_t* d_assignment, const uint64_t* d_values, uint64_t* d_old, hipStream_t st, size_t& bytes_later)
 {
     if (n_reqs < (api == 0 ? 1ull << 18 : 1ull << 17) || a->a->adt.n_ranges != 1) return false;
     const range_d_t<uint64_t>& r = a->a->h_ranges[0];
@@ -1907,9 +1911,12 @@ bool updates_by_bins(bam_array_t* a, int api, uint64_t n_reqs, const uint64_t* d
     const uint32_t bins = (uint32_t)((pages + (1ull << bin_log) - 1) >> bin_log);
     if (pages > r.cache.n_pages || r.page_start_offset % sizeof(uint64_t) || 1ull << bin_log > BAM_BIN_MAX_PAGES || page_elems << bin_log >= 1ull << 31 || is_captured(st)) return false;
     const uint64_t slice = std::min<uint64_t>(n_reqs, 1ull << 20), deals = (slice + BAM_DEAL_REQS - 1) / BAM_DEAL_REQS;
+    const size_t bytes = slice * (sizeof(update_rec_t) + sizeof(uint32_t)) + deals * bins * sizeof(uint32_t);
     std::lock_guard<std::mutex> guard(a->scratch.mu);
-    scratch_set* set = scratch_for(a, st, slice * (sizeof(update_rec_t) + sizeof(uint32_t)) + deals * bins * sizeof(uint32_t), 0);
-    if (!set) return false;
+    const bool worth_it = n_reqs >= (api == 0 ? 3ull << 18 : api == 1 ? 1ull << 19 : 1ull << 18);
+    scratch_set* set = worth_it ? scratch_for(a, st, bytes, 0)
+                                : a->scratch.get(st, st == hipStreamPerThread ? scratch_thread_number() : 0, bytes, 0, [](size_t) { return BufferPtr(); });
+    if (!set) { bytes_later = worth_it ? 0 : bytes; return false; }
     array_d_t<uint64_t>* d = a->a->d_array_ptr;
     update_bins_t g{};
     g.bins = bins;
@@ -1946,7 +1953,8 @@ int bam_array_update(bam_array_t* a, int api, uint64_t n_reqs, const uint64_t* d
     const dim3 grid(blocks_for(n_reqs, block_size)), block(block_size);
     hipStream_t st = (hipStream_t)stream;
     array_d_t<uint64_t>* d = a->a->d_array_ptr;
-    if (updates_by_bins(a, api, n_reqs, d_assignment, d_values, d_old, st)) return 0;
+    size_t bytes_later = 0;
+    if (updates_by_bins(a, api, n_reqs, d_assignment, d_values, d_old, st, bytes_later)) return 0;
     /* Several per lane: from where the waves left still fill the device (scattered, resident, one against four per lane: 16.6 and
      * 19.7 us for 64000, 28.9 and 27.6 for 128000, 57.7 and 43.2 for 256000), and not where the array outgrows its cache, so
      * that many of the elements miss (10^6 of them, first call: 0.67 s and 0.76 s). */
@@ -1956,6 +1964,10 @@ int bam_array_update(bam_array_t* a, int api, uint64_t n_reqs, const uint64_t* d
     else if (api == 1) hipLaunchKernelGGL(k_array_update<1>, grid, block, 0, st, d, n_reqs, d_assignment, d_values, d_old);
     else hipLaunchKernelGGL(k_array_update<2>, grid, block, 0, st, d, n_reqs, d_assignment, d_values, d_old);
     hip_err_chk(hipGetLastError());
+    if (bytes_later) {
+        std::lock_guard<std::mutex> guard(a->scratch.mu);
+        (void)scratch_for(a, st, bytes_later, 0);
+    }
     BAM_API_END
 }
 

@@ -87,7 +87,7 @@ struct bam_array32 { array_t<uint32_t>* a; BufferPtr partials; };      /* partia
  */
 inline scratch_set* scratch_for(bam_array_t* a, hipStream_t st, size_t notes_bytes, size_t wanted_bytes, size_t tiles_bytes = 0)
 {
-    auto alloc = [&](size_t bytes) -> BufferPtr {
+    auto alloc = [&](size_t bytes, bool clear = true) -> BufferPtr {
         const relaxed_capture relaxed;
         int current = a->device;
         (void)hipGetDevice(&current);
@@ -97,13 +97,13 @@ inline scratch_set* scratch_for(bam_array_t* a, hipStream_t st, size_t notes_byt
         hipError_t e = hipMalloc(&p, bytes);
         /* never on a stream that is being captured: those calls take no scratch.  `st` may be the null stream of the caller's
          * device, which does not wait for this one's */
-        if (e == hipSuccess) e = elsewhere ? hipMemset(p, 0, bytes) : hipMemsetAsync(p, 0, bytes, st);
-        if (e == hipSuccess && elsewhere) e = hipStreamSynchronize(0);
+        if (e == hipSuccess && clear) e = elsewhere ? hipMemset(p, 0, bytes) : hipMemsetAsync(p, 0, bytes, st);
+        if (e == hipSuccess && clear && elsewhere) e = hipStreamSynchronize(0);
         if (elsewhere) (void)hipSetDevice(current);
         if (e != hipSuccess) { (void)hipGetLastError(); if (p) (void)hipFree(p); return nullptr; }
         return BufferPtr(p, [](void* q) { (void)hipFree(q); });
     };
-    return a->scratch.get(st, st == hipStreamPerThread ? scratch_thread_number() : 0, notes_bytes, wanted_bytes, alloc, tiles_bytes);
+    return a->scratch.get(st, st == hipStreamPerThread ? scratch_thread_number() : 0, notes_bytes, wanted_bytes, alloc, tiles_bytes, [&](size_t bytes) { return alloc(bytes, false); });
 }
 
 // ---------------------------------------------------------------------------

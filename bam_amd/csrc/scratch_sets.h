@@ -60,11 +60,17 @@ struct scratch_sets {
     std::vector<std::shared_ptr<void>> replaced;
     /*
      * The set of `stream` (and of `thread`, 0 where the handle names one stream everywhere) with at least these sizes, with `mu` held; NULL where the memory is refused, and then the caller
-     * takes a route that needs none.  alloc(bytes) gives memory that is zero to what is queued on `stream` from now on, or NULL.
+     * takes a route that needs none.  alloc(bytes) gives memory that is zero to what is queued on `stream` from now on, or NULL;
+     * alloc_notes(bytes) memory for the notes, which every call writes before it reads them, whatever another left there.
      * A set is entered once all of it is there, and a buffer changes place with a larger one that is there.
      */
     template <typename Alloc>
     scratch_set* get(void* stream, uint64_t thread, size_t notes_bytes, size_t wanted_bytes, Alloc&& alloc, size_t tiles_bytes = 0)
+    {
+        return get(stream, thread, notes_bytes, wanted_bytes, alloc, tiles_bytes, alloc);
+    }
+    template <typename Alloc, typename AllocNotes>
+    scratch_set* get(void* stream, uint64_t thread, size_t notes_bytes, size_t wanted_bytes, Alloc&& alloc, size_t tiles_bytes, AllocNotes&& alloc_notes)
     {
         scratch_set* s = nullptr;
         for (auto& x : sets) if (x->stream == stream && x->thread == thread) s = x.get();
@@ -77,7 +83,7 @@ struct scratch_sets {
             sets.push_back(std::move(made));
             s = sets.back().get();
         }
-        return grown(s->notes, s->notes_bytes, notes_bytes, alloc) && grown(s->wanted, s->wanted_bytes, wanted_bytes, alloc) &&
+        return grown(s->notes, s->notes_bytes, notes_bytes, alloc_notes) && grown(s->wanted, s->wanted_bytes, wanted_bytes, alloc) &&
                grown(s->tiles, s->tiles_bytes, tiles_bytes, alloc) ? s : nullptr;
     }
 

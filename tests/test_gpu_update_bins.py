@@ -13,7 +13,7 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("api,n", [(0, 1 << 18), (0, (1 << 18) + 4095), (1, 1 << 17), (2, (1 << 17) + 1), (0, (1 << 20) - 1), (2, 1 << 20), (1, (1 << 20) + 1), (0, (2 << 20) + 77)])
 @pytest.mark.parametrize("page,spare,warm", [(4096, 3, 1.0), (4096, 3, 0.0), (512, 1, 0.5), (8192, 40000, 1.0)])
-@pytest.mark.parametrize("kind", ["scattered", "in_order"])
+@pytest.mark.parametrize("kind", ["scattered", "in_order", "in_order_at_once"])
 def test_updates_without_repeats(bam, api, n, page, spare, warm, kind):
     per = page // 8
     n_elems = n + spare * 7 + 5
@@ -24,6 +24,9 @@ def test_updates_without_repeats(bam, api, n, page, spare, warm, kind):
         a = r.array(n_elems, page, pages)
         if warm:
             a.gather(max(1, int(pages * warm)), None, stride=per)
+        # the first call of an array goes element by element, unless it is a large one, and leaves the memory for the bins behind
+        if kind != "in_order_at_once":
+            a.update(0, _dev(np.zeros(max(n, 1 << 18), dtype=np.uint64)), _dev(np.zeros(max(n, 1 << 18), dtype=np.uint64)))
         idx = (rng.permutation(n_elems)[:n] if kind == "scattered" else np.arange(n) + 5).astype(np.uint64)
         vals = rng.integers(1, 1 << 63, n).astype(np.uint64)
         outside = rng.integers(0, n, 3)
@@ -34,9 +37,9 @@ def test_updates_without_repeats(bam, api, n, page, spare, warm, kind):
             a.stats()
             old = _u64(a.update(api, _dev(idx), _dev(vals), block_size=64))
             st = a.stats()
-            assert np.array_equal(old[inside], model[idx[inside].astype(np.int64)]) and (api or not old[~inside].any()), rep
+            assert np.array_equal(old[inside], model[idx[inside].astype(np.int64)]) and not old[~inside].any(), rep
             model[idx[inside].astype(np.int64)] += vals[inside]
-            assert api or st["access_cnt"] == inside.sum(), st
+            assert st["access_cnt"] == inside.sum(), st
             assert rep == 0 and warm < 1 or st["read_io_cnt"] == 0, st
         r.objs[0][2].flush()
         assert np.array_equal(r.backing(n_elems), model) and not r.c.aborted()
