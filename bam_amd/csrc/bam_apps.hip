@@ -501,10 +501,14 @@ __global__ void k_scan_ptr_pc(array_d_t<uint64_t>* da, unsigned long long* outpu
 /*
  * The scan of elements that are resident, in one reading.  A workgroup holds a tile of 16384 elements in registers, tells the
  * others its sum, adds up what lies before it and writes the running sums.  What lies before: the tiles' sums, back to the nearest
- * tile that has told the sum of everything up to its end; a wave looks at 64 of them at a time.
- *   Tiles are taken in the order the workgroups are started in, which is that of their numbers on each cluster of compute
- * units, so the tile somebody waits for is running or will be next where it is to run; a wait that lasts longer than a second
- * is given up all the same.  (The number of the next tile, drawn from one word, would cost the device 20 ns a tile.)
+ * tile that has told the sum of everything up to its end; a wave looks at 64 of them at a time (the decoupled look-back of Merrill
+ * and Garland, "Single-pass parallel prefix scan with decoupled look-back", 2016).
+ *   The workgroups of a launch are started in the order of their numbers on each cluster of compute units, so of one scan the first
+ * unfinished tile runs, or will once something ends that waits for no tile.  Two scans at a time, on different streams,
+ * could each fill a cluster that a tile of the other's is to run on, and wait for each other: a scan that begins while another is on
+ * its way draws the numbers of its tiles from one word instead (next_tile), so that all before a tile have begun, and of those that do
+ * not draw there is never more than one (host_word::alone).  Always drawing costs the device 20 ns a tile: 2^26 elements 239 -> 257 us,
+ * 2^22 28.4 -> 33.1.  Against another process's scan there is the end of all waits, after 20 ms or when somebody has given up.
  *   A word of a tile is 32 bits of a sum and the number of the call: it says by itself whether it has been written, and nothing
  * has to be cleared or ordered.
  *   Bound by HBM: 16 bytes per element.  2^26 elements: 314 -> 245 us a call (4.4 TB/s; a copy of as much on this device 4.9), 2^25
@@ -515,6 +519,7 @@ __global__ void k_scan_ptr_pc(array_d_t<uint64_t>* da, unsigned long long* outpu
  */
 #define BAM_TILE_WAVES 16u
 #define BAM_TILE_ELEMS (BAM_TILE_WAVES * BAM_WAVE_ELEMS)
+#define BAM_SCAN_WAIT_TICKS 2000000ull      /* of the 100 MHz clock */
 #define BAM_COUNTED_WORD 98u      /* of the scratch's words: the call whose accesses were counted */
 __device__ __forceinline__ void scan_gives_up(uint32_t* finished, const uint32_t call, volatile uint32_t* host_left)
 {
@@ -556,20 +561,32 @@ __device__ __forceinline__ uint64_t scan_look_back(const scan_tile_t* tiles, con
             if ((looks & 1023u) == 0) {
                 const uint64_t now = wall_clock64();
                 if (!t0) t0 = now;
-                else if (now - t0 > 100000000ull) { scan_gives_up(finished, call, host_left); return acc; }
+                else if (now - t0 > BAM_SCAN_WAIT_TICKS) { scan_gives_up(finished, call, host_left); return acc; }
+                if (__hip_atomic_load(finished + BAM_LEFT_WORD, __ATOMIC_RELAXED, BAM_AGENT) == call) return acc;      /* nobody wants the result */
             }
         }
     }
 }
 /* n_access: what the scan counts, as the kernels that can miss count it */
 __global__ __launch_bounds__(BAM_TILE_WAVES * BAM_WAVE_SIZE) __attribute__((amdgpu_waves_per_eu(8))) void k_scan_tiles(array_d_t<uint64_t>* da, uint64_t* result, const uint64_t n, scan_tile_t* tiles, uint32_t* finished,
-                                                                               const uint32_t call, volatile uint32_t* host_left, const uint64_t n_access)
+                                                                               const uint32_t call, volatile uint32_t* host_left, const uint64_t n_access, uint32_t* next_tile)
 {
     __shared__ uint64_t wave_sums[BAM_TILE_WAVES], before_s;
+
     const uint32_t lane = bam::lane(), w = bam::first(threadIdx.x / BAM_WAVE_SIZE);
     bam::range_view<uint64_t> view;
     view.load(da->d_ranges);
-    const uint64_t tile = blockIdx.x, first = tile * BAM_TILE_ELEMS + w * BAM_WAVE_ELEMS;
+    uint32_t tile_drawn = blockIdx.x;
+    if (next_tile) {
+        __shared__ uint32_t drawn;
+        if (threadIdx.x == 0) {
+            drawn = __hip_atomic_fetch_add(next_tile, 1u, __ATOMIC_RELAXED, BAM_AGENT);
+            if (drawn == gridDim.x - 1) bam::st_relaxed(next_tile, 0u);      /* the last one: the next scan starts over */
+        }
+        __syncthreads();
+        tile_drawn = bam::first(drawn);
+    }
+    const uint64_t tile = tile_drawn, first = tile * BAM_TILE_ELEMS + w * BAM_WAVE_ELEMS;
     /* once somebody has given up the result is not wanted: the tile is told as it is */
     const bool given_up = __hip_atomic_load(finished + BAM_LEFT_WORD, __ATOMIC_RELAXED, BAM_AGENT) == call;
     bam::u64x2_t x[BAM_WAVE_ROWS];
@@ -610,7 +627,7 @@ __global__ __launch_bounds__(BAM_TILE_WAVES * BAM_WAVE_SIZE) __attribute__((amdg
             }
         }
     }
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
+    if (tile == 0 && threadIdx.x == 0) {
         bam_stat_shard_t* const sh = view.r->shard();
         __hip_atomic_fetch_add(&sh->access_cnt, (unsigned long long)n_access, __ATOMIC_RELAXED, BAM_AGENT);
         __hip_atomic_fetch_add(&sh->hit_cnt, (unsigned long long)n_access, __ATOMIC_RELAXED, BAM_AGENT);
@@ -706,6 +723,7 @@ uint64_t paired_accesses(uint64_t n, uint64_t half, uint64_t page_elems)
 struct host_word {
     volatile uint32_t* at = nullptr;
     bool idle = true;
+    bool alone = false;             /* no other word was out when this one was taken */
     host_word()
     {
         pool& p = shared();
@@ -715,7 +733,9 @@ struct host_word {
             void* mem = nullptr;
             if (hipHostMalloc(&mem, 64 * sizeof(uint32_t), hipHostMallocMapped | hipHostMallocPortable) != hipSuccess) { (void)hipGetLastError(); return; }
             for (uint32_t k = 0; k < 64; k++) p.free.push_back((volatile uint32_t*)mem + k);
+            p.made += 64;
         }
+        alone = p.free.size() == p.made;
         at = p.free.back();
         p.free.pop_back();
         at[0] = 0;                  /* never the number of a call */
@@ -731,7 +751,7 @@ struct host_word {
     host_word& operator=(const host_word&) = delete;
 
 private:
-    struct pool { std::mutex mu; std::vector<volatile uint32_t*> free; };
+    struct pool { std::mutex mu; std::vector<volatile uint32_t*> free; size_t made = 0; };
     static pool& shared() { static pool* p = new pool(); return *p; }      /* never taken down: the runtime may be gone by then */
 };
 
@@ -789,8 +809,9 @@ bool scan_resident(bam_array_t* a, uint64_t n_elems, uint32_t block_size, uint64
         if (!set) return false;
         call = set->next_call();
         finished = set->finished();
+        left.idle = false;          /* (until the wait is over) */
         hipLaunchKernelGGL(k_scan_tiles, dim3((uint32_t)n_tiles), dim3(BAM_TILE_WAVES * BAM_WAVE_SIZE), 0, st, a->a->d_array_ptr, d_result, n_elems, (scan_tile_t*)set->tiles.get(), finished, call,
-                           left.at, n_access);
+                           left.at, n_access, left.alone ? nullptr : set->next_tile());
         hip_err_chk(hipGetLastError());
     }
     const hipError_t e = hipStreamSynchronize(st);

@@ -32,6 +32,8 @@ struct scratch_set {
     /* how many pages a first launch has listed for the second, and which of them comes next: zero between calls, a line each */
     unsigned long long* listed() { return (unsigned long long*)(finished() + 160); }
     unsigned long long* next_chunk() { return (unsigned long long*)(finished() + 192); }
+    /* the number of the next tile of a scan that draws them: zero between calls */
+    uint32_t* next_tile() { return finished() + 208; }
     /* how many updates a slice has left for its last launch, by turns: the one's word is cleared by the other */
     unsigned long long* left_over(uint32_t which) { return (unsigned long long*)(finished() + (which ? 240 : 224)); }
 };

@@ -50,6 +50,22 @@ int main()
         }
         CHECK("all is given back", mem.live.empty() && mem.frees == mem.allocs);
     }
+    /* what the tiles of a scan tell each other, refused: the scan gets nothing, the calls that need none their set, the next scan all of it */
+    {
+        Memory mem;
+        scratch_sets sets;
+        auto alloc = [&](size_t b) { return mem(b); };
+        mem.refuse_from = 1;
+        CHECK("tiles refused", sets.get(stream(1), 0, 0, 0, alloc, 640) == nullptr);
+        scratch_set* s = sets.get(stream(1), 0, 0, 0, alloc);
+        CHECK("a call without tiles has its set", s && !s->tiles && mem.allocs == 1);
+        mem.refuse_from = -1;
+        CHECK("then tiles", sets.get(stream(1), 0, 0, 0, alloc, 640) == s && mem.holds(s->tiles, 640));
+        /* notes come from an allocator of their own */
+        Memory raw;
+        CHECK("notes apart", sets.get(stream(1), 0, 4096, 512, alloc, 640, [&](size_t b) { return raw(b); }) == s && raw.holds(s->notes, 4096) && mem.holds(s->wanted, 512));
+        s->notes.reset();
+    }
     /* one handle that is another stream in each thread: two threads share nothing, each finds its own again */
     {
         Memory mem;

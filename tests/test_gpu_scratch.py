@@ -134,3 +134,39 @@ def test_many_streams_by_turns(bam):
         for k in range(70):
             assert hip.hipStreamDestroy(ctypes.c_void_p(made[k])) == 0
         assert not r.c.aborted()
+
+
+@pytest.mark.parametrize("same", [False, True])
+def test_scans_of_two_threads_side_by_side(bam, same):
+    """two streams, many large scans each of resident elements: tiles that wait for tiles, of one array and of two"""
+    import threading
+    import torch
+    sizes = [(1 << 24) + 5, (1 << 24) - 16384 if same else (1 << 23) + 16384]
+    with Rig(bam, sum(-(-n // 512) for n in sizes) * 4096, n_queues=16, depth=256) as r:
+        first = r.array(sizes[0], 4096, -(-sizes[0] // 512))
+        arrs = [first, first if same else r.array(sizes[1], 4096, -(-sizes[1] // 512), -(-sizes[0] // 512) * 4096)]
+        want = []
+        for a, n in zip(arrs, sizes):
+            x = a.gather(n, None, stride=1)
+            want.append(torch.cat([torch.zeros(1, dtype=torch.int64, device="cuda"), torch.cumsum(x, 0)]))
+        streams = [torch.cuda.Stream() for _ in range(2)]
+        outs = [torch.empty(w.numel() + 1, dtype=torch.int64, device="cuda") for w in want]
+        torch.cuda.synchronize()
+        bad, start = [[], []], threading.Barrier(2)
+
+        def work(k):
+            torch.cuda.set_device(0)
+            with torch.cuda.stream(streams[k]):
+                start.wait()
+                for rep in range(25):
+                    outs[k].zero_()
+                    rc = arrs[k].L.bam_scan(arrs[k].h, sizes[k], 256, ctypes.c_void_p(outs[k].data_ptr()), ctypes.c_void_p(streams[k].cuda_stream))
+                    if rc or not torch.equal(outs[k][:-1], want[k]):
+                        bad[k].append(rep)
+
+        threads = [threading.Thread(target=work, args=(k,)) for k in range(2)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+        assert bad == [[], []] and not r.c.aborted()
