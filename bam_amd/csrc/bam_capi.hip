@@ -1896,10 +1896,11 @@ namespace {
 /*
  * Updates dealt out to bins of pages (k_update_deal), in slices of 2^20 requests; false, with nothing launched, where it does not
  * pay or the memory for the bins is not there.  The three routes to an element add the same (the third asks for indices that differ).
- *   That memory takes 70 us to get, more than the bins save a call of few requests: one that does not find it goes element by element
- * and leaves in bytes_later what there should be for the next one, which is allocated behind the launch, while that runs.  First
- * call of an array, element by element and with the memory got first, us: AtomicAdd 2^18 97 and 135, 2^19 136 and 158, 3 x 2^18 184 and 187,
- * 10^6 235 and 205; memref 2^17 71 and 124, 2^18 106 and 137, 2^19 161 and 158; += 2^17 93 and 125, 3 x 2^16 118 and 130, 2^18 159 and 130.
+ *   That memory takes 60 us to get where as much was given back before, 110 where not, more than the bins save a call of few requests:
+ * one that does not find it goes element by element and leaves in bytes_later what there should be for the next one, which is
+ * allocated behind the launch, while that runs.  First call of a new array, element by element and with the memory got first, us:
+ * 10^6 AtomicAdds 255 and 315; and where as much was given back AtomicAdd 2^18 97 and 135, 2^19 136 and 158, 3 x 2^18 184 and 187, 10^6 235
+ * and 205, memref 2^17 71 and 124, 2^19 161 and 158, 10^6 294 and 220, += 2^17 93 and 125, 2^18 159 and 130, 3 x 2^17 230 and 150.
  */
 bool updates_by_bins(bam_array_t* a, int api, uint64_t n_reqs, const uint64_t* d_assignment, const uint64_t* d_values, uint64_t* d_old, hipStream_t st, size_t& bytes_later)
 {
@@ -1913,7 +1914,7 @@ bool updates_by_bins(bam_array_t* a, int api, uint64_t n_reqs, const uint64_t* d
     const uint64_t slice = std::min<uint64_t>(n_reqs, 1ull << 20), deals = (slice + BAM_DEAL_REQS - 1) / BAM_DEAL_REQS;
     const size_t bytes = slice * (sizeof(update_rec_t) + sizeof(uint32_t)) + deals * bins * sizeof(uint32_t);
     std::lock_guard<std::mutex> guard(a->scratch.mu);
-    const bool worth_it = n_reqs >= (api == 0 ? 3ull << 18 : api == 1 ? 1ull << 19 : 1ull << 18);
+    const bool worth_it = n_reqs >= (api == 0 ? 1ull << 21 : api == 1 ? 1ull << 20 : 3ull << 17);
     scratch_set* set = worth_it ? scratch_for(a, st, bytes, 0)
                                 : a->scratch.get(st, st == hipStreamPerThread ? scratch_thread_number() : 0, bytes, 0, [](size_t) { return BufferPtr(); });
     if (!set) { bytes_later = worth_it ? 0 : bytes; return false; }
