@@ -1278,7 +1278,7 @@ struct graph_plan {
     bool bp_built = false;
     along_t along{};                         /* n_segs = 0: the array or its pages do not qualify, or there is no memory for the tables */
     along_tables along_mem;
-    uint32_t along_waves = 0, along_chunk = 0, along_again_waves = 0;
+    uint64_t along_budget = 0;               /* pages that the waves of a launch may hold */
     BufferPtr bytes_a, bytes_b, floats_a, floats_b, words_a;      /* per-vertex buffers: flags, PageRank's delta and residual, SSSP's new costs */
     BufferPtr queue_a, queue_b, queue_bits, queue_totals;         /* bam_bfs_frontier: the two queues, the bit map that puts a queue in order and its counts per 4096 vertices */
 
@@ -1414,7 +1414,6 @@ bool graph_plan::along_edges(bam_array_t* edges, hipStream_t st, const bool leve
                        [&](size_t bytes) { return spare_buffer(bytes, dev); })) return false;
     along.ahead = (uint64_t*)along_mem.bits.get();
     if (!along.n_segs) {
-        const uint64_t budget = r.cache.n_pages / 2;           /* pages all waves together may hold */
         uint64_t* const seg_first = seg_words ? (uint64_t*)along_mem.tables.get() : (uint64_t*)pl.first.get();
         along.offsets = offsets; along.n_vertices = n_vertices; along.n_edges = pl.n_edges; along.n_pages = pl.n_pages; along.n_segs = n_segs;
         along.seg_log = (uint32_t)__builtin_ctzll(segs_per_page);
@@ -1429,15 +1428,7 @@ bool graph_plan::along_edges(bam_array_t* edges, hipStream_t st, const bool leve
         along.next_chunk = count + BAM_PLAN_CHUNK(0);
         along.flags = count + BAM_PLAN_FLAGS(0);
         along.sure = 1;
-        /* as many waves as leave each a batch worth sending (pages a wave, ms: 29 500 cached, BFS of 2^21 vertices 64 11.8, 32 11.4, 16
-         * 11.6, 8 11.9; 7 500, 2^19 16 3.18, 8 3.11, 4 3.27; 3 700, 2^18 16 1.89, 8 1.73, 4 1.79; 2 048, 2^16 16 0.88, 8 0.72, 4 0.62, 2 0.70) */
-        along_chunk = 32;
-        while (along_chunk > 4 && budget / along_chunk < 256) along_chunk /= 2;
-        along_waves = (uint32_t)std::min<uint64_t>(BAM_ALONG_WAVES, std::max<uint64_t>(1, budget / along_chunk));
-        if (along_chunk > budget) along_chunk = (uint32_t)budget;
-        /* 128 of them where they reuse their slots; 1024 pages on their way all the same (2^18 vertices, 3 700 cached, chunks of 4: 256 waves 1.59
-         * ms, 128 1.93, all 469 1.58; the hand alone 1.76) */
-        along_again_waves = std::min(along_waves, std::max(128u, 1024u / along_chunk));
+        along_budget = r.cache.n_pages / 2;
         hip_err_chk(hipGetLastError());
     }
     return true;
@@ -1462,7 +1453,23 @@ void along_sweep(bam_array_t* edges, const graph_plan* pl, along_t g, const A& a
     g.stretches = A::joins && pl->all_cached && n_blk >= 4 * 768;
     const uint32_t blocks = (uint32_t)std::min<uint64_t>(!A::joins ? 1ull << 31 : g.stretches ? 768 : 1024, n_blk);
     hipLaunchKernelGGL(k_along_resident<A>, dim3(blocks), dim3(BAM_TRIP_WAVES * BAM_WAVE_SIZE), A::joins && !g.stretches ? 48u << 10 : 0, st, edges->a->d_array_ptr, g, algo);
-    hipLaunchKernelGGL(k_along_missing<A>, dim3(pl->along_waves), dim3(BAM_WAVE_SIZE), 0, st, edges->a->d_array_ptr, g, algo, pl->along_chunk, pl->along_again_waves);
+    /* As many waves as leave each a batch worth sending (pages a wave, ms: 29 500 cached, BFS of 2^21 vertices 64 11.8, 32 11.4, 16
+     * 11.6, 8 11.9; 7 500, 2^19 16 3.18, 8 3.11, 4 3.27; 3 700, 2^18 16 1.89, 8 1.73, 4 1.79; 2 048, 2^16 16 0.88, 8 0.72, 4 0.62, 2 0.70).
+     * Under four pages a wave where the cache is small and what a wave fetched, visited one page after the other, is much: for joins, which
+     * visit every entry, and for levels in pages of more than 8 KiB.  In batches of four and as here, and by k_bfs_by_page and k_cc_by_page, us:
+     * 2^19 vertices, 8 entries each, pages of 64 KiB, 40 cached, BFS 23 200, 8 100, 10 400, components 23 900, 7 000, 9 000; of 16 KiB, 128 cached,
+     * 8 900, 6 000, 6 000 and 8 600, 2 500, 3 100; components in pages of 8 KiB, 256 cached, 4 000, 1 800, 2 000, of 4 KiB, 256, 5 200, 3 400, 3 700.
+     * Levels in small pages gain as much from it while their store alone is served, and lose it where another's is too (2^16, 8 KiB, 64
+     * cached: 2.6 -> 1.6 ms, and 2.8 -> 3.7). */
+    const uint64_t budget = pl->along_budget, enough = A::joins ? 128 : 64;
+    const uint32_t least = A::joins || g.seg_log > 2 ? 1 : g.seg_log == 2 ? 2 : 4;
+    uint32_t chunk = 32;
+    while ((chunk > 4 && budget / chunk < 256) || (chunk > least && budget / chunk < enough)) chunk /= 2;
+    if (chunk > budget) chunk = (uint32_t)budget;
+    const uint32_t waves = (uint32_t)std::min<uint64_t>(BAM_ALONG_WAVES, budget / chunk);
+    /* 128 of them where they reuse their slots; 1024 pages on their way all the same (2^18 vertices, 3 700 cached, chunks of 4: 256 waves 1.59
+     * ms, 128 1.93, all 469 1.58; the hand alone 1.76) */
+    hipLaunchKernelGGL(k_along_missing<A>, dim3(waves), dim3(BAM_WAVE_SIZE), 0, st, edges->a->d_array_ptr, g, algo, chunk, std::min(waves, std::max(128u, 1024u / chunk)));
     hip_err_chk(hipGetLastError());
 }
 }
