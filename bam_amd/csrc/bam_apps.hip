@@ -168,8 +168,10 @@ __global__ __launch_bounds__(BAM_WAVE_SIZE) void k_vectoradd_resident(const vadd
     bam::range_view<uint64_t> va, vb, vc;
     va.load(g.a->d_ranges);
     const uint64_t per_page = va.page_size / 8;
-    if (blockIdx.x == gridDim.x - 1) {          /* what is behind the last full page */
-        if (g.n_full * per_page < g.n_elems) vadd_elements(g, g.n_full * per_page, g.n_elems);
+    const uint32_t n_main = (uint32_t)((g.n_full + BAM_VADD_PAGES - 1) / BAM_VADD_PAGES);
+    if (blockIdx.x >= n_main) {                 /* what is behind the last full page, 64 elements to a wave: one wave took 35 us for a page less one */
+        const uint64_t first = g.n_full * per_page + (uint64_t)(blockIdx.x - n_main) * BAM_WAVE_SIZE;
+        vadd_elements(g, first, first + BAM_WAVE_SIZE < g.n_elems ? first + BAM_WAVE_SIZE : g.n_elems);
         return;
     }
     vb.load(g.b->d_ranges);
@@ -786,7 +788,8 @@ bool vectoradd_by_page(bam_array_t* a, bam_array_t* b, bam_array_t* c, uint64_t 
     if (!set) return false;
     vadd_t g{a->a->d_array_ptr, b->a->d_array_ptr, c->a->d_array_ptr, n_elems, n_full, pages > cache->n_pages ? 1u : 0u, (uint8_t*)set->notes.get() + n_full * sizeof(uint32_t),
              (uint32_t*)set->notes.get(), set->listed(), set->next_chunk(), set->finished(), set->next_call()};
-    hipLaunchKernelGGL(k_vectoradd_resident, dim3((uint32_t)((n_full + BAM_VADD_PAGES - 1) / BAM_VADD_PAGES) + 1), dim3(BAM_WAVE_SIZE), 0, st, g);
+    hipLaunchKernelGGL(k_vectoradd_resident, dim3((uint32_t)((n_full + BAM_VADD_PAGES - 1) / BAM_VADD_PAGES) + blocks_for(n_elems - n_full * (cache->page_size / sizeof(uint64_t)), BAM_WAVE_SIZE)),
+                       dim3(BAM_WAVE_SIZE), 0, st, g);
     hipLaunchKernelGGL(k_vectoradd_missing, dim3((uint32_t)std::min<uint64_t>(waves, (n_full + chunk - 1) / chunk)), dim3(BAM_WAVE_SIZE), 0, st, g, chunk);
     hipLaunchKernelGGL(k_vectoradd_rest, dim3((uint32_t)std::min<uint64_t>(n_full, std::min<uint64_t>(4096, cache->n_pages / 8))), dim3(BAM_WAVE_SIZE), 0, st, g);      /* a wave holds a page of each array */
     hip_err_chk(hipGetLastError());
