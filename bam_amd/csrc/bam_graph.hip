@@ -1820,9 +1820,10 @@ int bam_cc_by_page(bam_array_t* edges, const uint64_t* d_offsets, uint64_t n_ver
     bool changed = true;
     /*
      * With every edge cached a sweep of label propagation costs 40 to 60 us up to 2^22 entries, and a reading that joins as much
-     * as its longest chain of loads and exchanges that failed: sweeps / joins in us for 0.03, 0.13, 0.26, 0.5, 1, 2.1, 4.2, 8.4
-     * million entries of a uniform random graph 116 / 78, 140 / 111, 164 / 164, 183 / 250, 219 / 253, 308 / 376, 413 / 336,
-     * 735 / 430; of a power-law graph of 0.1, 0.5, 1.9, 7.7, 15 million 105 / 83, 142 / 186, 197 / 337, 437 / 434, 886 / 691.
+     * as its longest chain of loads and exchanges that failed, which differs from call to call by twice and more: sweeps / joins in us, medians,
+     * for 0.03, 0.13, 0.26, 0.5, 1, 2.1, 4.2, 8.4 million entries of a uniform random graph 116 / 78, 140 / 106, 157 / 315, 177 / 495,
+     * 220 / 450, 290 / 450, 456 / 510, 735 / 560; of a power-law graph of 0.1, 0.5, 1.9, 7.7, 15 million 105 / 83, 140 / 106, 187 / 171,
+     * 437 / 254, 886 / 354; of a grid of 64 x 4096 (1 million, six sweeps and joins) 460 / 660.
      * A graph that is long rather than wide would take a sweep per step: after six the edges are joined, from the labels as they
      * are, each of which names a smaller vertex of the component or the vertex itself.
      */

@@ -452,10 +452,10 @@ def main():
             refs += list(ex.map(lambda x: oracle.bfs_levels(off_h, nb_u, int(x)), srcs[1:]))
         log("[bench] bfs oracle: %d sources, %.1fs" % (len(refs), time.time() - t1))
         legs = {}
-        # bam_bfs_by_page on every source, bam_bfs and bam_bfs_frontier on the first few: this array (one range that starts on a page,
-        # 4 KiB pages) all three read along its pages
-        for name, by_page, n_src, coarse in (("by_page", True, len(srcs), 1), ("per_vertex_bam_ptr", False, min(4, len(srcs)), 64),
-                                             ("queue_of_vertices", False, min(4, len(srcs)), 0)):
+        # the three entry points, named as they are: bam_bfs_by_page on every source, bam_bfs and bam_bfs_frontier on the first few.  This
+        # array (one range that starts on a page, 4 KiB pages) all three read along its pages
+        for name, by_page, n_src, coarse in (("bam_bfs_by_page", True, len(srcs), 1), ("bam_bfs", False, min(4, len(srcs)), 64),
+                                             ("bam_bfs_frontier", False, min(4, len(srcs)), 0)):
             tot_ms, tot_edges, levels_ok, iters = 0.0, 0, True, []
             ag.stats()
             for k, src in enumerate(srcs[:n_src]):
@@ -476,11 +476,11 @@ def main():
                           "frac_of_ceiling": st["read_io_cnt"] / tot_ms * 1e3 / ceiling,
                           "hit_rate": st["hit_cnt"] / max(st["access_cnt"], 1)}
             log("[bench] bfs %s: %s" % (name, legs[name]))
-        bfs = {"scale": args.bfs_scale, "edges": n_e, "cache_pages": cache_pages, "GTEPS": legs["by_page"]["GTEPS"]}
+        bfs = {"scale": args.bfs_scale, "edges": n_e, "cache_pages": cache_pages, "GTEPS": legs["bam_bfs_by_page"]["GTEPS"]}
         bfs.update(legs)
         # CPU figure: the oracle's uncached in-RAM serial BFS on one core, same graph, first source
         bfs["cpu_serial_GTEPS"] = cpu_bfs_edges / cpu_bfs_s / 1e9
-        bfs["frac_of_ceiling"] = bfs["by_page"]["frac_of_ceiling"]
+        bfs["frac_of_ceiling"] = bfs["bam_bfs_by_page"]["frac_of_ceiling"]
         ag.close(); rg.close(); pcg.close(); ctrl.close(); target.close()
         if not args.skip_cpu:
             # the reference's path on the host cores (oracle/cpu_path.c: its bam_ptr, page cache and queues restated per thread,
@@ -546,15 +546,15 @@ def main():
         ms2 = elapsed_ms(a2, b2)
         st2 = ac.stats()
         assert torch.equal(ref, lb2) and not ctrl.aborted(), "CC labels of bam_cc differ from the fixed point"
-        by_page = {"ms": ms, "iterations": it, "GTEPS": n_e / ms / 1e6, "read_ios": st["read_io_cnt"], "MIOPS": st["read_io_cnt"] / ms / 1e3,
-                   "frac_of_ceiling": st["read_io_cnt"] / ms * 1e3 / ceiling}
-        per_vertex = {"coarse": 64, "ms": ms2, "iterations": it2, "GTEPS": n_e / ms2 / 1e6, "read_ios": st2["read_io_cnt"], "MIOPS": st2["read_io_cnt"] / ms2 / 1e3,
-                      "frac_of_ceiling": st2["read_io_cnt"] / ms2 * 1e3 / ceiling}
-        # the headline of the leg is the faster of the two; both are reported (the second starts on what the first left in the cache)
-        lead, lead_name = (by_page, "by_page") if ms <= ms2 else (per_vertex, "per_vertex_bam_ptr")
+        cold = {"entry": "bam_cc_by_page", "ms": ms, "iterations": it, "GTEPS": n_e / ms / 1e6, "read_ios": st["read_io_cnt"], "MIOPS": st["read_io_cnt"] / ms / 1e3,
+                "frac_of_ceiling": st["read_io_cnt"] / ms * 1e3 / ceiling}
+        warm = {"entry": "bam_cc", "coarse": 64, "ms": ms2, "iterations": it2, "GTEPS": n_e / ms2 / 1e6, "read_ios": st2["read_io_cnt"], "MIOPS": st2["read_io_cnt"] / ms2 / 1e3,
+                "frac_of_ceiling": st2["read_io_cnt"] / ms2 * 1e3 / ceiling}
+        # the same kernels both times, with nothing cached and on what the first call left in the cache; the headline of the leg is the faster
+        lead, lead_name = (cold, "cold") if ms <= ms2 else (warm, "warm")
         cc = {"log2_vertices": args.cc_logv, "edges": n_e, "cache_pages": cache_pages, "ms": lead["ms"], "iterations": lead["iterations"],
               "GTEPS": lead["GTEPS"], "read_ios": lead["read_ios"], "MIOPS": lead["MIOPS"], "frac_of_ceiling": lead["frac_of_ceiling"],
-              "components": int(torch.unique(lb).numel()), "kernel": lead_name, "by_page": by_page, "per_vertex_bam_ptr": per_vertex}
+              "components": int(torch.unique(lb).numel()), "lead": lead_name, "cold": cold, "warm": warm}
         del src, ref, new, nb, off, lb, lb2, store_words
         ac.close(); rc_.close(); pcc.close(); ctrl.close(); target.close()
         target = ctrl = None

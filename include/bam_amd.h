@@ -96,7 +96,10 @@ int bam_range_create(bam_range_t** out, uint64_t index_start, uint64_t count, ui
 void bam_range_destroy(bam_range_t* r);
 int bam_array_create(bam_array_t** out, uint64_t n_elems, uint64_t disk_start_offset, bam_range_t** ranges, uint32_t n_ranges, uint32_t device);
 void bam_array_destroy(bam_array_t* a);
-/* array_t::print_reset_stats (include/page_cache.h:1731-1752) as numbers; out[4]: read_io_cnt, access_cnt, miss_cnt, hit_cnt */
+/* array_t::print_reset_stats (include/page_cache.h:1731-1752) as numbers; out[4]: read_io_cnt, access_cnt, miss_cnt, hit_cnt.
+ * An access is an element, or as many neighbouring elements as a bam_ptr has one window for; reads, writes and updates, reductions, scans
+ * and vectoradd count the same whichever kernels they run.  BFS and components along the edge pages (bam_bfs_by_page) count a page
+ * and sweep each. */
 int bam_array_stats(bam_array_t* a, uint64_t* out, int reset);
 
 /* ---- array benchmark kernels (benchmarks/array/main.cu:43-65) ----
@@ -147,7 +150,10 @@ int bam_array_write(bam_array_t* a, uint64_t n_reqs, const uint64_t* d_assignmen
  * d_old[t] (may be NULL) = what the element held before.  api 0: array_d_t::AtomicAdd (include/page_cache.h:1647), api 1:
  * an atomic add on the address bam_ptr::memref returns (:467), api 2: ptr[i] += v on a non-const bam_ptr (:478; a plain read
  * and write, so the indices of one launch must be distinct).  The pages touched are dirty afterwards and reach the store
- * on eviction or bam_page_cache_flush. */
+ * on eviction or bam_page_cache_flush.  An index that no range holds changes nothing, and d_old is 0 there.
+ * From 2^18 requests on for api 0, 2^17 for 1 and 2, of an array of one range that fits its cache, the requests are dealt out to bins of
+ * pages and added there, whatever api says (atomically, so the same elements and old values; counters too): except in a call
+ * that finds no memory for the bins, which then is got for the next one (large calls get it first), and under capture. */
 int bam_array_update(bam_array_t* a, int api, uint64_t n_reqs, const uint64_t* d_assignment, const uint64_t* d_values, uint64_t* d_old,
                      uint32_t block_size, void* stream);
 /* The submission entry the device path builds for one read or write (nvm_cmd_header / nvm_cmd_data_ptr / nvm_cmd_rw_blks,
@@ -227,8 +233,11 @@ int bam_array_set_graph(bam_array_t* edges, const uint64_t* d_offsets, uint64_t 
 /* ---- BFS (benchmarks/bfs/main.cu:658-689 kernel_coalesce_coarse_ptr_pc, host loop :1557-1566, 1577-1736) ----
  * Level-synchronous BFS from src: d_offsets[V+1] in device memory, neighbour ids read through the array,
  * d_labels[V] receives the level of every vertex (0xFFFFFFFF = unreachable).  *iterations = levels swept.
- * Where the array has one range that begins on a page boundary, and pages of 4 to 64 KiB, the edges are read along their pages
- * (bam_bfs_by_page), which is quicker whatever the graph; the same for bam_bfs_frontier and bam_cc.  Otherwise:
+ * Where the array has one range that begins on a page boundary, and pages of 4 to 64 KiB, and there is memory for the tables, the edges
+ * are read along their pages (bam_bfs_by_page); the same for bam_bfs_frontier and bam_cc.  That was quicker on power-law and uniform
+ * graphs of 2^12 to 2^24 vertices with all to 1 % of the edges cached, and on grids and paths of 2^13 to 2^26 vertices with up to 16 000
+ * levels (a level looks at the labels of all vertices: 2^26 vertices, 8192 x 8192, 67 us a level, over queues 260); not where next to
+ * nothing is reached (two vertices of 2^26 with 2^13 entries: 0.2 ms, over queues 0.1).  Otherwise:
  * The vertices are handed out in groups of max(coarse, 512) to as many waves as the device holds.  A wave first
  * touches the pages that hold the lists of its group's active vertices (what is not resident comes in as one batch of
  * commands), then reads the lists of 64 vertices at a time through bam_ptr, 64 entries per step across list ends.
@@ -252,7 +261,7 @@ int bam_cc_shaped(bam_array_t* edges, const uint64_t* d_offsets, uint64_t n_vert
                   int shape, uint32_t coarse, uint32_t stride, uint32_t* iterations, void* stream);
 /* ---- BFS over queues of vertices (benchmarks/bfs/main.cu:409-451 kernel_frontier_coalesce_ptr_pc, queues :1489-1492,
  * host loop :1561-1563, 1702-1711) ----
- * Instead of sweeping all labels, every level walks the queue of the vertices found by the level before and fills the
+ * Arrays that are read along their pages (bam_bfs) are here too, with no queue.  On others, instead of sweeping all labels, every level walks the queue of the vertices found by the level before and fills the
  * next one: a vertex enters it when the exchange on its label finds it unreached, the lanes of a wave that found one
  * at the same step take their places with one atomic.  Otherwise the walk of bam_bfs (lists packed 64 entries per
  * step, long lists in pieces).  Same levels and the same *iterations as bam_bfs; no result depends on the order of a

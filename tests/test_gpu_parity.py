@@ -925,8 +925,9 @@ def test_cc_labels_uniform_by_edge_page(bam, n_v, n_p, cache_pages):
 
 @pytest.mark.parametrize("cache_pages,coarse", [(24, 1), (256, 4), (4096, 64), (4096, 200)])
 def test_hub_lists_are_cut_into_pieces(bam, cache_pages, coarse):
-    """two hubs with lists of 9000 and 4096 entries (18 and 8 pages) on top of a sparse random graph: the per-vertex
-    kernels walk such lists in pieces, a wave each; levels and labels must not notice.  The hubs sit in
+    """two hubs with lists of 9000 and 4096 entries (18 and 8 pages) on top of a sparse random graph: PageRank's per-vertex
+    kernel walks such lists in pieces, a wave each; levels and labels, which are read along the pages of this array (the walks in
+    pieces: test_gpu_other_layouts.py), cross the pages of a list on several waves.  The hubs sit in
     different components until an edge of the random part joins them."""
     n_v = 20000
     pu = np.empty(6000, dtype=np.uint64); pv = np.empty(6000, dtype=np.uint64)
@@ -958,9 +959,8 @@ def test_hub_lists_are_cut_into_pieces(bam, cache_pages, coarse):
 @pytest.mark.parametrize("empty_every", [0, 4, 2])
 def test_lists_that_all_cross_a_page_boundary(bam, empty_every):
     """every list has 600 entries (a page holds 512), so each one ends on another page than it starts on, and every
-    `empty_every`-th vertex has none: the read-ahead of a group asks for the last pages on the lanes that have no first
-    page to ask for, and for the rest in a second batch (none empty: all in the second batch; every second one empty:
-    all in the first).  Neighbours are the next 600 vertices, so the levels step through the graph."""
+    `empty_every`-th vertex has none.  (Where the lists are walked vertex by vertex, test_gpu_other_layouts.py, the read-ahead of a
+    group asks for the last pages on the lanes that have no first page to ask for, and for the rest in a second batch.)  Neighbours are the next 600 vertices, so the levels step through the graph."""
     n_v, d = 4096, 600
     deg = np.full(n_v, d, dtype=np.uint64)
     if empty_every:
@@ -1039,8 +1039,8 @@ def test_sssp_float_costs(bam, scale, cache_pages):
 @pytest.mark.parametrize("scale,cache_pages", [(10, 4096), (14, 24), (16, 8192), (17, 700)])
 @pytest.mark.parametrize("sort", ["1", "0"])
 def test_bfs_levels_rmat_by_queue_of_vertices(bam, scale, cache_pages, sort, monkeypatch):
-    """the kernel that walks a queue of the level's vertices: same levels, same launch count, whether the queue is
-    sorted between levels (the default) or walked in the order of discovery"""
+    """bam_bfs_frontier: same levels, same count of levels, whatever the environment says about the order of queues, of which there are
+    none where the array is read along its pages as here (queues in both orders: test_gpu_other_layouts.py)"""
     monkeypatch.setenv("BAM_FRONTIER_SORT", sort)
     off, nb = oracle.rmat_csr(SEED, scale)
     r, a = _graph_rig(bam, nb, cache_pages, n_queues=16, depth=256)
