@@ -216,11 +216,13 @@ __device__ __forceinline__ void walk_packed(const uint64_t es, const uint64_t ee
 static_assert(BAM_PIECE_BUNDLE * 16u == BAM_WAVE_SIZE && BAM_PIECE_EDGES * 8u == 16u * 4096u, "a bundle's pages are shared out one per lane");
 struct heavy_piece_t { uint64_t v, first, last; };      /* entries [first, last) of the list of vertex v */
 
-__global__ void k_heavy_pieces(const uint64_t* vertexList, const uint64_t vertex_count, heavy_piece_t* pieces, unsigned long long* count)
+/* *lists_end: where the last list ends, for the host */
+__global__ void k_heavy_pieces(const uint64_t* vertexList, const uint64_t vertex_count, heavy_piece_t* pieces, unsigned long long* count, unsigned long long* lists_end)
 {
     const uint64_t v = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (v >= vertex_count) return;
     const uint64_t start = vertexList[v], end = vertexList[v + 1];
+    if (v == vertex_count - 1) *lists_end = end;
     if (end - start < BAM_HEAVY_EDGES) return;
     const uint64_t n = (end - start + BAM_PIECE_EDGES - 1) / BAM_PIECE_EDGES;
     const unsigned long long at = atomicAdd(count, (unsigned long long)n);
@@ -1228,7 +1230,7 @@ struct by_page_plan { uint64_t n_edges = 0, n_pages = 0; uint32_t epp = 0, ppw =
 
 /* the end of a level: the device's `changed` word goes to the host through pinned memory, and it and the counter the next
  * sweep takes its work from start the next level at zero.  One small launch instead of two copies and a fill. */
-/* words of a plan: [0] pieces, [1] next piece of work, [2] changed; then, written by many waves and on lines of their own, the words
+/* words of a plan: [0] pieces, [1] next piece of work, [2] changed, [3] where the last list ends; then, written by many waves and on lines of their own, the words
  * of along_t for each of the sweeps that are queued before the host looks */
 #define BAM_PLAN_SWEEPS 6u
 #define BAM_PLAN_WORDS (16u + BAM_PLAN_SWEEPS * 48u)
@@ -1259,6 +1261,7 @@ __global__ void k_sweeps_end(unsigned long long* words, volatile uint64_t* host_
 struct graph_plan {
     const uint64_t* offsets = nullptr;
     uint64_t n_vertices = 0, n_edges = 0;
+    uint64_t lists_end = 0;                  /* offsets[n_vertices] */
     BufferPtr buf, words, host_words;
     heavy_piece_t* pieces = nullptr;
     unsigned long long* count = nullptr;     /* [0] number of pieces, [1] next piece of work of the sweep */
@@ -1306,12 +1309,13 @@ struct graph_plan {
         if (cache_pages && resident > cache_pages / BAM_WAVE_SIZE) resident = cache_pages / BAM_WAVE_SIZE;
         if (resident < 2) resident = 2;
         hip_err_chk(hipMemsetAsync(words.get(), 0, BAM_PLAN_WORDS * sizeof(unsigned long long), st));
-        hipLaunchKernelGGL(k_heavy_pieces, dim3(blocks_for(n_vertices, 256)), dim3(256), 0, st, d_offsets, n_vertices, pieces, count);
+        hipLaunchKernelGGL(k_heavy_pieces, dim3(blocks_for(n_vertices, 256)), dim3(256), 0, st, d_offsets, n_vertices, pieces, count, count + 3);
         hip_err_chk(hipGetLastError());
-        unsigned long long n = 0;
-        hip_err_chk(hipMemcpyAsync(&n, count, sizeof(n), hipMemcpyDeviceToHost, st));
+        unsigned long long got[4] = {};
+        hip_err_chk(hipMemcpyAsync(got, count, sizeof(got), hipMemcpyDeviceToHost, st));
         hip_err_chk(hipStreamSynchronize(st));
-        n_pieces = n;
+        n_pieces = got[0];
+        lists_end = got[3];
         return 0;
     }
     /* workgroups of two waves for a sweep over `n_items` items in groups of `grp` */
@@ -1392,7 +1396,8 @@ int graph_plan::by_page(bam_array_t* edges, hipStream_t st, const bool can_do_wi
 
 /*
  * Whether BFS and components of an array are read along its pages, whichever entry point asks for them: the array has one
- * range that begins on a page boundary, and pages the two launches take.  Per vertex, and over a queue of vertices, the same
+ * range that begins on a page boundary, and pages the two launches take, and its number of elements covers the lists (it may be
+ * less than its range holds, and an entry behind it is found all the same by who looks it up in the range).  Per vertex, and over a queue of vertices, the same
  * levels took 2.9 ms (2^20 vertices, all cached; 0.47 along the pages), 10.4 and 13.6 ms (2^18, a quarter cached; 1.8), 0.72
  * and 1.27 (2^12; 0.12; without a plan made for the graph 0.80 and 1.44, 0.25).
  */
@@ -1404,7 +1409,7 @@ bool graph_plan::along_edges(bam_array_t* edges, hipStream_t st, const bool leve
     if (by_page(edges, st, true)) return false;
     by_page_plan& pl = bp;
     const uint64_t segs_per_page = r.cache.page_size / (BAM_SEG_EDGES * 8);
-    if (!segs_per_page || segs_per_page > BAM_TRIP_SEGS || !pl.n_pages || pl.n_pages > 0xFFFFFFFFull || n_vertices > 1ull << 32 || pl.n_edges > r.count) return false;
+    if (!segs_per_page || segs_per_page > BAM_TRIP_SEGS || !pl.n_pages || pl.n_pages > 0xFFFFFFFFull || n_vertices > 1ull << 32 || pl.n_edges > r.count || lists_end > pl.n_edges) return false;
     /* the first vertices of the segments where those are not the pages, the list of missing pages; and the bits, only where some edges
      * are on the store: there are no sweeps to spare otherwise */
     const uint64_t n_segs = (pl.n_edges + BAM_SEG_EDGES - 1) / BAM_SEG_EDGES, seg_words = segs_per_page > 1 ? n_segs + 1 : 0;

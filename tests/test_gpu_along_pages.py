@@ -109,6 +109,39 @@ def test_entries_that_are_in_no_list(bam, before, behind, filler, n_v, n_e, shar
         assert not r.c.aborted()
 
 
+@pytest.mark.parametrize("beyond", [1, 64, 700, 5000])
+@pytest.mark.parametrize("share", [1, 2])
+def test_lists_that_go_on_behind_the_number_of_elements(bam, beyond, share):
+    """an array created with fewer elements than its range holds: the entries behind them are looked up in the range"""
+    # a random graph, and behind it vertices with one entry each, of a vertex before them: nobody else's list names the last ones
+    n_v, n_more = 9001, 9000
+    off, nb = oracle.uniform_csr(SEED, n_v, 40009)
+    off = np.concatenate([off, off[-1] + np.arange(1, n_more + 1, dtype=np.uint64)])
+    nb = np.concatenate([nb, (n_v - 1 + np.random.default_rng(beyond).integers(0, np.arange(1, n_more + 1))).astype(np.uint64)])
+    src = n_v + n_more - 1
+    want, want_it = oracle.bfs_levels(off, nb, src)
+    labels, _ = oracle.cc_labels(off, nb)
+    assert want_it > 2 and labels[src] != src
+    pages = (len(nb) + 511) // 512
+    r = Rig(bam, pages * 4096, backing=True, n_queues=16, depth=256, stage_bytes=4096)
+    r.backing(len(nb))[:] = nb
+    with r:
+        cache = bam.PageCache(4096, pages // share + 1, 0, r.c)
+        held = bam.Range(0, len(nb), 0, pages, 0, 4096, cache, 0)
+        a = bam.Array(len(nb) - beyond, 0, [held], 0)
+        r.objs.append((a, held, cache))
+        d_off = _dev(off)
+        for kept in (False, True):
+            if kept:
+                a.set_graph(d_off)
+            for kw in KINDS[1:]:
+                lv, it = a.bfs(d_off, src, **kw)
+                assert np.array_equal(lv.cpu().numpy().view(np.uint32), want) and it == want_it, (kept, kw)
+            lb, _ = a.cc(d_off)
+            assert np.array_equal(_u64(lb), labels), kept
+        assert not r.c.aborted()
+
+
 # 4 x 768 workgroups' turns of four pages of 512 entries, one turn fewer, an entry and a segment more: by turns and in stretches
 @pytest.mark.parametrize("n_edges", [3071 * 2048, 3071 * 2048 + 1, 3071 * 2048 + 513, 3840 * 2048 - 1, 3840 * 2048 + 1])
 def test_labels_where_each_workgroup_has_a_stretch(bam, n_edges):
