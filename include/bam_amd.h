@@ -233,7 +233,8 @@ int bam_array_set_graph(bam_array_t* edges, const uint64_t* d_offsets, uint64_t 
 /* ---- BFS (benchmarks/bfs/main.cu:658-689 kernel_coalesce_coarse_ptr_pc, host loop :1557-1566, 1577-1736) ----
  * Level-synchronous BFS from src: d_offsets[V+1] in device memory, neighbour ids read through the array,
  * d_labels[V] receives the level of every vertex (0xFFFFFFFF = unreachable).  *iterations = levels swept.
- * Where the array has one range that begins on a page boundary, and pages of 4 to 64 KiB, and there is memory for the tables, the edges
+ * The array may be longer than the lists; what lies outside them is not looked at.
+ * Where it has one range that begins on a page boundary, and pages of 4 to 64 KiB, and there is memory for the tables, the edges
  * are read along their pages (bam_bfs_by_page); the same for bam_bfs_frontier and bam_cc.  That was quicker on power-law and uniform
  * graphs of 2^12 to 2^24 vertices with all to 1 % of the edges cached, and on grids and paths of 2^13 to 2^26 vertices with up to 16 000
  * levels (a level looks at the labels of all vertices: 2^26 vertices, 8192 x 8192, 67 us a level, over queues 260); not where next to
