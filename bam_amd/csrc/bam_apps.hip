@@ -950,7 +950,6 @@ unsigned long long* scan_scratch_of_current_device()
     return g_scratch_ptr[dev];
 }
 
-__global__ void k_store_zero64(unsigned long long* p) { *p = 0; }
 } // namespace
 
 extern "C" {

@@ -254,10 +254,13 @@ __device__ __forceinline__ void fetch_role(array_d_t<T>* const (&arrays)[N], con
     }
 }
 
+static __global__ void k_store_zero64(unsigned long long* p) { *p = 0; }
+
 /* fetch waves for a launch whose computing workgroups cover `elems_per_block` consecutive elements each: up to 512 waves
  * (32768 pages on their way; measured on 1 GiB read from the store: 32 waves 18 GB/s, 64 waves 29, 256 waves 34-42, 512 waves
  * 37-44, none 9-11), fewer where a quarter of the cache is less than that; BAM_FETCH_WAVES in the environment overrides the
- * number (0: none); `done` is cleared on the stream */
+ * number (0: none); `done` is cleared on the stream, by a kernel (the stream may be captured, and a memset's node is not to be relied
+ * on in replays), and got with the capture left alone; where it is refused nobody fetches ahead */
 inline fetch_plan make_fetch_plan(bam_array_t* a, int n_arrays, uint32_t block_size, uint64_t elems_per_block, hipStream_t st, unsigned long long* cleared = nullptr)
 {
     fetch_plan fp{nullptr, 0, 1u << 18, 0, elems_per_block};
@@ -275,9 +278,18 @@ inline fetch_plan make_fetch_plan(bam_array_t* a, int n_arrays, uint32_t block_s
     fp.blocks = (uint32_t)((waves + waves_per_block - 1) / waves_per_block);
     fp.lead_elems = budget_pages * (cache.page_size / sizeof(uint64_t));
     if (cleared) { fp.done = cleared; return fp; }      /* a word that an earlier launch on the stream clears */
-    if (!a->progress) a->progress = createBuffer(64, 0);
+    {
+        static std::mutex mu;
+        std::lock_guard<std::mutex> guard(mu);
+        if (!a->progress) {
+            const relaxed_capture relaxed;
+            void* p = nullptr;
+            if (hipMalloc(&p, 64) != hipSuccess) { (void)hipGetLastError(); fp.blocks = 0; return fp; }
+            a->progress = BufferPtr(p, [](void* q) { (void)hipFree(q); });
+        }
+    }
     fp.done = (unsigned long long*)a->progress.get();
-    hip_err_chk(hipMemsetAsync(fp.done, 0, sizeof(unsigned long long), st));
+    hipLaunchKernelGGL(k_store_zero64, dim3(1), dim3(1), 0, st, fp.done);
     return fp;
 }
 

@@ -170,3 +170,43 @@ def test_scans_of_two_threads_side_by_side(bam, same):
         for t in threads:
             t.join()
         assert bad == [[], []] and not r.c.aborted()
+
+
+@pytest.mark.parametrize("cold", [False, True])
+def test_captured_sums_of_arrays_read_by_pages(bam, cold):
+    """vectoradd and a reduction recorded into a graph after calls that take whole pages (or as the first calls at all), and replayed with other
+    elements and eager work between the replays"""
+    import torch
+    n, pages = 200_003, 391
+    with Rig(bam, 3 * pages * 4096, backing=True, n_queues=16, depth=256) as r:
+        pc = bam.PageCache(4096, 3 * pages + 30, 0, r.c)
+        rs = [bam.Range(0, n, k * pages, pages, 0, 4096, pc, 0) for k in range(3)]
+        a, b, c = arrs = [bam.Array(n, k * pages * 4096, [rs[k]], 0) for k in range(3)]
+        words = oracle.store(SEED, 0, 3 * pages * 512)
+        r.backing(len(words))[:] = words
+        x, y = words[:n].copy(), words[pages * 512:pages * 512 + n]
+        partials = torch.zeros(n // 128 + 1, dtype=torch.int64, device="cuda")
+        if not cold:
+            bam.vectoradd(a, b, c, n)
+            a.reduce(n, block_size=64)
+            torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            bam.vectoradd(a, b, c, n)
+            st = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+            assert a.L.bam_reduce(a.h, n, 64, ctypes.c_void_p(partials.data_ptr()), st) == 0
+        for rep in range(4):
+            graph.replay()
+            torch.cuda.synchronize()
+            assert np.array_equal(_u64(c.gather(n, None, stride=1)), x + y), rep
+            assert np.array_equal(_u64(partials), oracle.reduce_blocks(x, 64)), rep
+            idx = np.random.default_rng(rep).permutation(n)[:4096].astype(np.uint64)
+            a.update(0, _dev(idx), _dev(idx + np.uint64(7)))
+            x[idx.astype(np.int64)] += idx + np.uint64(7)
+            if rep == 1:
+                bam.vectoradd(a, b, c, n)
+                assert np.array_equal(_u64(a.reduce(n, block_size=256)), oracle.reduce_blocks(x, 256))
+        assert not r.c.aborted()
+        for z in arrs + rs:
+            z.close()
+        pc.close()
