@@ -186,3 +186,24 @@ def test_many_updates_element_by_element(bam, api, n, layout):
         x0[idx[inside].astype(np.int64)] += vals[inside]
         laid.pc.flush()
         assert np.array_equal(laid.get(), x0) and not r.c.aborted()
+
+
+@pytest.mark.parametrize("dist", [0, 1])
+def test_sums_over_two_controllers(bam, dist):
+    """arrays that are stored twice, and dealt out over two stores: element by element"""
+    n, pages = 40_003, 80
+    with Rig(bam, 3 * pages * 4096, backing=True, n_queues=8, depth=128) as r0, Rig(bam, 3 * pages * 4096, backing=True, n_queues=8, depth=128) as r1:
+        for r in (r0, r1):
+            r.backing(3 * pages * 512)[:] = oracle.store(SEED, 0, 3 * pages * 512)
+        pc = bam.PageCache(4096, 3 * pages + 30, 0, [r0.c, r1.c])
+        rs = [bam.Range(0, n, k * pages, pages, 0, 4096, pc, 0, dist) for k in range(3)]
+        arrs = [bam.Array(n, k * pages * 4096, [rs[k]], 0) for k in range(3)]
+        x, y = (_u64(z.gather(n, None, stride=1)).copy() for z in arrs[:2])
+        for rep in range(2):
+            bam.vectoradd(*arrs, n)
+            assert np.array_equal(_u64(arrs[2].gather(n, None, stride=1)), x + y), rep
+            pc.flush()
+        assert not r0.c.aborted() and not r1.c.aborted()
+        for z in arrs + rs:
+            z.close()
+        pc.close()

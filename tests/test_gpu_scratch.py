@@ -210,3 +210,33 @@ def test_captured_sums_of_arrays_read_by_pages(bam, cold):
         for z in arrs + rs:
             z.close()
         pc.close()
+
+
+def test_sums_beyond_the_sets_of_scratch(bam):
+    """vectoradd on seventy streams by turns: those that get no set of scratch go element by element"""
+    import torch
+    n, pages = 20_003, 40
+    hip = ctypes.CDLL("libamdhip64.so.7")
+    with Rig(bam, 3 * pages * 4096, backing=True, n_queues=16, depth=256) as r:
+        pc = bam.PageCache(4096, 3 * pages + 30, 0, r.c)
+        rs = [bam.Range(0, n, k * pages, pages, 0, 4096, pc, 0) for k in range(3)]
+        arrs = [bam.Array(n, k * pages * 4096, [rs[k]], 0) for k in range(3)]
+        words = oracle.store(SEED, 0, 3 * pages * 512)
+        r.backing(len(words))[:] = words
+        want = words[:n] + words[pages * 512:pages * 512 + n]
+        made = (ctypes.c_void_p * 70)()
+        for k in range(70):
+            assert hip.hipStreamCreateWithFlags(ctypes.byref(made, 8 * k), 1) == 0
+        for k in range(70):
+            arrs[2].update(0, _dev(np.arange(n, dtype=np.uint64)), _dev(np.ones(n, dtype=np.uint64)))      # not what the sums are
+            torch.cuda.synchronize()
+            assert arrs[0].L.bam_vectoradd(*[z.h for z in arrs], n, ctypes.c_void_p(made[k])) == 0
+            torch.cuda.synchronize()
+            if k in (0, 1, 63, 64, 69):
+                assert np.array_equal(_u64(arrs[2].gather(n, None, stride=1)), want), k
+        for k in range(70):
+            assert hip.hipStreamDestroy(ctypes.c_void_p(made[k])) == 0
+        assert not r.c.aborted()
+        for z in arrs + rs:
+            z.close()
+        pc.close()
