@@ -766,7 +766,7 @@ struct along_t {
     unsigned long long* next_chunk;             /* of the list, for the waves of the second launch */
     uint64_t* ahead;                            /* [n_segs * BAM_SEG_ROWS] a bit per entry (bfs_along) */
     unsigned long long* flags;                  /* [2] what the sweep tells the host, and the sweeps queued behind it */
-    bool stretches;
+    const unsigned long long* stretches;        /* not 0: a stretch of the array to each workgroup (k_cc_look); NULL: by turns */
     /* the sweep is made if it is sure to be wanted, or if one of these words, NULL or an earlier sweep's, says so */
     uint32_t sure;
     const unsigned long long* gate[2];
@@ -1001,6 +1001,23 @@ struct cc_along {
     }
 };
 
+/* Whether the graph's neighbours lie side by side, as far as its array is resident: 256 entries are looked at, and of most the two ends
+ * are less than a 64th of the vertices apart.  (A path, a grid of any but the widest rows; by chance, one entry in 32.) */
+__global__ __launch_bounds__(256) void k_cc_look(array_d_t<uint64_t>* da, const along_t g, unsigned long long* stretches)
+{
+    bam::range_view<uint64_t> view;
+    view.load(da->d_ranges);
+    const uint64_t begin = g.offsets[0], end = g.offsets[g.n_vertices];
+    if (begin >= end) { if (threadIdx.x == 0) *stretches = 0; return; }
+    const uint64_t e = begin + (end - begin) / 512 * (2 * threadIdx.x + 1), seg = e / BAM_SEG_EDGES;
+    uint64_t id = 0;
+    const bool there = bam_read_unpinned(view.pages + (view.pso >> view.page_size_log) + (seg >> g.seg_log), view.slot_addr(0), view.page_size_log, (e << 3) & (view.page_size - 1), id);
+    const uint64_t low = g.first[seg], high = g.first[seg + 1];
+    const bool near = there && (id < low ? low - id : id > high ? id - high : 0ull) < (g.n_vertices + 63) / 64;
+    const int n_there = __syncthreads_count(there), n_near = __syncthreads_count(near);
+    if (threadIdx.x == 0) *stretches = 2 * n_near > n_there;
+}
+
 /* a workgroup takes trips of 16 segments at most, a wave each, until there are none left */
 template <typename A>
 __global__ __launch_bounds__(BAM_TRIP_WAVES * BAM_WAVE_SIZE) void k_along_resident(array_d_t<uint64_t>* da, const along_t g, const A algo)
@@ -1016,8 +1033,9 @@ __global__ __launch_bounds__(BAM_TRIP_WAVES * BAM_WAVE_SIZE) void k_along_reside
     bool found = false, found_ahead = false;
     /* trips by turns, or, of joins, a stretch of them each (along_sweep) */
     const uint64_t n_blk = (g.n_segs + BAM_TRIP_WAVES * g.trip_segs - 1) / (BAM_TRIP_WAVES * g.trip_segs);
-    const uint64_t per = A::joins && g.stretches ? (n_blk + gridDim.x - 1) / gridDim.x : 1, step = A::joins && g.stretches ? 1 : gridDim.x;
-    const uint64_t blk_end = A::joins && g.stretches && (blockIdx.x + 1) * per < n_blk ? (blockIdx.x + 1) * per : n_blk;
+    const bool stretch = A::joins && g.stretches && *g.stretches;
+    const uint64_t per = stretch ? (n_blk + gridDim.x - 1) / gridDim.x : 1, step = stretch ? 1 : gridDim.x;
+    const uint64_t blk_end = stretch && (blockIdx.x + 1) * per < n_blk ? (blockIdx.x + 1) * per : n_blk;
     for (uint64_t blk = blockIdx.x * per; blk < blk_end; blk += step) {
         const uint64_t trip = blk * BAM_TRIP_WAVES + w_in_block, seg0 = trip * g.trip_segs;
         const uint64_t p0 = seg0 >> g.seg_log;
@@ -1230,9 +1248,10 @@ struct by_page_plan { uint64_t n_edges = 0, n_pages = 0; uint32_t epp = 0, ppw =
 
 /* the end of a level: the device's `changed` word goes to the host through pinned memory, and it and the counter the next
  * sweep takes its work from start the next level at zero.  One small launch instead of two copies and a fill. */
-/* words of a plan: [0] pieces, [1] next piece of work, [2] changed, [3] where the last list ends; then, written by many waves and on lines of their own, the words
+/* words of a plan: [0] pieces, [1] next piece of work, [2] changed, [3] where the last list ends, [4] along_t::stretches; then, written by many waves and on lines of their own, the words
  * of along_t for each of the sweeps that are queued before the host looks */
 #define BAM_PLAN_SWEEPS 6u
+#define BAM_PLAN_STRETCHES 4u
 #define BAM_PLAN_WORDS (16u + BAM_PLAN_SWEEPS * 48u)
 #define BAM_PLAN_FLAGS(k) (16u + (k) * 48u)          /* along_t::flags of sweep k, */
 #define BAM_PLAN_MISSING(k) (32u + (k) * 48u)        /* n_missing, */
@@ -1443,21 +1462,28 @@ extern "C++" {
 /*
  * One reading of the edge array, or of what the algorithm wants of it, with the words g names.
  * Joins: chains grow with the entries that are joined at a time (2^22 vertices, all cached, 2.6 ms with 16384 waves), and where they meet.
- * Where all edges are cached, and make four turns or more, each of the workgroups that are there at a time, three on a compute unit, has a
- * stretch of the array: on a graph of neighbours side by side grow along the array, and waves that take its next pieces by turns hook them
- * to each other as they grow.  By turns with two workgroups on a unit, and stretches, ms: grids of 512 x 8192, 4096 x 4096 and 8192 x 8192
- * 2.8, 13.2, 49 and 0.64, 2.9, 7.1; paths of 2^22 and 2^24 1.6, 5.3 and 1.3, 5.1; uniform, 2^22 and 2^24 vertices 1.45, 5.0 and 1.22, 4.9;
- * a power-law graph of 2^20 0.65 and 0.55.
- * Where some are on the store, those that are not often lie together, and stretches would leave the most of them to few: a quarter of 2^22
+ * On a graph of neighbours side by side they grow along the array, and waves that take its next pieces by turns hook them to each other
+ * as they grow: a stretch of the array to each workgroup.  On a graph without such an order stretches join trees all over it before there
+ * is a large one, which the pieces in order grow from the front.  So where all edges are cached and make six turns or more, a
+ * look at some of them (k_cc_look, 5 us) says which.  By turns and in stretches, two workgroups on a compute unit, us, medians: grids of 64 x 32768,
+ * 1024 x 2048, 512 x 8192, 2048 x 2048, 4096 x 4096 3580, 2000, 2780, 2790, 9200 and 830, 860, 630, 1140, 2580; paths of 2^22 and 2^24 1560,
+ * 5360 and 1340, 5130; uniform, 2^20, 2^21, 2^22 vertices 370, 610, 1200 and 570, 660, 1250; power-law, 2^18, 2^19, 2^20 310, 690, 620 and
+ * 260, 400, 670.  Three workgroups on a unit, in stretches, took 620, 650, 1400 on the uniform ones and 1600 and 2300 on square grids.
+ * Where some edges are on the store, those that are not often lie together, and stretches would leave the most of them to few: a quarter of 2^22
  * vertices' cached 5.6 by turns, 6.2 in stretches; a half 4.1 and 4.2 (4.4 and more by turns with three workgroups on a unit, hence the LDS).
  */
 template <typename A>
 void along_sweep(bam_array_t* edges, const graph_plan* pl, along_t g, const A& algo, hipStream_t st)
 {
     const uint64_t n_blk = (g.n_segs + BAM_TRIP_WAVES * g.trip_segs - 1) / (BAM_TRIP_WAVES * g.trip_segs);
-    g.stretches = A::joins && pl->all_cached && n_blk >= 4 * 768;
-    const uint32_t blocks = (uint32_t)std::min<uint64_t>(!A::joins ? 1ull << 31 : g.stretches ? 768 : 1024, n_blk);
-    hipLaunchKernelGGL(k_along_resident<A>, dim3(blocks), dim3(BAM_TRIP_WAVES * BAM_WAVE_SIZE), A::joins && !g.stretches ? 48u << 10 : 0, st, edges->a->d_array_ptr, g, algo);
+    const bool look = A::joins && pl->all_cached && n_blk >= 6 * 512;
+    if (look) {
+        unsigned long long* const stretches = pl->count + BAM_PLAN_STRETCHES;
+        hipLaunchKernelGGL(k_cc_look, dim3(1), dim3(256), 0, st, edges->a->d_array_ptr, g, stretches);
+        g.stretches = stretches;
+    }
+    const uint32_t blocks = (uint32_t)std::min<uint64_t>(!A::joins ? 1ull << 31 : look ? 512 : 1024, n_blk);
+    hipLaunchKernelGGL(k_along_resident<A>, dim3(blocks), dim3(BAM_TRIP_WAVES * BAM_WAVE_SIZE), A::joins ? 48u << 10 : 0, st, edges->a->d_array_ptr, g, algo);
     /* As many waves as leave each a batch worth sending (pages a wave, ms: 29 500 cached, BFS of 2^21 vertices 64 11.8, 32 11.4, 16
      * 11.6, 8 11.9; 7 500, 2^19 16 3.18, 8 3.11, 4 3.27; 3 700, 2^18 16 1.89, 8 1.73, 4 1.79; 2 048, 2^16 16 0.88, 8 0.72, 4 0.62, 2 0.70).
      * Under four pages a wave where the cache is small and what a wave fetched, visited one page after the other, is much: for joins, which

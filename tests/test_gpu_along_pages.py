@@ -142,8 +142,8 @@ def test_lists_that_go_on_behind_the_number_of_elements(bam, beyond, share):
         assert not r.c.aborted()
 
 
-# 4 x 768 workgroups' turns of four pages of 512 entries, one turn fewer, an entry and a segment more: by turns and in stretches
-@pytest.mark.parametrize("n_edges", [3071 * 2048, 3071 * 2048 + 1, 3071 * 2048 + 513, 3840 * 2048 - 1, 3840 * 2048 + 1])
+# 6 x 512 workgroups' turns of four pages of 512 entries, one turn fewer, an entry and a segment more: by turns and in stretches
+@pytest.mark.parametrize("n_edges", [3071 * 2048, 3071 * 2048 + 1, 3071 * 2048 + 513, 3584 * 2048 - 1, 3584 * 2048 + 1, 3840 * 2048 - 1, 3840 * 2048 + 1])
 def test_labels_where_each_workgroup_has_a_stretch(bam, n_edges):
     """paths of 1 to 5000 vertices one after the other, all edges cached"""
     rng = np.random.default_rng(n_edges)
@@ -169,6 +169,40 @@ def test_labels_where_each_workgroup_has_a_stretch(bam, n_edges):
         for by_page in (False, True, False):
             lb, _ = a.cc(d_off, by_page=by_page)
             assert np.array_equal(_u64(lb), labels), by_page
+        assert not r.c.aborted()
+
+
+# the number of vertices over how far a neighbour is at most: neighbours side by side just so, just not, and all over the graph
+@pytest.mark.parametrize("part", [70, 24, 16, 2])
+@pytest.mark.parametrize("before,behind", [(0, 0), (700, 5000)])
+def test_labels_of_long_arrays_by_how_far_the_neighbours_are(bam, part, before, behind):
+    """all edges cached and six turns of the workgroups or more, where a look at the neighbours says how the array is shared out; the
+    rest of the array, which is in no list, holds numbers of vertices too"""
+    from scipy.sparse import csr_matrix
+    from scipy.sparse.csgraph import connected_components
+    rng = np.random.default_rng(part)
+    n_v, d = 910003, 7
+    deg = np.where(rng.random(n_v) < 0.2, 0, rng.integers(6, 2 * d + 2, n_v))
+    off = np.concatenate([[0], np.cumsum(deg)]) + before
+    owner = np.repeat(np.arange(n_v), deg)
+    far = n_v // part
+    nb = rng.integers(0, n_v, len(owner) + before + behind)
+    # of the last vertices within the thousandth that they are in, so that there are several components
+    most = n_v // 4 * 3
+    nb[before:before + len(owner)] = np.where(owner < most, (owner + rng.integers(-far, far + 1, len(owner))) % most,
+                                              owner // 910 * 910 + rng.integers(0, 900, len(owner)) % np.minimum(910, n_v - owner // 910 * 910))
+    assert len(nb) > 3072 * 2048
+    graph = csr_matrix((np.ones(len(owner), dtype=np.int8), nb[before:before + len(owner)], off - before), shape=(n_v, n_v))
+    _, comp = connected_components(graph, directed=False)
+    least = np.full(comp.max() + 1, n_v, dtype=np.int64)
+    np.minimum.at(least, comp, np.arange(n_v))
+    want = least[comp].astype(np.uint64)
+    r, a = _rig(bam, nb.astype(np.uint64), 4096, (len(nb) + 511) // 512)
+    with r:
+        d_off = _dev(off.astype(np.uint64))
+        for by_page in (False, True, False):                       # nothing cached, all cached
+            lb, _ = a.cc(d_off, by_page=by_page)
+            assert np.array_equal(_u64(lb), want), by_page
         assert not r.c.aborted()
 
 
