@@ -76,8 +76,8 @@ def splitmix_block_sums(torch, seed, first_word, n_words):
 
 
 def usable_cores():
-    """the cores this process may use: what the scheduler allows it, capped by the share the environment names (a GPU box
-    exports the share of its one GPU as OMP_NUM_THREADS while os.cpu_count() shows the whole machine)"""
+    """the cores this process may use: what the scheduler allows it, capped by the share the environment names (a shared machine
+    may export the share of one GPU as OMP_NUM_THREADS while os.cpu_count() shows the whole machine)"""
     try:
         n = len(os.sched_getaffinity(0))
     except AttributeError:
@@ -115,7 +115,7 @@ def main():
                     help="hit-path leg and a plain 1 GiB copy only (short; what the counter passes of the profiler are run on)")
     args = ap.parse_args()
     if args.gpus != 1:
-        sys.exit("bench.py: this path runs on one GPU; --gpus %d is not supported (a GPU box here has one GPU, "
+        sys.exit("bench.py: this path runs on one GPU; --gpus %d is not supported (one process drives one GPU, "
                  "and the path has no collective step to scale)" % args.gpus)
 
     import numpy as np

@@ -1,6 +1,6 @@
 /*
  * CPU restatement of the reference's GPU-side storage-access path.
- * TEST INFRASTRUCTURE ONLY (checker and CPU baseline); the shipped library
+ * TEST INFRASTRUCTURE ONLY (what the tests compare with, and the CPU baseline); the shipped library
  * never links or calls this file.
  *
  * One software lane per POSIX thread, C11 atomics where the reference uses

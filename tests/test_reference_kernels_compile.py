@@ -1,6 +1,6 @@
 """The drop-in claim, by compilation: the text of the reference's benchmark kernels, read from the reference tree at test
 time (never committed; written to a temporary directory), is compiled for gfx950 in a translation unit that includes only
-this repository's include/ headers.  Skipped where the reference tree is absent (the GPU box).  No GPU is needed.
+this repository's include/ headers.  Skipped where the reference tree is absent.  No GPU is needed.
 
 What a maintainer of the reference has to touch is listed in EDITS and nowhere else: a kernel that does not appear there
 compiles letter for letter."""
