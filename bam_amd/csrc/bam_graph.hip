@@ -587,6 +587,24 @@ __device__ __forceinline__ void cc_join(unsigned long long* comp, const uint64_t
     const unsigned long long u = bam::ld_relaxed(comp + a), v = bam::ld_relaxed(comp + b);
     if (u != v) cc_join_trees(comp, u, v);
 }
+/*
+ * Every vertex to the root of its tree, where trees are long: label propagation that was broken off leaves chains of as many steps as
+ * the component is long, over how many it made.  A lane moves its own vertex alone, and always down; those with smaller numbers, which
+ * it comes to, began earlier or at the same time, so that chains halve together.  Joined as they were, a path of 2^21 vertices took
+ * 360 ms, since some waves walked down chains of vertices whose own waves had not begun; with this launch, 168 us there, 1.05.
+ */
+__global__ void k_cc_shorten(unsigned long long* comp, uint64_t vertex_count)
+{
+    const uint64_t v = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (v >= vertex_count) return;
+    unsigned long long up = bam::ld_relaxed(comp + v);
+    for (;;) {
+        const unsigned long long upper = bam::ld_relaxed(comp + up);
+        if (upper == up) return;
+        bam::st_relaxed(comp + v, upper);
+        up = upper;
+    }
+}
 /* n_missing, next_chunk: along_t's, of the reading before, which are zero between sweeps (NULL: it had none) */
 __global__ void k_cc_settle(unsigned long long* comp, uint64_t vertex_count, unsigned long long* n_missing, unsigned long long* next_chunk)
 {
@@ -1856,7 +1874,7 @@ int bam_cc_by_page(bam_array_t* edges, const uint64_t* d_offsets, uint64_t n_ver
      * 220 / 450, 290 / 450, 456 / 510, 735 / 560; of a power-law graph of 0.1, 0.5, 1.9, 7.7, 15 million 105 / 83, 140 / 106, 187 / 171,
      * 437 / 254, 886 / 354; of a grid of 64 x 4096 (1 million, six sweeps and joins) 460 / 660.
      * A graph that is long rather than wide would take a sweep per step: after six the edges are joined, from the labels as they
-     * are, each of which names a smaller vertex of the component or the vertex itself.
+     * are, each of which names a smaller vertex of the component or the vertex itself, and so the roots the labels lead to do.
      */
     if (pl->bp.n_pages && pl->all_cached && pl->bp.n_edges > (1ull << 17) && pl->bp.n_edges < (1ull << 22)) {
         bool* curr = (bool*)graph_plan::sized(pl->bytes_a, n_vertices);
@@ -1874,6 +1892,7 @@ int bam_cc_by_page(bam_array_t* edges, const uint64_t* d_offsets, uint64_t n_ver
         }
     }
     if (changed) {
+        if (iter) hipLaunchKernelGGL(k_cc_shorten, dim3(blocks_for(n_vertices, 256)), dim3(256), 0, st, comp, n_vertices);
         cc_read_edges(edges, pl, comp, st);
         hipLaunchKernelGGL(k_cc_settle, dim3(blocks_for(n_vertices, 256)), dim3(256), 0, st, comp, n_vertices, pl->along.n_missing, pl->along.next_chunk);
         hip_err_chk(hipGetLastError());

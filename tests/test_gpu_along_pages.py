@@ -271,6 +271,41 @@ def test_a_run_of_vertices_without_lists_is_not_gone_over(bam):
             assert min(took) < 0.04, took
 
 
+@pytest.mark.parametrize("n_v", [70001, 1048575, 1600003, (1 << 21) - 1])
+@pytest.mark.parametrize("cut", [2, 1000])
+def test_components_that_label_propagation_was_broken_off_in(bam, n_v, cut):
+    """two paths, the shorter below or in the middle of the longer: six sweeps leave chains of a sixth of their length.  Joined as they were
+    they took 0.36 s from 1.6 million vertices on, where some waves walked down what others had not come to (1.4 ms before)"""
+    import time
+    import torch
+    v = np.arange(n_v, dtype=np.int64)
+    low, high = (0, n_v // cut) if cut == 2 else (n_v // 3, n_v // 3 + n_v // cut)      # the shorter path: [low, high)
+    path = (v >= low) & (v < high)
+    order = np.concatenate([v[path], v[~path]])                # neighbours along it, but for the step from the one path to the other
+    linked = np.ones(n_v - 1, dtype=bool)
+    linked[path.sum() - 1] = False
+    src, dst = order[:-1][linked], order[1:][linked]
+    u, w = np.concatenate([src, dst]), np.concatenate([dst, src])
+    by = np.lexsort((w, u))
+    off = np.concatenate([[0], np.cumsum(np.bincount(u, minlength=n_v))]).astype(np.uint64)
+    nb = w[by].astype(np.uint64)
+    want = np.where(path, low, 0 if low else high).astype(np.uint64)
+    r, a = _rig(bam, nb, 4096, (len(nb) + 511) // 512)
+    with r:
+        d_off = _dev(off)
+        a.set_graph(d_off)
+        took = []
+        for _ in range(4):
+            torch.cuda.synchronize()
+            t = time.perf_counter()
+            lb, it = a.cc(d_off, by_page=True)
+            torch.cuda.synchronize()
+            took.append(time.perf_counter() - t)
+            assert np.array_equal(_u64(lb), want) and (it == 8 or len(nb) <= 1 << 17), it
+        assert min(took) < 0.04, took
+        assert not r.c.aborted()
+
+
 @pytest.mark.parametrize("n_levels", [1, 2, 5, 6, 7, 11, 12, 13, 19])
 @pytest.mark.parametrize("entries,cache_pages", [(1, 64), (700, 6)])
 def test_as_many_levels_as_are_queued_at_a_time(bam, n_levels, entries, cache_pages):
