@@ -1482,11 +1482,12 @@ extern "C++" {
  * Joins: chains grow with the entries that are joined at a time (2^22 vertices, all cached, 2.6 ms with 16384 waves), and where they meet.
  * On a graph of neighbours side by side they grow along the array, and waves that take its next pieces by turns hook them to each other
  * as they grow: a stretch of the array to each workgroup.  On a graph without such an order stretches join trees all over it before there
- * is a large one, which the pieces in order grow from the front.  So where all edges are cached and make six turns or more, a
+ * is a large one, which the pieces in order grow from the front.  So where all edges are cached and make two turns or more, a
  * look at some of them (k_cc_look, 5 us) says which.  By turns and in stretches, two workgroups on a compute unit, us, medians: grids of 64 x 32768,
  * 1024 x 2048, 512 x 8192, 2048 x 2048, 4096 x 4096 3580, 2000, 2780, 2790, 9200 and 830, 860, 630, 1140, 2580; paths of 2^22 and 2^24 1560,
  * 5360 and 1340, 5130; uniform, 2^20, 2^21, 2^22 vertices 370, 610, 1200 and 570, 660, 1250; power-law, 2^18, 2^19, 2^20 310, 690, 620 and
- * 260, 400, 670.  Three workgroups on a unit, in stretches, took 620, 650, 1400 on the uniform ones and 1600 and 2300 on square grids.
+ * 260, 400, 670; with two to five turns, grids of 64 x 8192, 1024 x 1024, 64 x 16384, 512 x 2048, 256 x 5095 1150, 1290, 1880, 1690, 2500 and
+ * 1100, 1400, 840, 600, 450, paths of 2^20 and 2^21 445, 840 and 410, 750.  Three workgroups on a unit, in stretches, took 620, 650, 1400 on the uniform ones and 1600 and 2300 on square grids.
  * Where some edges are on the store, those that are not often lie together, and stretches would leave the most of them to few: a quarter of 2^22
  * vertices' cached 5.6 by turns, 6.2 in stretches; a half 4.1 and 4.2 (4.4 and more by turns with three workgroups on a unit, hence the LDS).
  */
@@ -1494,7 +1495,7 @@ template <typename A>
 void along_sweep(bam_array_t* edges, const graph_plan* pl, along_t g, const A& algo, hipStream_t st)
 {
     const uint64_t n_blk = (g.n_segs + BAM_TRIP_WAVES * g.trip_segs - 1) / (BAM_TRIP_WAVES * g.trip_segs);
-    const bool look = A::joins && pl->all_cached && n_blk >= 6 * 512;
+    const bool look = A::joins && pl->all_cached && n_blk >= 2 * 512;
     if (look) {
         unsigned long long* const stretches = pl->count + BAM_PLAN_STRETCHES;
         hipLaunchKernelGGL(k_cc_look, dim3(1), dim3(256), 0, st, edges->a->d_array_ptr, g, stretches);

@@ -142,8 +142,8 @@ def test_lists_that_go_on_behind_the_number_of_elements(bam, beyond, share):
         assert not r.c.aborted()
 
 
-# 6 x 512 workgroups' turns of four pages of 512 entries, one turn fewer, an entry and a segment more: by turns and in stretches
-@pytest.mark.parametrize("n_edges", [3071 * 2048, 3071 * 2048 + 1, 3071 * 2048 + 513, 3584 * 2048 - 1, 3584 * 2048 + 1, 3840 * 2048 - 1, 3840 * 2048 + 1])
+# 2 x 512 workgroups' turns of four pages of 512 entries, one turn fewer, an entry and a segment more: by turns and in stretches
+@pytest.mark.parametrize("n_edges", [1023 * 2048, 1023 * 2048 + 1, 1023 * 2048 + 513, 1024 * 2048, 1024 * 2048 + 1, 1535 * 2048 + 511, 3071 * 2048, 3071 * 2048 + 1, 3071 * 2048 + 513, 3584 * 2048 - 1, 3584 * 2048 + 1, 3840 * 2048 - 1, 3840 * 2048 + 1])
 def test_labels_where_each_workgroup_has_a_stretch(bam, n_edges):
     """paths of 1 to 5000 vertices one after the other, all edges cached"""
     rng = np.random.default_rng(n_edges)
@@ -176,7 +176,7 @@ def test_labels_where_each_workgroup_has_a_stretch(bam, n_edges):
 @pytest.mark.parametrize("part", [70, 24, 16, 2])
 @pytest.mark.parametrize("before,behind", [(0, 0), (700, 5000)])
 def test_labels_of_long_arrays_by_how_far_the_neighbours_are(bam, part, before, behind):
-    """all edges cached and six turns of the workgroups or more, where a look at the neighbours says how the array is shared out; the
+    """all edges cached and two turns of the workgroups or more, where a look at the neighbours says how the array is shared out; the
     rest of the array, which is in no list, holds numbers of vertices too"""
     from scipy.sparse import csr_matrix
     from scipy.sparse.csgraph import connected_components
@@ -191,7 +191,7 @@ def test_labels_of_long_arrays_by_how_far_the_neighbours_are(bam, part, before, 
     most = n_v // 4 * 3
     nb[before:before + len(owner)] = np.where(owner < most, (owner + rng.integers(-far, far + 1, len(owner))) % most,
                                               owner // 910 * 910 + rng.integers(0, 900, len(owner)) % np.minimum(910, n_v - owner // 910 * 910))
-    assert len(nb) > 3072 * 2048
+    assert len(nb) > 1024 * 2048
     graph = csr_matrix((np.ones(len(owner), dtype=np.int8), nb[before:before + len(owner)], off - before), shape=(n_v, n_v))
     _, comp = connected_components(graph, directed=False)
     least = np.full(comp.max() + 1, n_v, dtype=np.int64)
