@@ -1995,6 +1995,8 @@ struct bam_ptr_tlb {
  * compute unit eleven waves went to eleven queues, of which the last to be served set the time (vectoradd and its flush, three stores
  * by turns, 116 668, 400 003, 10^6 and 3 x 10^6 elements: a queue per wave 432, 499, 642 and 1024 us, per four 215, 510, 685 and 1088, per
  * eight 220, 332, 645 and 1077, per sixteen 245, 295, 514 and 1092, per 64 250, 440, 622 and 996).
+ * Pages that do not fit a staging page are read out of the cache by whoever serves the queue, a matter of 50 us for 8 KiB, and want
+ * as many of those as there are: by compute unit (195 and 2931 pages 7 and 30 ms, in sixteens 10 and 56).
  */
 #define BAM_FLUSH_WAVES_PER_QUEUE 16u
 static __global__ void __flush(page_cache_d_t* pc)
@@ -2012,9 +2014,10 @@ static __global__ void __flush(page_cache_d_t* pc)
     const uint64_t index = get_backing_page_(pc->ranges_page_starts[range], addr, pc->n_ctrls, dist);
     uint64_t c = get_backing_ctrl_(addr, pc->n_ctrls, dist);
     const uint64_t c_end = c == ALL_CTRLS ? pc->n_ctrls : c + 1;
+    const uint32_t queue = pc->page_size <= pc->stage_bytes ? blockIdx.x / BAM_FLUSH_WAVES_PER_QUEUE : get_smid();
     for (c = c == ALL_CTRLS ? 0 : c; c < c_end; c++) {
         Controller* ctl = pc->d_ctrls[c];
-        write_data(pc, ctl->d_qps + ((blockIdx.x / BAM_FLUSH_WAVES_PER_QUEUE) % ctl->n_qps), index * pc->n_blocks_per_page, pc->n_blocks_per_page, page);
+        write_data(pc, ctl->d_qps + (queue % ctl->n_qps), index * pc->n_blocks_per_page, pc->n_blocks_per_page, page);
     }
     __hip_atomic_fetch_and(&dp->state, ~DIRTY, __ATOMIC_RELEASE, BAM_AGENT);
 }
