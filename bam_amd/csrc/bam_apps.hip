@@ -12,21 +12,21 @@ __global__ __launch_bounds__(64) void k_vectoradd_ptr_pc(array_d_t<uint64_t>* da
         fetch_role(arrays, n_elems, fp);
         return;
     }
-    const uint64_t bid = blockIdx.x - (fp.done ? fp.blocks : 0u);
-    const uint64_t tid = (uint64_t)blockDim.x * bid + threadIdx.x;
-    bam_ptr<uint64_t> Aptr(da);
-    bam_ptr<uint64_t> Bptr(db);
-    bam_ptr<uint64_t> Cptr(dc);
-    const bam_ptr<uint64_t>& A = Aptr;
-    const bam_ptr<uint64_t>& B = Bptr;
-    const uint64_t first = tid - threadIdx.x % BAM_WAVE_SIZE;
-    if (first < n_elems) {
+    /* once each, or by turns where the cache does not let as many waves hold pages at a time (bam_vectoradd) */
+    const uint32_t fetching = fp.done ? fp.blocks : 0u;
+    for (uint64_t first = (uint64_t)(blockIdx.x - fetching) * BAM_WAVE_SIZE; first < n_elems; first += (uint64_t)(gridDim.x - fetching) * BAM_WAVE_SIZE) {
+        const uint64_t tid = first + threadIdx.x;
+        bam_ptr<uint64_t> Aptr(da);
+        bam_ptr<uint64_t> Bptr(db);
+        bam_ptr<uint64_t> Cptr(dc);
+        const bam_ptr<uint64_t>& A = Aptr;
+        const bam_ptr<uint64_t>& B = Bptr;
         touch_ahead(da, first, n_elems, BAM_WAVE_SIZE, 0);
         touch_ahead(db, first, n_elems, BAM_WAVE_SIZE, 1);
         touch_ahead(dc, first, n_elems, BAM_WAVE_SIZE, 2);
+        if (tid < n_elems) Cptr[tid] = A[tid] + B[tid];
+        if (fp.done && threadIdx.x == 0) __hip_atomic_fetch_add(fp.done, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-    if (tid < n_elems) Cptr[tid] = A[tid] + B[tid];
-    if (fp.done && threadIdx.x == 0) __hip_atomic_fetch_add(fp.done, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 /*
@@ -796,6 +796,33 @@ bool vectoradd_by_page(bam_array_t* a, bam_array_t* b, bam_array_t* c, uint64_t 
     return true;
 }
 
+/*
+ * Waves for k_vectoradd_ptr_pc: one per 64 elements, unless those that the device runs at a time could hold the pages of all slots.  A
+ * wave keeps its page of A while it waits for a slot for B's, and both while it waits for C's, so that they then wait for each
+ * other until the bounded waits give up, and the sums are wrong (three times 65 pages of 8 KiB behind 97 slots: now and then).  As
+ * many as have a slot for each of their three pages do not.
+ */
+uint32_t vectoradd_waves(bam_array_t* a, bam_array_t* b, bam_array_t* c, uint64_t n_elems)
+{
+    uint64_t slots = ~0ull, held = 0;
+    for (bam_array_t* x : {a, b, c}) {
+        uint64_t pages = 0;
+        for (uint32_t k = 0; k < x->a->adt.n_ranges; k++) {
+            const range_d_t<uint64_t>& r = x->a->h_ranges[k];
+            slots = std::min<uint64_t>(slots, r.cache.n_pages);
+            pages += r.page_count;
+        }
+        if (x != c) held += pages;                /* who holds a page of C waits for nothing */
+    }
+    const uint32_t waves = blocks_for(n_elems, BAM_WAVE_SIZE);
+    int dev = 0, units = 0, per_unit = 0;
+    hip_err_chk(hipGetDevice(&dev));
+    hip_err_chk(hipDeviceGetAttribute(&units, hipDeviceAttributeMultiprocessorCount, dev));
+    hip_err_chk(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_unit, k_vectoradd_ptr_pc, BAM_WAVE_SIZE, 0));
+    held = std::min(held, 2 * std::min<uint64_t>(waves, (uint64_t)units * per_unit));
+    return held < slots ? waves : (uint32_t)std::min<uint64_t>(waves, std::max<uint64_t>(1, slots / 3));
+}
+
 /* the scan of resident elements; false if some were not, and then the result is not written in full, or if there is no
  * memory for the sums */
 bool scan_resident(bam_array_t* a, uint64_t n_elems, uint32_t block_size, uint64_t* d_result, hipStream_t st)
@@ -838,7 +865,7 @@ int bam_vectoradd(bam_array_t* a, bam_array_t* b, bam_array_t* c, uint64_t n_ele
     BAM_API_BEGIN
     if (vectoradd_by_page(a, b, c, n_elems, (hipStream_t)stream)) return 0;
     const fetch_plan fp = make_fetch_plan(a, 3, 64, 64, (hipStream_t)stream);
-    hipLaunchKernelGGL(k_vectoradd_ptr_pc, dim3(blocks_for(n_elems, 64) + fp.blocks), dim3(64), 0, (hipStream_t)stream,
+    hipLaunchKernelGGL(k_vectoradd_ptr_pc, dim3(vectoradd_waves(a, b, c, n_elems) + fp.blocks), dim3(64), 0, (hipStream_t)stream,
                        a->a->d_array_ptr, b->a->d_array_ptr, n_elems, c->a->d_array_ptr, fp);
     hip_err_chk(hipGetLastError());
     BAM_API_END

@@ -164,6 +164,29 @@ def test_sums_element_by_element(bam, page, offset, n):
         pc.close()
 
 
+# caches that waves which hold a page of A and of B can fill, and one page more or less than those of A and B
+@pytest.mark.parametrize("page,slots,n", [(8192, 97, 66001), (8192, 3, 5000), (8192, 130, 66001), (8192, 131, 66001), (512, 24, 20011), (512, 626, 20011), (512, 627, 20011), (512, 2000, 300007)])
+def test_sums_where_the_waves_could_fill_the_cache(bam, page, slots, n):
+    """element by element: a wave keeps its pages of A and B while it waits for one of C, so fewer waves run than the cache has slots"""
+    pages = (n * 8 + page - 1) // page
+    r = Rig(bam, 3 * pages * page, backing=True, n_queues=16, depth=256, stage_bytes=4096)
+    store = r.backing(3 * pages * page // 8)
+    store[:] = oracle.store(SEED, 0, len(store))
+    with r:
+        pc = bam.PageCache(page, slots, 0, r.c)
+        rs = [bam.Range(0, n, k * pages, pages, 0, page, pc, 0) for k in range(3)]
+        arrs = [bam.Array(n, k * pages * page, [rs[k]], 0) for k in range(3)]
+        part = [store[k * pages * page // 8:][:n] for k in range(3)]
+        for rep in range(3):
+            bam.vectoradd(*arrs, n)
+            pc.flush()
+            assert not r.c.aborted(), rep
+            assert np.array_equal(part[2], part[0] + part[1]), rep
+        for x in arrs + rs:
+            x.close()
+        pc.close()
+
+
 # as many requests as go to bins where the array fits its cache
 @pytest.mark.parametrize("api,n", [(0, 1 << 18), (1, 1 << 17), (2, (1 << 17) + 77)])
 @pytest.mark.parametrize("layout", ["two", "inside"])
