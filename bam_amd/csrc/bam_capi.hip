@@ -438,6 +438,9 @@ __attribute__((noinline)) __device__ uint64_t update_call(const array_d_t<uint64
  * add, some 50 of them the atomics on the elements), through memref 255 and 108, through ptr[i] += v 515 and 108; within a sixteenth of
  * it 166 and 97, sorted 92 and 89, in order 73 and 52, on 100 pages 693 and 96, on one 443 and 283, on 64 elements 1305 and 1228.
  * From where it pays on (scattered): 2^18 updates 65 and 60, 2^17 51 and 53 (memref 61 and 53, += 83 and 54).
+ * Requests in an order gain later than that, and lose before: AtomicAdd of 2^18 and 2^19 sorted 40 and 54, 54 and 65, in order 32 and 39,
+ * 41 and 44.  The line is drawn by the scattered ones, since what those gain is more, the more of them meet on a page: 2^18 over 4 MiB in pages
+ * of 4 KiB 103 and 56, of 8 KiB 143 and 56, 2^19 180 and 71, 258 and 72.
  */
 #define BAM_BINS 512u                           /* at most: a power of two of pages to a bin */
 #define BAM_BIN_MAX_PAGES 4096u
