@@ -654,7 +654,7 @@ __global__ void k_page_first_vertex(const uint64_t* offsets, uint64_t n_vertices
 }
 
 /*
- * For PageRank, and for BFS and components where a page is smaller than 4 KiB or larger than 64 (else k_along_resident):
+ * For PageRank, and for BFS and components where a page is larger than 64 KiB (else k_along_resident; components also as cc_read_edges has it):
  * one wave, `ppw` consecutive pages of the edge array per trip (lane l looks after page l of the trip), trips
  * handed out wave by wave along the array.  A page is wanted when one of its vertices is active; the wanted pages
  * of a trip are taken with one acquire, so their misses go to the store as one batch of commands, and the whole
@@ -770,6 +770,7 @@ __global__ __launch_bounds__(64) void k_cc_by_page(array_d_t<uint64_t>* da, cons
  */
 #define BAM_SEG_ROWS 8u
 #define BAM_SEG_EDGES (BAM_SEG_ROWS * BAM_WAVE_SIZE)
+#define BAM_ALL_ROWS ((1u << BAM_SEG_ROWS) - 1u)
 #define BAM_TRIP_SEGS 16u
 #define BAM_TRIP_WAVES 4u                       /* waves to a workgroup of the first launch: they share an add to the list */
 struct along_t {
@@ -777,7 +778,8 @@ struct along_t {
     uint64_t n_vertices;
     const uint64_t* first;                      /* [n_segs + 1] the vertex whose list holds the segment's first entry */
     uint64_t n_edges, n_pages, n_segs;          /* of the array, which may hold more than the lists */
-    uint32_t seg_log;                           /* log2 of the segments in a page, at most that of BAM_TRIP_SEGS */
+    uint32_t seg_log;                           /* log2 of the segments in a page, at most that of BAM_TRIP_SEGS (0 where a page is less than one) */
+    uint32_t part_log;                          /* log2 of the pages in a segment (0 where a page is one or more) */
     uint32_t trip_segs;                         /* segments a wave of the first launch looks after: whole pages, BAM_TRIP_SEGS at most */
     uint32_t* missing;                          /* [n_pages] the pages the first launch leaves to the second */
     unsigned long long* n_missing;              /* zero between sweeps, like the next one */
@@ -925,8 +927,16 @@ struct bfs_along {
         wave_lds_fence();
         return wanted;
     }
-    /* the entries of the segment, the k-th of those prepared: lane l holds entry 64 r + l in id[r] */
-    __device__ __forceinline__ void visit(const along_t& g, lds_t& s, const uint64_t seg, const uint32_t k, const uint64_t (&id)[BAM_SEG_ROWS], bool& found, bool& found_ahead) const
+    /* whether entries of rows [row, row + n) of those prepared are wanted */
+    __device__ __forceinline__ bool wants(const along_t&, lds_t& s, const uint64_t, const uint32_t row, const uint32_t n) const
+    {
+        unsigned long long any = 0;
+        for (uint32_t r = 0; r < n; r++) any |= s.now[row + r];
+        return any != 0;
+    }
+    /* the entries of the segment, the k-th of those prepared: lane l holds entry 64 r + l in id[r]; of the rows that `rows` has a bit for */
+    __device__ __forceinline__ void visit(const along_t& g, lds_t& s, const uint64_t seg, const uint32_t k, const uint64_t (&id)[BAM_SEG_ROWS], bool& found, bool& found_ahead,
+                                          const uint32_t rows = BAM_ALL_ROWS) const
     {
         const uint32_t lane = bam::lane();
         uint32_t have[BAM_SEG_ROWS];
@@ -935,6 +945,7 @@ struct bfs_along {
         for (uint32_t r = 0; r < BAM_SEG_ROWS; r++) {
             next[r] = AHEAD ? bam::first((uint64_t)s.next[k * BAM_SEG_ROWS + r]) : 0ull;
             all[r] = bam::first((uint64_t)s.now[k * BAM_SEG_ROWS + r]) | next[r];
+            if (!((rows >> r) & 1)) all[r] = 0;
             have[r] = 0;
             if ((all[r] >> lane) & 1) have[r] = bam::ld_relaxed(label + id[r]);
         }
@@ -948,7 +959,7 @@ struct bfs_along {
                 found |= !on; found_ahead |= on;
             }
         }
-        if (AHEAD && lane < BAM_SEG_ROWS) g.ahead[seg * BAM_SEG_ROWS + lane] = s.next[k * BAM_SEG_ROWS + lane];
+        if (AHEAD && lane < BAM_SEG_ROWS && ((rows >> lane) & 1)) g.ahead[seg * BAM_SEG_ROWS + lane] = s.next[k * BAM_SEG_ROWS + lane];
     }
 };
 
@@ -967,7 +978,13 @@ struct cc_along {
             if ((seg0 + k) * BAM_SEG_EDGES < end && (seg0 + k + 1) * BAM_SEG_EDGES > begin) wanted |= 1u << k;
         return wanted;
     }
-    __device__ __forceinline__ void visit(const along_t& g, lds_t& s, const uint64_t seg, const uint32_t, const uint64_t (&id)[BAM_SEG_ROWS], bool&, bool&) const
+    __device__ __forceinline__ bool wants(const along_t& g, lds_t&, const uint64_t seg0, const uint32_t row, const uint32_t n) const
+    {
+        const uint64_t e = seg0 * BAM_SEG_EDGES + row * BAM_WAVE_SIZE;
+        return e < g.offsets[g.n_vertices] && e + n * BAM_WAVE_SIZE > g.offsets[0];
+    }
+    __device__ __forceinline__ void visit(const along_t& g, lds_t& s, const uint64_t seg, const uint32_t, const uint64_t (&id)[BAM_SEG_ROWS], bool&, bool&,
+                                          const uint32_t rows = BAM_ALL_ROWS) const
     {
         const uint32_t lane = bam::lane();
         const uint64_t e0 = seg * BAM_SEG_EDGES, begin_all = g.offsets[0], end_all = g.offsets[g.n_vertices];
@@ -1008,7 +1025,7 @@ struct cc_along {
             if (m) begin = r * BAM_WAVE_SIZE + 63u - (uint32_t)__builtin_clzll(m);
             u[r] = w[r] = 0;
             const uint64_t e = e0 + r * BAM_WAVE_SIZE + lane;
-            if (e >= begin_all && e < e1) { u[r] = bam::ld_relaxed(comp + src); w[r] = bam::ld_relaxed(comp + id[r]); }
+            if (((rows >> r) & 1) && e >= begin_all && e < e1) { u[r] = bam::ld_relaxed(comp + src); w[r] = bam::ld_relaxed(comp + id[r]); }
         }
 #pragma unroll
         for (uint32_t r = 0; r < BAM_SEG_ROWS; r++) {
@@ -1029,15 +1046,40 @@ __global__ __launch_bounds__(256) void k_cc_look(array_d_t<uint64_t>* da, const 
     if (begin >= end) { if (threadIdx.x == 0) *stretches = 0; return; }
     const uint64_t e = begin + (end - begin) / 512 * (2 * threadIdx.x + 1), seg = e / BAM_SEG_EDGES;
     uint64_t id = 0;
-    const bool there = bam_read_unpinned(view.pages + (view.pso >> view.page_size_log) + (seg >> g.seg_log), view.slot_addr(0), view.page_size_log, (e << 3) & (view.page_size - 1), id);
+    const bool there = bam_read_unpinned(view.pages + (view.pso >> view.page_size_log) + ((e << 3) >> view.page_size_log), view.slot_addr(0), view.page_size_log, (e << 3) & (view.page_size - 1), id);
     const uint64_t low = g.first[seg], high = g.first[seg + 1];
     const bool near = there && (id < low ? low - id : id > high ? id - high : 0ull) < (g.n_vertices + 63) / 64;
     const int n_there = __syncthreads_count(there), n_near = __syncthreads_count(near);
     if (threadIdx.x == 0) *stretches = 2 * n_near > n_there;
 }
 
-/* a workgroup takes trips of 16 segments at most, a wave each, until there are none left */
+/*
+ * Pages of less than a segment: those of one segment that a wave holds (bit q of `held`: its q-th, in slot `slot` of lane lane0 + q; one at least)
+ * are visited together, since where the lists begin is worked out for all of it.  The rows of the others are loaded
+ * from a page that is held, and not looked at.  Pages of 512 bytes, 2^20 vertices of a power-law graph, all, a half and a quarter of the edges
+ * cached, by page and by vertex, ms: levels 1.63, 9.5, 11.8 and 4.6, 48.7, 61.0 -> 0.42, 3.9, 6.1; components of 2^21 vertices of a uniform one,
+ * a half and a quarter, 3.7, 4.6 and 20.2, 9.7 -> 2.4, 4.2.
+ */
 template <typename A>
+__device__ __forceinline__ void visit_parts(const A& algo, const along_t& g, typename A::lds_t& s, const bam::range_view<uint64_t>& view, const uint64_t seg, const uint32_t k,
+                                            const uint64_t held, const uint32_t lane0, const uint32_t slot, bool& found, bool& found_ahead)
+{
+    const uint32_t row_log = 3u - g.part_log, lane = bam::lane();          /* log2 of the rows in a page */
+    static_assert(BAM_SEG_ROWS == 8u, "eight rows to a segment");
+    uint64_t id[BAM_SEG_ROWS];
+    uint32_t rows = 0;
+#pragma unroll
+    for (uint32_t r = 0; r < BAM_SEG_ROWS; r++) {
+        const uint32_t q = r >> row_log;
+        const bool in = ((held >> q) & 1) != 0;
+        rows |= in ? 1u << r : 0u;
+        id[r] = bam::ld_payload((const uint64_t*)view.slot_addr(bam::bcast(slot, lane0 + (in ? q : bam::first_lane(held)))) + (r & ((1u << row_log) - 1u)) * BAM_WAVE_SIZE + lane);
+    }
+    algo.visit(g, s, seg, k, id, found, found_ahead, rows);
+}
+
+/* a workgroup takes trips of 16 segments at most, a wave each, until there are none left */
+template <typename A, bool PARTS>
 __global__ __launch_bounds__(BAM_TRIP_WAVES * BAM_WAVE_SIZE) void k_along_resident(array_d_t<uint64_t>* da, const along_t g, const A algo)
 {
     if (!g.sure && !(g.gate[0] && *g.gate[0]) && !(g.gate[1] && *g.gate[1])) return;
@@ -1056,14 +1098,18 @@ __global__ __launch_bounds__(BAM_TRIP_WAVES * BAM_WAVE_SIZE) void k_along_reside
     const uint64_t blk_end = stretch && (blockIdx.x + 1) * per < n_blk ? (blockIdx.x + 1) * per : n_blk;
     for (uint64_t blk = blockIdx.x * per; blk < blk_end; blk += step) {
         const uint64_t trip = blk * BAM_TRIP_WAVES + w_in_block, seg0 = trip * g.trip_segs;
-        const uint64_t p0 = seg0 >> g.seg_log;
+        const uint64_t p0 = PARTS ? seg0 << g.part_log : seg0 >> g.seg_log;
         bool miss = false;
         if (seg0 < g.n_segs) {
             const uint32_t n_segs = (uint32_t)(g.n_segs - seg0 < g.trip_segs ? g.n_segs - seg0 : g.trip_segs);
             const uint32_t wanted = algo.prepare(g, s, seg0, n_segs);
             /* lane j: the trip's j-th page */
-            const uint32_t per = 1u << g.seg_log;
-            const bool want = lane < (g.trip_segs >> g.seg_log) && ((wanted >> (lane << g.seg_log)) & ((1u << per) - 1u)) != 0;
+            const uint32_t per = 1u << (PARTS ? g.part_log : g.seg_log);
+            bool want;
+            if constexpr (PARTS) {
+                const uint32_t rows = BAM_SEG_ROWS >> g.part_log;
+                want = lane < (n_segs << g.part_log) && p0 + lane < g.n_pages && algo.wants(g, s, seg0, lane * rows, rows);
+            } else want = lane < (g.trip_segs >> g.seg_log) && ((wanted >> (lane << g.seg_log)) & ((1u << per) - 1u)) != 0;
             data_page_t* const dp = view.pages + (view.pso >> view.page_size_log) + p0 + (want ? lane : 0);
             uint64_t sv = 0;
             uint32_t slot = 0;
@@ -1075,7 +1121,13 @@ __global__ __launch_bounds__(BAM_TRIP_WAVES * BAM_WAVE_SIZE) void k_along_reside
             miss = want && !have;
             view.n_access += have ? 1u : 0u;
             view.n_hit = view.n_access;
-            for (uint64_t m = bam::ballot(have); m; m &= m - 1) {
+            if constexpr (PARTS) {
+                const uint64_t here = bam::ballot(have);
+                for (uint32_t k = 0; k < n_segs; k++) {
+                    const uint64_t m = (here >> (k << g.part_log)) & ((1ull << per) - 1ull);
+                    if (m) visit_parts(algo, g, s, view, seg0 + k, k, m, k << g.part_log, slot, found, found_ahead);
+                }
+            } else for (uint64_t m = bam::ballot(have); m; m &= m - 1) {
                 const uint32_t j = bam::first_lane(m);
                 const uint64_t* payload = (const uint64_t*)view.slot_addr(bam::bcast(slot, j)) + lane;
                 for (uint32_t k = j << g.seg_log; k < (j + 1) << g.seg_log; k++) {
@@ -1113,7 +1165,7 @@ __global__ __launch_bounds__(BAM_TRIP_WAVES * BAM_WAVE_SIZE) void k_along_reside
  * before, with 512, 256 and 128 waves of 32 pages: 124 100 11.36, 108 100 9.83, 102 000 9.14, 98 000 8.88; 2^20 vertices, half cached,
  * 46 700 4.78, 32 900 3.32, 30 900 3.19, 30 700 3.20; 2^19, half, 28 500 3.17, 21 700 2.38, 18 400 2.07, 16 100 1.96.
  */
-template <typename A>
+template <typename A, bool PARTS>
 __global__ __launch_bounds__(BAM_WAVE_SIZE) void k_along_missing(array_d_t<uint64_t>* da, const along_t g, const A algo, const uint32_t chunk, const uint32_t again_waves)
 {
     __shared__ typename A::lds_t s;
@@ -1139,7 +1191,27 @@ __global__ __launch_bounds__(BAM_WAVE_SIZE) void k_along_missing(array_d_t<uint6
         auto keep = [&](uint32_t s_) { slot = s_; return false; };
         view.acquire_helped(p + pso_pages, want, false, keep, keep);
         /* a page whose wait was given up (the controller is marked aborted) has no slot and is not visited */
-        for (uint64_t m = bam::ballot(want && slot != BAM_NO_SLOT); m; m &= m - 1) {
+        if constexpr (PARTS) {
+            /* the pages of a segment follow one another in the list, but for those that are not in it */
+            const uint32_t per = 1u << g.part_log;
+            for (uint64_t m = bam::ballot(want && slot != BAM_NO_SLOT); m;) {
+                const uint32_t j = bam::first_lane(m);
+                const uint64_t seg = bam::bcast(p, j) >> g.part_log;
+                const uint64_t same = bam::ballot(want && slot != BAM_NO_SLOT && p >> g.part_log == seg);
+                m &= ~same;
+                /* lane q: the slot of the segment's q-th page */
+                uint64_t held = 0;
+                uint32_t at = 0;
+                for (uint32_t q = 0; q < per; q++) {
+                    const uint64_t of = bam::ballot((p & (per - 1u)) == q) & same;
+                    if (!of) continue;
+                    held |= 1ull << q;
+                    const uint32_t s_q = bam::bcast(slot, bam::first_lane(of));
+                    if (lane == q) at = s_q;
+                }
+                if (algo.prepare(g, s, seg, 1)) visit_parts(algo, g, s, view, seg, 0, held, 0, at, found, found_ahead);
+            }
+        } else for (uint64_t m = bam::ballot(want && slot != BAM_NO_SLOT); m; m &= m - 1) {
             const uint32_t j = bam::first_lane(m);
             const uint64_t seg0 = bam::bcast(p, j) << g.seg_log;
             const uint64_t* payload = (const uint64_t*)view.slot_addr(bam::bcast(slot, j)) + lane;
@@ -1445,11 +1517,13 @@ bool graph_plan::along_edges(bam_array_t* edges, hipStream_t st, const bool leve
     if (r.index_start != 0 || r.page_start_offset % r.cache.page_size || r.cache.n_pages < 2) return false;
     if (by_page(edges, st, true)) return false;
     by_page_plan& pl = bp;
-    const uint64_t segs_per_page = r.cache.page_size / (BAM_SEG_EDGES * 8);
-    if (!segs_per_page || segs_per_page > BAM_TRIP_SEGS || !pl.n_pages || pl.n_pages > 0xFFFFFFFFull || n_vertices > 1ull << 32 || pl.n_edges > r.count || lists_end > pl.n_edges) return false;
+    /* pages of less than a segment: of a row or more, as many to a trip of the first launch as a wave has lanes */
+    const uint64_t segs_per_page = std::max<uint64_t>(1, r.cache.page_size / (BAM_SEG_EDGES * 8));
+    const uint64_t pages_per_seg = std::max<uint64_t>(1, BAM_SEG_EDGES * 8 / r.cache.page_size);
+    if (pages_per_seg > BAM_SEG_ROWS || segs_per_page > BAM_TRIP_SEGS || !pl.n_pages || pl.n_pages > 0xFFFFFFFFull || n_vertices > 1ull << 32 || pl.n_edges > r.count || lists_end > pl.n_edges) return false;
     /* the first vertices of the segments where those are not the pages, the list of missing pages; and the bits, only where some edges
      * are on the store: there are no sweeps to spare otherwise */
-    const uint64_t n_segs = (pl.n_edges + BAM_SEG_EDGES - 1) / BAM_SEG_EDGES, seg_words = segs_per_page > 1 ? n_segs + 1 : 0;
+    const uint64_t n_segs = (pl.n_edges + BAM_SEG_EDGES - 1) / BAM_SEG_EDGES, seg_words = segs_per_page > 1 || pages_per_seg > 1 ? n_segs + 1 : 0;
     int dev = 0;
     hip_err_chk(hipGetDevice(&dev));
     if (!along_mem.get(seg_words * sizeof(uint64_t) + pl.n_pages * sizeof(uint32_t), levels && !all_cached ? n_segs * BAM_SEG_ROWS * sizeof(uint64_t) : 0,
@@ -1459,9 +1533,10 @@ bool graph_plan::along_edges(bam_array_t* edges, hipStream_t st, const bool leve
         uint64_t* const seg_first = seg_words ? (uint64_t*)along_mem.tables.get() : (uint64_t*)pl.first.get();
         along.offsets = offsets; along.n_vertices = n_vertices; along.n_edges = pl.n_edges; along.n_pages = pl.n_pages; along.n_segs = n_segs;
         along.seg_log = (uint32_t)__builtin_ctzll(segs_per_page);
+        along.part_log = (uint32_t)__builtin_ctzll(pages_per_seg);
         along.trip_segs = (uint32_t)segs_per_page;
         /* a wave's share as small as leaves 16384 waves or more (2^20 vertices, all cached, BFS: 0.47 ms, with 8192 0.50, 4096 0.56, 2048 0.70) */
-        while (along.trip_segs < BAM_TRIP_SEGS && n_segs / along.trip_segs >= 32768) along.trip_segs *= 2;
+        while (along.trip_segs < std::min<uint64_t>(BAM_TRIP_SEGS, BAM_WAVE_SIZE / pages_per_seg) && n_segs / along.trip_segs >= 32768) along.trip_segs *= 2;
         along.first = seg_first;
         if (seg_words)
             hipLaunchKernelGGL(k_page_first_vertex, dim3(blocks_for(n_segs + 1, 256)), dim3(256), 0, st, offsets, n_vertices, (uint64_t)BAM_SEG_EDGES, n_segs, seg_first);
@@ -1502,7 +1577,9 @@ void along_sweep(bam_array_t* edges, const graph_plan* pl, along_t g, const A& a
         g.stretches = stretches;
     }
     const uint32_t blocks = (uint32_t)std::min<uint64_t>(!A::joins ? 1ull << 31 : look ? 512 : 1024, n_blk);
-    hipLaunchKernelGGL(k_along_resident<A>, dim3(blocks), dim3(BAM_TRIP_WAVES * BAM_WAVE_SIZE), A::joins ? 48u << 10 : 0, st, edges->a->d_array_ptr, g, algo);
+    const uint32_t lds = A::joins ? 48u << 10 : 0;
+    if (g.part_log) hipLaunchKernelGGL((k_along_resident<A, true>), dim3(blocks), dim3(BAM_TRIP_WAVES * BAM_WAVE_SIZE), lds, st, edges->a->d_array_ptr, g, algo);
+    else hipLaunchKernelGGL((k_along_resident<A, false>), dim3(blocks), dim3(BAM_TRIP_WAVES * BAM_WAVE_SIZE), lds, st, edges->a->d_array_ptr, g, algo);
     /* As many waves as leave each a batch worth sending (pages a wave, ms: 29 500 cached, BFS of 2^21 vertices 64 11.8, 32 11.4, 16
      * 11.6, 8 11.9; 7 500, 2^19 16 3.18, 8 3.11, 4 3.27; 3 700, 2^18 16 1.89, 8 1.73, 4 1.79; 2 048, 2^16 16 0.88, 8 0.72, 4 0.62, 2 0.70).
      * Under four pages a wave where the cache is small and what a wave fetched, visited one page after the other, is much: for joins, which
@@ -1513,13 +1590,20 @@ void along_sweep(bam_array_t* edges, const graph_plan* pl, along_t g, const A& a
      * cached: 2.6 -> 1.6 ms, and 2.8 -> 3.7). */
     const uint64_t budget = pl->along_budget, enough = A::joins ? 128 : 64;
     const uint32_t least = A::joins || g.seg_log > 2 ? 1 : g.seg_log == 2 ? 2 : 4;
-    uint32_t chunk = 32;
+    const bool parts = g.part_log != 0;
+    uint32_t chunk = parts ? 64 : 32;
     while ((chunk > 4 && budget / chunk < 256) || (chunk > least && budget / chunk < enough)) chunk /= 2;
     if (chunk > budget) chunk = (uint32_t)budget;
-    const uint32_t waves = (uint32_t)std::min<uint64_t>(BAM_ALONG_WAVES, budget / chunk);
+    /* Pages of less than a segment come in several times as fast: more of them to a wave, and more waves, as long as the cache is not
+     * small (pages of 512 bytes, 64 to a wave with 1024 waves, 512 where slots are used again / 32 with 512 and 128 / 64 with 512 and 256, ms: BFS of 2^20
+     * vertices, half cached, 3.9 / 7.7 / 4.9, a quarter 6.0 / 10.9 / 8.0; 2^16 vertices, a quarter, batches of 4, with 468, 256 and 128 waves 1.39,
+     * 1.21, 1.23; components of 2^21, a quarter, 4.1 / 4.9 / 3.8). */
+    const uint32_t waves = (uint32_t)std::min<uint64_t>(parts ? 2 * BAM_ALONG_WAVES : BAM_ALONG_WAVES, budget / chunk);
     /* 128 of them where they reuse their slots; 1024 pages on their way all the same (2^18 vertices, 3 700 cached, chunks of 4: 256 waves 1.59
      * ms, 128 1.93, all 469 1.58; the hand alone 1.76) */
-    hipLaunchKernelGGL(k_along_missing<A>, dim3(waves), dim3(BAM_WAVE_SIZE), 0, st, edges->a->d_array_ptr, g, algo, chunk, std::min(waves, std::max(128u, 1024u / chunk)));
+    const uint32_t again_waves = std::min(waves, parts ? chunk == 64 ? 512u : 256u : std::max(128u, 1024u / chunk));
+    if (parts) hipLaunchKernelGGL((k_along_missing<A, true>), dim3(waves), dim3(BAM_WAVE_SIZE), 0, st, edges->a->d_array_ptr, g, algo, chunk, again_waves);
+    else hipLaunchKernelGGL((k_along_missing<A, false>), dim3(waves), dim3(BAM_WAVE_SIZE), 0, st, edges->a->d_array_ptr, g, algo, chunk, again_waves);
     hip_err_chk(hipGetLastError());
 }
 }
@@ -1563,10 +1647,14 @@ uint32_t bfs_along_levels(bam_array_t* edges, graph_plan* pl, uint32_t* d_labels
 }
 
 /* one reading of the edges that joins the trees of their ends.  In one launch where all are cached and few: 2^15 entries take 80 us, in two
- * 88; but that one goes over the vertices between the lists of a page, so not where there may be many */
-void cc_read_edges(bam_array_t* edges, graph_plan* pl, unsigned long long* comp, hipStream_t st)
+ * 88 (in pages of 512 and 1024 bytes, which that launch goes over one after the other, 271 and 144, and 85); but that one goes over
+ * the vertices between the lists of a page, so not where there may be many.  By page (bam_cc_by_page), in pages of less than 4 KiB, also where
+ * all are cached and many: 2^24 entries of a uniform graph in pages of 512, 1024, 2048 bytes 690, 660, 630 us, in two launches 725, 730, 775
+ * (vertex by vertex 990, 970, 1070). */
+void cc_read_edges(bam_array_t* edges, graph_plan* pl, unsigned long long* comp, hipStream_t st, const bool by_page)
 {
-    if (pl->along.n_segs && !(pl->all_cached && pl->bp.n_edges <= 1ull << 17 && pl->n_vertices <= pl->bp.n_edges / 4)) along_sweep(edges, pl, pl->along, cc_along{comp}, st);
+    const bool one = pl->bp.n_edges <= 1ull << 17 ? pl->along.part_log < 2 : by_page && pl->along.part_log;
+    if (pl->along.n_segs && !(one && pl->all_cached && pl->n_vertices <= pl->bp.n_edges / 4)) along_sweep(edges, pl, pl->along, cc_along{comp}, st);
     else if (pl->bp.n_pages)
         hipLaunchKernelGGL(k_cc_by_page, dim3(pl->bp.blocks), dim3(BAM_WAVE_SIZE), 0, st, edges->a->d_array_ptr, pl->offsets, (const uint64_t*)pl->bp.first.get(), pl->bp.n_edges, pl->bp.ppw,
                            pl->cc_backwards(), comp);
@@ -1811,7 +1899,7 @@ int bam_cc(bam_array_t* edges, const uint64_t* d_offsets, uint64_t n_vertices, u
     unsigned long long* comp = (unsigned long long*)d_labels;
     const bool along = pl->along_edges(edges, st, false);
     hipLaunchKernelGGL(k_iota, dim3(blocks_for(n_vertices, 256)), dim3(256), 0, st, comp, n_vertices);
-    if (along) cc_read_edges(edges, pl, comp, st);
+    if (along) cc_read_edges(edges, pl, comp, st, false);
     else
         hipLaunchKernelGGL(k_cc_coalesce_coarse_ptr_pc, dim3(pl->blocks(n_vertices, group)), dim3(128), 0, st, edges->a->d_array_ptr, n_vertices, d_offsets, comp, group,
                        pl->pieces, pl->n_pieces, pl->next_work(), pl->cc_backwards());
@@ -1894,7 +1982,7 @@ int bam_cc_by_page(bam_array_t* edges, const uint64_t* d_offsets, uint64_t n_ver
     }
     if (changed) {
         if (iter) hipLaunchKernelGGL(k_cc_shorten, dim3(blocks_for(n_vertices, 256)), dim3(256), 0, st, comp, n_vertices);
-        cc_read_edges(edges, pl, comp, st);
+        cc_read_edges(edges, pl, comp, st, true);
         hipLaunchKernelGGL(k_cc_settle, dim3(blocks_for(n_vertices, 256)), dim3(256), 0, st, comp, n_vertices, pl->along.n_missing, pl->along.next_chunk);
         hip_err_chk(hipGetLastError());
         hip_err_chk(hipStreamSynchronize(st));

@@ -234,7 +234,7 @@ int bam_array_set_graph(bam_array_t* edges, const uint64_t* d_offsets, uint64_t 
  * Level-synchronous BFS from src: d_offsets[V+1] in device memory, neighbour ids read through the array,
  * d_labels[V] receives the level of every vertex (0xFFFFFFFF = unreachable).  *iterations = levels swept.
  * The array may be longer than the lists; what lies outside them is not looked at.
- * Where it has one range that begins on a page boundary, and pages of 4 to 64 KiB, and there is memory for the tables, the edges
+ * Where it has one range that begins on a page boundary, and pages of 512 bytes to 64 KiB, and there is memory for the tables, the edges
  * are read along their pages (bam_bfs_by_page); the same for bam_bfs_frontier and bam_cc.  That was quicker on power-law and uniform
  * graphs of 2^12 to 2^24 vertices with all to 1 % of the edges cached, and on grids and paths of 2^13 to 2^26 vertices with up to 16 000
  * levels (a level looks at the labels of all vertices: 2^26 vertices, 8192 x 8192, 67 us a level, over queues 260); not where next to
@@ -289,8 +289,8 @@ int bam_cc(bam_array_t* edges, const uint64_t* d_offsets, uint64_t n_vertices, u
  * page of the edge array, which it walks vertex by vertex.  Here a sweep is two launches: the pages that hold edges of active
  * vertices and are resident are visited, the others listed, and then fetched in batches and visited; the table is built
  * by binary search.  Where some edges are on the store, edges of the next level's vertices are visited along with a level's
- * own where their page is there anyway, and their pages need not come in for them again.  (Pages smaller than 4 KiB or larger
- * than 64: a wave takes a run of up to 64 consecutive pages, and acquires those that hold edges of active vertices with one call.)
+ * own where their page is there anyway, and their pages need not come in for them again.  (Pages larger than 64 KiB:
+ * a wave takes a run of up to 64 consecutive pages, and acquires those that hold edges of active vertices with one call.)
  * Same inputs, same outputs as bam_bfs / bam_cc (levels and labels are unique, so they are bit-identical).
  * The array must consist of one range that starts on a page boundary. */
 int bam_bfs_by_page(bam_array_t* edges, const uint64_t* d_offsets, uint64_t n_vertices, uint64_t src, uint32_t* d_labels,
