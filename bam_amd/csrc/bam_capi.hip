@@ -3,6 +3,7 @@
 // pattern and block benchmarks.  Kernel shapes follow the reference's benchmark
 // kernels (cited per kernel); lane arithmetic is for 64-wide waves.  The graph
 // kernels are in bam_graph.hip, vectoradd / reduction / scan in bam_apps.hip.
+#include <cmath>
 #include "bam_capi_internal.h"
 
 std::string& bam_err()
@@ -99,6 +100,18 @@ __global__ void k_array_read_n_whole(array_d_t<uint64_t>* dr, uint64_t n_reqs, c
     block_accumulate(sum, v);
 }
 
+/* requests of a first launch that wait for pages from the store, dealt out page by page (k_reads_begin, k_reads_deal, k_reads_fetch) */
+struct dealt_reads_t {
+    uint32_t* counts;            /* [pages] requests for the page; zero between calls */
+    uint32_t* begin;             /* [pages] where they begin */
+    uint32_t* ranks;             /* [n] which of its page's the request is */
+    uint64_t* idx;               /* [n] page after page: index of the request's element */
+    uint32_t* ids;               /* [n] and which request it is (what is handed out, not what is summed) */
+    uint32_t* cursor;            /* requests dealt so far, and turns taken: zero when the first launch has ended */
+    uint32_t* turns;
+    uint32_t pages, turn, batch; /* neighbouring pages to a turn of a wave, and how many of them are asked for at a time: powers of two, BAM_BEGIN_PAGES and 64 at most */
+    uint32_t hits;               /* whether requests count as hits but for the one that its page is asked for by */
+};
 /*
  * A launch of scattered requests in several launches (arrays of one range).  The first, this kernel: a wave takes
  * 64 * N * rounds consecutive requests, N per lane at a time, and reads those whose page is resident, without a reference
@@ -112,11 +125,13 @@ __global__ void k_array_read_n_whole(array_d_t<uint64_t>* dr, uint64_t n_reqs, c
  * line of HBM behind each element.  2^26 reads of a resident 1 GiB: 1.52 ms summed, 1.83 ms handed out (2.03 as one launch with
  * one read per thread); N = 4 instead of 8: 1.91.
  */
-template <int N, bool GATHER>
+template <int N, bool GATHER, bool DEALT = false>
 __global__ __launch_bounds__(256) void k_array_read_n(array_d_t<uint64_t>* dr, uint64_t n_reqs, const uint64_t* __restrict__ assignment, uint32_t rounds,
-                                                      unsigned long long* partials, uint64_t* missed, uint64_t n_words, uint8_t* wanted, unsigned long long* sum, uint64_t* out_list, uint32_t* finished, uint32_t call)
+                                                      unsigned long long* partials, uint64_t* missed, uint64_t n_words, uint8_t* wanted, unsigned long long* sum, uint64_t* out_list, uint32_t* finished, uint32_t call,
+                                                      const dealt_reads_t g)
 {
     const uint32_t lane = bam::lane();
+    if constexpr (DEALT) { if (blockIdx.x == 0 && threadIdx.x == 0) *g.cursor = *g.turns = 0; }
     /* the wave's requests: 64 * N * rounds consecutive ones, lane l taking l, l + 64, ..., N at a time: what a wave, a workgroup
      * and the launch do once (the range's descriptor, the counters, the checksum) is shared by more reads the more rounds there are */
     const uint64_t wave = bam::first(((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) / BAM_WAVE_SIZE), w0 = wave * N * rounds, t0 = w0 * BAM_WAVE_SIZE + lane;
@@ -152,6 +167,7 @@ __global__ __launch_bounds__(256) void k_array_read_n(array_d_t<uint64_t>* dr, u
         dr->template seq_read_n_resident<N, true>(idx, want, out, got, view);
         /* the N words of notes of the round with one store: lane j writes the j-th */
         uint64_t mine = 0;
+        uint32_t rank[N];
 #pragma unroll
         for (int j = 0; j < N; j++) {
             const bool left = want[j] & !got[j] & (idx[j] - view.index_start < view.index_end - view.index_start);
@@ -160,7 +176,12 @@ __global__ __launch_bounds__(256) void k_array_read_n(array_d_t<uint64_t>* dr, u
             const uint64_t m = bam::ballot(left);
             if (lane == (uint32_t)j) mine = m;
             any_left |= m;
-            if (m && wanted && left) wanted[view.page_of(idx[j])] = 1;
+            if constexpr (DEALT) { rank[j] = 0; got[j] = left; if (left) rank[j] = __hip_atomic_fetch_add(g.counts + view.page_of(idx[j]), 1u, __ATOMIC_RELAXED, BAM_AGENT); }
+            else if (m && wanted && left) wanted[view.page_of(idx[j])] = 1;
+        }
+        if constexpr (DEALT) {
+#pragma unroll
+            for (int j = 0; j < N; j++) if (got[j]) g.ranks[t0 + (r * N + j) * BAM_WAVE_SIZE] = rank[j];
         }
         if (lane < (uint32_t)N && w0 + r * N + lane < n_words) missed[w0 + r * N + lane] = mine;
     }
@@ -309,6 +330,216 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
         if (bam::ballot(any)) block_accumulate(partials, v);
         fold_by_last_block(partials, sum, finished);
     }
+}
+
+/*
+ * Page by page, each page asked for once and visited as soon as it is there, whatever the cache holds: the first launch has
+ * counted the requests of each page as it found them missing (DEALT above), the next two put them in order of their pages, and a
+ * wave of the last (k_reads_fetch) takes a turn of neighbouring pages, asks for those that somebody waits for in batches and
+ * reads the batch's requests, which lie side by side.  Stretches of the range (k_fetch_wanted) need a drain of the queues
+ * each, and caches of thousands of pages.
+ *   A wave holds its batch while it waits for the rest of it, as k_along_missing does, and the pages that are held so are counted in a
+ * word of the cache, for all arrays and streams together: beyond half the cache batches are not held, and a page that goes
+ * before its requests are read is read on demand.
+ *   Bound by the store.  Gathers of elements at random, request by request or in stretches, and here, ms (pages of 4 KiB): 8404 behind 2101,
+ * 20000 requests 1.06 and 0.70, 277608 7.3 and 0.72, 2^22 458 and 1.10; 16384 behind 8192, 2^20 1.33 and 0.74; 65536 behind 16384, 2^17 5.9 and
+ * 3.3, 2^22 4.94 and 4.04; 65536 behind 32768, 2^19 2.78 and 2.65; 512 behind 256, 10^5 0.65 and 0.12; 192076 of 512 bytes behind 96038, 426105
+ * 2.1 and 1.6.  Turns of as many pages as have a batch wanted among them: 2^21 pages of 512 bytes, half cached, 2^20 requests, 7.8, with turns of
+ * a batch's size 11.7.
+ */
+#define BAM_BEGIN_PAGES 1024u
+#define BAM_PLEDGED_WORD 1u          /* of the cache's miss_tokens: pages held so, beside the count of the first compute unit */
+/* what lanes of a wave have written to LDS, for all of its lanes: a wave's LDS operations run in order */
+__device__ __forceinline__ void wave_lds_fence()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+__global__ __launch_bounds__(256) void k_reads_begin(const dealt_reads_t g, const uint32_t* finished, uint32_t call)
+{
+    __shared__ uint32_t wave_total[256 / BAM_WAVE_SIZE], base;
+    if (__hip_atomic_load(finished + BAM_LEFT_WORD, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != call) return;
+    const uint32_t p = blockIdx.x * BAM_BEGIN_PAGES + threadIdx.x * 4u, w = threadIdx.x / BAM_WAVE_SIZE;
+    uint32_t c[4];
+#pragma unroll
+    for (uint32_t k = 0; k < 4; k++) c[k] = p + k < g.pages ? g.counts[p + k] : 0;
+    const uint32_t mine = c[0] + c[1] + c[2] + c[3], incl = (uint32_t)bam::wave_running_sum(mine);
+    if (bam::lane() == BAM_WAVE_SIZE - 1) wave_total[w] = incl;
+    __syncthreads();
+    /* in whatever order the workgroups come: what matters is that the pages of a turn follow one another */
+    if (threadIdx.x == 0) base = __hip_atomic_fetch_add(g.cursor, wave_total[0] + wave_total[1] + wave_total[2] + wave_total[3], __ATOMIC_RELAXED, BAM_AGENT);
+    __syncthreads();
+    uint32_t at = base + incl - mine;
+    for (uint32_t k = 0; k < w; k++) at += wave_total[k];
+#pragma unroll
+    for (uint32_t k = 0; k < 4; k++) { if (p + k < g.pages) g.begin[p + k] = at; at += c[k]; }
+}
+template <bool GATHER>
+__global__ __launch_bounds__(256) void k_reads_deal(array_d_t<uint64_t>* dr, const dealt_reads_t g, const uint64_t* __restrict__ assignment, const uint64_t* __restrict__ missed, uint64_t n_words,
+                                                    const uint32_t* finished, uint32_t call)
+{
+    constexpr uint32_t N = 4;
+    if (__hip_atomic_load(finished + BAM_LEFT_WORD, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != call) return;
+    const uint32_t lane = bam::lane();
+    const uint64_t w0 = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) / BAM_WAVE_SIZE * N;
+    bam::range_view<uint64_t> view;
+    view.load(dr->d_ranges);
+    bool take[N];
+    uint64_t i[N];
+    uint32_t rank[N], begin[N];
+#pragma unroll
+    for (uint32_t j = 0; j < N; j++) take[j] = w0 + j < n_words && ((missed[w0 + j] >> lane) & 1);
+#pragma unroll
+    for (uint32_t j = 0; j < N; j++) {
+        const uint64_t t = take[j] ? (w0 + j) * BAM_WAVE_SIZE + lane : 0;
+        i[j] = assignment[t];
+        rank[j] = g.ranks[t];
+    }
+#pragma unroll
+    for (uint32_t j = 0; j < N; j++) begin[j] = take[j] ? g.begin[view.page_of(i[j])] : 0;
+#pragma unroll
+    for (uint32_t j = 0; j < N; j++)
+        if (take[j]) {
+            g.idx[begin[j] + rank[j]] = i[j];
+            if constexpr (GATHER) g.ids[begin[j] + rank[j]] = (uint32_t)((w0 + j) * BAM_WAVE_SIZE + lane);
+        }
+}
+template <bool GATHER>
+__global__ __launch_bounds__(64) void k_reads_fetch(array_d_t<uint64_t>* dr, const dealt_reads_t g, unsigned long long* partials, unsigned long long* sum, uint64_t* out_list, uint32_t* finished, uint32_t call)
+{
+    constexpr int N = 4;
+    __shared__ uint32_t list[BAM_WAVE_SIZE * 2], counts[BAM_WAVE_SIZE * 2], slots[BAM_BEGIN_PAGES];
+    if (__hip_atomic_load(finished + BAM_LEFT_WORD, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != call) return;
+    const uint32_t lane = bam::lane();
+    bam::range_view<uint64_t> view;
+    view.load(dr->d_ranges);
+    view.place = BAM_PLACE_PULLED;
+    const page_cache_d_t* const cache = &dr->d_ranges->cache;
+    uint32_t* const pledged = cache->miss_tokens + BAM_PLEDGED_WORD;
+    const uint32_t most = (uint32_t)(cache->n_pages / 2);
+    uint64_t v = 0;
+    uint32_t n_read = 0, n_pages = 0;
+    for (;;) {
+        uint32_t turn = 0;
+        if (lane == 0) turn = __hip_atomic_fetch_add(g.turns, 1u, __ATOMIC_RELAXED, BAM_AGENT);
+        const uint64_t first = (uint64_t)bam::bcast(turn, 0) * g.turn;
+        if (first >= g.pages) break;
+        const uint64_t last = first + g.turn < g.pages ? first + g.turn : g.pages;
+        uint32_t begin = bam::first(g.begin[first]), have = 0;
+        for (uint64_t p = first; p < last || have;) {
+            /* the next pages that somebody waits for, as many as are asked for together */
+            while (have < g.batch && p < last) {
+                const uint32_t n_mine = p + lane < last ? g.counts[p + lane] : 0;
+                const uint64_t m = bam::ballot(n_mine != 0);
+                if (n_mine) {
+                    const uint32_t at = have + bam::popc(m & bam::lanes_below(lane));
+                    list[at] = (uint32_t)p + lane;
+                    counts[at] = n_mine;
+                    g.counts[p + lane] = 0;
+                }
+                have += bam::popc(m);
+                p += BAM_WAVE_SIZE;
+            }
+            wave_lds_fence();
+            const uint32_t pages = have < g.batch ? have : g.batch;
+            if (!pages) break;
+            const bool mine = lane < pages;
+            const uint64_t page = list[mine ? lane : 0];
+            const uint32_t n = bam::bcast((uint32_t)bam::wave_running_sum(mine ? counts[lane] : 0), BAM_WAVE_SIZE - 1);
+            const uint32_t next = list[pages + lane < have ? pages + lane : 0], next_count = counts[pages + lane < have ? pages + lane : 0];
+            wave_lds_fence();
+            if (pages + lane < have) { list[lane] = next; counts[lane] = next_count; }
+            have -= pages;
+            uint32_t hold = 0;
+            if (lane == 0) {
+                hold = __hip_atomic_fetch_add(pledged, pages, __ATOMIC_RELAXED, BAM_AGENT) + pages <= most;
+                if (!hold) __hip_atomic_fetch_add(pledged, 0u - pages, __ATOMIC_RELAXED, BAM_AGENT);
+            }
+            hold = bam::bcast(hold, 0);
+            uint32_t slot = BAM_NO_SLOT;
+            auto arrive = [&](uint32_t at) { slot = hold ? at : BAM_NO_SLOT; return !hold; };
+            view.acquire_helped(page, mine, false, arrive, arrive);
+            if (mine) slots[page - first] = slot;
+            const bool held = bam::ballot(mine && slot == BAM_NO_SLOT) == 0;
+            if (!held && slot != BAM_NO_SLOT) bam_release_refs(view.pages + page, 1, false);        /* a wait was given up */
+            wave_lds_fence();
+            n_pages += pages;
+            for (uint32_t b = 0; b < n; b += N * BAM_WAVE_SIZE) {
+                size_t idx[N];
+                bool want[N], got[N];
+                uint64_t x[N];
+#pragma unroll
+                for (int j = 0; j < N; j++) {
+                    const uint32_t k = b + j * BAM_WAVE_SIZE + lane;
+                    want[j] = k < n;
+                    idx[j] = g.idx[begin + (want[j] ? k : 0)];
+                }
+                if (held) {
+                    const uint64_t* at[N];
+#pragma unroll
+                    for (int j = 0; j < N; j++) {
+                        const uint64_t byte = view.byte_of(idx[j]);
+                        at[j] = (const uint64_t*)(view.slot_addr(slots[(byte >> view.page_size_log) - first]) + (byte & (view.page_size - 1)));
+                        n_read += bam::popc(bam::ballot(want[j]));
+                    }
+                    bam::ld_payload_nt(at, x);
+                } else {
+                    dr->template seq_read_n_resident<N, true>(idx, want, x, got, view);
+#pragma unroll 1
+                    for (int j = 0; j < N; j++) {
+                        n_read += bam::popc(bam::ballot(got[j]));
+                        if (want[j] && !got[j]) x[j] = dr->seq_read_call(idx[j]);
+                    }
+                }
+#pragma unroll
+                for (int j = 0; j < N; j++) {
+                    if constexpr (GATHER) { if (want[j]) __builtin_nontemporal_store(x[j], out_list + g.ids[begin + b + j * BAM_WAVE_SIZE + lane]); }
+                    else v += want[j] ? x[j] : 0;
+                }
+            }
+            if (held && mine) bam_release_refs(view.pages + page, 1, false);
+            if (hold && lane == 0) __hip_atomic_fetch_add(pledged, 0u - pages, __ATOMIC_RELAXED, BAM_AGENT);
+            begin += n;
+        }
+    }
+    view.n_access = lane == 0 ? n_read : 0;
+    view.n_hit = lane == 0 && g.hits && n_read > n_pages ? n_read - n_pages : 0;
+    view.flush_stats();
+    if constexpr (!GATHER) {
+        block_accumulate(partials, v);
+        fold_by_last_block(partials, sum, finished);
+    }
+}
+
+/*
+ * Few requests of an array larger than its cache: `each` of them to a wave (a power of two), whose other lanes help to move
+ * their pages.  Bound by the time a wave takes for its batch, which grows with the batch: of 1000 requests of 4096 pages behind 2048 with
+ * ten of their pages missing 183 us with 64 to a wave, 37 with 4; all missing pages, 3000 requests, 250 and 182, 512 pages behind 256, 700
+ * requests, 185 and 66; all resident 6 to 7 us either way.
+ */
+template <bool GATHER>
+__global__ __launch_bounds__(256) void k_array_read_few(array_d_t<uint64_t>* dr, uint64_t n_reqs, const uint64_t* __restrict__ assignment, uint32_t each, unsigned long long* partials, uint64_t* out_list)
+{
+    const uint32_t lane = bam::lane();
+    const uint64_t t = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) / BAM_WAVE_SIZE * each + lane;
+    const bool mine = lane < each && t < n_reqs;
+    const size_t idx[1] = {mine ? assignment[t] : 0};
+    const bool want[1] = {mine};
+    bam::range_view<uint64_t> view;
+    view.load(dr->d_ranges);
+    uint64_t x[1];
+    bool got[1];
+    dr->template seq_read_n_resident<1, true>(idx, want, x, got, view);
+    const bool absent = mine && !got[0] && view.holds(idx[0]);
+    if (bam::ballot(absent)) {
+        const uint64_t byte = absent ? view.byte_of(idx[0]) : 0;
+        auto use = [&](uint32_t slot) { x[0] = bam::ld_payload((const uint64_t*)(view.slot_addr(slot) + (byte & (view.page_size - 1)))); return true; };
+        view.acquire_helped(byte >> view.page_size_log, absent, false, use, use);
+    }
+    if constexpr (GATHER) { if (mine) out_list[t] = x[0]; }
+    else block_accumulate(partials, mine ? x[0] : 0);
+    view.template flush_stats<false>();
 }
 
 /* thread t hands out the element it read instead of adding it to a sum */
@@ -1723,6 +1954,97 @@ bool scattered_launches_pay(bam_array_t* a, uint64_t n_reqs, hipStream_t st)
     return !is_captured(st);
 }
 /*
+ * Few requests, so that most have a page to themselves: spread over more waves than there are 64 of them (k_array_read_few), 256 waves in
+ * pages of 4 KiB or less and as many bytes in larger ones.  A wave for 64, at least 256 and at least 512 waves, us: 4096 pages behind 2048, 1000 requests 183, 37, 37,
+ * 8000 252, 219, 247; 16384 behind 8192, 5000 258, 155, 172, 30000 608, 614, 620; 65536 behind 16384, 20000 1088, 1086, 1130.
+ */
+bool few_reads_pay(bam_array_t* a, uint64_t n_reqs)
+{
+    const range_d_t<uint64_t>& range = a->a->h_ranges[0];
+    return two_launches_ok(a) && range.page_count > range.cache.n_pages && n_reqs <= BAM_REQS_AT_A_TIME;
+}
+template <bool GATHER>
+void few_reads(bam_array_t* a, uint64_t n_reqs, const uint64_t* d_assignment, uint64_t* d_out, hipStream_t st)
+{
+    const uint64_t least = std::min<uint64_t>(256, (1ull << 20) / a->a->h_ranges[0].cache.page_size);
+    uint32_t each = BAM_WAVE_SIZE;
+    while (each > 4 && n_reqs / each < least) each /= 2;
+    hipLaunchKernelGGL(k_array_read_few<GATHER>, dim3(blocks_for((n_reqs + each - 1) / each * BAM_WAVE_SIZE, 256)), dim3(256), 0, st, a->a->d_array_ptr, n_reqs, d_assignment, each,
+                       (unsigned long long*)a->partials.get(), d_out);
+}
+/*
+ * Whether requests are put in order of their pages: where there are more than one for each page and two for each slot (below, few of them
+ * share a page, and each waits for its own: us that way and in order, 4096 pages behind 2048, 8000 219 and 244, 16000 258 and 242; 16384
+ * behind 8192, 30000 614 and 646, 60000 735 and 725; 8404 behind 2101, 8404 436 and 538, 12000 700 and 609), and always where they are not all on
+ * their way together; but not where requests spread evenly ask for no more pages than the cache holds, and so find them all
+ * the next time (that takes three launches more, 16 us for 6).
+ *   Large launches go by stretches all the same where those have the whole array in two, and where there would be several
+ * slices, each of which asks for all pages (2^19 pages behind 2^18, 2^22 requests 19.9 and 20.3 ms; 2^16 behind 2^15, 2^24 3.3 and 11.1).
+ */
+#define BAM_DEALT_SLICE (1ull << 22)
+bool dealt_reads_pay(bam_array_t* a, uint64_t n_reqs, hipStream_t st)
+{
+    if (!two_launches_ok(a)) return false;
+    const range_d_t<uint64_t>& range = a->a->h_ranges[0];
+    const uint64_t pages = range.page_count, cache_pages = range.cache.n_pages;
+    if (pages <= cache_pages || pages >= 1ull << 32) return false;
+    if (n_reqs <= BAM_REQS_AT_A_TIME && n_reqs < pages + 2 * cache_pages) return false;
+    if ((double)n_reqs < -std::log1p(-(double)cache_pages / (double)pages) * (double)pages) return false;
+    if (page_by_page(range, n_reqs) && (n_reqs > BAM_DEALT_SLICE || (pages <= 2 * cache_pages && cache_pages >= 1ull << 18))) return false;
+    return !is_captured(st);
+}
+/* the requests in slices, each slice's put in order of their pages; false, with nothing launched, where there is no memory for that */
+template <bool GATHER>
+bool dealt_reads(bam_array_t* a, uint64_t n_reqs, const uint64_t* d_assignment, unsigned long long* sum, uint64_t* d_out, hipStream_t st)
+{
+    const range_d_t<uint64_t>& range = a->a->h_ranges[0];
+    array_d_t<uint64_t>* d = a->a->d_array_ptr;
+    const uint64_t slice = std::min<uint64_t>(n_reqs, BAM_DEALT_SLICE), slice_words = (slice + BAM_WAVE_SIZE - 1) / BAM_WAVE_SIZE, pages = range.page_count;
+    std::lock_guard<std::mutex> guard(a->scratch.mu);
+    scratch_set* set = scratch_for(a, st, (slice_words + slice) * sizeof(uint64_t) + (2 * slice + pages) * sizeof(uint32_t), pages * sizeof(uint32_t));
+    if (!set) return false;
+    uint64_t* missed = (uint64_t*)set->notes.get();
+    dealt_reads_t g{};
+    g.counts = (uint32_t*)set->wanted.get();
+    g.idx = missed + slice_words;
+    g.ids = (uint32_t*)(g.idx + slice);
+    g.ranks = g.ids + slice;
+    g.begin = g.ranks + slice;
+    g.cursor = set->cursor();
+    g.turns = set->turns();
+    g.pages = (uint32_t)pages;
+    g.hits = !page_by_page(range, n_reqs);
+    const uint64_t budget = range.cache.n_pages / 2;
+    /* batches as for k_along_missing (16384 pages of 4 KiB behind 8192, 2^20 requests, 4, 8, 16, 32 to a batch: 0.80, 0.75, 0.75, 0.75 ms; 30000 0.81, 0.76, 0.65, 0.64) */
+    const bool small = range.cache.page_size < 4096;
+    const uint64_t most_waves = small ? 1024 : 512;
+    g.batch = small ? 64 : 32;
+    while (g.batch > 4 && budget / g.batch < 256) g.batch /= 2;
+    /* a turn as long as has about a batch's pages missing and asked for, if there are several for each wave all the same */
+    const uint64_t asked = std::min<uint64_t>(slice, pages) * (pages - range.cache.n_pages) / pages;
+    g.turn = g.batch;
+    while (g.turn < BAM_BEGIN_PAGES && g.turn * asked < g.batch * pages && pages / (2 * g.turn) >= 4 * most_waves) g.turn *= 2;
+    const uint32_t waves = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>({most_waves, budget / g.batch, (pages + g.turn - 1) / g.turn}));
+    unsigned long long* part = set->partials();
+    uint32_t* fin = set->finished();
+    for (uint64_t t = 0; t < n_reqs; t += slice) {
+        const uint64_t n = std::min(slice, n_reqs - t), n_words = (n + BAM_WAVE_SIZE - 1) / BAM_WAVE_SIZE;
+        const uint64_t* const asg = d_assignment + t;
+        uint64_t* const out = GATHER ? d_out + t : nullptr;
+        const uint32_t call = set->next_call();
+        const uint32_t N = n < 1ull << 17 ? 1 : n < 1ull << 20 ? 4 : 8;
+        const dim3 grid(blocks_for((n_words + N - 1) / N * BAM_WAVE_SIZE, 256)), block(256);
+        if (N == 1) hipLaunchKernelGGL((k_array_read_n<1, GATHER, true>), grid, block, 0, st, d, n, asg, 1u, part, missed, n_words, (uint8_t*)nullptr, sum, out, fin, call, g);
+        else if (N == 4) hipLaunchKernelGGL((k_array_read_n<4, GATHER, true>), grid, block, 0, st, d, n, asg, 1u, part, missed, n_words, (uint8_t*)nullptr, sum, out, fin, call, g);
+        else hipLaunchKernelGGL((k_array_read_n<8, GATHER, true>), grid, block, 0, st, d, n, asg, 1u, part, missed, n_words, (uint8_t*)nullptr, sum, out, fin, call, g);
+        hipLaunchKernelGGL(k_reads_begin, dim3(blocks_for(pages, BAM_BEGIN_PAGES)), block, 0, st, g, fin, call);
+        hipLaunchKernelGGL(k_reads_deal<GATHER>, dim3(blocks_for((n_words + 3) / 4 * BAM_WAVE_SIZE, 256)), block, 0, st, d, g, asg, missed, n_words, fin, call);
+        hipLaunchKernelGGL(k_reads_fetch<GATHER>, dim3(waves), dim3(BAM_WAVE_SIZE), 0, st, d, g, part, sum, out, fin, call);
+    }
+    hip_err_chk(hipGetLastError());
+    return true;
+}
+/*
  * Scattered reads in several launches: what is resident (k_array_read_n), then the rest.  Where the array is larger than
  * its cache and there are enough requests for them to meet on pages, the rest goes page by page: the pages somebody waits
  * for are fetched, each once, in whole batches (k_fetch_wanted), and then the requests for them are read
@@ -1752,11 +2074,12 @@ bool scattered_reads(bam_array_t* a, uint64_t n_reqs, const uint64_t* d_assignme
     uint32_t* fin = set->finished();
     const uint32_t call = set->next_call();
     const dim3 grid(blocks_for(n_waves * BAM_WAVE_SIZE, 256)), block(256);
+    const dealt_reads_t none{};
     switch (N) {
-    case 1: hipLaunchKernelGGL((k_array_read_n<1, GATHER>), grid, block, 0, st, d, n_reqs, d_assignment, rounds, part, missed, n_words, wanted, sum, d_out, fin, call); break;
-    case 2: hipLaunchKernelGGL((k_array_read_n<2, GATHER>), grid, block, 0, st, d, n_reqs, d_assignment, rounds, part, missed, n_words, wanted, sum, d_out, fin, call); break;
-    case 4: hipLaunchKernelGGL((k_array_read_n<4, GATHER>), grid, block, 0, st, d, n_reqs, d_assignment, rounds, part, missed, n_words, wanted, sum, d_out, fin, call); break;
-    default: hipLaunchKernelGGL((k_array_read_n<8, GATHER>), grid, block, 0, st, d, n_reqs, d_assignment, rounds, part, missed, n_words, wanted, sum, d_out, fin, call); break;
+    case 1: hipLaunchKernelGGL((k_array_read_n<1, GATHER>), grid, block, 0, st, d, n_reqs, d_assignment, rounds, part, missed, n_words, wanted, sum, d_out, fin, call, none); break;
+    case 2: hipLaunchKernelGGL((k_array_read_n<2, GATHER>), grid, block, 0, st, d, n_reqs, d_assignment, rounds, part, missed, n_words, wanted, sum, d_out, fin, call, none); break;
+    case 4: hipLaunchKernelGGL((k_array_read_n<4, GATHER>), grid, block, 0, st, d, n_reqs, d_assignment, rounds, part, missed, n_words, wanted, sum, d_out, fin, call, none); break;
+    default: hipLaunchKernelGGL((k_array_read_n<8, GATHER>), grid, block, 0, st, d, n_reqs, d_assignment, rounds, part, missed, n_words, wanted, sum, d_out, fin, call, none); break;
     }
     /* the later launches: as many words per wave as leave some eight thousand waves' worth of chunks */
     uint32_t words = 1;
@@ -1797,6 +2120,7 @@ int bam_array_read_shaped(bam_array_t* a, uint64_t n_reqs, const uint64_t* d_ass
     hipStream_t st = (hipStream_t)stream;
     /* a graph keeps the addresses it was recorded with and may be replayed beside other calls: it gets the shape that keeps no
      * notes between launches (the same sum), as does a call for whose notes there is no memory */
+    if (shape == BAM_READ_TWO_LAUNCHES && dealt_reads_pay(a, n_reqs, st) && dealt_reads<false>(a, n_reqs, d_assignment, (unsigned long long*)d_sum, nullptr, st)) return 0;
     if (shape == BAM_READ_TWO_LAUNCHES && !is_captured(st) && scattered_reads<false>(a, n_reqs, d_assignment, reads_per_lane, (unsigned long long*)d_sum, nullptr, st)) return 0;
     array_d_t<uint64_t>* d = a->a->d_array_ptr;
     unsigned long long* part = (unsigned long long*)a->partials.get();
@@ -1830,7 +2154,9 @@ int bam_array_read(bam_array_t* a, uint64_t n_reqs, const uint64_t* d_assignment
         return bam_array_read_shaped(a, n_reqs, d_assignment, shape, (uint32_t)lanes_env, block_size, d_sum, stream);
     }
     BAM_API_BEGIN
-    hipLaunchKernelGGL(k_array_read, dim3(blocks_for(n_reqs, block_size)), dim3(block_size), 0, (hipStream_t)stream,
+    if (d_assignment && reqs_per_thread == 1 && dealt_reads_pay(a, n_reqs, (hipStream_t)stream) && dealt_reads<false>(a, n_reqs, d_assignment, (unsigned long long*)d_sum, nullptr, (hipStream_t)stream)) return 0;
+    if (d_assignment && reqs_per_thread == 1 && few_reads_pay(a, n_reqs)) few_reads<false>(a, n_reqs, d_assignment, nullptr, (hipStream_t)stream);
+    else hipLaunchKernelGGL(k_array_read, dim3(blocks_for(n_reqs, block_size)), dim3(block_size), 0, (hipStream_t)stream,
                        a->a->d_array_ptr, n_reqs, d_assignment, stride, reqs_per_thread, (unsigned long long*)a->partials.get());
     hipLaunchKernelGGL(k_fold_partials, dim3(1), dim3(1024), 0, (hipStream_t)stream, (unsigned long long*)a->partials.get(), (unsigned long long*)d_sum);
     hip_err_chk(hipGetLastError());
@@ -1843,8 +2169,10 @@ int bam_array_gather(bam_array_t* a, uint64_t n_reqs, const uint64_t* d_assignme
     if (!block_size || block_size % BAM_WAVE_SIZE || block_size > 1024) return fail(EINVAL, "bam_array_gather: block size must be a multiple of 64, at most 1024");
     if (!n_reqs) return 0;
     BAM_API_BEGIN
+    if (d_assignment && dealt_reads_pay(a, n_reqs, (hipStream_t)stream) && dealt_reads<true>(a, n_reqs, d_assignment, nullptr, d_out, (hipStream_t)stream)) return 0;
     if (d_assignment && scattered_launches_pay(a, n_reqs, (hipStream_t)stream) && scattered_reads<true>(a, n_reqs, d_assignment, 8, nullptr, d_out, (hipStream_t)stream)) return 0;
-    hipLaunchKernelGGL(k_array_gather, dim3(blocks_for(n_reqs, block_size)), dim3(block_size), 0, (hipStream_t)stream,
+    if (d_assignment && few_reads_pay(a, n_reqs)) few_reads<true>(a, n_reqs, d_assignment, d_out, (hipStream_t)stream);
+    else hipLaunchKernelGGL(k_array_gather, dim3(blocks_for(n_reqs, block_size)), dim3(block_size), 0, (hipStream_t)stream,
                        a->a->d_array_ptr, n_reqs, d_assignment, stride, d_out);
     hip_err_chk(hipGetLastError());
     BAM_API_END

@@ -14,7 +14,8 @@
 #define BAM_SCRATCH_WORDS_BYTES (BAM_SUM_PARTIALS * sizeof(uint64_t) + 1024)
 
 /*
- * The bits of the requests a first launch leaves, a byte per page of the range that somebody waits for (zero between calls),
+ * The bits of the requests a first launch leaves, a byte per page of the range that somebody waits for
+ * or a count of its requests (zero between calls),
  * what the tiles of a scan tell each other (words that carry the number of their call), checksum shards and the count of finished
  * workgroups.
  */
@@ -32,6 +33,9 @@ struct scratch_set {
     /* how many pages a first launch has listed for the second, and which of them comes next: zero between calls, a line each */
     unsigned long long* listed() { return (unsigned long long*)(finished() + 160); }
     unsigned long long* next_chunk() { return (unsigned long long*)(finished() + 192); }
+    /* requests dealt out to their pages so far, and turns of pages taken: the first launch clears them */
+    uint32_t* cursor() { return finished() + 144; }
+    uint32_t* turns() { return finished() + 176; }
     /* the number of the next tile of a scan that draws them: zero between calls */
     uint32_t* next_tile() { return finished() + 208; }
     /* how many updates a slice has left for its last launch, by turns: the one's word is cleared by the other */

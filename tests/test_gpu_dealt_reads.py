@@ -1,0 +1,113 @@
+"""Scattered reads of arrays larger than their cache: requests put in order of their pages, and few requests spread over waves."""
+import numpy as np
+import pytest
+
+import oracle
+from test_gpu_parity import Rig, SEED, bam, _dev, _u64  # noqa: F401  (bam is the module fixture)
+
+pytestmark = pytest.mark.gpu
+
+
+def _check(a, n, idx, words, base=0, reps=2):
+    inside = idx - np.uint64(base) < len(words)
+    want = np.where(inside, words[np.where(inside, idx - np.uint64(base), 0).astype(np.int64)], 0).astype(np.uint64)
+    d = _dev(idx)
+    for rep in range(reps):
+        assert np.array_equal(_u64(a.gather(n, d)), want), rep
+        st = a.stats()
+        assert st["access_cnt"] == inside.sum() and st["hit_cnt"] + st["miss_cnt"] == st["access_cnt"], st
+        assert a.read(n, d) == int(np.sum(want, dtype=np.uint64)), rep
+        assert a.stats()["access_cnt"] == inside.sum()
+
+
+# caches of two pages up, turns of 4 pages to 1024, a range's last turn and its last 1024 pages cut short; requests: one, around a wave's
+# and where more are spread over each, on both sides of where they are put in order, more than one slice
+@pytest.mark.parametrize("page,pages,cache_pages", [(4096, 3, 2), (4096, 11, 8), (4096, 65, 17), (4096, 1025, 256), (8192, 1030, 515), (65536, 70, 20), (512, 2049, 700),
+                                                    (512, 70001, 17000), (4096, 4100, 3900)])
+def test_every_element(bam, page, pages, cache_pages):
+    n_elems = pages * page // 8 - 5
+    words = oracle.store(SEED, 0, n_elems)
+    rng = np.random.default_rng(pages)
+    line = pages + 2 * cache_pages
+    with Rig(bam, pages * page // 65536 * 65536 + 65536, n_queues=16, depth=256) as r:
+        a = r.array(n_elems, page, cache_pages)
+        for n in (1, 63, 65, 1023, line - 1, line, 4 * line + 1, (1 << 18) + 65):
+            idx = rng.integers(0, n_elems, n).astype(np.uint64)
+            idx[rng.integers(0, n, 3)] = np.array([n_elems, (1 << 64) - 1, 1 << 45], dtype=np.uint64)
+            _check(a, n, idx, words)
+        assert not r.c.aborted() and r.c.info()["error_completions"] == 0
+
+
+@pytest.mark.parametrize("kind", ["one element", "one page", "skewed", "in order", "backwards"])
+def test_orders_and_concentrations(bam, kind):
+    """cold each time: the requests for a page are as many as there are, and each page is read from the store once while half the cache holds what is asked for together"""
+    pages, cache_pages, n = 3000, 1000, 200001
+    n_elems = pages * 512 - 1
+    words = oracle.store(SEED, 0, n_elems)
+    rng = np.random.default_rng(3)
+    idx = {"one element": np.full(n, 77 * 512 + 5), "one page": 77 * 512 + rng.integers(0, 512, n), "skewed": rng.random(n) ** 6 * n_elems,
+           "in order": np.arange(n) * 7, "backwards": n_elems - 1 - np.arange(n) * 7}[kind].astype(np.uint64)
+    with Rig(bam, pages * 4096, n_queues=16, depth=256) as r:
+        a = r.array(n_elems, 4096, cache_pages)
+        assert np.array_equal(_u64(a.gather(n, _dev(idx))), words[idx.astype(np.int64)])
+        assert a.stats()["read_io_cnt"] == len(np.unique(idx // 512))
+        _check(a, n, idx, words)
+        assert not r.c.aborted()
+
+
+def test_more_requests_than_a_slice(bam):
+    pages, cache_pages, n = 2000, 700, (1 << 22) + 12345
+    words = oracle.store(SEED, 0, pages * 512)
+    with Rig(bam, pages * 4096, n_queues=16, depth=256) as r:
+        a = r.array(pages * 512, 4096, cache_pages)
+        _check(a, n, np.random.default_rng(1).integers(0, pages * 512, n).astype(np.uint64), words, reps=1)
+        assert not r.c.aborted()
+
+
+@pytest.mark.parametrize("page,offset,first", [(512, 0, 1000), (4096, 24, 0), (8192, 504, 777)])
+def test_ranges_that_begin_inside_a_page(bam, page, offset, first):
+    from bam_amd import Array, PageCache, Range
+    per, pages, cache_pages = page // 8, 600, 300
+    n_elems = (pages * page - offset) // 8 - 3
+    words = oracle.store(SEED, 3 * per + offset // 8, n_elems)
+    rng = np.random.default_rng(page)
+    with Rig(bam, (pages + 4) * page // 65536 * 65536 + 65536, n_queues=16, depth=256) as r:
+        pc = PageCache(page, cache_pages, 0, r.c)
+        rg = Range(first, first + n_elems, 3, pages, offset, page, pc, 0)
+        a = Array(first + n_elems, 0, [rg], 0)
+        for n in (100, 1199, 20000):
+            idx = (rng.integers(0, n_elems, n) + first).astype(np.uint64)
+            idx[:3] = np.array([(first - 1) % (1 << 64), first + n_elems, (1 << 64) - 1], dtype=np.uint64)
+            _check(a, n, idx, words, first)
+        assert not r.c.aborted()
+        a.close(); rg.close(); pc.close()
+
+
+def test_many_streams_and_arrays_of_one_cache(bam):
+    """Eight streams over two arrays behind one small cache: together they may hold no more than half of it."""
+    import torch
+    from bam_amd import Array, PageCache, Range
+    pages, n = 900, 9001
+    words = oracle.store(SEED, 0, 2 * pages * 512)
+    rng = np.random.default_rng(5)
+    with Rig(bam, 2 * pages * 4096, n_queues=16, depth=256) as r:
+        pc = PageCache(4096, 256, 0, r.c)
+        rgs = [Range(0, pages * 512, k * pages, pages, 0, 4096, pc, 0) for k in range(2)]
+        arrays = [Array(pages * 512, 0, [rg], 0) for rg in rgs]
+        reqs = [rng.integers(0, pages * 512, n).astype(np.uint64) for _ in range(8)]
+        d = [_dev(x) for x in reqs]
+        torch.cuda.synchronize()
+        streams = [torch.cuda.Stream() for _ in d]
+        outs = [[] for _ in d]
+        for rep in range(4):
+            for k, s in enumerate(streams):
+                with torch.cuda.stream(s):
+                    outs[k].append(arrays[k % 2].gather(n, d[k]))
+        torch.cuda.synchronize()
+        for k, x in enumerate(reqs):
+            for o in outs[k]:
+                assert np.array_equal(_u64(o), words[x.astype(np.int64) + k % 2 * pages * 512]), k
+        assert not r.c.aborted()
+        for a in arrays: a.close()
+        for rg in rgs: rg.close()
+        pc.close()
