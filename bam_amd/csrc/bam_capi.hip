@@ -995,6 +995,46 @@ __device__ __forceinline__ void stream_fetch_role(array_d_t<uint64_t>* dr, const
  * page side by side, array_d_t::seq_read_n); otherwise through bam_ptr per element.  DEFER: the page is read only if it is
  * resident; true (for the whole wave) if it was not, and then nothing of it is counted, neither in `v` nor in the views.
  */
+/*
+ * Eight rows of 64 elements from element `first` on, which begins a row of a page: the pages they lie in (stream_group_pages) are looked at, read and
+ * looked at again side by side, without references.  `seen`: the words of their descriptors, lane k the k-th's, as an earlier look found
+ * them; those of the eight rows from `next` on when the call returns.  False, with nothing added, where a page is not resident or did not
+ * stay.
+ *   Pages of 512 bytes one after the other are a chain of trips to memory for 512 bytes each.  1 GiB resident in such pages, one, four and 16
+ * to a wave, through operator[] 3188, 2064, 1766 -> 237 us, bam_ptr 2818, 908, 696 -> 209, page-wise 2120, 856, 514 -> 232; in pages of 4 and 8 KiB,
+ * operator[], which looks at a page's descriptor lane by lane for every eight elements, 325 -> 209 and 324 -> 197.  bam_ptr in pages of 4 KiB and more
+ * keeps to its own window, opened a page ahead: 202 us.
+ */
+__device__ __forceinline__ uint32_t stream_group_pages(const bam::range_view<uint64_t>& view) { return view.page_size < 4096 ? 4096u >> view.page_size_log : 1u; }
+__device__ __forceinline__ uint64_t stream_group_look(const bam::range_view<uint64_t>& view, const uint64_t first, const uint32_t lane)
+{
+    const uint32_t k = lane < stream_group_pages(view) ? lane : 0;
+    return __hip_atomic_load((const uint64_t*)(view.pages + (first * sizeof(uint64_t) >> view.page_size_log) + k), __ATOMIC_RELAXED, BAM_AGENT);
+}
+__device__ __forceinline__ bool stream_group(const bam::range_view<uint64_t>& view, const uint64_t first, const uint64_t next, const uint32_t lane, uint64_t& seen, uint64_t& v)
+{
+    const uint64_t was = seen;
+    if (bam::ballot(((uint32_t)was >> (CNT_SHIFT + 1)) != V_NB)) { seen = stream_group_look(view, next, lane); return false; }
+    const uint32_t slot = (uint32_t)(was >> 32) & BAM_SLOT_MASK, in_page = (uint32_t)(first * sizeof(uint64_t)) & (view.page_size - 1);
+    const uint64_t* at[8];
+#pragma unroll
+    for (uint32_t r = 0; r < 8; r++) {
+        const uint32_t byte = in_page + r * BAM_WAVE_SIZE * (uint32_t)sizeof(uint64_t);
+        at[r] = (const uint64_t*)(view.slot_addr(bam::bcast(slot, byte >> view.page_size_log)) + (byte & (view.page_size - 1))) + lane;
+    }
+    seen = stream_group_look(view, next, lane);
+    uint64_t x[8];
+    bam::ld_payload_nt(at, x);
+    if (bam::ballot(((stream_group_look(view, first, lane) ^ was) & 0xFFFFFFFFC0000000ull) != 0)) return false;
+    v += ((x[0] + x[1]) + (x[2] + x[3])) + ((x[4] + x[5]) + (x[6] + x[7]));
+    return true;
+}
+/* whether pages are read so: of a range whose first element is the first of a page */
+__device__ __forceinline__ bool stream_by_groups(const bam::range_view<uint64_t>& view)
+{
+    return view.page_size >= 512 && view.page_size < 4096 && view.index_start == 0 && view.pso == 0 && view.r->cache.fast_reads;
+}
+
 template <bool ELEM, bool DEFER, typename PTR>
 __device__ __forceinline__ bool stream_page(array_d_t<uint64_t>* dr, PTR& ptr, bam::range_view<uint64_t>& elem_view, const uint64_t first, const uint64_t epp,
                                             const uint32_t lane, uint64_t& v)
@@ -1060,11 +1100,11 @@ __device__ __forceinline__ bool stream_page(array_d_t<uint64_t>* dr, PTR& ptr, b
 }
 
 template <int MODE>
-__device__ __forceinline__ void cache_stream_body(array_d_t<uint64_t>* dr, uint64_t n_waves, uint64_t n_pages_per_wave, const uint64_t* assignment, unsigned long long* sum,
+__device__ __forceinline__ void cache_stream_body(array_d_t<uint64_t>* dr, uint64_t n_waves, uint64_t n_pages_per_wave_, const uint64_t total, const uint64_t* assignment, unsigned long long* sum,
                                                   const fetch_plan fp = fetch_plan{nullptr, 0, 0, 0, 0})
 {
     if (MODE >= 3 && fp.done && blockIdx.x < fp.blocks) {
-        stream_fetch_role(dr, n_waves, n_pages_per_wave, assignment, fp);
+        stream_fetch_role(dr, n_waves, n_pages_per_wave_, assignment, fp);
         return;
     }
     const uint64_t tid = (uint64_t)(blockIdx.x - (MODE >= 3 && fp.done ? fp.blocks : 0u)) * blockDim.x + threadIdx.x;
@@ -1072,9 +1112,10 @@ __device__ __forceinline__ void cache_stream_body(array_d_t<uint64_t>* dr, uint6
     const uint64_t wave = bam::first(tid / BAM_WAVE_SIZE), lane = tid % BAM_WAVE_SIZE;
     uint64_t v = 0;
     if (wave < n_waves) {
+        const uint64_t n_pages_per_wave = MODE == 2 && (wave + 1) * n_pages_per_wave_ > total ? total - wave * n_pages_per_wave_ : n_pages_per_wave_;
         range_d_t<uint64_t>* r0 = dr->d_ranges;
         const uint64_t epp = bam::first(r0->n_elems_per_page);
-        const uint64_t start_page = bam::first(assignment ? assignment[wave] : wave * n_pages_per_wave);
+        const uint64_t start_page = bam::first(assignment ? assignment[wave] : wave * n_pages_per_wave_);
         if (MODE == 2) {
             /*
              * Descriptor read once.  Pages are taken sixteen at a time: lane l of the wave asks for page l of the
@@ -1085,7 +1126,22 @@ __device__ __forceinline__ void cache_stream_body(array_d_t<uint64_t>* dr, uint6
             view.load(r0);
             const uint32_t n8 = view.page_size / 8;
             uint64_t a0 = 0, a1 = 0;
+            const bool by_groups = stream_by_groups(view);
+            const uint32_t group = by_groups ? stream_group_pages(view) : 1;
+            uint64_t seen = 0, seen_first = ~0ull;
             for (uint64_t p0 = 0; p0 < n_pages_per_wave; p0 += 16) {
+                if (by_groups) {
+                    const uint64_t first = (start_page + p0) * epp, next = first + 8 * BAM_WAVE_SIZE;
+                    if (p0 + group <= n_pages_per_wave && first < next && next <= view.index_end) {
+                        if (seen_first != first) seen = stream_group_look(view, first, lane);
+                        seen_first = next + 8 * BAM_WAVE_SIZE <= view.index_end ? next : first;
+                        if (stream_group(view, first, seen_first, lane, seen, a0)) {
+                            if (lane < group) view.account(true);
+                            p0 += (uint64_t)group - 16;           /* (the loop's 16 on top) */
+                            continue;
+                        }
+                    }
+                }
                 const uint32_t nb = (uint32_t)(n_pages_per_wave - p0 < 16 ? n_pages_per_wave - p0 : 16);
                 uint32_t slot = BAM_NO_SLOT;
                 const uint64_t page = view.page_of((start_page + p0 + (lane < nb ? lane : 0)) * epp);
@@ -1152,29 +1208,30 @@ __device__ __forceinline__ void cache_stream_body(array_d_t<uint64_t>* dr, uint6
 template <int MODE>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MODE == 1 ? 4 : 1))) void k_cache_stream_whole(array_d_t<uint64_t>* dr, uint64_t n_waves, uint64_t n_pages_per_wave, const uint64_t* assignment, unsigned long long* sum)
 {
-    cache_stream_body<MODE>(dr, n_waves, n_pages_per_wave, assignment, sum);
+    cache_stream_body<MODE>(dr, n_waves, n_pages_per_wave, n_waves * n_pages_per_wave, assignment, sum);
 }
 /* modes 3 and 4 with fetch waves at the front of the grid */
 template <int MODE>
 __global__ __launch_bounds__(256) void k_cache_stream_fetched(array_d_t<uint64_t>* dr, uint64_t n_waves, uint64_t n_pages_per_wave, const uint64_t* assignment, unsigned long long* sum,
                                                              const fetch_plan fp)
 {
-    cache_stream_body<MODE>(dr, n_waves, n_pages_per_wave, assignment, sum, fp);
+    cache_stream_body<MODE>(dr, n_waves, n_pages_per_wave, n_waves * n_pages_per_wave, assignment, sum, fp);
 }
-__global__ __launch_bounds__(256) void k_cache_stream_pages(array_d_t<uint64_t>* dr, uint64_t n_waves, uint64_t n_pages_per_wave, const uint64_t* assignment, unsigned long long* sum)
+__global__ __launch_bounds__(256) void k_cache_stream_pages(array_d_t<uint64_t>* dr, uint64_t n_waves, uint64_t n_pages_per_wave, const uint64_t total, const uint64_t* assignment, unsigned long long* sum)
 {
-    cache_stream_body<2>(dr, n_waves, n_pages_per_wave, assignment, sum);
+    cache_stream_body<2>(dr, n_waves, n_pages_per_wave, total, assignment, sum);
 }
 
 /*
- * Modes 0 and 1 in two launches (arrays of one range).  The first, this kernel, is the reference's kernel
+ * Modes 0 and 1 in two launches (arrays of one range).  GROUPS: eight rows at a time as long as their pages are resident
+ * (stream_group), page by page otherwise.  The first, this kernel, is the reference's kernel
  * (benchmarks/cache/main.cu:44-114: a wave per run of pages, every element through bam_ptr or operator[]) with pointers
  * that do not load: a page that is not resident is noted in deferred[wave * n_pages_per_wave + p] and left to the second
  * launch (k_cache_stream_deferred), which has the miss path.  A kernel that can miss carries the registers and the stack of
  * the miss path through every page visit (four waves per SIMD, a frame in scratch memory); this one has neither.
  */
-template <int MODE>
-__global__ __launch_bounds__(256) void k_cache_stream(array_d_t<uint64_t>* dr, uint64_t n_waves, uint64_t n_pages_per_wave, const uint64_t* assignment, unsigned long long* partials,
+template <int MODE, bool GROUPS>
+__global__ __launch_bounds__(256) void k_cache_stream(array_d_t<uint64_t>* dr, uint64_t n_waves, uint64_t run_pages, const uint64_t total, const uint64_t* assignment, unsigned long long* partials,
                                                       uint8_t* deferred, unsigned long long* sum, uint32_t* finished, uint32_t call)
 {
     static_assert(MODE == 0 || MODE == 1, "the page-wise mode and the fetching modes are kernels of their own");
@@ -1183,19 +1240,49 @@ __global__ __launch_bounds__(256) void k_cache_stream(array_d_t<uint64_t>* dr, u
     const uint32_t lane = bam::lane();
     uint64_t v = 0;
     if (wave < n_waves) {
+        const uint64_t n_pages_per_wave = (wave + 1) * run_pages > total ? total - wave * run_pages : run_pages;
         range_d_t<uint64_t>* r0 = dr->d_ranges;
         const uint64_t epp = bam::first(r0->n_elems_per_page);
-        const uint64_t start_page = bam::first(assignment ? assignment[wave] : wave * n_pages_per_wave);
+        const uint64_t start_page = bam::first(assignment ? assignment[wave] : wave * run_pages);
         bam_ptr<uint64_t, true> ptr(dr);
         bam::range_view<uint64_t> elem_view;
-        if (MODE == 0) elem_view.load(r0);
+        if (MODE == 0 || GROUPS) elem_view.load(r0);
         uint64_t later = 0;                 /* bit p % 64: page p is left to the second launch (the same in every lane) */
+        uint64_t seen = 0, seen_first = ~0ull;
         for (uint64_t p = 0; p < n_pages_per_wave; p++) {
+            if constexpr (GROUPS) {
+                constexpr uint64_t rows8 = 8 * BAM_WAVE_SIZE;
+                const uint32_t pages = stream_group_pages(elem_view);
+                const uint64_t first = (start_page + p) * epp, last = first + (epp < rows8 ? rows8 : epp), end = elem_view.index_end;
+                if (p % pages == 0 && p + pages <= n_pages_per_wave && first < last && last <= end) {
+                    if (seen_first != first) seen = stream_group_look(elem_view, first, lane);
+                    uint64_t sum = 0, at = first;
+                    for (bool good = true; good && at < last; at += rows8) {
+                        seen_first = at + 2 * rows8 <= end ? at + rows8 : first;
+                        good = stream_group(elem_view, at, seen_first, lane, seen, sum);
+                        if (!good) at = last;           /* (ends behind `last`) */
+                    }
+                    if (at == last) {
+                        v += sum;
+                        /* as page after page counts: operator[] every element, a pointer the page, lane by lane */
+                        const uint32_t counted = MODE == 0 ? (uint32_t)((last - first) / BAM_WAVE_SIZE) : pages;
+                        elem_view.n_access += counted; elem_view.n_hit += counted;
+                        p += pages - 1;
+                        if ((p & 63u) == 63u || p + 1 == n_pages_per_wave) {
+                            const uint64_t from = p & ~63ull;
+                            if (from + lane <= p) deferred[wave * run_pages + from + lane] = (uint8_t)((later >> lane) & 1u);
+                            if (later) note_work_left(finished, call);
+                            later = 0;
+                        }
+                        continue;
+                    }
+                }
+            }
             if (stream_page<MODE == 0, true>(dr, ptr, elem_view, (start_page + p) * epp, epp, lane, v)) later |= 1ull << (p & 63u);
             if ((p & 63u) == 63u || p + 1 == n_pages_per_wave) {
                 /* the notes of up to 64 pages with one store, a byte per lane */
                 const uint64_t first = p & ~63ull;
-                if (first + lane <= p) deferred[wave * n_pages_per_wave + first + lane] = (uint8_t)((later >> lane) & 1u);
+                if (first + lane <= p) deferred[wave * run_pages + first + lane] = (uint8_t)((later >> lane) & 1u);
                 if (later) note_work_left(finished, call);
                 later = 0;
             }
@@ -2332,18 +2419,33 @@ int bam_cache_stream(bam_array_t* a, uint64_t n_waves, uint64_t n_pages_per_wave
     if (!n_waves || !n_pages_per_wave) return 0;
     BAM_API_BEGIN
     const uint32_t bs = 256;
-    const dim3 grid(blocks_for(n_waves * BAM_WAVE_SIZE, bs)), block(bs);
+    const range_d_t<uint64_t>& r = a->a->h_ranges[0];
+    const uint64_t total = n_waves * n_pages_per_wave, unit = r.cache.page_size < 4096 ? 4096 / r.cache.page_size : 1;
+    /*
+     * Where the runs follow one another the pages may be shared out to other runs: of up to 64 KiB, as many as leave 4096 waves something, 4 KiB
+     * at least.  1 GiB resident in pages of 4 KiB, a page, four and 16 to a wave, through bam_ptr 390, 217, 202 us; 8 MiB, four and 16, 36, 46; 128 MiB
+     * 59, 61.  Pages in batches (mode 2) are held while others are waited for: only where the cache has room for all of them.
+     */
+    uint64_t run_waves = n_waves, run_pages = n_pages_per_wave;
+    if (!d_assignment && mode <= 2 && a->a->adt.n_ranges == 1 && n_waves < 1ull << 32 && n_pages_per_wave < 1ull << 32 && (mode < 2 || (total <= r.cache.n_pages && r.page_count <= r.cache.n_pages))) {
+        run_pages = 16 * unit;
+        while (run_pages > unit && total / run_pages < 4096) run_pages /= 2;
+        run_waves = (total + run_pages - 1) / run_pages;
+    }
+    const dim3 grid(blocks_for(n_waves * BAM_WAVE_SIZE, bs)), block(bs), grid_runs(blocks_for(run_waves * BAM_WAVE_SIZE, bs));
     array_d_t<uint64_t>* d = a->a->d_array_ptr;
     unsigned long long* s = (unsigned long long*)a->partials.get();
     if (mode <= 1 && two_launches_ok(a)) {
         /* the kernel that reads what is resident, then the one that reads what it noted (and folds the checksum) */
-        const uint64_t total = n_waves * n_pages_per_wave;
         uint8_t* notes = (uint8_t*)a->notes_for(total);
         unsigned long long* sum = (unsigned long long*)d_sum;
         uint32_t* fin = (uint32_t*)a->finished.get();
         const uint32_t call = a->next_call();
-        if (mode == 0) hipLaunchKernelGGL(k_cache_stream<0>, grid, block, 0, (hipStream_t)stream, d, n_waves, n_pages_per_wave, d_assignment, s, notes, sum, fin, call);
-        else hipLaunchKernelGGL(k_cache_stream<1>, grid, block, 0, (hipStream_t)stream, d, n_waves, n_pages_per_wave, d_assignment, s, notes, sum, fin, call);
+        const bool groups = (mode == 0 || unit > 1) && r.cache.page_size >= 512 && r.index_start == 0 && r.page_start_offset == 0 && run_pages >= unit;
+        if (mode == 0 && groups) hipLaunchKernelGGL((k_cache_stream<0, true>), grid_runs, block, 0, (hipStream_t)stream, d, run_waves, run_pages, total, d_assignment, s, notes, sum, fin, call);
+        else if (groups) hipLaunchKernelGGL((k_cache_stream<1, true>), grid_runs, block, 0, (hipStream_t)stream, d, run_waves, run_pages, total, d_assignment, s, notes, sum, fin, call);
+        else if (mode == 0) hipLaunchKernelGGL((k_cache_stream<0, false>), grid_runs, block, 0, (hipStream_t)stream, d, run_waves, run_pages, total, d_assignment, s, notes, sum, fin, call);
+        else hipLaunchKernelGGL((k_cache_stream<1, false>), grid_runs, block, 0, (hipStream_t)stream, d, run_waves, run_pages, total, d_assignment, s, notes, sum, fin, call);
         const uint64_t n_chunks = (total + BAM_WAVE_SIZE - 1) / BAM_WAVE_SIZE;
         const dim3 grid2(blocks_for((n_chunks < 1024 ? n_chunks : 1024) * BAM_WAVE_SIZE, bs));      /* a thousand waves with 64 pages each keep the store busy; when nothing was noted the fewer the better */
         if (mode == 0) hipLaunchKernelGGL(k_cache_stream_deferred<0>, grid2, block, 0, (hipStream_t)stream, d, n_waves, n_pages_per_wave, d_assignment, s, notes, sum, fin, call);
@@ -2361,7 +2463,7 @@ int bam_cache_stream(bam_array_t* a, uint64_t n_waves, uint64_t n_pages_per_wave
         if (mode == 3) hipLaunchKernelGGL(k_cache_stream_fetched<3>, grid_f, block, 0, (hipStream_t)stream, d, n_waves, n_pages_per_wave, d_assignment, s, fp);
         else hipLaunchKernelGGL(k_cache_stream_fetched<4>, grid_f, block, 0, (hipStream_t)stream, d, n_waves, n_pages_per_wave, d_assignment, s, fp);
     }
-    else hipLaunchKernelGGL(k_cache_stream_pages, grid, block, 0, (hipStream_t)stream, d, n_waves, n_pages_per_wave, d_assignment, s);
+    else hipLaunchKernelGGL(k_cache_stream_pages, grid_runs, block, 0, (hipStream_t)stream, d, run_waves, run_pages, total, d_assignment, s);
     hipLaunchKernelGGL(k_fold_partials, dim3(1), dim3(1024), 0, (hipStream_t)stream, s, (unsigned long long*)d_sum);
     hip_err_chk(hipGetLastError());
     BAM_API_END

@@ -164,7 +164,8 @@ int bam_sqe_image(uint16_t cid, uint8_t opcode, uint32_t nsid, uint64_t prp1, ui
                   uint32_t* host_out16, uint32_t* d_out64x16, void* stream);
 
 /* ---- cache / pattern benchmark kernels (benchmarks/cache/main.cu:44-114, benchmarks/pattern/main.cu:105-170) ----
- * One wave per run of n_pages_per_wave whole pages starting at page d_assignment[w] (or w * n_pages_per_wave),
+ * One wave per run of n_pages_per_wave whole pages starting at page d_assignment[w] (or w * n_pages_per_wave: then
+ * modes 0 to 2 may share the same pages out to runs of another length),
  * every element read once and summed into *d_sum.  mode 0: array_d_t::operator[] per element,
  * mode 1: bam_ptr per element (the reference's kernel, 64-wide), mode 2: one acquire per page and
  * streamed 8-byte loads; modes 3 and 4: modes 1 and 0 for data that is not
