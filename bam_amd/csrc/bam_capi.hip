@@ -951,8 +951,10 @@ __device__ __attribute__((noinline)) void stream_touch(range_d_t<uint64_t>* r, c
     view.load(r);
     auto touch = [](uint32_t) { return true; };
     const uint64_t lane = bam::lane(), epp = r->n_elems_per_page;
-    const uint64_t page = view.page_of((first + (lane < n ? lane : 0)) * epp);
-    const bool take = lane < n && page_absent(view, page);
+    const uint64_t elem = (first + (lane < n ? lane : 0)) * epp;
+    const bool in = lane < n && view.holds(elem);           /* in front of the range and behind it there are no descriptors */
+    const uint64_t page = view.page_of(in ? elem : view.index_start);
+    const bool take = in && page_absent(view, page);
     if (bam::ballot(take)) view.template acquire_helped<true>(page, take, false, touch, touch);
     view.n_access = view.n_hit = 0;
 }
@@ -981,8 +983,8 @@ __device__ __forceinline__ void stream_fetch_role(array_d_t<uint64_t>* dr, const
         const uint64_t at = b * BAM_WAVE_SIZE + bam::lane();
         const uint64_t cw = at < total ? at / ppw : 0;
         const uint64_t elem = ((assignment ? assignment[cw] : cw * ppw) + at % ppw) * epp;
-        const bool in = at < total && elem < dr->n_elems;
-        const uint64_t page = view.page_of(in ? elem : 0);
+        const bool in = at < total && view.holds(elem);
+        const uint64_t page = view.page_of(in ? elem : view.index_start);
         const bool take = in && page_absent(view, page);
         if (bam::ballot(take)) view.acquire_helped(page, take, false, touch, touch);
         view.n_access = view.n_hit = 0;
@@ -1324,8 +1326,8 @@ __global__ __launch_bounds__(256) void k_cache_stream_deferred(array_d_t<uint64_
             view.load(r0);
             const uint32_t reach = (uint32_t)(r0->cache.n_pages >> 6 > BAM_WAVE_SIZE ? BAM_WAVE_SIZE : r0->cache.n_pages >> 6);
             auto touch = [](uint32_t) { return true; };
-            const bool in = noted && page * epp < dr->n_elems;
-            const uint64_t pg = view.page_of(in ? page * epp : 0);
+            const bool in = noted && view.holds(page * epp);
+            const uint64_t pg = view.page_of(in ? page * epp : view.index_start);
             const bool absent = in && page_absent(view, pg);
             if (reach >= 2)
                 for (uint32_t b = 0; b < BAM_WAVE_SIZE; b += reach) {

@@ -55,3 +55,22 @@ def test_a_run_far_outside_is_not_read(bam):
         for mode in (0, 1):
             assert a.stream(3, 1, _dev(starts), mode=mode) == 0
         assert not r.c.aborted()
+
+
+@pytest.mark.parametrize("page,offset,first", [(512, 0, 1000), (1024, 24, 0)])
+def test_ranges_that_begin_elsewhere(bam, page, offset, first):
+    """page by page there; elements in front of the range read as 0 and nobody looks for their pages"""
+    from bam_amd import Array, PageCache, Range
+    pages = 300
+    n_elems = (pages * page - offset) // 8
+    with Rig(bam, (pages + 8) * page // 65536 * 65536 + 65536, n_queues=8, depth=256) as r:
+        pc = PageCache(page, pages, 0, r.c)
+        rg = Range(first, first + n_elems, 0, pages, offset, page, pc, 0)
+        a = Array(first + n_elems, 0, [rg], 0)
+        words = oracle.store(SEED, offset // 8, n_elems)
+        want = int(np.sum(words[:210 * page // 8 - first], dtype=np.uint64))
+        for mode in (5, 6, 0, 1, 3, 4):
+            for rep in range(2):
+                assert a.stream(30, 7, mode=mode) == want, (mode, rep)
+        assert not r.c.aborted()
+        a.close(); rg.close(); pc.close()
