@@ -576,6 +576,8 @@ __device__ __forceinline__ void cc_join_trees(unsigned long long* comp, unsigned
     u = cc_root(comp, u); v = cc_root(comp, v);
     while (u != v) {
         if (u < v) { const unsigned long long t = u; u = v; v = t; }
+        /* one lane of those that would exchange the same root's word as the first: exchanges on one address are performed one after the other */
+        if (u == bam::first((uint64_t)u) && bam::lane() != bam::first_lane(bam::active_mask())) { u = cc_root(comp, u); continue; }
         const unsigned long long was = atomicCAS(comp + u, u, v);
         if (was == u) break;
         u = cc_root(comp, was);
@@ -604,6 +606,62 @@ __global__ void k_cc_shorten(unsigned long long* comp, uint64_t vertex_count)
         bam::st_relaxed(comp + v, upper);
         up = upper;
     }
+}
+/*
+ * The forest that the joins begin with, from the first BAM_CC_FIRST neighbours of lists, as far as those lie in one page that is resident.  First
+ * (ROUND false, all vertices) each vertex is put under the smallest of its own, if that is smaller than itself: no exchange, and no
+ * tree that another wave is joining meanwhile.  Then, with trees shortened (k_cc_shorten), rounds over every `each`-th vertex point the
+ * larger root of an entry's two ends at the smaller one, by a minimum that nobody waits for: of several for one root the smallest stays, and
+ * what the others would have joined is joined when the edges are read, as all are.  What makes a reading of the edges slow is
+ * that most of them meet on a few roots which are being joined, each exchange waiting for the others on its word; with nearly all of a component
+ * under one root before it begins, both ends of most name that.
+ *   Uniform random graphs, 8 entries a vertex, all cached, medians in us of two graphs before, with one launch of the first kind and with three rounds: 2^14 vertices 99 149, 158, 76
+ * 74; 2^16 237 269, 378, 92 93; 2^17 670 406, 890, 121 111; 2^18 378 605, 638, 154 161; 2^19 362 885, 635, 254 258; 2^20 399 560, 606, 369 371; half
+ * cached 2^19 819 1349, 901, 653 655, 2^22 3950 3788, 4042, 3806 3806, within 1 % from call to call instead of 20.  From 2^21 vertices on, all cached, two
+ * rounds: 620 840 -> 577 575 (three 630 628), 2^22 1198 1124 -> 1116 1146.  Power-law 2^16, 2^18, 2^20 126, 217, 559 -> 73, 137, 381; grids of
+ * 64 x 4096, 1024 x 1024, 2048 x 2048 454, 825, 902 -> 77, 184, 525; a path of 2^21 723 -> 281.  Rounds over all vertices: 2^17 229, 2^22 1535.
+ */
+#define BAM_CC_FIRST 4
+template <bool ROUND>
+__global__ __launch_bounds__(256) void k_cc_begin(array_d_t<uint64_t>* da, const uint64_t* offsets, const uint64_t n_vertices, unsigned long long* comp, const uint32_t each)
+{
+    const uint64_t v = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) * (ROUND ? each : 1u);
+    bam::range_view<uint64_t> view;
+    view.load(da->d_ranges);
+    if (v >= n_vertices) return;
+    const uint64_t e = offsets[v], end = offsets[v + 1];
+    unsigned long long up = ROUND ? bam::ld_relaxed(comp + v) : v;
+    if (e < end && end <= view.index_end) {
+        const uint64_t byte = view.byte_of(e);
+        const uint32_t in_page = (uint32_t)byte & (view.page_size - 1), here = (view.page_size - in_page) / (uint32_t)sizeof(uint64_t);
+        const uint32_t n = end - e < here ? (uint32_t)(end - e) : here;
+        const data_page_t* const dp = view.pages + (byte >> view.page_size_log);
+        const uint64_t was = __hip_atomic_load((const uint64_t*)dp, __ATOMIC_RELAXED, BAM_AGENT);
+        if (((uint32_t)was >> (CNT_SHIFT + 1)) == V_NB) {
+            const uint64_t* at[BAM_CC_FIRST];
+            uint64_t x[BAM_CC_FIRST];
+            /* (the first entry again where there are fewer) */
+#pragma unroll
+            for (uint32_t j = 0; j < BAM_CC_FIRST; j++) at[j] = (const uint64_t*)(view.slot_addr((uint32_t)(was >> 32) & BAM_SLOT_MASK) + in_page) + (j < n ? j : 0);
+            bam::ld_payload_nt(at, x);
+            if (((__hip_atomic_load((const uint64_t*)dp, __ATOMIC_RELAXED, BAM_AGENT) ^ was) & 0xFFFFFFFFC0000000ull) == 0) {
+                if constexpr (!ROUND) {
+#pragma unroll
+                    for (uint32_t j = 0; j < BAM_CC_FIRST; j++) up = x[j] < up ? x[j] : up;
+                } else {
+                    unsigned long long high[BAM_CC_FIRST], low[BAM_CC_FIRST];
+#pragma unroll
+                    for (uint32_t j = 0; j < BAM_CC_FIRST; j++) high[j] = bam::ld_relaxed(comp + x[j]);
+#pragma unroll
+                    for (uint32_t j = 0; j < BAM_CC_FIRST; j++) { low[j] = high[j] < up ? high[j] : up; high[j] = high[j] < up ? up : high[j]; }
+#pragma unroll
+                    for (uint32_t j = 0; j < BAM_CC_FIRST; j++)
+                        if (low[j] != high[j] && bam::ld_relaxed(comp + high[j]) > low[j]) __hip_atomic_fetch_min(comp + high[j], low[j], __ATOMIC_RELAXED, BAM_AGENT);
+                }
+            }
+        }
+    }
+    if constexpr (!ROUND) bam::st_relaxed(comp + v, up);
 }
 /* n_missing, next_chunk: along_t's, of the reading before, which are zero between sweeps (NULL: it had none) */
 __global__ void k_cc_settle(unsigned long long* comp, uint64_t vertex_count, unsigned long long* n_missing, unsigned long long* next_chunk)
@@ -1646,6 +1704,20 @@ uint32_t bfs_along_levels(bam_array_t* edges, graph_plan* pl, uint32_t* d_labels
     }
 }
 
+/* the forest that cc_read_edges begins with: k_cc_begin, for the arrays whose pages are read along (elsewhere every vertex by itself) */
+void cc_begin(bam_array_t* edges, graph_plan* pl, unsigned long long* comp, hipStream_t st)
+{
+    const uint64_t nv = pl->n_vertices;
+    if (!pl->along.n_segs) { hipLaunchKernelGGL(k_iota, dim3(blocks_for(nv, 256)), dim3(256), 0, st, comp, nv); return; }
+    const bool large = pl->all_cached && nv >= 1ull << 21;
+    hipLaunchKernelGGL(k_cc_begin<false>, dim3(blocks_for(nv, 256)), dim3(256), 0, st, edges->a->d_array_ptr, pl->offsets, nv, comp, 1u);
+    hipLaunchKernelGGL(k_cc_shorten, dim3(blocks_for(nv, 256)), dim3(256), 0, st, comp, nv);
+    for (uint32_t round = large ? 1 : 0; round < 3; round++) {
+        const uint32_t each = round < 2 ? 4 : 8;
+        hipLaunchKernelGGL(k_cc_begin<true>, dim3(blocks_for((nv + each - 1) / each, 256)), dim3(256), 0, st, edges->a->d_array_ptr, pl->offsets, nv, comp, each);
+        hipLaunchKernelGGL(k_cc_shorten, dim3(blocks_for(nv, 256)), dim3(256), 0, st, comp, nv);
+    }
+}
 /* one reading of the edges that joins the trees of their ends.  In one launch where all are cached and few: 2^15 entries take 80 us, in two
  * 88 (in pages of 512 and 1024 bytes, which that launch goes over one after the other, 271 and 144, and 85); but that one goes over
  * the vertices between the lists of a page, so not where there may be many.  By page (bam_cc_by_page), in pages of less than 4 KiB, also where
@@ -1898,11 +1970,12 @@ int bam_cc(bam_array_t* edges, const uint64_t* d_offsets, uint64_t n_vertices, u
     const uint64_t group = coarse > 512 ? coarse : 512;
     unsigned long long* comp = (unsigned long long*)d_labels;
     const bool along = pl->along_edges(edges, st, false);
-    hipLaunchKernelGGL(k_iota, dim3(blocks_for(n_vertices, 256)), dim3(256), 0, st, comp, n_vertices);
-    if (along) cc_read_edges(edges, pl, comp, st, false);
-    else
+    if (along) { cc_begin(edges, pl, comp, st); cc_read_edges(edges, pl, comp, st, false); }
+    else {
+        hipLaunchKernelGGL(k_iota, dim3(blocks_for(n_vertices, 256)), dim3(256), 0, st, comp, n_vertices);
         hipLaunchKernelGGL(k_cc_coalesce_coarse_ptr_pc, dim3(pl->blocks(n_vertices, group)), dim3(128), 0, st, edges->a->d_array_ptr, n_vertices, d_offsets, comp, group,
                        pl->pieces, pl->n_pieces, pl->next_work(), pl->cc_backwards());
+    }
     hipLaunchKernelGGL(k_cc_settle, dim3(blocks_for(n_vertices, 256)), dim3(256), 0, st, comp, n_vertices, pl->along.n_missing, pl->along.next_chunk);
     hip_err_chk(hipGetLastError());
     if (along) { hip_err_chk(hipStreamSynchronize(st)); }
@@ -1953,7 +2026,6 @@ int bam_cc_by_page(bam_array_t* edges, const uint64_t* d_offsets, uint64_t n_ver
     if (int rc = pl->by_page(edges, st)) return rc;
     pl->along_edges(edges, st, false);
     unsigned long long* comp = (unsigned long long*)d_labels;
-    hipLaunchKernelGGL(k_iota, dim3(blocks_for(n_vertices, 256)), dim3(256), 0, st, comp, n_vertices);
     uint32_t iter = 0;
     bool changed = true;
     /*
@@ -1968,6 +2040,7 @@ int bam_cc_by_page(bam_array_t* edges, const uint64_t* d_offsets, uint64_t n_ver
     if (pl->bp.n_pages && pl->all_cached && pl->bp.n_edges > (1ull << 17) && pl->bp.n_edges < (1ull << 22)) {
         bool* curr = (bool*)graph_plan::sized(pl->bytes_a, n_vertices);
         bool* next = (bool*)graph_plan::sized(pl->bytes_b, n_vertices);
+        hipLaunchKernelGGL(k_iota, dim3(blocks_for(n_vertices, 256)), dim3(256), 0, st, comp, n_vertices);
         hip_err_chk(hipMemsetAsync(curr, 0x01, n_vertices, st));
         hip_err_chk(hipMemsetAsync(next, 0x00, n_vertices, st));
         while (changed && iter < 6) {
@@ -1982,6 +2055,7 @@ int bam_cc_by_page(bam_array_t* edges, const uint64_t* d_offsets, uint64_t n_ver
     }
     if (changed) {
         if (iter) hipLaunchKernelGGL(k_cc_shorten, dim3(blocks_for(n_vertices, 256)), dim3(256), 0, st, comp, n_vertices);
+        else cc_begin(edges, pl, comp, st);
         cc_read_edges(edges, pl, comp, st, true);
         hipLaunchKernelGGL(k_cc_settle, dim3(blocks_for(n_vertices, 256)), dim3(256), 0, st, comp, n_vertices, pl->along.n_missing, pl->along.next_chunk);
         hip_err_chk(hipGetLastError());
