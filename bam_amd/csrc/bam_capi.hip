@@ -77,6 +77,33 @@ __global__ void k_array_read(array_d_t<uint64_t>* dr, uint64_t n_reqs, const uin
     block_accumulate(sum, v);
 }
 
+/* a workgroup's values into the launch's checksum: `sum` itself where few workgroups do, else the shards that k_fold_partials folds */
+__device__ __forceinline__ void workgroup_accumulate(unsigned long long* partials, unsigned long long* sum, uint64_t v)
+{
+    __shared__ unsigned long long total;
+    if (threadIdx.x == 0) total = 0;
+    __syncthreads();
+    v = wave_sum(v);
+    if (bam::lane() == 0 && v) atomicAdd(&total, (unsigned long long)v);
+    __syncthreads();
+    if (threadIdx.x == 0 && total) atomicAdd(sum ? sum : &partials[(blockIdx.x * 0x9E3779B1u) >> 20], total);
+}
+/*
+ * The same for requests of an array that fits its cache, a read to a thread, as long as one launch answers them sooner than two
+ * (bam_array_read).  Bound by the launches and the sum's way to the host: with sums added up by wave, folded by a launch of its own (two launches from
+ * 2^16 requests on), and here, us a call that waits for its sum, 16 million elements in pages of 4 KiB: 1000 reads 25.6 and 22.6, 60000 26.2 and 23.9, 65536 37.9 and
+ * 24.0, 300000 41.5 and 34.2, 2^20 57.1 and 51.7.  (Cold, 2^18 and 2^20 of them 3.17 and 3.15 ms, 3.33 and 3.23.)
+ */
+#define BAM_DIRECT_GROUPS 128u       /* as many workgroups add to the sum themselves: 256 as well as a launch that folds takes (27.0 and 27.4 us), 600 longer (35.7 and 34.2) */
+#define BAM_READ_EACH_THREADS 512u
+__global__ __launch_bounds__(BAM_READ_EACH_THREADS) void k_array_read_each(array_d_t<uint64_t>* dr, uint64_t n_reqs, const uint64_t* __restrict__ assignment, unsigned long long* partials, unsigned long long* sum)
+{
+    const uint64_t tid = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    uint64_t v = 0;
+    if (tid < n_reqs) v = (*dr)[assignment[tid]];
+    workgroup_accumulate(partials, sum, v);
+}
+
 /* the same sum for a launch of scattered requests, BAM_READS_PER_LANE of them per thread a quarter of the launch apart
  * (request t + j * threads for j = 0 .. 3), read side by side (array_d_t::seq_read_n): what the lanes of a wave ask for
  * together is as scattered as with one request per thread, and each lane keeps four requests in flight instead of one */
@@ -519,7 +546,7 @@ __global__ __launch_bounds__(64) void k_reads_fetch(array_d_t<uint64_t>* dr, con
  * requests, 185 and 66; all resident 6 to 7 us either way.
  */
 template <bool GATHER>
-__global__ __launch_bounds__(256) void k_array_read_few(array_d_t<uint64_t>* dr, uint64_t n_reqs, const uint64_t* __restrict__ assignment, uint32_t each, unsigned long long* partials, uint64_t* out_list)
+__global__ __launch_bounds__(256) void k_array_read_few(array_d_t<uint64_t>* dr, uint64_t n_reqs, const uint64_t* __restrict__ assignment, uint32_t each, unsigned long long* partials, unsigned long long* sum, uint64_t* out_list)
 {
     const uint32_t lane = bam::lane();
     const uint64_t t = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) / BAM_WAVE_SIZE * each + lane;
@@ -538,7 +565,7 @@ __global__ __launch_bounds__(256) void k_array_read_few(array_d_t<uint64_t>* dr,
         view.acquire_helped(byte >> view.page_size_log, absent, false, use, use);
     }
     if constexpr (GATHER) { if (mine) out_list[t] = x[0]; }
-    else block_accumulate(partials, mine ? x[0] : 0);
+    else workgroup_accumulate(partials, sum, mine ? x[0] : 0);
     view.template flush_stats<false>();
 }
 
@@ -2053,13 +2080,16 @@ bool few_reads_pay(bam_array_t* a, uint64_t n_reqs)
     return two_launches_ok(a) && range.page_count > range.cache.n_pages && n_reqs <= BAM_REQS_AT_A_TIME;
 }
 template <bool GATHER>
-void few_reads(bam_array_t* a, uint64_t n_reqs, const uint64_t* d_assignment, uint64_t* d_out, hipStream_t st)
+void few_reads(bam_array_t* a, uint64_t n_reqs, const uint64_t* d_assignment, unsigned long long* sum, uint64_t* d_out, hipStream_t st)
 {
+    unsigned long long* const part = (unsigned long long*)a->partials.get();
     const uint64_t least = std::min<uint64_t>(256, (1ull << 20) / a->a->h_ranges[0].cache.page_size);
     uint32_t each = BAM_WAVE_SIZE;
     while (each > 4 && n_reqs / each < least) each /= 2;
-    hipLaunchKernelGGL(k_array_read_few<GATHER>, dim3(blocks_for((n_reqs + each - 1) / each * BAM_WAVE_SIZE, 256)), dim3(256), 0, st, a->a->d_array_ptr, n_reqs, d_assignment, each,
-                       (unsigned long long*)a->partials.get(), d_out);
+    const uint32_t groups = blocks_for((n_reqs + each - 1) / each * BAM_WAVE_SIZE, 256);
+    const bool fold = !GATHER && groups > BAM_DIRECT_GROUPS;
+    hipLaunchKernelGGL(k_array_read_few<GATHER>, dim3(groups), dim3(256), 0, st, a->a->d_array_ptr, n_reqs, d_assignment, each, part, fold ? nullptr : sum, d_out);
+    if (fold) hipLaunchKernelGGL(k_fold_partials, dim3(1), dim3(1024), 0, st, part, sum);
 }
 /*
  * Whether requests are put in order of their pages: where there are more than one for each page and two for each slot (below, few of them
@@ -2192,6 +2222,29 @@ bool scattered_reads(bam_array_t* a, uint64_t n_reqs, const uint64_t* d_assignme
     hip_err_chk(hipGetLastError());
     return true;
 }
+/* the sum of scattered reads of an array of one range, where there is a better way than bam_array_read_shaped's; false, with nothing launched, where not */
+bool summed_reads(bam_array_t* a, uint64_t n_reqs, const uint64_t* d_assignment, unsigned long long* sum, hipStream_t st)
+{
+    if (!two_launches_ok(a)) return false;
+    const range_d_t<uint64_t>& range = a->a->h_ranges[0];
+    if (range.page_count > range.cache.n_pages) {
+        if (dealt_reads_pay(a, n_reqs, st) && dealt_reads<false>(a, n_reqs, d_assignment, sum, nullptr, st)) return true;
+        /* (from 2^16 on what is resident first: 200000 of 2^19 pages behind 2^18, three such sets by turns, 9.4 ms in one launch and 5.1 in two) */
+        if (n_reqs >= 1ull << 16 || !few_reads_pay(a, n_reqs)) return false;
+        few_reads<false>(a, n_reqs, d_assignment, sum, nullptr, st);
+    } else {
+        /* up to 2^20, one launch (k_array_read_each): then two, of 2^22 16 million elements in pages of 4 KiB 133 us and, a read to a thread, 120, of
+         * 128 million 139 and 162 */
+        if (n_reqs > 1ull << 20) return false;
+        unsigned long long* const part = (unsigned long long*)a->partials.get();
+        const uint32_t groups = blocks_for(n_reqs, BAM_READ_EACH_THREADS);
+        const bool fold = groups > BAM_DIRECT_GROUPS;
+        hipLaunchKernelGGL(k_array_read_each, dim3(groups), dim3(BAM_READ_EACH_THREADS), 0, st, a->a->d_array_ptr, n_reqs, d_assignment, part, fold ? nullptr : sum);
+        if (fold) hipLaunchKernelGGL(k_fold_partials, dim3(1), dim3(1024), 0, st, part, sum);
+    }
+    hip_err_chk(hipGetLastError());
+    return true;
+}
 } // namespace
 } // extern "C++"
 
@@ -2233,8 +2286,10 @@ int bam_array_read(bam_array_t* a, uint64_t n_reqs, const uint64_t* d_assignment
     if (!n_reqs) return 0;
     /* a large launch of scattered requests, one read each: in two launches where the array allows it, else four requests per
      * thread (results and counters are the same) */
+    BAM_API_BEGIN
+    static const int shape_env = getenv("BAM_READ_SHAPE") ? atoi(getenv("BAM_READ_SHAPE")) : 0;
+    if (d_assignment && reqs_per_thread == 1 && !shape_env && summed_reads(a, n_reqs, d_assignment, (unsigned long long*)d_sum, (hipStream_t)stream)) return 0;
     if (d_assignment && reqs_per_thread == 1 && n_reqs >= (1ull << 16)) {
-        static const int shape_env = getenv("BAM_READ_SHAPE") ? atoi(getenv("BAM_READ_SHAPE")) : 0;
         /* eight reads per lane in the first launch: 44 thousand million reads a second on resident data against 39 with four
          * (what bounds the kernel is how many requests a compute unit's L1 keeps in flight, and for how long each) */
         static const int lanes_env = getenv("BAM_READS_PER_LANE") ? atoi(getenv("BAM_READS_PER_LANE")) : 8;
@@ -2242,10 +2297,7 @@ int bam_array_read(bam_array_t* a, uint64_t n_reqs, const uint64_t* d_assignment
         if (shape_env >= BAM_READ_ONE_PER_THREAD && shape_env <= BAM_READ_TWO_LAUNCHES && (shape_env != BAM_READ_TWO_LAUNCHES || two_launches_ok(a))) shape = shape_env;
         return bam_array_read_shaped(a, n_reqs, d_assignment, shape, (uint32_t)lanes_env, block_size, d_sum, stream);
     }
-    BAM_API_BEGIN
-    if (d_assignment && reqs_per_thread == 1 && dealt_reads_pay(a, n_reqs, (hipStream_t)stream) && dealt_reads<false>(a, n_reqs, d_assignment, (unsigned long long*)d_sum, nullptr, (hipStream_t)stream)) return 0;
-    if (d_assignment && reqs_per_thread == 1 && few_reads_pay(a, n_reqs)) few_reads<false>(a, n_reqs, d_assignment, nullptr, (hipStream_t)stream);
-    else hipLaunchKernelGGL(k_array_read, dim3(blocks_for(n_reqs, block_size)), dim3(block_size), 0, (hipStream_t)stream,
+    hipLaunchKernelGGL(k_array_read, dim3(blocks_for(n_reqs, block_size)), dim3(block_size), 0, (hipStream_t)stream,
                        a->a->d_array_ptr, n_reqs, d_assignment, stride, reqs_per_thread, (unsigned long long*)a->partials.get());
     hipLaunchKernelGGL(k_fold_partials, dim3(1), dim3(1024), 0, (hipStream_t)stream, (unsigned long long*)a->partials.get(), (unsigned long long*)d_sum);
     hip_err_chk(hipGetLastError());
@@ -2260,7 +2312,7 @@ int bam_array_gather(bam_array_t* a, uint64_t n_reqs, const uint64_t* d_assignme
     BAM_API_BEGIN
     if (d_assignment && dealt_reads_pay(a, n_reqs, (hipStream_t)stream) && dealt_reads<true>(a, n_reqs, d_assignment, nullptr, d_out, (hipStream_t)stream)) return 0;
     if (d_assignment && scattered_launches_pay(a, n_reqs, (hipStream_t)stream) && scattered_reads<true>(a, n_reqs, d_assignment, 8, nullptr, d_out, (hipStream_t)stream)) return 0;
-    if (d_assignment && few_reads_pay(a, n_reqs)) few_reads<true>(a, n_reqs, d_assignment, d_out, (hipStream_t)stream);
+    if (d_assignment && few_reads_pay(a, n_reqs)) few_reads<true>(a, n_reqs, d_assignment, nullptr, d_out, (hipStream_t)stream);
     else hipLaunchKernelGGL(k_array_gather, dim3(blocks_for(n_reqs, block_size)), dim3(block_size), 0, (hipStream_t)stream,
                        a->a->d_array_ptr, n_reqs, d_assignment, stride, d_out);
     hip_err_chk(hipGetLastError());
