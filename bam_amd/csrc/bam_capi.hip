@@ -2376,9 +2376,18 @@ namespace {
  */
 bool updates_by_bins(bam_array_t* a, int api, uint64_t n_reqs, const uint64_t* d_assignment, const uint64_t* d_values, uint64_t* d_old, hipStream_t st, size_t& bytes_later)
 {
-    if (n_reqs < (api == 0 ? 1ull << 18 : 1ull << 17) || a->a->adt.n_ranges != 1) return false;
+    if (a->a->adt.n_ranges != 1) return false;
     const range_d_t<uint64_t>& r = a->a->h_ranges[0];
     const uint64_t page_elems = r.cache.page_size / sizeof(uint64_t), pages = r.page_count;
+    /*
+     * From as many on as the bins gain from, scattered over any number of pages; and through pointers from fewer where many meet on a page, since the
+     * ones that do wait for each other's references: us element by element (memref, +=) and in bins, of 2^10 pages of 8 KiB, 48000 27 37 and 30,
+     * 65000 34 48 and 31, 125000 60 85 and 35; 2^11 of 4 KiB, 65000 26 43 and 31, 100000 36 61 and 33; 2^9, 32000 29 32 and 29, 65000 50 58 and 31; 2^13,
+     * 65000 22 29 and 32, 80000 25 42 and 32, 125000 35 63 and 35.  Sorted, 65000 of 2^10 pages 24 36 and 29, 100000 of 2^11 28 44 and 30; in order 209 190
+     * and 23, 115 122 and 23.  AtomicAdd gains as much there scattered (48 and 35), but loses as much in an order (20 and 31, 20 and 24).
+     */
+    const uint64_t enough = api == 0 ? 1ull << 18 : api == 1 ? 1ull << 17 : 9ull << 13, meet = api == 1 ? 3600000 : 1700000;
+    if (n_reqs < enough && (api == 0 || n_reqs < 1ull << 14 || n_reqs * n_reqs < meet * pages)) return false;
     uint32_t bin_log = 0;
     while ((pages + (1ull << bin_log) - 1) >> bin_log > BAM_BINS) bin_log++;
     const uint32_t bins = (uint32_t)((pages + (1ull << bin_log) - 1) >> bin_log);

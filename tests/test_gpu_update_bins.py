@@ -65,3 +65,25 @@ def test_updates_that_meet(bam, pages, span):
         np.add.at(model, idx.astype(np.int64), vals)
         r.objs[0][2].flush()
         assert np.array_equal(r.backing(n_elems), model) and not r.c.aborted()
+
+
+# through pointers from fewer requests on, the fewer the pages: on both sides of each line
+@pytest.mark.parametrize("api,pages,n", [(1, 200, (1 << 14) - 1), (1, 74, 1 << 14), (1, 1000, 59999), (1, 1000, 60000), (1, 6000, (1 << 17) - 1), (2, 1000, 41231), (2, 1000, 41232),
+                                         (2, 6000, (9 << 13) - 1), (2, 6000, 9 << 13), (2, 157, 1 << 14), (0, 100, (1 << 18) - 1)])
+@pytest.mark.parametrize("kind", ["scattered", "in_order", "one_page"])
+def test_updates_of_few_pages(bam, api, pages, n, kind):
+    n_elems = pages * 512 - 3
+    rng = np.random.default_rng(n)
+    with Rig(bam, pages * 4096, backing=True, n_queues=16, depth=256) as r:
+        model = r.backing(n_elems).copy()
+        a = r.array(n_elems, 4096, pages)
+        a.gather(pages, None, stride=512)
+        a.update(0, _dev(np.zeros(1 << 18, dtype=np.uint64)), _dev(np.zeros(1 << 18, dtype=np.uint64)))      # leaves the memory for the bins behind
+        idx = (rng.integers(0, n_elems, n) if kind == "scattered" else np.arange(n) % n_elems if kind == "in_order" else rng.integers(512, 1024, n)).astype(np.uint64)
+        if api:                                               # no two at a time on an element
+            idx = np.unique(idx) if kind != "scattered" else rng.permutation(n_elems)[:n].astype(np.uint64)
+        vals = rng.integers(1, 1 << 63, len(idx)).astype(np.uint64)
+        for rep in range(2):
+            a.update(api, _dev(idx), _dev(vals))
+            np.add.at(model, idx.astype(np.int64), vals)
+        assert np.array_equal(_u64(a.gather(n_elems, None)), model) and not r.c.aborted()
