@@ -2082,12 +2082,17 @@ bool few_reads_pay(bam_array_t* a, uint64_t n_reqs)
 template <bool GATHER>
 void few_reads(bam_array_t* a, uint64_t n_reqs, const uint64_t* d_assignment, unsigned long long* sum, uint64_t* d_out, hipStream_t st)
 {
-    unsigned long long* const part = (unsigned long long*)a->partials.get();
+    unsigned long long* part = (unsigned long long*)a->partials.get();
     const uint64_t least = std::min<uint64_t>(256, (1ull << 20) / a->a->h_ranges[0].cache.page_size);
     uint32_t each = BAM_WAVE_SIZE;
     while (each > 4 && n_reqs / each < least) each /= 2;
     const uint32_t groups = blocks_for((n_reqs + each - 1) / each * BAM_WAVE_SIZE, 256);
     const bool fold = !GATHER && groups > BAM_DIRECT_GROUPS;
+    std::unique_lock<std::mutex> guard(a->scratch.mu, std::defer_lock);
+    if (fold && !is_captured(st)) {
+        guard.lock();
+        if (scratch_set* set = scratch_for(a, st, 0, 0)) part = set->partials();
+    }
     hipLaunchKernelGGL(k_array_read_few<GATHER>, dim3(groups), dim3(256), 0, st, a->a->d_array_ptr, n_reqs, d_assignment, each, part, fold ? nullptr : sum, d_out);
     if (fold) hipLaunchKernelGGL(k_fold_partials, dim3(1), dim3(1024), 0, st, part, sum);
 }
@@ -2236,11 +2241,17 @@ bool summed_reads(bam_array_t* a, uint64_t n_reqs, const uint64_t* d_assignment,
         /* up to 2^20, one launch (k_array_read_each): then two, of 2^22 16 million elements in pages of 4 KiB 133 us and, a read to a thread, 120, of
          * 128 million 139 and 162 */
         if (n_reqs > 1ull << 20) return false;
-        unsigned long long* const part = (unsigned long long*)a->partials.get();
         const uint32_t groups = blocks_for(n_reqs, BAM_READ_EACH_THREADS);
-        const bool fold = groups > BAM_DIRECT_GROUPS;
-        hipLaunchKernelGGL(k_array_read_each, dim3(groups), dim3(BAM_READ_EACH_THREADS), 0, st, a->a->d_array_ptr, n_reqs, d_assignment, part, fold ? nullptr : sum);
-        if (fold) hipLaunchKernelGGL(k_fold_partials, dim3(1), dim3(1024), 0, st, part, sum);
+        if (groups <= BAM_DIRECT_GROUPS) hipLaunchKernelGGL(k_array_read_each, dim3(groups), dim3(BAM_READ_EACH_THREADS), 0, st, a->a->d_array_ptr, n_reqs, d_assignment, nullptr, sum);
+        else {
+            /* the shards of this stream: calls on several streams must not fold each other's */
+            if (is_captured(st)) return false;
+            std::lock_guard<std::mutex> guard(a->scratch.mu);
+            scratch_set* set = scratch_for(a, st, 0, 0);
+            if (!set) return false;
+            hipLaunchKernelGGL(k_array_read_each, dim3(groups), dim3(BAM_READ_EACH_THREADS), 0, st, a->a->d_array_ptr, n_reqs, d_assignment, set->partials(), nullptr);
+            hipLaunchKernelGGL(k_fold_partials, dim3(1), dim3(1024), 0, st, set->partials(), sum);
+        }
     }
     hip_err_chk(hipGetLastError());
     return true;

@@ -105,9 +105,9 @@ int bam_array_stats(bam_array_t* a, uint64_t* out, int reset);
 /* ---- array benchmark kernels (benchmarks/array/main.cu:43-65) ----
  * One thread per request: thread t reads element d_assignment[t] (or t * stride when d_assignment is NULL)
  * reqs_per_thread times through array_d_t::operator[] and the launch adds every value read into *d_sum
- * (mod 2^64).  The reference discards the values; the checksum is what makes the result checkable.  A launch of 2^16 or
- * more scattered requests read once each takes another shape (bam_array_read_shaped): the same reads, sum and counters of
- * accesses, several of them in flight per lane. */
+ * (mod 2^64).  The reference discards the values; the checksum is what makes the result checkable.  Scattered requests read
+ * once each take other shapes by how many there are and whether the array fits its cache (below, and bam_array_read_shaped): the same reads,
+ * sum and counters of accesses. */
 int bam_array_read(bam_array_t* a, uint64_t n_reqs, const uint64_t* d_assignment, uint64_t stride, uint64_t reqs_per_thread,
                    uint32_t block_size, uint64_t* d_sum, void* stream);
 /* The same scattered requests (thread t reads element d_assignment[t] once; sum into *d_sum) with the launch shape named,
@@ -123,8 +123,10 @@ int bam_array_read(bam_array_t* a, uint64_t n_reqs, const uint64_t* d_assignment
  *                             one range only (EINVAL otherwise); on a stream that is being captured the
  *                             call runs as BAM_READ_FOUR_PER_THREAD.  A request whose page these launches
  *                             fetched counts as a miss, any other by what it finds when it is read.
- * bam_array_read picks BAM_READ_TWO_LAUNCHES with eight reads per lane for launches of 2^16 requests and more where the array
- * allows it (BAM_READ_FOUR_PER_THREAD where not) and BAM_READ_ONE_PER_THREAD below that. */
+ * bam_array_read picks, for arrays of one range, one launch of a read per thread up to 2^20 requests of an array that fits its cache and
+ * BAM_READ_TWO_LAUNCHES with eight reads per lane beyond; for one that does not fit, what BAM_READ_TWO_LAUNCHES does, with the requests
+ * put in order of their pages where they share them, or from 2^16 on, and below that few requests to a wave.  Other arrays:
+ * BAM_READ_FOUR_PER_THREAD from 2^16 on and BAM_READ_ONE_PER_THREAD below. */
 #define BAM_READ_ONE_PER_THREAD  1
 #define BAM_READ_FOUR_PER_THREAD 2
 #define BAM_READ_TWO_LAUNCHES    3
