@@ -2101,7 +2101,10 @@ void few_reads(bam_array_t* a, uint64_t n_reqs, const uint64_t* d_assignment, un
  * share a page, and each waits for its own: us that way and in order, 4096 pages behind 2048, 8000 219 and 244, 16000 258 and 242; 16384
  * behind 8192, 30000 614 and 646, 60000 735 and 725; 8404 behind 2101, 8404 436 and 538, 12000 700 and 609), and always where they are not all on
  * their way together; but not where requests spread evenly ask for no more pages than the cache holds, and so find them all
- * the next time (that takes three launches more, 16 us for 6).
+ * the next time (that takes three launches more, 16 us for 6; beside two launches, from 2^18 requests on, 59 and 57, and they do not find all of
+ * them while they ask for nine tenths as many: 2^20 of 2^18 pages behind 2000 less 1.61 ms in two launches and 0.33 here).
+ *   Few missing pages gain as well: 2^22 of those 1.30 and 0.44 ms, 10^5 and 2^20 of 9000 behind 8500 0.31 and 0.10, 0.57 and 0.17; 2^24, several
+ * slices, no more.
  *   Large launches go by stretches all the same where those have the whole array in two, and where there would be several
  * slices, each of which asks for all pages (2^19 pages behind 2^18, 2^22 requests 19.9 and 20.3 ms; 2^16 behind 2^15, 2^24 3.3 and 11.1).
  */
@@ -2113,7 +2116,9 @@ bool dealt_reads_pay(bam_array_t* a, uint64_t n_reqs, hipStream_t st)
     const uint64_t pages = range.page_count, cache_pages = range.cache.n_pages;
     if (pages <= cache_pages || pages >= 1ull << 32) return false;
     if (n_reqs <= BAM_REQS_AT_A_TIME && n_reqs < pages + 2 * cache_pages) return false;
-    if ((double)n_reqs < -std::log1p(-(double)cache_pages / (double)pages) * (double)pages) return false;
+    const double asked = (double)pages * -std::expm1(-(double)n_reqs / (double)pages);
+    if (asked < (n_reqs <= BAM_REQS_AT_A_TIME ? 1.0 : 0.9) * (double)cache_pages) return false;
+    if (n_reqs > BAM_DEALT_SLICE && pages <= 2 * cache_pages) return false;
     if (page_by_page(range, n_reqs) && (n_reqs > BAM_DEALT_SLICE || (pages <= 2 * cache_pages && cache_pages >= 1ull << 18))) return false;
     return !is_captured(st);
 }
