@@ -365,9 +365,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
  * wave of the last (k_reads_fetch) takes a turn of neighbouring pages, asks for those that somebody waits for in batches and
  * reads the batch's requests, which lie side by side.  Stretches of the range (k_fetch_wanted) need a drain of the queues
  * each, and caches of thousands of pages.
- *   A wave holds its batch while it waits for the rest of it, as k_along_missing does, and the pages that are held so are counted in a
- * word of the cache, for all arrays and streams together: beyond half the cache batches are not held, and a page that goes
- * before its requests are read is read on demand.
+ *   A wave that waits holds nothing but the slots it is loading: a batch is held if all of its pages were there, or came, together, as they
+ * do where nobody else asks for them and slots are not short, and then nothing is waited for until it is read.  Otherwise each page is given
+ * back as it arrives, the requests are read as those of the first launch are, and those whose page has gone again on demand.  (Were
+ * pages held while others are waited for, this launch and whatever else holds pages of the cache, a sweep over a graph or pointers of a
+ * caller's kernel, could each wait for slots that the other has.)
  *   Bound by the store.  Gathers of elements at random, request by request or in stretches, and here, ms (pages of 4 KiB): 8404 behind 2101,
  * 20000 requests 1.06 and 0.70, 277608 7.3 and 0.72, 2^22 458 and 1.10; 16384 behind 8192, 2^20 1.33 and 0.74; 65536 behind 16384, 2^17 5.9 and
  * 3.3, 2^22 4.94 and 4.04; 65536 behind 32768, 2^19 2.78 and 2.65; 512 behind 256, 10^5 0.65 and 0.12; 192076 of 512 bytes behind 96038, 426105
@@ -375,7 +377,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
  * a batch's size 11.7.
  */
 #define BAM_BEGIN_PAGES 1024u
-#define BAM_PLEDGED_WORD 1u          /* of the cache's miss_tokens: pages held so, beside the count of the first compute unit */
 /* what lanes of a wave have written to LDS, for all of its lanes: a wave's LDS operations run in order */
 __device__ __forceinline__ void wave_lds_fence()
 {
@@ -442,9 +443,6 @@ __global__ __launch_bounds__(64) void k_reads_fetch(array_d_t<uint64_t>* dr, con
     bam::range_view<uint64_t> view;
     view.load(dr->d_ranges);
     view.place = BAM_PLACE_PULLED;
-    const page_cache_d_t* const cache = &dr->d_ranges->cache;
-    uint32_t* const pledged = cache->miss_tokens + BAM_PLEDGED_WORD;
-    const uint32_t most = (uint32_t)(cache->n_pages / 2);
     uint64_t v = 0;
     uint32_t n_read = 0, n_pages = 0;
     for (;;) {
@@ -478,18 +476,15 @@ __global__ __launch_bounds__(64) void k_reads_fetch(array_d_t<uint64_t>* dr, con
             wave_lds_fence();
             if (pages + lane < have) { list[lane] = next; counts[lane] = next_count; }
             have -= pages;
-            uint32_t hold = 0;
-            if (lane == 0) {
-                hold = __hip_atomic_fetch_add(pledged, pages, __ATOMIC_RELAXED, BAM_AGENT) + pages <= most;
-                if (!hold) __hip_atomic_fetch_add(pledged, 0u - pages, __ATOMIC_RELAXED, BAM_AGENT);
-            }
-            hold = bam::bcast(hold, 0);
             uint32_t slot = BAM_NO_SLOT;
-            auto arrive = [&](uint32_t at) { slot = hold ? at : BAM_NO_SLOT; return !hold; };
+            auto arrive = [&](uint32_t at) {
+                const bool all = bam::popc(bam::active_mask()) == pages;
+                if (all) slot = at;
+                return !all;
+            };
             view.acquire_helped(page, mine, false, arrive, arrive);
             if (mine) slots[page - first] = slot;
             const bool held = bam::ballot(mine && slot == BAM_NO_SLOT) == 0;
-            if (!held && slot != BAM_NO_SLOT) bam_release_refs(view.pages + page, 1, false);        /* a wait was given up */
             wave_lds_fence();
             n_pages += pages;
             for (uint32_t b = 0; b < n; b += N * BAM_WAVE_SIZE) {
@@ -526,7 +521,6 @@ __global__ __launch_bounds__(64) void k_reads_fetch(array_d_t<uint64_t>* dr, con
                 }
             }
             if (held && mine) bam_release_refs(view.pages + page, 1, false);
-            if (hold && lane == 0) __hip_atomic_fetch_add(pledged, 0u - pages, __ATOMIC_RELAXED, BAM_AGENT);
             begin += n;
         }
     }

@@ -83,8 +83,43 @@ def test_ranges_that_begin_inside_a_page(bam, page, offset, first):
         a.close(); rg.close(); pc.close()
 
 
+@pytest.mark.parametrize("cache_pages", [64, 300])
+def test_beside_a_sweep_that_holds_pages(bam, cache_pages):
+    """A sweep over a graph holds up to half of the cache while it waits for more: gathers of another array, on two streams, hold none while they wait"""
+    import torch
+    from test_gpu_beside_evictions import OTHER, Shared
+    off, nb = oracle.uniform_csr(SEED, 20011, 150007)
+    src = int(oracle.bfs_sources(SEED, off, 1)[0])
+    levels, n_levels = oracle.bfs_levels(off, nb, src)
+    labels, _ = oracle.cc_labels(off, nb)
+    n = 8001
+    with Shared(bam, [len(nb)], cache_pages) as s:
+        s.of(0, len(nb))[:] = nb
+        d_off = _dev(off)
+        s.arrs[0].set_graph(d_off)
+        reqs = [np.random.default_rng(k).integers(0, OTHER * 512, n).astype(np.uint64) for k in range(2)]
+        d, streams = [_dev(x) for x in reqs], [torch.cuda.Stream() for _ in reqs]
+        for rep in range(4):
+            torch.cuda.synchronize()
+            outs = []
+            for k in range(2):
+                with torch.cuda.stream(streams[k]):
+                    outs.append([s.arrs[-1].gather(n, d[k]) for _ in range(3)])
+            if rep & 1:
+                lb, _ = s.arrs[0].cc(d_off)
+                assert np.array_equal(_u64(lb), labels), rep
+            else:
+                lv, it = s.arrs[0].bfs(d_off, src)
+                assert np.array_equal(lv.cpu().numpy().view(np.uint32), levels) and it == n_levels, rep
+            torch.cuda.synchronize()
+            for k in range(2):
+                for o in outs[k]:
+                    assert np.array_equal(_u64(o), s.of(1, OTHER * 512)[reqs[k].astype(np.int64)]), (rep, k)
+            assert not s.r.c.aborted()
+
+
 def test_many_streams_and_arrays_of_one_cache(bam):
-    """Eight streams over two arrays behind one small cache: together they may hold no more than half of it."""
+    """Eight streams over two arrays behind one small cache, most of whose batches come in parts."""
     import torch
     from bam_amd import Array, PageCache, Range
     pages, n = 900, 9001
