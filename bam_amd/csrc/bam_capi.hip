@@ -1144,6 +1144,8 @@ __device__ __forceinline__ void cache_stream_body(array_d_t<uint64_t>* dr, uint6
              * Descriptor read once.  Pages are taken sixteen at a time: lane l of the wave asks for page l of the
              * batch, so the sixteen reference counts go out as one vector atomic; then the whole wave streams the
              * sixteen pages, eight 8-byte loads in flight per lane, and the sixteen references are dropped together.
+             * What cannot be had without waiting is asked for again when the others have been read and dropped: there may be any number of
+             * waves, and other streams beside them, and none waits while it holds pages.
              */
             bam::range_view<uint64_t> view;
             view.load(r0);
@@ -1152,7 +1154,7 @@ __device__ __forceinline__ void cache_stream_body(array_d_t<uint64_t>* dr, uint6
             const bool by_groups = stream_by_groups(view);
             const uint32_t group = by_groups ? stream_group_pages(view) : 1;
             uint64_t seen = 0, seen_first = ~0ull;
-            for (uint64_t p0 = 0; p0 < n_pages_per_wave; p0 += 16) {
+            for (uint64_t p0 = 0; p0 < n_pages_per_wave;) {
                 if (by_groups) {
                     const uint64_t first = (start_page + p0) * epp, next = first + 8 * BAM_WAVE_SIZE;
                     if (p0 + group <= n_pages_per_wave && first < next && next <= view.index_end) {
@@ -1160,43 +1162,47 @@ __device__ __forceinline__ void cache_stream_body(array_d_t<uint64_t>* dr, uint6
                         seen_first = next + 8 * BAM_WAVE_SIZE <= view.index_end ? next : first;
                         if (stream_group(view, first, seen_first, lane, seen, a0)) {
                             if (lane < group) view.account(true);
-                            p0 += (uint64_t)group - 16;           /* (the loop's 16 on top) */
+                            p0 += group;
                             continue;
                         }
                     }
                 }
                 const uint32_t nb = (uint32_t)(n_pages_per_wave - p0 < 16 ? n_pages_per_wave - p0 : 16);
-                uint32_t slot = BAM_NO_SLOT;
                 const uint64_t page = view.page_of((start_page + p0 + (lane < nb ? lane : 0)) * epp);
-                if (lane < nb) {
-                    auto keep = [&](uint32_t s_) { slot = s_; return false; };
-                    view.acquire<true>(page, false, keep, keep);
-                }
-                /* a page whose wait was given up (the controller is marked aborted) has no slot: nothing of the batch is read */
-                const bool all_in = bam::ballot(lane < nb && slot == BAM_NO_SLOT) == 0;
-                uint32_t k = all_in ? 0 : nb;
-                if (n8 == 8 * BAM_WAVE_SIZE)            /* 4 KiB pages: two at a time */
-                    for (; k + 1 < nb; k += 2) {
-                        uint64_t x[16];
-                        bam::ld_payload_stream16((const uint64_t*)view.slot_addr(bam::bcast(slot, k)) + lane,
-                                                 (const uint64_t*)view.slot_addr(bam::bcast(slot, k + 1)) + lane, x);
-                        a0 += ((x[0] + x[2]) + (x[4] + x[6])) + ((x[8] + x[10]) + (x[12] + x[14]));
-                        a1 += ((x[1] + x[3]) + (x[5] + x[7])) + ((x[9] + x[11]) + (x[13] + x[15]));
-                    }
-                for (; k < nb; k++) {
-                    const uint64_t* base = (const uint64_t*)view.slot_addr(bam::bcast(slot, k));
-                    for (uint32_t i = (uint32_t)lane; i < n8; i += 8 * BAM_WAVE_SIZE) {
-                        uint64_t x[8];
-                        if (i + 7 * BAM_WAVE_SIZE < n8) bam::ld_payload_stream8(base + i, x);
-                        else {
-#pragma unroll
-                            for (int j = 0; j < 8; j++) x[j] = i + j * BAM_WAVE_SIZE < n8 ? bam::ld_payload(base + i + j * BAM_WAVE_SIZE) : 0;
+                for (uint32_t left = (1u << nb) - 1u; left;) {
+                    uint32_t slot;
+                    const bool in = view.acquire_some<true>(page, lane < nb && ((left >> lane) & 1u), slot);
+                    uint32_t m = (uint32_t)bam::ballot(in);
+                    if (!m) break;                          /* the wait was given up (the controller is marked aborted): the rest is not read */
+                    left &= ~m;
+                    if (n8 == 8 * BAM_WAVE_SIZE)            /* 4 KiB pages: two at a time */
+                        while (m & (m - 1)) {
+                            const uint32_t k = (uint32_t)__builtin_ctz(m);
+                            m &= m - 1;
+                            const uint32_t k1 = (uint32_t)__builtin_ctz(m);
+                            m &= m - 1;
+                            uint64_t x[16];
+                            bam::ld_payload_stream16((const uint64_t*)view.slot_addr(bam::bcast(slot, k)) + lane,
+                                                     (const uint64_t*)view.slot_addr(bam::bcast(slot, k1)) + lane, x);
+                            a0 += ((x[0] + x[2]) + (x[4] + x[6])) + ((x[8] + x[10]) + (x[12] + x[14]));
+                            a1 += ((x[1] + x[3]) + (x[5] + x[7])) + ((x[9] + x[11]) + (x[13] + x[15]));
                         }
-                        a0 += x[0] + x[2] + x[4] + x[6];
-                        a1 += x[1] + x[3] + x[5] + x[7];
+                    for (; m; m &= m - 1) {
+                        const uint64_t* base = (const uint64_t*)view.slot_addr(bam::bcast(slot, (uint32_t)__builtin_ctz(m)));
+                        for (uint32_t i = (uint32_t)lane; i < n8; i += 8 * BAM_WAVE_SIZE) {
+                            uint64_t x[8];
+                            if (i + 7 * BAM_WAVE_SIZE < n8) bam::ld_payload_stream8(base + i, x);
+                            else {
+#pragma unroll
+                                for (int j = 0; j < 8; j++) x[j] = i + j * BAM_WAVE_SIZE < n8 ? bam::ld_payload(base + i + j * BAM_WAVE_SIZE) : 0;
+                            }
+                            a0 += x[0] + x[2] + x[4] + x[6];
+                            a1 += x[1] + x[3] + x[5] + x[7];
+                        }
                     }
+                    if (in) bam_release_refs(view.pages + page, 1, false);
                 }
-                if (lane < nb) view.release(page, false);
+                p0 += nb;
             }
             v += a0 + a1;
             view.flush_stats();
@@ -2497,7 +2503,7 @@ int bam_cache_stream(bam_array_t* a, uint64_t n_waves, uint64_t n_pages_per_wave
     /*
      * Where the runs follow one another the pages may be shared out to other runs: of up to 64 KiB, as many as leave 4096 waves something, 4 KiB
      * at least.  1 GiB resident in pages of 4 KiB, a page, four and 16 to a wave, through bam_ptr 390, 217, 202 us; 8 MiB, four and 16, 36, 46; 128 MiB
-     * 59, 61.  Pages in batches (mode 2) are held while others are waited for: only where the cache has room for all of them.
+     * 59, 61.  Mode 2 only where the cache has room for all of them.
      */
     uint64_t run_waves = n_waves, run_pages = n_pages_per_wave;
     if (!d_assignment && mode <= 2 && a->a->adt.n_ranges == 1 && n_waves < 1ull << 32 && n_pages_per_wave < 1ull << 32 && (mode < 2 || (total <= r.cache.n_pages && r.page_count <= r.cache.n_pages))) {

@@ -1040,6 +1040,71 @@ struct range_view {
     {
         acquire_<OUTLINE, true>(page, write, on_hit, on_miss, take);
     }
+    /*
+     * As many of the pages of the lanes with `take`, each another one and for reading, as can be had without waiting while one is held: true, with the
+     * slot and a reference, for the lanes whose page was resident, or whose pages are the first that came if none was; the other
+     * lanes hold nothing, and ask again when the caller has given back what it got.  Whoever keeps pages while it waits for more
+     * (acquire with callbacks that answer false) has to be one of so few that the cache holds all they ask for, or they wait for each other's
+     * slots.  All lanes of the wave call; those that take nothing help.  False for all of them: the wait was given up.
+     */
+    template <bool OUTLINE = false>
+    __forceinline__ __device__ bool acquire_some(const uint64_t page, const bool take, uint32_t& slot)
+    {
+        const uint32_t me = lane();
+        data_page_t* const dp = pages + (take ? page : 0);
+        uint64_t sv = 0;
+        slot = BAM_NO_SLOT;
+        bool in = false, open = take;                     /* open: a reference on a page that is not there yet */
+        if (take && bam_try_hit(dp, 1, false, sv, slot)) { in = true; open = false; account(true); }
+        if (__builtin_expect(ballot(open) != 0, 0)) {
+            const uint32_t queue = wave_slot_hash();
+            spin_t sp;
+            page_cache_d_t* const cache = (page_cache_d_t*)first((uint64_t)&r->cache);
+            /* admission to the miss path as in acquire_ */
+            const uint32_t limit = cache->miss_waves;
+            uint32_t* const tokens = cache->miss_tokens + (cu_id() & (BAM_TOKEN_SLOTS - 1)) * 16;
+            bool admitted = limit == 0;
+            for (;;) {
+                const bam_pass_t ps = bam_slow_pass<OUTLINE>(r, page, queue, sv, slot, (open ? BAM_PASS_TAKE_PART : 0u) | (admitted ? BAM_PASS_MAY_LOAD : 0u) | (place << BAM_PASS_PLACE_SHIFT));
+                const bool wants = (ps.flags & BAM_PASS_WANTS) != 0;
+                if (open) {
+                    sv = ps.sv;
+                    if (ps.flags & BAM_PASS_RESOLVED) { slot = ps.slot; in = true; open = false; account((ps.flags & BAM_PASS_HIT) != 0); }
+                }
+                if (ballot(in)) break;
+                if (!admitted && ballot(wants)) {
+                    uint32_t ok = 0;
+                    if (open) __hip_atomic_fetch_add(&dp->state, 0u - 1u, __ATOMIC_RELAXED, BAM_AGENT);
+                    if (me == 0) {
+                        for (uint32_t i = 1;; i++) {
+                            if (ld_relaxed(tokens) < limit) {
+                                if (__hip_atomic_fetch_add(tokens, 1u, __ATOMIC_RELAXED, BAM_AGENT) < limit) { ok = 1; break; }
+                                __hip_atomic_fetch_add(tokens, 0u - 1u, __ATOMIC_RELAXED, BAM_AGENT);
+                            }
+                            __builtin_amdgcn_s_sleep(127);
+                            __builtin_amdgcn_s_sleep(127);
+                            __builtin_amdgcn_s_sleep(127);
+                            __builtin_amdgcn_s_sleep(127);
+                            if ((i & 15u) == 0 && cache->guard && ld_relaxed_sys(&cache->guard->abort)) break;
+                        }
+                    }
+                    if (open) bam_try_hit(dp, 1, false, sv, slot);             /* the next pass reads the outcome from sv */
+                    admitted = bcast(ok, 0) != 0;
+                    if (!admitted) break;
+                    continue;
+                }
+                if (limit && admitted) {
+                    if (me == 0) __hip_atomic_fetch_add(tokens, 0u - 1u, __ATOMIC_RELAXED, BAM_AGENT);
+                    admitted = false;
+                }
+                if (cache->spin_giveup(sp)) break;
+            }
+            if (limit && admitted && me == 0) __hip_atomic_fetch_add(tokens, 0u - 1u, __ATOMIC_RELAXED, BAM_AGENT);
+            if (open) __hip_atomic_fetch_add(&dp->state, 0u - 1u, __ATOMIC_RELAXED, BAM_AGENT);
+            fill();
+        }
+        return in;
+    }
     template <bool OUTLINE, bool HELPERS, typename FH, typename FM>
     __forceinline__ __device__ void acquire_(const uint64_t page_, const bool write, FH&& on_hit, FM&& on_miss, const bool take)
     {

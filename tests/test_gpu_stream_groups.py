@@ -74,3 +74,36 @@ def test_ranges_that_begin_elsewhere(bam, page, offset, first):
                 assert a.stream(30, 7, mode=mode) == want, (mode, rep)
         assert not r.c.aborted()
         a.close(); rg.close(); pc.close()
+
+
+@pytest.mark.parametrize("page", [512, 4096])
+@pytest.mark.parametrize("pages,cache_pages", [(240, 256), (1200, 64), (33, 17)])
+def test_page_wise_streams_that_share_a_cache(bam, page, pages, cache_pages):
+    """Three arrays behind one cache that holds one of them, or less, each streamed page by page on a stream of its own: waves hold nothing while
+    they wait, so all of them end, and every page counts once however often it is asked for"""
+    import torch
+    from bam_amd import Array, PageCache, Range
+    per, ppw = page // 8, 17 if pages > 33 else 11
+    waves = pages // ppw
+    words = oracle.store(SEED, 0, 3 * pages * per).reshape(3, -1)
+    with Rig(bam, (3 * pages * page + 65535) // 65536 * 65536, n_queues=8, depth=256) as r:
+        pc = PageCache(page, cache_pages, 0, r.c)
+        rgs = [Range(0, pages * per, k * pages, pages, 0, page, pc, 0) for k in range(3)]
+        arrays = [Array(pages * per, 0, [rg], 0) for rg in rgs]
+        want = [int(np.sum(words[k, :waves * ppw * per], dtype=np.uint64)) for k in range(3)]
+        streams = [torch.cuda.Stream() for _ in arrays]
+        sums = torch.zeros((6, 3), dtype=torch.int64, device="cuda")
+        torch.cuda.synchronize()
+        for rep in range(6):
+            for k, s in enumerate(streams):
+                with torch.cuda.stream(s):
+                    arrays[k].stream_async(waves, ppw, sums[rep, k:], mode=2)
+        torch.cuda.synchronize()
+        for k, a in enumerate(arrays):
+            assert [int(x) & MASK for x in sums[:, k]] == [want[k]] * 6, k
+            st = a.stats()
+            assert st["access_cnt"] == 6 * waves * ppw and st["read_io_cnt"] >= waves * ppw, st
+        assert not r.c.aborted()
+        for a in arrays: a.close()
+        for rg in rgs: rg.close()
+        pc.close()
