@@ -2501,14 +2501,18 @@ int bam_cache_stream(bam_array_t* a, uint64_t n_waves, uint64_t n_pages_per_wave
     const range_d_t<uint64_t>& r = a->a->h_ranges[0];
     const uint64_t total = n_waves * n_pages_per_wave, unit = r.cache.page_size < 4096 ? 4096 / r.cache.page_size : 1;
     /*
-     * Where the runs follow one another the pages may be shared out to other runs: of up to 64 KiB, as many as leave 4096 waves something, 4 KiB
-     * at least.  1 GiB resident in pages of 4 KiB, a page, four and 16 to a wave, through bam_ptr 390, 217, 202 us; 8 MiB, four and 16, 36, 46; 128 MiB
-     * 59, 61.  Mode 2 only where the cache has room for all of them.
+     * Where the runs follow one another the pages may be shared out to other runs: 16 pages or, of less than 4 KiB, 64 KiB, or less where that leaves
+     * fewer than 4096 waves; 4 KiB at least.  1 GiB resident in pages of 4 KiB, a page, four and 16 to a wave, through bam_ptr 390, 217, 202 us; 8 MiB,
+     * four and 16, 36, 46; 128 MiB 59, 61.  Mode 2 only where the cache has room for all of them, and for pages of up to 8 KiB as few as 1792 waves, since a
+     * wave has sixteen references on their way at a time: us with a page, two, four, eight and 16 to a wave, 4 KiB, 6909 pages 33.7 32.0 31.6 31.8 34.2,
+     * 12797 43.1 37.7 35.5 35.2 35.2, 32765 68.7 55.6 48.9 46.8 46.4; 8 KiB, 3453 30.5 32.1 33.8 38.6 48.8, 6397 37.4 36.4 35.3 39.4 49.7, 16381 55.4 49.8
+     * 48.2 46.4 52.5; of 512 bytes, 16, 32, 64 and 128, 49149 31.1 33.1 36.7 47.0, 524285 93.3 83.4 73.9 69.6.  (64 KiB, 4093, one and four 66.6 74.9.)
      */
     uint64_t run_waves = n_waves, run_pages = n_pages_per_wave;
     if (!d_assignment && mode <= 2 && a->a->adt.n_ranges == 1 && n_waves < 1ull << 32 && n_pages_per_wave < 1ull << 32 && (mode < 2 || (total <= r.cache.n_pages && r.page_count <= r.cache.n_pages))) {
         run_pages = 16 * unit;
-        while (run_pages > unit && total / run_pages < 4096) run_pages /= 2;
+        const uint64_t enough = mode == 2 && r.cache.page_size <= 8192 ? 1792 : 4096;
+        while (run_pages > unit && total / run_pages < enough) run_pages /= 2;
         run_waves = (total + run_pages - 1) / run_pages;
     }
     const dim3 grid(blocks_for(n_waves * BAM_WAVE_SIZE, bs)), block(bs), grid_runs(blocks_for(run_waves * BAM_WAVE_SIZE, bs));
