@@ -2107,18 +2107,28 @@ void few_reads(bam_array_t* a, uint64_t n_reqs, const uint64_t* d_assignment, un
  * slices, no more.
  *   Large launches go by stretches all the same where those have the whole array in two, and where there would be several
  * slices, each of which asks for all pages (2^19 pages behind 2^18, 2^22 requests 19.9 and 20.3 ms; 2^16 behind 2^15, 2^24 3.3 and 11.1).
+ *   Nor where an array has many pages for each request: a count and a beginning are looked at and kept for every page (8 bytes, and 0.1 ns of a
+ * call in pages of 4 KiB, 0.3 in pages of 512 bytes), and a turn has few pages that anybody waits for.  What it gains there is that waves of 64 requests, as many as there are,
+ * wait for each other's slots in a small cache: so fewer pages to a request the more slots there are.  Gathers, ms, two launches and
+ * in order, 2^18 + 1 requests of 2^20, 2^22, 2^24, 2^26 pages of 4 KiB: behind 2^13 65 59 57 57 and 19 21 22 28; 2^14 32 31 30 30 and 17 19 21 28; 2^15 19.1
+ * 21.0 21.6 21.6 and 17.1 19.2 20.8 27.8; 2^16 17.6 20.0 20.6 21.0 and 16.6 19.1 20.8 27.8; 2^17 15.7 19.0 20.0 20.5 and 15.7 18.8 20.7 27.7; of 512
+ * bytes, 2^22 and 2^24 pages, behind 2^14 30 29 and 5.3 7.3; 2^16 6.5 6.0 and 3.6 6.1; 2^17 3.8 3.9 and 3.7 4.7; behind 2^18, 2^20, 2^21, 2^22 pages 2.67 3.07 3.34 and 2.70
+ * 3.23 3.58; 2^20 requests of 2^21, 2^22, 2^24 10.4 11.7 12.8 and 9.7 11.5 13.5.
  */
 #define BAM_DEALT_SLICE (1ull << 22)
+#define BAM_DEALT_PAGES (1ull << 26)          /* at most: 512 MiB of counts and beginnings to a stream, as much as the pages' descriptors take */
 bool dealt_reads_pay(bam_array_t* a, uint64_t n_reqs, hipStream_t st)
 {
     if (!two_launches_ok(a)) return false;
     const range_d_t<uint64_t>& range = a->a->h_ranges[0];
     const uint64_t pages = range.page_count, cache_pages = range.cache.n_pages;
-    if (pages <= cache_pages || pages >= 1ull << 32) return false;
+    if (pages <= cache_pages) return false;
     if (n_reqs <= BAM_REQS_AT_A_TIME && n_reqs < pages + 2 * cache_pages) return false;
     const double asked = (double)pages * -std::expm1(-(double)n_reqs / (double)pages);
     if (asked < (n_reqs <= BAM_REQS_AT_A_TIME ? 1.0 : 0.9) * (double)cache_pages) return false;
     if (n_reqs > BAM_DEALT_SLICE && pages <= 2 * cache_pages) return false;
+    const uint64_t per_request = std::max<uint64_t>(4, (range.cache.page_size < 4096 ? 1ull << 20 : 1ull << 21) / cache_pages);
+    if (pages > BAM_DEALT_PAGES || pages / per_request >= std::min<uint64_t>(n_reqs, BAM_DEALT_SLICE)) return false;
     if (page_by_page(range, n_reqs) && (n_reqs > BAM_DEALT_SLICE || (pages <= 2 * cache_pages && cache_pages >= 1ull << 18))) return false;
     return !is_captured(st);
 }

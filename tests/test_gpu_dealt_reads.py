@@ -146,3 +146,29 @@ def test_many_streams_and_arrays_of_one_cache(bam):
         for a in arrays: a.close()
         for rg in rgs: rg.close()
         pc.close()
+
+
+# many pages for each request: the most with 2^14 and 2^18 slots and one more, and a range with more pages than counts are kept for
+@pytest.mark.parametrize("page,pages,cache_pages,n,dealt", [(512, 1 << 22, 1 << 18, (1 << 20) + 1, True), (512, (1 << 22) + 4, 1 << 18, 1 << 20, False), (512, 1 << 24, 1 << 18, (1 << 18) + 1, False),
+                                                            (4096, (1 << 25) - 8, 1 << 14, (1 << 18) + 1, True), (4096, (1 << 25) + 256, 1 << 14, (1 << 18) + 1, False),
+                                                            (512, (1 << 26) + 8, 1 << 12, (1 << 18) + 1, False)])
+def test_many_pages_to_a_request(bam, page, pages, cache_pages, n, dealt):
+    """scattered reads keep a count and a beginning for every page only while there are not too many pages for each request (and slot), and
+    no more of them than are worth it: seen by the memory that the first calls on a stream take"""
+    import torch
+    from bam_amd import gen
+    n_elems = pages * page // 8
+    want = oracle.lib().bo_gather_sum(SEED, SEED, 0, n, n_elems)
+    with Rig(bam, pages * page, n_queues=16, depth=256) as r:
+        a = r.array(n_elems, page, cache_pages)
+        idx = gen.gather_indices(SEED, n, n_elems)
+        out = torch.empty(n, dtype=torch.int64, device="cuda")
+        assert int(out.sum()) is not None                              # what torch itself needs is there
+        torch.cuda.synchronize()
+        free = torch.cuda.mem_get_info()[0]
+        got = a.read(n, idx)
+        taken = free - torch.cuda.mem_get_info()[0]
+        assert got == want
+        assert int(a.gather(n, idx).sum()) % (1 << 64) == want
+        assert a.stats()["access_cnt"] == 2 * n and not r.c.aborted()
+        assert taken >= 8 * pages if dealt else taken < 8 * pages // 2, (taken, pages)
