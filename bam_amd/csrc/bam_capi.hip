@@ -2288,7 +2288,6 @@ int bam_array_read_shaped(bam_array_t* a, uint64_t n_reqs, const uint64_t* d_ass
     hipStream_t st = (hipStream_t)stream;
     /* a graph keeps the addresses it was recorded with and may be replayed beside other calls: it gets the shape that keeps no
      * notes between launches (the same sum), as does a call for whose notes there is no memory */
-    if (shape == BAM_READ_TWO_LAUNCHES && dealt_reads_pay(a, n_reqs, st) && dealt_reads<false>(a, n_reqs, d_assignment, (unsigned long long*)d_sum, nullptr, st)) return 0;
     if (shape == BAM_READ_TWO_LAUNCHES && !is_captured(st) && scattered_reads<false>(a, n_reqs, d_assignment, reads_per_lane, (unsigned long long*)d_sum, nullptr, st)) return 0;
     array_d_t<uint64_t>* d = a->a->d_array_ptr;
     unsigned long long* part = (unsigned long long*)a->partials.get();

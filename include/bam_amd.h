@@ -124,8 +124,9 @@ int bam_array_read(bam_array_t* a, uint64_t n_reqs, const uint64_t* d_assignment
  *                             call runs as BAM_READ_FOUR_PER_THREAD.  A request whose page these launches
  *                             fetched counts as a miss, any other by what it finds when it is read.
  * bam_array_read picks, for arrays of one range, one launch of a read per thread up to 2^20 requests of an array that fits its cache and
- * BAM_READ_TWO_LAUNCHES with eight reads per lane beyond; for one that does not fit, what BAM_READ_TWO_LAUNCHES does, with the requests
- * put in order of their pages where they share them, or from 2^16 on, and below that few requests to a wave.  Other arrays:
+ * BAM_READ_TWO_LAUNCHES with eight reads per lane beyond.  For one that does not fit: requests that share pages are put in order of them
+ * behind the first launch, each page fetched once and its requests read, in batches of pages, a shape that has no name here (a request counts
+ * as above); others go as BAM_READ_TWO_LAUNCHES from 2^16 on, and below that 4 to 64 requests to a wave in one launch.  Other arrays:
  * BAM_READ_FOUR_PER_THREAD from 2^16 on and BAM_READ_ONE_PER_THREAD below. */
 #define BAM_READ_ONE_PER_THREAD  1
 #define BAM_READ_FOUR_PER_THREAD 2

@@ -172,3 +172,28 @@ def test_many_pages_to_a_request(bam, page, pages, cache_pages, n, dealt):
         assert int(a.gather(n, idx).sum()) % (1 << 64) == want
         assert a.stats()["access_cnt"] == 2 * n and not r.c.aborted()
         assert taken >= 8 * pages if dealt else taken < 8 * pages // 2, (taken, pages)
+
+
+@pytest.mark.parametrize("lanes", [1, 2, 4, 8])
+def test_a_shape_that_is_named_is_the_one_that_runs(bam, lanes):
+    """two launches keep a bit for each request between them, requests in order of their pages 16 bytes, and those only bam_array_read may have: seen by the memory taken"""
+    import torch
+    from bam_amd import gen
+    pages, cache_pages, n = 8192, 2048, (1 << 20) + 37
+    want = oracle.lib().bo_gather_sum(SEED, SEED, 0, n, pages * 512)
+    with Rig(bam, pages * 4096, n_queues=16, depth=256) as r:
+        a = r.array(pages * 512, 4096, cache_pages)
+        idx = gen.gather_indices(SEED, n, pages * 512)
+        for few in (64, 1 << 16):                                                  # what torch and the kernels' own frames take is there, and the words of the stream
+            a.read_shaped(few, idx, a.TWO_LAUNCHES, lanes)
+        a.stats()
+        torch.cuda.synchronize()
+        free = torch.cuda.mem_get_info()[0]
+        for rep in range(2):
+            assert a.read_shaped(n, idx, a.TWO_LAUNCHES, lanes, block_size=64) == want
+            st = a.stats()
+            assert st["access_cnt"] == n and st["hit_cnt"] + st["miss_cnt"] == st["access_cnt"], st
+        assert free - torch.cuda.mem_get_info()[0] < 4 * n
+        assert a.read(n, idx) == want
+        assert free - torch.cuda.mem_get_info()[0] >= 16 * n
+        assert not r.c.aborted()
