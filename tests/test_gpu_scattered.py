@@ -1,4 +1,6 @@
-"""Scattered reads in several launches (bam_array_gather, bam_array_read): what is resident first, then the rest page by page."""
+"""Scattered reads in several launches (bam_array_gather, bam_array_read): what is resident first, then the rest, in order of its pages or in stretches of the range."""
+import math
+
 import numpy as np
 import pytest
 
@@ -9,9 +11,11 @@ pytestmark = pytest.mark.gpu
 
 
 IN_FLIGHT = 1 << 18        # requests that are on their way together in a launch that can miss
+SLICE = 1 << 22            # requests that are put in order of their pages together
 
 
 def _page_by_page(pages, cache_pages, n):
+    """whether a page that somebody waits for is fetched once, and all requests that wait for it count as misses, whichever launches do it (_in_order)"""
     if pages <= cache_pages or 2 * n < pages - 1 or cache_pages < 4096:
         return False
     if 2 * pages > 5 * cache_pages:
@@ -20,6 +24,17 @@ def _page_by_page(pages, cache_pages, n):
         beyond = (n >> 17) * (pages - 2 * cache_pages)
         return n >= 3 << 17 or beyond >= cache_pages if pages - cache_pages >= 24576 else beyond > cache_pages
     return n > IN_FLIGHT and pages - cache_pages >= (16384 if pages == 2 * cache_pages else 24576)
+
+
+def _in_order(pages, cache_pages, n, page=4096):
+    """whether the requests that the first launch leaves are put in order of their pages"""
+    if pages <= cache_pages or n <= IN_FLIGHT and n < pages + 2 * cache_pages:
+        return False
+    if -math.expm1(-n / pages) * pages < (1.0 if n <= IN_FLIGHT else 0.9) * cache_pages or n > SLICE and pages <= 2 * cache_pages:
+        return False
+    if pages > 1 << 26 or pages // max(4, (1 << (20 if page < 4096 else 21)) // cache_pages) >= min(n, SLICE):
+        return False
+    return not (_page_by_page(pages, cache_pages, n) and (n > SLICE or pages <= 2 * cache_pages and cache_pages >= 1 << 18))
 
 
 # pages of data and of cache: everything resident; just below and at the smallest cache that is fetched for page by page, one
@@ -34,7 +49,9 @@ def _page_by_page(pages, cache_pages, n):
 def test_scattered_reads_element_by_element(bam, pages, cache_pages, n):
     """Every element of a gather and the sum of the same requests, twice (the second call finds what the first left behind),
     with a few requests outside the array (they read as 0 and are not counted) and a skewed half; every request inside is
-    counted once and misses cover the reads from the store.  Page by page each page asked for is read once, cold or not."""
+    counted once and misses cover the reads from the store.  Page by page each page asked for is read once, cold or not.  (All sizes that are
+    fetched for page by page go in order of their pages here; in stretches: below.)"""
+    assert not _page_by_page(pages, cache_pages, n) or _in_order(pages, cache_pages, n)
     n_elems = pages * 512 - 37
     words = oracle.store(SEED, 0, n_elems)
     rng = np.random.default_rng(n)
@@ -61,6 +78,36 @@ def test_scattered_reads_element_by_element(bam, pages, cache_pages, n):
             a.stats()
             a.gather(n, d_idx)
             assert a.stats()["hit_cnt"] == inside.sum()
+        assert not r.c.aborted() and r.c.info()["error_completions"] == 0
+
+
+# two stretches, three (the last cut short), four (of 512 pages more than a quarter); the smallest cache; one request more than goes in order
+@pytest.mark.parametrize("pages,cache_pages,n", [(65536, 32768, SLICE + 13), (49157, 24576, SLICE + 64), (40000, 16384, SLICE + 1), (12289, 4096, SLICE + 77), (16384, 4096, 2 * SLICE + 5)])
+@pytest.mark.parametrize("page", [512, 4096])
+def test_stretches_element_by_element(bam, page, pages, cache_pages, n):
+    """more requests than are put in order together: the pages that somebody waits for are fetched a stretch of the range at a time, each once, and then
+    the requests for them are read; a skewed half, some outside the array, one page that most ask for"""
+    assert _page_by_page(pages, cache_pages, n) and not _in_order(pages, cache_pages, n, page)
+    n_elems = pages * page // 8 - 37
+    words = oracle.store(SEED, 0, n_elems)
+    rng = np.random.default_rng(n)
+    with Rig(bam, pages * page // 65536 * 65536 + 65536, n_queues=16, depth=256) as r:
+        a = r.array(n_elems, page, cache_pages)
+        idx = rng.integers(0, n_elems, n).astype(np.uint64)
+        idx[::2] = (rng.random(len(idx[::2])) ** 4 * n_elems).astype(np.uint64)
+        idx[n // 3:n // 3 + 9999] = 5 * (page // 8) + 3
+        idx[rng.integers(0, n, 5)] = np.array([n_elems, n_elems + 1, 1 << 40, (1 << 64) - 1, 1 << 63], dtype=np.uint64)
+        inside = idx < n_elems
+        want = np.where(inside, words[np.where(inside, idx, 0).astype(np.int64)], 0).astype(np.uint64)
+        d_idx = _dev(idx)
+        asked = len(np.unique(idx[inside] // (page // 8)))
+        for rep in range(2):
+            assert np.array_equal(_u64(a.gather(n, d_idx)), want), rep
+            st = a.stats()
+            assert st["read_io_cnt"] == asked if rep == 0 else st["read_io_cnt"] <= asked, (st, asked)
+            assert st["access_cnt"] == inside.sum() and st["hit_cnt"] + st["miss_cnt"] == st["access_cnt"], st
+            assert a.read(n, d_idx) == int(np.sum(want, dtype=np.uint64)), rep
+            assert a.stats()["access_cnt"] == inside.sum()
         assert not r.c.aborted() and r.c.info()["error_completions"] == 0
 
 
