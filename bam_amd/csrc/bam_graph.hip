@@ -1628,7 +1628,7 @@ template <typename A>
 void along_sweep(bam_array_t* edges, const graph_plan* pl, along_t g, const A& algo, hipStream_t st)
 {
     const uint64_t n_blk = (g.n_segs + BAM_TRIP_WAVES * g.trip_segs - 1) / (BAM_TRIP_WAVES * g.trip_segs);
-    const bool look = A::joins && pl->all_cached && n_blk >= 2 * 512;
+    const bool look = A::joins && pl->all_cached && n_blk >= 2 * 512 && edges->a->h_ranges[0].cache.fast_reads;
     if (look) {
         unsigned long long* const stretches = pl->count + BAM_PLAN_STRETCHES;
         hipLaunchKernelGGL(k_cc_look, dim3(1), dim3(256), 0, st, edges->a->d_array_ptr, g, stretches);
@@ -1704,11 +1704,12 @@ uint32_t bfs_along_levels(bam_array_t* edges, graph_plan* pl, uint32_t* d_labels
     }
 }
 
-/* the forest that cc_read_edges begins with: k_cc_begin, for the arrays whose pages are read along (elsewhere every vertex by itself) */
+/* the forest that cc_read_edges begins with: k_cc_begin, for the arrays whose pages are read along (elsewhere, and where entries are not read without a
+ * reference on their page, every vertex by itself) */
 void cc_begin(bam_array_t* edges, graph_plan* pl, unsigned long long* comp, hipStream_t st)
 {
     const uint64_t nv = pl->n_vertices;
-    if (!pl->along.n_segs) { hipLaunchKernelGGL(k_iota, dim3(blocks_for(nv, 256)), dim3(256), 0, st, comp, nv); return; }
+    if (!pl->along.n_segs || !edges->a->h_ranges[0].cache.fast_reads) { hipLaunchKernelGGL(k_iota, dim3(blocks_for(nv, 256)), dim3(256), 0, st, comp, nv); return; }
     const bool large = pl->all_cached && nv >= 1ull << 21;
     hipLaunchKernelGGL(k_cc_begin<false>, dim3(blocks_for(nv, 256)), dim3(256), 0, st, edges->a->d_array_ptr, pl->offsets, nv, comp, 1u);
     hipLaunchKernelGGL(k_cc_shorten, dim3(blocks_for(nv, 256)), dim3(256), 0, st, comp, nv);

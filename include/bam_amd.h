@@ -99,7 +99,7 @@ void bam_array_destroy(bam_array_t* a);
 /* array_t::print_reset_stats (include/page_cache.h:1731-1752) as numbers; out[4]: read_io_cnt, access_cnt, miss_cnt, hit_cnt.
  * An access is an element, or as many neighbouring elements as a bam_ptr has one window for; reads, writes and updates, reductions, scans
  * and vectoradd count the same whichever kernels they run.  BFS and components along the edge pages (bam_bfs_by_page) count a page
- * and sweep each. */
+ * and sweep each; what components look at of resident lists before the sweep that joins them does not count. */
 int bam_array_stats(bam_array_t* a, uint64_t* out, int reset);
 
 /* ---- array benchmark kernels (benchmarks/array/main.cu:43-65) ----

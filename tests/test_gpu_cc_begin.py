@@ -51,3 +51,14 @@ def test_labels_where_a_round_is_left_out(bam, n_v, shape):
     u, v = _pairs(shape, n_v, rng) if shape == "path" else (rng.integers(0, n_v, n_v), rng.integers(0, n_v, n_v))
     off, nb = _csr(n_v, u, v)
     _check(bam, off, nb, 4096, -(-len(nb) // 512), calls=1)
+
+
+@pytest.mark.parametrize("shape,n_v", [("wide", 30011), ("path", (1 << 20) + 3)])
+@pytest.mark.parametrize("page,share", [(512, 2), (4096, 1)])
+def test_without_reads_that_hold_no_reference(bam, shape, n_v, page, share, monkeypatch):
+    """BAM_FAST_READS=0: every vertex begins by itself, and nothing is looked at before the pages of the edges are held"""
+    monkeypatch.setenv("BAM_FAST_READS", "0")
+    rng = np.random.default_rng(page)
+    u, v = _pairs(shape, n_v, rng) if shape == "path" else (rng.integers(0, n_v, 4 * n_v), rng.integers(0, n_v, 4 * n_v))
+    off, nb = _csr(n_v, u, v)
+    _check(bam, off, nb, page, max(2, -(-len(nb) * 8 // page) // share), calls=2)
