@@ -2406,12 +2406,15 @@ bool updates_by_bins(bam_array_t* a, int api, uint64_t n_reqs, const uint64_t* d
     const uint64_t page_elems = r.cache.page_size / sizeof(uint64_t), pages = r.page_count;
     /*
      * From as many on as the bins gain from, scattered over any number of pages; and through pointers from fewer where many meet on a page, since the
-     * ones that do wait for each other's references: us element by element (memref, +=) and in bins, of 2^10 pages of 8 KiB, 48000 27 37 and 30,
-     * 65000 34 48 and 31, 125000 60 85 and 35; 2^11 of 4 KiB, 65000 26 43 and 31, 100000 36 61 and 33; 2^9, 32000 29 32 and 29, 65000 50 58 and 31; 2^13,
-     * 65000 22 29 and 32, 80000 25 42 and 32, 125000 35 63 and 35.  Sorted, 65000 of 2^10 pages 24 36 and 29, 100000 of 2^11 28 44 and 30; in order 209 190
-     * and 23, 115 122 and 23.  AtomicAdd gains as much there scattered (48 and 35), but loses as much in an order (20 and 31, 20 and 24).
+     * ones that do wait for each other's references, though not from as few as those that are sorted would take longer in bins for.  us element by element (memref,
+     * +=) and in bins, scattered; sorted: of 2^7 pages, 25000 36 40 and 22; 39 41 and 23; of 2^8, 30000 34 39 and 24; 27 31 and 24; 36000 40 45 and 25;
+     * 31 37 and 25; of 384, 36000 34 40 and 27; 24 30 and 26; 48000 43 51 and 28; 30 38 and 27; of 2^9, 33000 31 35 and 31; 18 23 and 29; 48000 39 47 and 33; 24 32 and
+     * 30; 65000 52 59 and 33; 33 43 and 30; of 2^10, 48000 29 40 and 32; 18 27 and 29; 65000 36 51 and 33; 25 36 and 30; 90000 46 67 and 35; 35 48 and 31; of 2^11,
+     * 65000 28 44 and 34; 19 31 and 30; 110000 40 68 and 36; 33 51 and 32; of 2^12, 74000 26 41 and 34; 19 32 and 31; 125000 36 68 and 37; 30 51 and 33.  In order, 48000 of
+     * 2^9 95 93 and 25.  AtomicAdd gains as much there scattered (48 and 35), but loses as much in an order (20 and 31, 20 and 24).
      */
-    const uint64_t enough = api == 0 ? 1ull << 18 : api == 1 ? 1ull << 17 : 9ull << 13, meet = api == 1 ? 3600000 : 1700000;
+    const uint64_t enough = api == 0 ? 1ull << 18 : api == 1 ? 1ull << 17 : 9ull << 13;
+    const uint64_t meet = pages <= 256 ? (api == 1 ? 3600000 : 1700000) : api == 1 ? 6000000 : 3400000;
     if (n_reqs < enough && (api == 0 || n_reqs < 1ull << 14 || n_reqs * n_reqs < meet * pages)) return false;
     uint32_t bin_log = 0;
     while ((pages + (1ull << bin_log) - 1) >> bin_log > BAM_BINS) bin_log++;

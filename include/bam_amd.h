@@ -154,7 +154,8 @@ int bam_array_write(bam_array_t* a, uint64_t n_reqs, const uint64_t* d_assignmen
  * an atomic add on the address bam_ptr::memref returns (:467), api 2: ptr[i] += v on a non-const bam_ptr (:478; a plain read
  * and write, so the indices of one launch must be distinct).  The pages touched are dirty afterwards and reach the store
  * on eviction or bam_page_cache_flush.  An index that no range holds changes nothing, and d_old is 0 there.
- * From 2^18 requests on for api 0, 2^17 for 1 and 2, of an array of one range that fits its cache, the requests are dealt out to bins of
+ * From 2^18 requests on for api 0, 2^17 for 1 and 73728 for 2 (for 1 and 2 also from 2^14 on where the square of their number is 6000000 and 3400000 for
+ * each page or more, up to 256 pages 3600000 and 1700000), of an array of one range that fits its cache, the requests are dealt out to bins of
  * pages and added there, whatever api says (atomically, so the same elements and old values; counters too): except in a call
  * that finds no memory for the bins, which then is got for the next one (large calls get it first), and under capture. */
 int bam_array_update(bam_array_t* a, int api, uint64_t n_reqs, const uint64_t* d_assignment, const uint64_t* d_values, uint64_t* d_old,

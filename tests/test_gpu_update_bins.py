@@ -87,3 +87,37 @@ def test_updates_of_few_pages(bam, api, pages, n, kind):
             a.update(api, _dev(idx), _dev(vals))
             np.add.at(model, idx.astype(np.int64), vals)
         assert np.array_equal(_u64(a.gather(n_elems, None)), model) and not r.c.aborted()
+
+
+# fewer than 2^17 and 73728 requests through pointers: both sides of where they meet often enough, up to 256 pages and beyond
+@pytest.mark.parametrize("api,pages,n,bins", [(1, 256, 30357, False), (1, 256, 30358, True), (1, 512, 55425, False), (1, 512, 55426, True), (1, 2048, 110850, False), (1, 2048, 110852, True),
+                                              (2, 256, 20861, False), (2, 256, 20862, True), (2, 257, 29560, False), (2, 512, 41722, False), (2, 512, 41723, True), (2, 1024, 59005, False), (2, 1024, 59006, True)])
+def test_where_few_updates_take_bins(bam, api, pages, n, bins):
+    """seen by the memory that a first call on each of 24 streams leaves for the next; below the line there is none"""
+    import torch
+    n_elems = pages * 512
+    with Rig(bam, pages * 4096, backing=True, n_queues=8, depth=256) as r:
+        model = r.backing(n_elems).copy()
+        a = r.array(n_elems, 4096, pages)
+        a.gather(pages, None, stride=512)
+        idx = np.random.default_rng(n).permutation(n_elems)[:n].astype(np.uint64)
+        d, v = _dev(idx), _dev(np.full(n, 3, dtype=np.uint64))
+        streams = [torch.cuda.Stream() for _ in range(24)]
+        old = torch.zeros(n, dtype=torch.int64, device="cuda")
+        p = ctypes.c_void_p
+
+        def calls(m):
+            for s in streams:
+                assert a.L.bam_array_update(a.h, api, m, p(d.data_ptr()), p(v.data_ptr()), p(old.data_ptr()), 64, p(s.cuda_stream)) == 0
+                s.synchronize()
+
+        calls(1000)                                           # what the kernels' own frames take is there
+        free = torch.cuda.mem_get_info()[0]
+        calls(n)
+        taken = free - torch.cuda.mem_get_info()[0]
+        assert taken >= 24 * 20 * n // 2 if bins else taken < 24 * 20 * n // 8, taken
+        calls(n)
+        want = model.copy()
+        want[idx.astype(np.int64)] += np.uint64(2 * 24 * 3)
+        want[idx[:1000].astype(np.int64)] += np.uint64(24 * 3)
+        assert np.array_equal(_u64(a.gather(n_elems, None)), want) and not r.c.aborted()
