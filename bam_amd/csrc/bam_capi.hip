@@ -259,9 +259,7 @@ __global__ __launch_bounds__(256) void k_fetch_wanted(array_d_t<uint64_t>* dr, u
             uint32_t at = have + incl - n;
             for (; f; f &= f - 1) mine[at++] = (uint32_t)(p - first) + (uint32_t)__builtin_ctzll(f) / 8u;
             have += bam::bcast(incl, BAM_WAVE_SIZE - 1);
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            wave_lds_fence();
         }
         while (have >= BAM_WAVE_SIZE || (!more && have)) {
             const uint32_t n = have < BAM_WAVE_SIZE ? have : BAM_WAVE_SIZE;
@@ -324,10 +322,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
         if (!total) continue;
         any = true;
         if (rest != bits) missed[w0 + lane] = rest;
-        /* written and read by the lanes of one wave, which runs its LDS operations in order */
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        wave_lds_fence();
         for (uint32_t b = 0; b < total; b += 4 * BAM_WAVE_SIZE) {
             size_t idx[4];
             bool want[4], got[4];
@@ -377,13 +372,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
  * a batch's size 11.7.
  */
 #define BAM_BEGIN_PAGES 1024u
-/* what lanes of a wave have written to LDS, for all of its lanes: a wave's LDS operations run in order */
-__device__ __forceinline__ void wave_lds_fence()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
 __global__ __launch_bounds__(256) void k_reads_begin(const dealt_reads_t g, const uint32_t* finished, uint32_t call)
 {
     __shared__ uint32_t wave_total[256 / BAM_WAVE_SIZE], base;
@@ -1013,12 +1001,6 @@ __device__ __forceinline__ void stream_fetch_role(array_d_t<uint64_t>* dr, const
 }
 
 /*
- * One page of a streaming wave, every element read once and added up: lane l reads elements l, l + 64, ... of the page
- * whose first element is `first`.  ELEM: through array_d_t::operator[] per element (the eight elements a lane reads of a
- * page side by side, array_d_t::seq_read_n); otherwise through bam_ptr per element.  DEFER: the page is read only if it is
- * resident; true (for the whole wave) if it was not, and then nothing of it is counted, neither in `v` nor in the views.
- */
-/*
  * Eight rows of 64 elements from element `first` on, which begins a row of a page: the pages they lie in (stream_group_pages) are looked at, read and
  * looked at again side by side, without references.  `seen`: the words of their descriptors, lane k the k-th's, as an earlier look found
  * them; those of the eight rows from `next` on when the call returns.  False, with nothing added, where a page is not resident or did not
@@ -1058,6 +1040,12 @@ __device__ __forceinline__ bool stream_by_groups(const bam::range_view<uint64_t>
     return view.page_size >= 512 && view.page_size < 4096 && view.index_start == 0 && view.pso == 0 && view.r->cache.fast_reads;
 }
 
+/*
+ * One page of a streaming wave, every element read once and added up: lane l reads elements l, l + 64, ... of the page
+ * whose first element is `first`.  ELEM: through array_d_t::operator[] per element (the eight elements a lane reads of a
+ * page side by side, array_d_t::seq_read_n); otherwise through bam_ptr per element.  DEFER: the page is read only if it is
+ * resident; true (for the whole wave) if it was not, and then nothing of it is counted, neither in `v` nor in the views.
+ */
 template <bool ELEM, bool DEFER, typename PTR>
 __device__ __forceinline__ bool stream_page(array_d_t<uint64_t>* dr, PTR& ptr, bam::range_view<uint64_t>& elem_view, const uint64_t first, const uint64_t epp,
                                             const uint32_t lane, uint64_t& v)

@@ -127,6 +127,14 @@ __device__ __forceinline__ uint64_t wave_sum(uint64_t v)
     return v;
 }
 
+/* what lanes of a wave have written to LDS, for all of its lanes: a wave's LDS operations run in order */
+__device__ __forceinline__ void wave_lds_fence()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 /*
  * Add the wave's values into the launch's checksum.  A single word would take one atomic per wave of the
  * whole grid, all serialised on one address (about 12 ns each: a million waves cost more than the reads they

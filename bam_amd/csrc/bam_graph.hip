@@ -849,13 +849,6 @@ struct along_t {
     uint32_t sure;
     const unsigned long long* gate[2];
 };
-/* written and read by the lanes of one wave, which runs its LDS operations in order */
-__device__ __forceinline__ void wave_lds_fence()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
 __device__ __forceinline__ void raise_flag(unsigned long long* flag, const bool mine)
 {
     const uint64_t m = bam::ballot(mine);
