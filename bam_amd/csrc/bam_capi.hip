@@ -2094,7 +2094,10 @@ void few_reads(bam_array_t* a, uint64_t n_reqs, const uint64_t* d_assignment, un
  *   Few missing pages gain as well: 2^22 of those 1.30 and 0.44 ms, 10^5 and 2^20 of 9000 behind 8500 0.31 and 0.10, 0.57 and 0.17; 2^24, several
  * slices, no more.
  *   Large launches go by stretches all the same where those have the whole array in two, and where there would be several
- * slices, each of which asks for all pages (2^19 pages behind 2^18, 2^22 requests 19.9 and 20.3 ms; 2^16 behind 2^15, 2^24 3.3 and 11.1).
+ * slices, each of which asks for all pages (2^16 behind 2^15, 2^24 3.3 and 11.1 ms).  The first from 2^18 slots on, in stretches and in order, ms, of 2^19, 2^20,
+ * 2^22 requests: 2^19 pages of 4 KiB behind 2^18 13.0 17.2 19.9 and 13.2 17.5 19.9, of 8 KiB 31.1 41.5 48.4 and 31.0 41.2 48.2, of 512 bytes 2.9 3.7 3.9 and 2.9 3.4
+ * 4.0; 2^20 of 4 KiB behind 2^19 (2^20, 2^22) 25.6 38.5 and 26.4 40.0, of 512 bytes 5.3 7.2 and 5.1 7.6; 3 x 2^17 behind 2^18 7.9 10.2 10.5 and 7.7 10.0 10.1, of 512 bytes
+ * 2.2 2.9 2.8 and 2.0 2.5 2.0.
  *   Nor where an array has many pages for each request: a count and a beginning are looked at and kept for every page (8 bytes, and 0.1 ns of a
  * call in pages of 4 KiB, 0.3 in pages of 512 bytes), and a turn has few pages that anybody waits for.  What it gains there is that waves of 64 requests, as many as there are,
  * wait for each other's slots in a small cache: so fewer pages to a request the more slots there are.  Gathers, ms, two launches and
