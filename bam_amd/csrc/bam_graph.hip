@@ -755,31 +755,33 @@ __device__ __forceinline__ void graph_by_page(array_d_t<uint64_t>* da, const uin
         const bool want = ((marks >> lane) & 1) != 0;
         uint64_t va = 0, vb = 0;
         if (want) { va = first[p]; vb = first[p + 1]; }
-        uint32_t slot = BAM_NO_SLOT;
-        if (bam::ballot(want)) {
+        /* those that can be had without waiting are walked and given back before the others are waited for; a page whose wait was given up (the
+         * controller is marked aborted) is not walked */
+        for (bool left = want; bam::ballot(left);) {
+            uint32_t slot;
             /* the lanes without a page of their own come along and help move what the others load */
-            auto keep = [&](uint32_t s_) { slot = s_; return false; };
-            view.acquire_helped(p + pso_pages, want, false, keep, keep);
-        }
-        /* a page whose wait was given up (the controller is marked aborted) has no slot and is not walked */
-        for (uint64_t m = bam::ballot(want && slot != BAM_NO_SLOT); m; m &= m - 1) {
-            const uint32_t j = bam::first_lane(m);
-            const uint64_t va_j = bam::bcast(va, j), vb_j = bam::bcast(vb, j);
-            const uint64_t ps = (p0 + j) * epp, pe = ps + epp < n_edges ? ps + epp : n_edges;
-            const uint64_t* payload = (const uint64_t*)view.slot_addr(bam::bcast(slot, j));
-            for (uint64_t vbase = va_j; vbase <= vb_j; vbase += BAM_WAVE_SIZE) {
-                const uint64_t v = vbase + lane;
-                uint64_t es = 0, ee = 0;
-                if (v <= vb_j && active(v)) {
-                    es = offsets[v]; ee = offsets[v + 1];
-                    if (es < ps) es = ps;
-                    if (ee > pe) ee = pe;
+            const bool in = view.acquire_some(p + pso_pages, left, slot);
+            if (!bam::ballot(in)) break;
+            left = left && !in;
+            for (uint64_t m = bam::ballot(in); m; m &= m - 1) {
+                const uint32_t j = bam::first_lane(m);
+                const uint64_t va_j = bam::bcast(va, j), vb_j = bam::bcast(vb, j);
+                const uint64_t ps = (p0 + j) * epp, pe = ps + epp < n_edges ? ps + epp : n_edges;
+                const uint64_t* payload = (const uint64_t*)view.slot_addr(bam::bcast(slot, j));
+                for (uint64_t vbase = va_j; vbase <= vb_j; vbase += BAM_WAVE_SIZE) {
+                    const uint64_t v = vbase + lane;
+                    uint64_t es = 0, ee = 0;
+                    if (v <= vb_j && active(v)) {
+                        es = offsets[v]; ee = offsets[v + 1];
+                        if (es < ps) es = ps;
+                        if (ee > pe) ee = pe;
+                    }
+                    if (ee < es) ee = es;
+                    walk_packed(es, ee, v, [&](uint64_t i) { return bam::ld_payload(payload + (i - ps)); }, visit);
                 }
-                if (ee < es) ee = es;
-                walk_packed(es, ee, v, [&](uint64_t i) { return bam::ld_payload(payload + (i - ps)); }, visit);
             }
+            if (in) bam_release_refs(view.pages + p + pso_pages, 1, false);
         }
-        if (want) view.release(p + pso_pages, false);
     }
     view.flush_stats();
 }
@@ -1238,43 +1240,48 @@ __global__ __launch_bounds__(BAM_WAVE_SIZE) void k_along_missing(array_d_t<uint6
         if (c >= n) break;
         const bool want = lane < chunk && c + lane < n;
         const uint64_t p = g.missing[want ? c + lane : c];
-        uint32_t slot = BAM_NO_SLOT;
-        auto keep = [&](uint32_t s_) { slot = s_; return false; };
-        view.acquire_helped(p + pso_pages, want, false, keep, keep);
-        /* a page whose wait was given up (the controller is marked aborted) has no slot and is not visited */
-        if constexpr (PARTS) {
-            /* the pages of a segment follow one another in the list, but for those that are not in it */
-            const uint32_t per = 1u << g.part_log;
-            for (uint64_t m = bam::ballot(want && slot != BAM_NO_SLOT); m;) {
-                const uint32_t j = bam::first_lane(m);
-                const uint64_t seg = bam::bcast(p, j) >> g.part_log;
-                const uint64_t same = bam::ballot(want && slot != BAM_NO_SLOT && p >> g.part_log == seg);
-                m &= ~same;
-                /* lane q: the slot of the segment's q-th page */
-                uint64_t held = 0;
-                uint32_t at = 0;
-                for (uint32_t q = 0; q < per; q++) {
-                    const uint64_t of = bam::ballot((p & (per - 1u)) == q) & same;
-                    if (!of) continue;
-                    held |= 1ull << q;
-                    const uint32_t s_q = bam::bcast(slot, bam::first_lane(of));
-                    if (lane == q) at = s_q;
+        uint32_t last = BAM_NO_SLOT;
+        /* as graph_by_page has it: no page is held while another is waited for */
+        for (bool left = want; bam::ballot(left);) {
+            uint32_t slot;
+            const bool in = view.acquire_some(p + pso_pages, left, slot);
+            if (!bam::ballot(in)) break;                      /* the wait was given up (the controller is marked aborted): the rest is not visited */
+            left = left && !in;
+            if (in) last = slot;
+            if constexpr (PARTS) {
+                /* the pages of a segment follow one another in the list, but for those that are not in it */
+                const uint32_t per = 1u << g.part_log;
+                for (uint64_t m = bam::ballot(in); m;) {
+                    const uint32_t j = bam::first_lane(m);
+                    const uint64_t seg = bam::bcast(p, j) >> g.part_log;
+                    const uint64_t same = bam::ballot(in && p >> g.part_log == seg);
+                    m &= ~same;
+                    /* lane q: the slot of the segment's q-th page */
+                    uint64_t held = 0;
+                    uint32_t at = 0;
+                    for (uint32_t q = 0; q < per; q++) {
+                        const uint64_t of = bam::ballot((p & (per - 1u)) == q) & same;
+                        if (!of) continue;
+                        held |= 1ull << q;
+                        const uint32_t s_q = bam::bcast(slot, bam::first_lane(of));
+                        if (lane == q) at = s_q;
+                    }
+                    if (algo.prepare(g, s, seg, 1)) visit_parts(algo, g, s, view, seg, 0, held, 0, at, found, found_ahead);
                 }
-                if (algo.prepare(g, s, seg, 1)) visit_parts(algo, g, s, view, seg, 0, held, 0, at, found, found_ahead);
-            }
-        } else for (uint64_t m = bam::ballot(want && slot != BAM_NO_SLOT); m; m &= m - 1) {
-            const uint32_t j = bam::first_lane(m);
-            const uint64_t seg0 = bam::bcast(p, j) << g.seg_log;
-            const uint64_t* payload = (const uint64_t*)view.slot_addr(bam::bcast(slot, j)) + lane;
-            for (uint32_t k = 0; k < 1u << g.seg_log && seg0 + k < g.n_segs; k++) {
-                uint64_t id[BAM_SEG_ROWS];
+            } else for (uint64_t m = bam::ballot(in); m; m &= m - 1) {
+                const uint32_t j = bam::first_lane(m);
+                const uint64_t seg0 = bam::bcast(p, j) << g.seg_log;
+                const uint64_t* payload = (const uint64_t*)view.slot_addr(bam::bcast(slot, j)) + lane;
+                for (uint32_t k = 0; k < 1u << g.seg_log && seg0 + k < g.n_segs; k++) {
+                    uint64_t id[BAM_SEG_ROWS];
 #pragma unroll
-                for (uint32_t r = 0; r < BAM_SEG_ROWS; r++) id[r] = bam::ld_payload(payload + k * BAM_SEG_EDGES + r * BAM_WAVE_SIZE);
-                if (algo.prepare(g, s, seg0 + k, 1)) algo.visit(g, s, seg0 + k, 0, id, found, found_ahead);
+                    for (uint32_t r = 0; r < BAM_SEG_ROWS; r++) id[r] = bam::ld_payload(payload + k * BAM_SEG_EDGES + r * BAM_WAVE_SIZE);
+                    if (algo.prepare(g, s, seg0 + k, 1)) algo.visit(g, s, seg0 + k, 0, id, found, found_ahead);
+                }
             }
+            if (in) bam_release_refs(view.pages + p + pso_pages, 1, false);
         }
-        if (want) view.release(p + pso_pages, false);
-        if (A::again && again) { view.place = BAM_PLACE_AGAIN; view.again = slot; }       /* the slots of the next chunk, unless the hand stands at others */
+        if (A::again && again) { view.place = BAM_PLACE_AGAIN; view.again = last; }       /* the slots of the next chunk, unless the hand stands at others */
     }
     raise_flag(g.flags, found);
     raise_flag(g.flags + 1, found_ahead);

@@ -1053,7 +1053,7 @@ struct range_view {
         const uint32_t me = lane();
         data_page_t* const dp = pages + (take ? page : 0);
         uint64_t sv = 0;
-        slot = BAM_NO_SLOT;
+        slot = again;
         bool in = false, open = take;                     /* open: a reference on a page that is not there yet */
         if (take && bam_try_hit(dp, 1, false, sv, slot)) { in = true; open = false; account(true); }
         if (__builtin_expect(ballot(open) != 0, 0)) {
