@@ -134,9 +134,10 @@ int bam_array_read(bam_array_t* a, uint64_t n_reqs, const uint64_t* d_assignment
 int bam_array_read_shaped(bam_array_t* a, uint64_t n_reqs, const uint64_t* d_assignment, int shape, uint32_t reads_per_lane, uint32_t block_size,
                           uint64_t* d_sum, void* stream);
 /* the same requests with the values handed out: d_out[t] = element d_assignment[t] (or t * stride); what a kernel of the
- * reference's benchmark would hold in its register after array_d_t::operator[] (benchmarks/array/main.cu:57).  Launches of
- * more than 2^18 requests where the array is larger than its cache, and of 2^21 and more where it is larger than 512 MiB, run as
- * BAM_READ_TWO_LAUNCHES does (arrays of one range, streams that are not being captured) */
+ * reference's benchmark would hold in its register after array_d_t::operator[] (benchmarks/array/main.cu:57).  Of an array of one range larger than
+ * its cache, as bam_array_read: requests that share pages in order of them (from as many as there are pages and twice the slots on), others
+ * of more than 2^18 as BAM_READ_TWO_LAUNCHES does, and fewer 4 to 64 to a wave; of one that fits, 2^21 and more where it is larger than 512 MiB in two launches.
+ * Streams that are being captured, and all others: one launch */
 int bam_array_gather(bam_array_t* a, uint64_t n_reqs, const uint64_t* d_assignment, uint64_t stride, uint32_t block_size, uint64_t* d_out, void* stream);
 /* The read pattern of bam_array_read (one thread per request, element d_assignment[t] or t * span) through the other
  * access routes of array_d_t (include/page_cache.h:1240-1716, 414-485): api 1 get_raw/release_raw, 2 get_page_gid +
@@ -169,7 +170,7 @@ int bam_sqe_image(uint16_t cid, uint8_t opcode, uint32_t nsid, uint64_t prp1, ui
 
 /* ---- cache / pattern benchmark kernels (benchmarks/cache/main.cu:44-114, benchmarks/pattern/main.cu:105-170) ----
  * One wave per run of n_pages_per_wave whole pages starting at page d_assignment[w] (or w * n_pages_per_wave: then
- * modes 0 to 2 may share the same pages out to runs of another length),
+ * modes 0 to 2 may share the same pages out to runs of another length; who wants runs of n_pages_per_wave names them in d_assignment),
  * every element read once and summed into *d_sum.  mode 0: array_d_t::operator[] per element,
  * mode 1: bam_ptr per element (the reference's kernel, 64-wide), mode 2: one acquire per page and
  * streamed 8-byte loads; modes 3 and 4: modes 1 and 0 for data that is not
