@@ -1156,8 +1156,11 @@ __device__ __forceinline__ void cache_stream_body(array_d_t<uint64_t>* dr, uint6
                     }
                 }
                 const uint32_t nb = (uint32_t)(n_pages_per_wave - p0 < 16 ? n_pages_per_wave - p0 : 16);
-                const uint64_t page = view.page_of((start_page + p0 + (lane < nb ? lane : 0)) * epp);
-                for (uint32_t left = (1u << nb) - 1u; left;) {
+                /* pages in front of the range and behind it have no descriptors and are not read */
+                const uint64_t elem = (start_page + p0 + (lane < nb ? lane : 0)) * epp;
+                const bool there = elem >= view.index_start && view.page_of(elem) < r0->page_count;
+                const uint64_t page = there ? view.page_of(elem) : 0;
+                for (uint32_t left = (uint32_t)bam::ballot(there && lane < nb); left;) {
                     uint32_t slot;
                     const bool in = view.acquire_some<true>(page, lane < nb && ((left >> lane) & 1u), slot);
                     uint32_t m = (uint32_t)bam::ballot(in);

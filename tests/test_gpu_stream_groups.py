@@ -107,3 +107,33 @@ def test_page_wise_streams_that_share_a_cache(bam, page, pages, cache_pages):
         for a in arrays: a.close()
         for rg in rgs: rg.close()
         pc.close()
+
+
+@pytest.mark.parametrize("page,offset,first", [(512, 0, 0), (512, 0, 1000), (4096, 24, 0), (8192, 504, 70000)])
+def test_page_wise_runs_that_leave_the_range(bam, page, offset, first):
+    """pages in front of the range and behind its last one are not read and not counted; runs named and by turns, resident and not"""
+    from bam_amd import Array, PageCache, Range
+    pages, per, ppw = 300, page // 8, 21
+    n_elems = (pages * page - offset) // 8
+    words = oracle.store(SEED, 0, pages * per).reshape(pages, per)
+
+    def model(starts):
+        elem = (np.asarray(starts, dtype=np.int64)[:, None] + np.arange(ppw)).ravel() * per
+        at = ((elem - first) * 8 + offset) // page
+        at = at[(elem >= first) & (at < pages)]
+        return int(np.sum(words[at], dtype=np.uint64)), len(at)
+
+    with Rig(bam, (pages + 8) * page // 65536 * 65536 + 65536, n_queues=8, depth=256, stage_bytes=max(4096, page)) as r:
+        for cache_pages in (pages, 40):
+            pc = PageCache(page, cache_pages, 0, r.c)
+            rg = Range(first, first + n_elems, 0, pages, offset, page, pc, 0)
+            a = Array(first + n_elems, 0, [rg], 0)
+            at = first // per
+            named = np.array([0, at + 3, at + pages - 5, at + pages, at + pages + 1, 1 << 40, (1 << 58) // per], dtype=np.uint64)
+            for rep in range(2):
+                for starts, d in ((named, _dev(named)), (np.arange(40) * ppw, None)):
+                    want, n = model(starts)
+                    assert a.stream(len(starts), ppw, d, mode=2) == want, (cache_pages, rep)
+                    assert a.stats()["access_cnt"] == n
+            assert not r.c.aborted()
+            a.close(); rg.close(); pc.close()
